@@ -25,6 +25,11 @@ int check_tensor(const m3_tensor& t, const char* name, int dims, int64_t inner_e
 // After a launch: translate hipGetLastError into a status.
 int check_launch(const char* what);
 
+// Workspace bytes of a scan call and the call itself (scan.hip). `rows` false: without the 16-wave
+// kernel, whose q / k rows take most of a 16-bit call's workspace.
+size_t scan_need(const m3_scan_args& a, bool rows);
+int scan_run(const m3_scan_args& a, bool rows, hipStream_t stream);
+
 // The recurrent scan (rscan.hip) for the shapes the chunked MFMA kernel does not tile, and a
 // decode step run as a one-token recurrent scan for the shapes the step kernels do not take.
 bool rscan_fits(const m3_scan_args& a);

@@ -8,7 +8,7 @@
 // that device passes the kept address as the scan's workspace.
 //
 // The scan's workspace needs no clearing between calls: prep writes every region the scan reads
-// (the RMSNorm factors, the angle tiles, the scalar blocks), and a split call's segment buffers
+// (the RMSNorm factors or q / k rows, the angle tiles, the scalar blocks), and a split call's segment buffers
 // are written by its pass 1 and composition before pass 2 reads them. So nothing is zeroed here,
 // and no call allocates, frees or synchronises.
 #include <hip/hip_runtime.h>
@@ -57,19 +57,30 @@ extern "C" int m3_scan_fwd_noalloc(const m3_scan_args* args, hipStream_t stream)
   using namespace m3;
   clear_error();
   if (args == nullptr) return fail(M3_EINVAL, "m3_scan_fwd_noalloc: args is NULL");
-  size_t need = 0;
-  int rc = m3_scan_workspace_size(args, &need);
-  if (rc != M3_OK) return rc;
+  // the call as m3_scan_fwd would run it, or, where that outgrows the scratch, unsplit, then on
+  // the kernels that keep no q / k rows
+  m3_scan_args a = *args;
+  bool rows = true;
+  const size_t want = scan_need(a, rows);
+  size_t need = want;
+  if (need > M3_SCRATCH_BYTES && a.segments == 0) {
+    a.segments = 1;
+    need = scan_need(a, rows);
+  }
+  if (need > M3_SCRATCH_BYTES) {
+    rows = false;
+    need = scan_need(a, rows);
+  }
   if (need > M3_SCRATCH_BYTES) {
     return fail(M3_EWORKSPACE,
                 "m3_scan_fwd_noalloc: the call needs %zu bytes of scratch, above the %u-byte "
                 "maximum (use m3_scan_fwd with a workspace)",
-                need, static_cast<unsigned>(M3_SCRATCH_BYTES));
+                want, static_cast<unsigned>(M3_SCRATCH_BYTES));
   }
   void* ptr = nullptr;
-  if ((rc = scratch_address(&ptr)) != M3_OK) return rc;
-  m3_scan_args a = *args;
+  const int rc = scratch_address(&ptr);
+  if (rc != M3_OK) return rc;
   a.workspace = ptr;
   a.workspace_bytes = M3_SCRATCH_BYTES;
-  return m3_scan_fwd(&a, stream);
+  return scan_run(a, rows, stream);
 }

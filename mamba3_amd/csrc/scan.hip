@@ -4,7 +4,8 @@
 //   prep_kernel  head-independent per-token work, once per token instead of once per head:
 //                the RMSNorm factors of the raw B / C rows (model.py:190-191) and
 //                pi * tanh(angle) of the phase increments (model.py:225-228), into a workspace.
-//   scan_kernel  one persistent workgroup (8 waves) per (batch, head) walks the sequence in
+//   scan16_kernel (scan16_kernel.hpp) the 16-bit calls whose rows can be read as vectors;
+//   scan_kernel  the others. One persistent workgroup per (batch, head) walks the sequence in
 //                sub-chunks of ROWS flattened (token, rank) rows. The FP32 state lives in MFMA
 //                accumulator registers for the whole sequence (stored transposed, S^T [N, P],
 //                as 16x16 tiles spread over the waves), so the per-chunk state update that the
@@ -34,374 +35,11 @@
 // Replaces ops._fused_chunk_scan (ops.py:253-367) / its driver (ops.py:370-505) and the Triton
 // kernels _chunk_main_kernel (_triton.py:74-291) and _chunk_state_kernel (_triton.py:294-413);
 // the same kernel serves the portable entry ops.mamba3_scan (ops.py:544-822).
-#include "m3_common.hpp"
-#include "m3_host.hpp"
-#include "m3_math.h"
+#include "scan_common.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 namespace m3 {
-
-constexpr int kThreads = 512;
-constexpr int kWaves = 8;
-constexpr int kTiles = 4;  // 16x16 state tiles per wave (N_pad * P_pad <= 128 * 64)
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// MFMA policy per activation type: 16-bit types use 16x16x32 (K = 32, 8 elements per lane),
-// FP32 uses 16x16x4 (K = 4, one element per lane). ROWS is the sub-chunk height.
-template <typename T> struct Mma;
-template <> struct Mma<__bf16> {
-  static constexpr int ROWS = 64, PAD = 8;
-  typedef bf16x8 v8;
-  typedef bf16x4 v4;
-  typedef bf16x2 v2;
-  static __device__ __forceinline__ f4 mma(v8 a, v8 b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mma<_Float16> {
-  static constexpr int ROWS = 64, PAD = 8;
-  typedef f16x8 v8;
-  typedef f16x4 v4;
-  typedef f16x2 v2;
-  static __device__ __forceinline__ f4 mma(v8 a, v8 b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mma<float> {
-  static constexpr int ROWS = 32, PAD = 4;
-  typedef float v8;  // unused: FP32 operands are single elements
-  typedef f4 v4;
-  typedef f32x2 v2;
-  static __device__ __forceinline__ f4 mma(float a, float b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-
-// Compile-time LDS layout. Operand tiles are padded to N = 128 and P = 64 (the largest shapes
-// the kernel takes; every Mamba3 configuration has P <= 64), so every offset and loop bound is a
-// constant; smaller shapes run on zero padding.
-constexpr int kNPad = 128, kPPad = 64, kSMax = 32, kRMax = 8;
-constexpr int kNT = kNPad / 16, kPT = kPPad / 16;  // 16-row tiles of N and P
-
-template <typename T> struct Layout {
-  static constexpr int ROWS = Mma<T>::ROWS, PAD = Mma<T>::PAD, ES = sizeof(T);
-  static constexpr int LQ = kNPad + PAD;   // row stride (elements) of Qs, Ks, Sb
-  static constexpr int LR = ROWS + PAD;    // row stride (elements) of KT, VT
-  static constexpr int LP = kPPad + PAD;   // row stride (elements) of VR, ZR
-  static constexpr int al(int x) { return (x + 15) / 16 * 16; }
-  static constexpr int QS = 0;
-  static constexpr int KS = al(QS + ROWS * LQ * ES);
-  static constexpr int KT = al(KS + ROWS * LQ * ES);
-  static constexpr int VT = al(KT + kNPad * LR * ES);
-  static constexpr int VR = al(VT + kPPad * LR * ES);
-  static constexpr int ZR = al(VR + ROWS * LP * ES);
-  static constexpr int SB = al(ZR + ROWS * LP * ES);
-  static constexpr int FB = al(SB + kPPad * LQ * ES);
-  // float scratch, offsets in floats from FB, sized for TM = ROWS tokens (rank 1): two side
-  // blocks alternating (a sub-chunk's scalar block, ScBlk, then the (q, k) RMSNorm factors of
-  // its rows), the angle tile, two cos / sin tables ([token][angle][cos, sin], token stride CST
-  // for 16-byte aligned rows)
-  static constexpr int TM = ROWS;
-  static constexpr int SCB = 5 * TM + 8 + 2 * ROWS, SC0 = 0;
-  static constexpr int ANG = SC0 + 2 * SCB;  // [TM / 4][kSMax][4]
-  static constexpr int CST = 2 * kSMax + 4, CSB = TM * CST;
-  static constexpr int CS0 = ANG + TM * kSMax, PBASE = CS0 + 2 * CSB;
-  static constexpr int POFF = PBASE + kSMax, MX = POFF + kSMax, MZ = MX + kRMax * kPPad;
-  static constexpr int MO = MZ + kRMax * kPPad;
-  static constexpr int BYTES = FB + 4 * (MO + kRMax * kPPad);
-};
-
-// Per-token scalar block of one sub-chunk of TOK tokens (floats, token-indexed arrays): dt, the
-// within-chunk cumsum of adt, the exp-trapezoid scale, gamma, scale * decay to the end of the
-// token's 16-row tile; then the cumsum at each tile end, exp of the last cumsum and the last
-// cumsum itself. The prep pass writes them; the scan copies them to LDS (and takes exp(cum) and
-// scale * exp(cum_last - cum) from them itself, an exp per lane).
-template <int TOK> struct ScBlk {
-  static constexpr int DTV = 0, CUM = TOK, SCL = 2 * TOK, GAM = 3 * TOK, BSC = 4 * TOK;
-  static constexpr int CEND = 5 * TOK, ECL = 5 * TOK + 4, CL = 5 * TOK + 5;
-  static constexpr int SIZE = 5 * TOK + 8;
-};
-
-// Per-launch values shared by host and device.
-struct ScanGeom {
-  int xcd_map;           // 1: map blocks so each XCD holds consecutive (b, h)
-  int vec_qk, vec_vz;    // 1: q/k rows and v/z rows may be loaded with 16 / 8-byte vectors
-  int vec_nw;            // 1: both norm weights unit-stride and 8-byte aligned (4-element loads)
-  int norm_factors;      // 1: prep stores the RMSNorm factors (every scan kernel but the 16-wave
-                         // one, which reads the normalized rows instead)
-  // prep workspace, float offsets of its regions (-1: absent): RMSNorm factors [B][L][G*R][2]
-  // (q, k), pi tanh(angle) [B][L4][S][4] (4 consecutive tokens of one angle together, L4 =
-  // ceil(L / 4)), scalar blocks [B*H][nsub][scw] of `tok`-token sub-chunks
-  int64_t ws_norm, ws_ang, ws_sc;
-  int L4, tok, nsub, scw;
-  int ws_bytes;  // workspace bytes when below 2^31 (the projection form addresses it in 32 bits)
-  // the model's 16-bit shape at ranks 1 and 4 (scan16_kernel): the RMS-normalized q / k rows
-  // [B][L][R][2][N] in the activation dtype, after the regions above (byte offset, -1: absent)
-  // and their bytes when below 2^31 (read through a buffer resource of their own)
-  int64_t ws_qk;
-  int qk_bytes;
-  // projection form (the full-shape kernel): q, k, value, gate, dt, a, trap are slices of one
-  // projection row; byte offsets of each slice from `proj`, the batch / token strides and the
-  // group / rank / head strides of the slices, in bytes
-  const char* proj;
-  int64_t proj_b, out_b;
-  int tok_b, o_q, o_k, o_v, o_z, o_dt, o_a, o_tr, qk_g, qk_r, vz_h, sc_h, out_t, out_h;
-  // the output's physical start and the offset of logical token 0 from it (non-zero when the
-  // call runs backwards: token strides < 0, logical token t at physical token L - 1 - t)
-  const char* out_base;
-  int out_o0;
-};
-
-__device__ __forceinline__ f4 zero4() {
-  f4 z;
-  z[0] = z[1] = z[2] = z[3] = 0.f;
-  return z;
-}
-
-template <typename T>
-__device__ __forceinline__ T* lds_t(char* base, int off) {
-  return reinterpret_cast<T*>(base + off);
-}
-
-// ------------------------------------------------------------------ raw register tiles
-
-// Activation elements held as raw bits until they are used: W8 words hold 8 elements,
-// W4 words hold 4 (two 16-bit elements per word, or one FP32 element per word).
-template <typename T> struct Words {
-  static constexpr int W8 = sizeof(T) == 4 ? 8 : 4;
-  static constexpr int W4 = sizeof(T) == 4 ? 4 : 2;
-};
-
-__device__ __forceinline__ float bits_to_f(uint32_t bits16, __bf16*) {
-  return __uint_as_float(bits16 << 16);
-}
-__device__ __forceinline__ float bits_to_f(uint32_t bits16, _Float16*) {
-  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(bits16)));
-}
-
-template <typename T, int NW>
-__device__ __forceinline__ float raw_get(const uint32_t (&w)[NW], int i) {
-  if constexpr (sizeof(T) == 4) {
-    return __uint_as_float(w[i]);
-  } else {
-    const uint32_t x = w[i >> 1];
-    return bits_to_f((i & 1) ? (x >> 16) : (x & 0xffffu), static_cast<T*>(nullptr));
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ uint32_t elem_bits(const T* p) {
-  if constexpr (sizeof(T) == 4) {
-    return __float_as_uint(*p);
-  } else {
-    return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, *p));
-  }
-}
-
-// Load up to E elements (n valid, the rest zero) into raw words; one vector load when `vec`
-// and all E are valid (16 bytes, or 8 bytes for four 16-bit elements).
-template <typename T, int E, int NW>
-__device__ __forceinline__ void load_words(uint32_t (&w)[NW], const T* p, int n, bool vec) {
-  if (vec && n >= E) {
-    if constexpr (NW == 2) {
-      const uint2 q = *reinterpret_cast<const uint2*>(p);
-      w[0] = q.x; w[1] = q.y;
-    } else {
-#pragma unroll
-      for (int j = 0; j < NW; j += 4) {
-        const uint4 q = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint32_t*>(p) + j);
-        w[j] = q.x; w[j + 1] = q.y; w[j + 2] = q.z; w[j + 3] = q.w;
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < NW; ++j) w[j] = 0u;
-#pragma unroll
-  for (int i = 0; i < E; ++i) {
-    if (i < n) {
-      const uint32_t e = elem_bits(p + i);
-      if constexpr (sizeof(T) == 4) {
-        w[i] = e;
-      } else {
-        w[i >> 1] |= e << (16 * (i & 1));
-      }
-    }
-  }
-}
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef short i16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// Two values rounded to a 16-bit type (round to nearest even) and packed into one word, a
-// first: one packed convert for bf16.
-template <typename T>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  typedef T t2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, t2));
-}
-
-// Two adjacent activation values stored with one LDS write.
-template <typename T>
-__device__ __forceinline__ void st_pair(T* dst, float a, float b) {
-  if constexpr (sizeof(T) == 4) {
-    *reinterpret_cast<f32x2*>(dst) = (f32x2){a, b};
-  } else {
-    *reinterpret_cast<uint32_t*>(dst) = pack2<T>(a, b);
-  }
-}
-
-// Four adjacent activation values stored with one LDS write.
-template <typename T>
-__device__ __forceinline__ void st_quad(T* dst, f4 x) {
-  if constexpr (sizeof(T) == 4) {
-    *reinterpret_cast<f4*>(dst) = x;
-  } else {
-    *reinterpret_cast<u32x2*>(dst) = (u32x2){pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3])};
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void st_row8(T* dst, const float* x) {
-  if constexpr (sizeof(T) == 4) {
-    f4 a, b;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { a[i] = x[i]; b[i] = x[4 + i]; }
-    reinterpret_cast<f4*>(dst)[0] = a;
-    reinterpret_cast<f4*>(dst)[1] = b;
-  } else {
-    *reinterpret_cast<u32x4*>(dst) = (u32x4){pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]),
-                                             pack2<T>(x[4], x[5]), pack2<T>(x[6], x[7])};
-  }
-}
-
-// ------------------------------------------------------------------ scan
-
-// Wave-level scans with DPP row shifts (no LDS traffic). row_shr:n = 0x110 + n; lanes whose
-// source lies before their 16-lane row read 0.
-template <int CTRL>
-__device__ __forceinline__ float dpp_shr(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
-                                                               CTRL, 0xf, 0xf, true));
-}
-
-// Inclusive scan within aligned segments of SEG lanes (SEG a power of 2, <= 16). For SEG = 16
-// the segment is the DPP row, whose shifts already read 0 before the row's first lane (the
-// same +0 the masks add), so no mask is applied.
-template <int SEG>
-__device__ __forceinline__ float seg_incl_scan(float x, int lane) {
-  const int j = lane & (SEG - 1);
-  constexpr bool ROW = SEG == 16;
-  if constexpr (SEG > 1) { const float u = dpp_shr<0x111>(x); x += (ROW || j >= 1) ? u : 0.f; }
-  if constexpr (SEG > 2) { const float u = dpp_shr<0x112>(x); x += (ROW || j >= 2) ? u : 0.f; }
-  if constexpr (SEG > 4) { const float u = dpp_shr<0x114>(x); x += (ROW || j >= 4) ? u : 0.f; }
-  if constexpr (SEG > 8) { const float u = dpp_shr<0x118>(x); x += (ROW || j >= 8) ? u : 0.f; }
-  return x;
-}
-
-// Sum over each 16-lane row, in every lane of the row: DPP row rotations by 8, 4, 2 and 1.
-__device__ __forceinline__ float row16_sum(float x) {
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128,
-                                                             0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124,
-                                                             0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122,
-                                                             0xf, 0xf, false));
-  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121,
-                                                             0xf, 0xf, false));
-  return x;
-}
-
-__device__ __forceinline__ float readlane_f(float x, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l));
-}
-
-// Inclusive scan over the 64 lanes of a wave.
-__device__ __forceinline__ float wave_incl_scan(float x, int lane) {
-  x = seg_incl_scan<16>(x, lane);
-  const float r0 = readlane_f(x, 15), r1 = readlane_f(x, 31), r2 = readlane_f(x, 47);
-  const int row = lane >> 4;
-  x += row >= 1 ? r0 : 0.f;
-  x += row >= 2 ? r1 : 0.f;
-  x += row >= 3 ? r2 : 0.f;
-  return x;
-}
-
-// Transposed operand tiles ([n or p][row]) XOR-swizzle their 8-row groups by a key taken from
-// the tile row (n or p) so that the column-wise stores of the staging spread over the LDS banks;
-// every reader applies the same swizzle. Groups of 8 (16-bit: 16 bytes) stay contiguous.
-template <int ROWS>
-__device__ __forceinline__ int swz(int row, int key) {
-  return row ^ (8 * (key & (ROWS / 8 - 1)));
-}
-
-// Column col of row row of the Ks tile when swizzled: its 16-byte chunk c sits at c ^ 2 (row & 3)
-// (16-bit). The scores' reads of one chunk in 16 consecutive rows (rows 272 bytes apart) still
-// cover 16 bank groups, and the carry's transposing reads of 4 rows x 32 bytes no longer overlap.
-template <bool PLAIN>
-__device__ __forceinline__ int ks_col(int row, int col) {
-  if constexpr (PLAIN) {
-    return col;
-  } else {
-    return (((col >> 3) ^ (2 * (row & 3))) << 3) | (col & 7);
-  }
-}
-
-// Buffer resource over `bytes` bytes from `base` (raw, stride 0): loads at offsets beyond the
-// extent return zero, stores there are dropped.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0), bytes,
-                                           0x00020000);
-}
-
-// NW raw words (NW in {2, 4, 8}) from a buffer at byte offset `off`.
-template <int NW>
-__device__ __forceinline__ void bload_words(uint32_t (&w)[NW], __amdgpu_buffer_rsrc_t r, int off) {
-  if constexpr (NW == 2) {
-    const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
-    w[0] = v[0];
-    w[1] = v[1];
-  } else {
-#pragma unroll
-    for (int j = 0; j < NW; j += 4) {
-      const u32x4 v =
-          __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 4 * j, 0, 0));
-      w[j] = v[0];
-      w[j + 1] = v[1];
-      w[j + 2] = v[2];
-      w[j + 3] = v[3];
-    }
-  }
-}
-
-__device__ __forceinline__ float bload_f32(__amdgpu_buffer_rsrc_t r, int off) {
-  return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-}
-
-// Four consecutive activation values stored as one vector (8 bytes for 16-bit types).
-template <typename T>
-__device__ __forceinline__ void bstore_quad(f4 x, __amdgpu_buffer_rsrc_t r, int off) {
-  if constexpr (sizeof(T) == 4) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), r, off, 0, 0);
-  } else {
-    typename Mma<T>::v4 v;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = from_f<T>(x[i]);
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 0);
-  }
-}
 
 // Global reads of one (batch, head). Per sub-chunk: the q / k and value / gate words of each
 // lane's rows, and the side data the block stages through LDS: its scalar block followed by the
@@ -421,7 +59,6 @@ struct Feed {
   // FULL
   __amdgpu_buffer_rsrc_t rs_p, rs_w;
   int o_qk, o_vz, d_q1, d_k, d_z, tok_b;  // per-lane byte offsets at token 0, uniform deltas
-  int d_hi = 8;  // MIMO projection form: byte offset of a row's second 4-column chunk
   int side_o, side_s, ang_o, ang_s;        // per-lane workspace byte offsets at sub-chunk 0, strides
   // BUF: resources of q, k, value, gate and the given phases; per-lane byte offsets at token 0,
   // the byte strides of a token and the second row's delta
@@ -581,20 +218,7 @@ struct Feed {
 
   __device__ __forceinline__ void words_qk(int t0, int nw, bool qk_on, uint32_t (&rq)[2][W8],
                                            uint32_t (&rk)[2][W8]) const {
-    if constexpr (FULL && R > 1 && ES == 2) {
-      // MIMO: two 4-column chunks per row, d_hi apart (a rotation pair's partners, or adjacent)
-      const int tb = t0 * tok_b;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        uint32_t lo[2], hi[2];
-        bload_words<2>(lo, rs_p, o_qk + tb + j * d_q1);
-        bload_words<2>(hi, rs_p, o_qk + tb + j * d_q1 + d_hi);
-        rq[j][0] = lo[0]; rq[j][1] = lo[1]; rq[j][2] = hi[0]; rq[j][3] = hi[1];
-        bload_words<2>(lo, rs_p, o_qk + tb + j * d_q1 + d_k);
-        bload_words<2>(hi, rs_p, o_qk + tb + j * d_q1 + d_k + d_hi);
-        rk[j][0] = lo[0]; rk[j][1] = lo[1]; rk[j][2] = hi[0]; rk[j][3] = hi[1];
-      }
-    } else if constexpr (FULL) {
+    if constexpr (FULL) {
       // unconditional, also for lanes without a q/k or v/z role: every offset stays inside a
       // buffer or past its extent, where the load returns zero
       const int tb = t0 * tok_b;
@@ -705,99 +329,6 @@ struct Feed {
     }
   }
 };
-
-// Column of angle `col` in the cos / sin table row of token tt. SWZ (64-token sub-chunks, 32
-// angles): blocks of 4 angles are XOR-swizzled by the token's 16-token block, spreading the
-// phase stage's column writes over the LDS banks, and the two angle pairs of a block swap places
-// in every other token pair, so the 16-byte reads of two token rows 2 apart (136 floats: the
-// same banks shifted by 8) fall into different halves of each 8-float group. A reader takes a
-// block as two pairs, each at its own cs_col.
-template <bool SWZ>
-__device__ __forceinline__ int cs_col(int col, int tt) {
-  return SWZ ? col ^ (4 * ((tt >> 4) & 3)) ^ (2 * ((tt >> 1) & 1)) : col;
-}
-
-// Bounded phase (model.py:215-256) of tokens TPL pg .. TPL pg + TPL-1 of the sub-chunk at t0 for
-// angle ps: fmod-reduced increments summed within 64-token blocks, an fmod-reduced carry between
-// blocks, the running block sum and carry in pbase / poff; cos / sin into the table of angle ps.
-template <int PG, int TPL, int CST, bool SWZ, bool EXACT>
-__device__ __forceinline__ void phase_stage(float* tab, int ps, float* pbase, float* poff,
-                                            const float* dtv, int t0, int L, int pg, int lane,
-                                            bool angles, const float (&pa)[TPL], float* fph,
-                                            float* fblk, int64_t blk_stride) {
-  float ph[TPL];
-  if (angles) {
-    float x[TPL];
-    float mx = 0.f;  // largest |increment| of the lane (NaN and inf reduce like any x below)
-#pragma unroll
-    for (int i = 0; i < TPL; ++i) {
-      x[i] = __fmul_rn(pa[i], dtv[TPL * pg + i]);  // dt is 0 past the sub-chunk's last token
-      mx = fmaxf(mx, fabsf(x[i]));
-    }
-    // fmodf(x, 2 pi) is x itself for |x| < 2 pi (dt < 2, the usual case); the reductions are
-    // chosen per wave, so no lane branches on its own elements
-    float inc[TPL];
-    if (__builtin_amdgcn_ballot_w64(!(mx < M3_TWO_PI_F)) == 0) {
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) inc[i] = x[i];
-    } else if (__builtin_amdgcn_ballot_w64(!(mx < 1048576.0f)) == 0) {
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) inc[i] = m3_fmod_2pi_small(x[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) inc[i] = m3_fmod_2pi(x[i]);
-    }
-    float cpre[TPL];
-    float run = 0.f;
-#pragma unroll
-    for (int i = 0; i < TPL; ++i) {
-      run = __fadd_rn(run, inc[i]);
-      cpre[i] = run;
-    }
-    const float incl = seg_incl_scan<PG>(run, lane);
-    // the previous lane's inclusive sum: sums of earlier tokens only (incl - run would round in
-    // the later tokens of this lane's group)
-    float excl = dpp_shr<0x111>(incl);
-    if (pg == 0) excl = 0.f;
-    float base = *pbase, off = *poff;
-    if ((t0 & 63) == 0 && t0 > 0) {
-      // the block that just ended: its increment sum, when asked for (block_phase)
-      if (fblk != nullptr && pg == 0) fblk[((t0 >> 6) - 1) * blk_stride] = base;
-      off = m3_fmod_2pi_small(__fadd_rn(off, base));
-      base = 0.f;
-    }
-    // the final phase (token L - 1), when this sub-chunk holds it (wave-uniform test)
-    const bool last = fph != nullptr && t0 <= L - 1 && L - 1 - t0 < PG * TPL;
-#pragma unroll
-    for (int i = 0; i < TPL; ++i) {
-      // |base|, |excl + cpre| <= 64 * 2 pi and |off| < 2 pi: within the reduction's range.
-      // !EXACT (16-bit activations): sin / cos reduce the phase themselves (below 66 turns, the
-      // hardware's range), a difference far below the 16-bit rounding of the rotated values.
-      const float raw = __fadd_rn(__fadd_rn(base, __fadd_rn(excl, cpre[i])), off);
-      ph[i] = EXACT ? m3_fmod_2pi_small(raw) : raw;
-    }
-    if (last) {  // one wave-uniform branch instead of a lane test per token
-#pragma unroll
-      for (int i = 0; i < TPL; ++i) {
-        if (t0 + TPL * pg + i == L - 1) *fph = EXACT ? ph[i] : m3_fmod_2pi_small(ph[i]);
-      }
-    }
-    if (pg == PG - 1) {
-      *pbase = __fadd_rn(base, incl);
-      *poff = off;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TPL; ++i) ph[i] = pa[i];
-  }
-#pragma unroll
-  for (int i = 0; i < TPL; ++i) {
-    const int tt = TPL * pg + i;
-    float2 v;
-    __sincosf(ph[i], &v.y, &v.x);
-    *reinterpret_cast<float2*>(tab + tt * CST + 2 * cs_col<SWZ>(ps, tt)) = v;
-  }
-}
 
 // ------------------------------------------------------------------ prep
 
@@ -915,7 +446,7 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
 // Head-independent and per-(head, sub-chunk) work ahead of the scan, three block ranges:
 //  [0, nb_norm)  one 16-lane group per norm_rows() raw q / k rows (token, group, rank, q|k), 8
 //                elements per lane: each row's RMSNorm factor 1 / sqrt(mean(x^2) + eps)
-//                (model.py:190-191);
+//                (model.py:190-191), or for the 16-wave scan the finished row in slot order;
 //  [.., +nb_ang) one lane per kAngQuads (4-token group, angle) pairs, tokens padded to a multiple
 //                of 4: pi * tanh(angle) (model.py:225-228), 0 in the padding;
 // The first two give each workgroup several rows' loads in flight: with one round trip per
@@ -956,6 +487,15 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     const int l16 = tid & 15, row0 = blk * 16 * kNormRows + (tid >> 4);
     const int N = a.d_state;
     const bool in = 8 * l16 < N;  // lanes past column N load column 0 and count zeros
+    // rows_out (the 16-wave scan): lane l16 holds the slots 8 l16 .. 8 l16 + 7 (slot_col) instead
+    // of the columns, as two 4-column chunks at ca and cb (a pair's two columns with the MIMO
+    // rotation, interleaved below); a chunk past column N counts zeros
+    const bool rows_out = sizeof(T) == 2 && g.form16 >= 0;
+    const bool pairs = rows_out && g.perm && 8 * l16 < 2 * a.num_angles;
+    const bool in_b = 8 * l16 + 4 < N;
+    const int ca = !in ? 0 : pairs ? 4 * l16 : slot_col(8 * l16, g.perm, a.num_angles);
+    const int cb = !in_b ? 0 : pairs ? 4 * l16 + 2 * a.num_angles
+                                     : slot_col(8 * l16 + 4, g.perm, a.num_angles);
     // Rows (token, group, rank, q | k): a lane's rows row0 + 16 k all have row0's parity, so one
     // tensor (q or k). When 2 gr_n divides 16 they also share its (group, rank), the token
     // advancing by 8 / gr_n per k: the addresses follow from row0's by additions (a division
@@ -963,7 +503,8 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     // instructions). Rows past the end re-read the last batch row's last token.
     const int which = row0 & 1;
     const m3_tensor& xt = which ? a.k : a.q;
-    const T* xbase = static_cast<const T*>(xt.ptr) + (in ? 8 * l16 : 0);
+    // (rows_out: the chunks are added to the row's start below)
+    const T* xbase = static_cast<const T*>(xt.ptr) + (in && !rows_out ? 8 * l16 : 0);
     const int64_t xs0 = xt.stride[0], xs1 = xt.stride[1];
     const bool step_rows = 16 % (2 * gr_n) == 0;
     const int dtok = step_rows ? 8 / gr_n : 0;
@@ -992,26 +533,47 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
       const int b2 = tok / L, t2 = tok - b2 * L;
       const m3_tensor& x = wh ? a.k : a.q;
       return static_cast<const T*>(x.ptr) + b2 * x.stride[0] + t2 * x.stride[1] +
-             g2i * x.stride[2] + r2 * x.stride[3] + (in ? 8 * l16 : 0);
+             g2i * x.stride[2] + r2 * x.stride[3] + (in && !rows_out ? 8 * l16 : 0);
     };
     float ss[kNormRows];
     uint32_t w8[kNormRows][Words<T>::W8];
-    // the normalized rows' weights for this lane's 8 columns, raw, issued with the rows (after
-    // the factor stores below they would be a second round trip)
-    const bool rows_out = sizeof(T) == 2 && g.ws_qk >= 0 && g.vec_qk;
+    // the rows' weights for this lane's two chunks, raw, issued with the rows (after the factor
+    // stores below they would be a second round trip)
     const bool nw_vec = rows_out && g.vec_nw;
     Raw4 nw_r[2][2] = {};
     if (nw_vec) {
-      nw_r[0][0] = ldraw4(a.q_norm_w, 8 * l16);
-      nw_r[0][1] = ldraw4(a.q_norm_w, 8 * l16 + 4);
-      nw_r[1][0] = ldraw4(a.k_norm_w, 8 * l16);
-      nw_r[1][1] = ldraw4(a.k_norm_w, 8 * l16 + 4);
+      nw_r[0][0] = ldraw4(a.q_norm_w, ca);
+      nw_r[0][1] = ldraw4(a.q_norm_w, cb);
+      nw_r[1][0] = ldraw4(a.k_norm_w, ca);
+      nw_r[1][1] = ldraw4(a.k_norm_w, cb);
     }
-    if (g.vec_qk) {
+    if (rows_out && !(g.vec_qk && !g.perm)) {
+      if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int k = 0; k < kNormRows; ++k) {
+          const T* p = row_ptr(k);
+          const uint2 x = *reinterpret_cast<const uint2*>(p + ca);
+          const uint2 y = *reinterpret_cast<const uint2*>(p + cb);
+          w8[k][0] = in ? x.x : 0u;
+          w8[k][1] = in ? x.y : 0u;
+          w8[k][2] = in_b ? y.x : 0u;
+          w8[k][3] = in_b ? y.y : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kNormRows; ++k) {
+          ss[k] = 0.f;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float v = raw_get<T>(w8[k], i);
+            ss[k] = fmaf(v, v, ss[k]);
+          }
+        }
+      }
+    } else if (g.vec_qk) {
 #pragma unroll
       for (int k = 0; k < kNormRows; ++k) {
         // rows past the end re-read an earlier row; their sums are not stored
-        const T* p = row_ptr(k);
+        const T* p = row_ptr(k) + (rows_out && in ? 8 * l16 : 0);
 #pragma unroll
         for (int j = 0; j < Words<T>::W8; j += 4) {
           const uint4 q = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint32_t*>(p) + j);
@@ -1050,16 +612,18 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
       ss[k] = row16_sum(ss[k]);  // the row's 16 lanes
       const int row = row0 + 16 * k;
       fac[k] = 1.f / sqrtf(ss[k] / static_cast<float>(N) + a.norm_eps);
-      if (l16 == 0 && row < nrows && g.norm_factors) ws[g.ws_norm + static_cast<int64_t>(row)] = fac[k];
+      if (l16 == 0 && row < nrows && !rows_out) ws[g.ws_norm + static_cast<int64_t>(row)] = fac[k];
     }
     if constexpr (sizeof(T) == 2) {
       if (rows_out) {
-        // the model's shape at ranks 1 and 4 (N = 128, one group, vector rows): the normalized rows
-        // themselves, rnd(x * factor * rnd(w)) (model.py:48-55: F.rms_norm with the weight in the
-        // activation dtype, the result in it), rows (token, q | k) at N elements each
-        // the lane's tensor's weights (every row of the lane is q, or every row k), chosen by
+        // the rows themselves, 128 slots (zeros past the call's columns): rnd(x * factor * rnd(w))
+        // for the model's shape (model.py:48-55: F.rms_norm with the weight in the activation
+        // dtype, the result in it), the same product in FP32 for form kProj, the given values
+        // without norm weights (the hook form). Rows (token, group, rank, q | k).
+        // The lane's tensor's weights (every row of the lane is q, or every row k) are chosen by
         // bit masks on the raw words: a select between two weight arrays by `which` became a
         // dynamically indexed array in scratch memory
+        const bool norm = a.q_norm_w.ptr != nullptr;
         float wl[8];
         if (nw_vec) {
           const uint32_t msk = 0u - static_cast<uint32_t>(which);
@@ -1076,9 +640,13 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
         } else {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            const float wq = ldx(a.q_norm_w.ptr, a.q_norm_w.dtype, (8 * l16 + i) * a.q_norm_w.stride[0]);
-            const float wk = ldx(a.k_norm_w.ptr, a.k_norm_w.dtype, (8 * l16 + i) * a.k_norm_w.stride[0]);
-            wl[i] = rnd<T>(which ? wk : wq);
+            const int n = min((i < 4 ? ca : cb) + (i & 3), N - 1);
+            wl[i] = 1.f;
+            if (norm) {
+              const float wq = ldx(a.q_norm_w.ptr, a.q_norm_w.dtype, n * a.q_norm_w.stride[0]);
+              const float wk = ldx(a.k_norm_w.ptr, a.k_norm_w.dtype, n * a.k_norm_w.stride[0]);
+              wl[i] = rnd<T>(which ? wk : wq);
+            }
           }
         }
         char* qk = reinterpret_cast<char*>(ws) + g.ws_qk;
@@ -1086,10 +654,24 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
         for (int k = 0; k < kNormRows; ++k) {
           const int row = row0 + 16 * k;
           if (row >= nrows) continue;
-          float x[8];
+          float x[8], y[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) x[i] = raw_get<T>(w8[k], i) * fac[k] * wl[i];
-          st_row8<T>(reinterpret_cast<T*>(qk + (static_cast<int64_t>(row) * N + 8 * l16) * 2), x);
+          for (int i = 0; i < 8; ++i) {
+            const float v = raw_get<T>(w8[k], i);
+            x[i] = norm ? v * fac[k] * wl[i] : v;
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            // a pair's two columns side by side
+            y[2 * i] = pairs ? x[i] : x[2 * i];
+            y[2 * i + 1] = pairs ? x[4 + i] : x[2 * i + 1];
+          }
+          const int64_t o = static_cast<int64_t>(row) * kNPad + 8 * l16;
+          if (g.form16 == kProj) {
+            st_row8<float>(reinterpret_cast<float*>(qk) + o, y);
+          } else {
+            st_row8<T>(reinterpret_cast<T*>(qk) + o, y);
+          }
         }
       }
     }
@@ -1198,16 +780,11 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
   }
 }
 
-// SO (state only, with FULL): the segmented scan's first pass, which needs the end state, log
-// decay, last k and phase block sums but no outputs. The stores of Qs, VR, ZR, Sb and the output
-// are left out, and with them (dead code) the q math, the scores, the decay weights, the intra
-// and inter products and the epilogue; k, the carry tiles and products and the phase remain.
-//
-// SHAPE (without FULL): the model's shape (N = 128, P = 64, 32 angles when rotating, aligned
-// 16-byte rows) with the generic inputs (the hook form): the dimensions and the vector-load
+// FULL and SHAPE are FP32 forms (16-bit calls of those shapes take scan16_kernel). SHAPE: the
+// model's shape (N = 128, P = 64, 32 angles when rotating, aligned 16-byte rows) with the generic inputs (the hook form): the dimensions and the vector-load
 // choice are compile-time constants, the features stay runtime; every read and the output go
 // through buffer resources at per-lane offsets, issued unconditionally as in the FULL form.
-template <typename T, int R, bool FULL, bool SO = false, bool SHAPE = false>
+template <typename T, int R, bool FULL, bool SHAPE = false>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, const ScanGeom g,
                                                         const float* __restrict__ prep) {
   using M = Mma<T>;
@@ -1217,22 +794,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   constexpr int WPR = kWaves / RT;     // waves sharing one query row tile
   constexpr int TOK = ROWS / R;        // tokens per sub-chunk
   constexpr bool F32 = sizeof(T) == 4;
-  // the swizzled Ks layout (ks_col): rank 1 in 16 bits (config 2 442 against 445 us); at rank 4
-  // it measured within the 1% spread of these comparisons, and the plain rows are kept
-  constexpr bool KSW = !F32 && R == 1;
+  static_assert(F32 || !(FULL || SHAPE), "16-bit calls of the model's shapes take scan16_kernel");
   constexpr int ES = sizeof(T);
   constexpr int LQ = Lay::LQ, LR = Lay::LR, LP = Lay::LP, NP = kNPad, CST = Lay::CST;
   using SB_ = ScBlk<TOK>;
-  // SISO model shape: q / k lanes split by column half, waves 0-3 holding the rotated columns;
-  // the phase on waves 0-3 only, 8 tokens per lane (their compute interval is the shorter one)
-  constexpr bool SPLIT = (FULL || SHAPE) && R == 1 && !F32;
-  // MIMO model shape in projection form: q / k lanes split by rotation role as well. Waves 0-3
-  // hold the rotated pairs (n, n + 64), n < 32, four pairs per lane (the MIMO rotation pairs
-  // quarter 1 with quarter 3, model.py:201-213, ops.py:35-84), waves 4-7 eight consecutive
-  // columns of the unrotated quarters 2 and 4: no lane exchanges a partner, and only the rotated
-  // half does rotation arithmetic.
-  constexpr bool MSPLIT = FULL && R > 1 && !F32;
-  constexpr int TPL = SPLIT ? 8 : 4;   // tokens per phase lane
+  constexpr int TPL = 4;               // tokens per phase lane
   constexpr int PG = TOK / TPL;        // phase lanes per angle
   // swizzle keys of the FP32 transposed tiles, n >> KSH for KT and p >> VSH for VT
   constexpr int KSH = F32 ? 3 : 4, VSH = F32 ? 2 : 4;
@@ -1279,24 +845,13 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   const float Dh = ldx(a.D.ptr, a.D.dtype, h * a.D.stride[0]);
 
   // ---- lane roles
-  // q / k: row pair rp (rows 2rp, 2rp+1), columns n0 .. n0+7 (SPLIT: waves 0-3 columns 0-63,
-  // waves 4-7 columns 64-127)
-  const int rp = (SPLIT || MSPLIT) ? (tid & 255) >> 3 : tid >> 4;
-  const int n0 = SPLIT    ? 64 * (tid >> 8) + 8 * (tid & 7)
-                 : MSPLIT ? (tid < 256 ? 4 * (tid & 7)
-                                       : ((tid & 7) < 4 ? 32 + 8 * (tid & 7) : 64 + 8 * (tid & 7)))
-                          : 8 * (tid & 15);
-  // the lane's i-th column (MSPLIT rotated lanes: n0 .. n0+3, then their partners n0+64 ..)
-  auto col_of = [&](int i) {
-    return (MSPLIT && tid < 256) ? (i < 4 ? n0 + i : n0 + 60 + i) : n0 + i;
-  };
-  // (SPLIT / MSPLIT: every lane has both roles, 512 threads covering 64 rows x 128 columns and
-  // 64 rows x 64 columns)
-  const bool qk_on = SPLIT || MSPLIT || (rp < ROWS / 2 && n0 < N);
+  // q / k: row pair rp (rows 2rp, 2rp+1), columns n0 .. n0+7
+  const int rp = tid >> 4, n0 = 8 * (tid & 15);
+  const bool qk_on = rp < ROWS / 2 && n0 < N;
   // v / z: row pair vp (rows 2vp, 2vp+1; tokens 2vp, 2vp+1 for R = 1), columns p0 .. p0+3
   constexpr int P4 = kPPad / 4;
   const int vp = tid / P4, p0 = 4 * (tid % P4);
-  const bool vz_on = SPLIT || (2 * vp < TOK * R && p0 < P);
+  const bool vz_on = 2 * vp < TOK * R && p0 < P;
   // phase: angle ps, token group pg (tokens TPL pg .. TPL pg + TPL-1)
   const int pg = tid % PG, ps = tid / PG;
   const bool ph_on = rotate && ps < S;
@@ -1352,7 +907,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   float wq[8], wk[8], bq[NB][8], bk[NB][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int n = col_of(i);
+    const int n = n0 + i;
     const bool ok = qk_on && n < N;
     wq[i] = (ok && norm) ? rnd<T>(ldx(a.q_norm_w.ptr, a.q_norm_w.dtype, n * a.q_norm_w.stride[0]))
                          : 1.f;
@@ -1436,7 +991,6 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   // ---- per-token reads
   Feed<T, R, FULL, SHAPE> fd;
   fd.init(a, g, prep, b, h, grp, rp, n0, vp, p0, N, P, norm);
-  if constexpr (MSPLIT) fd.d_hi = (col_of(4) - n0) * ES;
   float* fph = a.final_phase.ptr != nullptr
                    ? static_cast<float*>(a.final_phase.ptr) + b * a.final_phase.stride[0] +
                          h * a.final_phase.stride[1] + ps * a.final_phase.stride[2]
@@ -1526,7 +1080,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   if (ph_on && nsub > 0) {
     float pa[TPL];
     angles_of(pa);
-    phase_stage<PG, TPL, CST, SPLIT, F32>(csb(0), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
+    phase_stage<PG, TPL, CST, false, F32>(csb(0), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
                                      scb(0) + SB_::DTV, 0, L, pg, lane, angles, pa, fph, fblk,
                                      blk_stride);
   }
@@ -1545,10 +1099,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       ang_store(ang);
     }
     // q / k rows -> Qs, Ks (row-major), FP32 KT (transposed, swizzled); rows 2rp, 2rp+1.
-    // SPLIT: one copy of the code per column half, rotated (waves 0-3) or not, so no values
-    // merge between the two.
-    auto stage_qk = [&](auto rot_tag) {
-      constexpr bool ROT = decltype(rot_tag)::value;
+    if (qk_on) {
       // (q, k) RMSNorm factors of rows 2rp, 2rp+1
       float fq[2] = {1.f, 1.f}, fk[2] = {1.f, 1.f};
       if (norm) {
@@ -1568,45 +1119,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           q[i] = fmaf(raw_get<T>(rq[j], i), fq[j] * wq[i], bq[R == 1 ? 0 : j][i]);
           k[i] = fmaf(raw_get<T>(rk[j], i), fk[j] * wk[i], bk[R == 1 ? 0 : j][i]);
         }
-        if constexpr (MSPLIT) {
-          // pairs (n0 + i, n0 + 64 + i), angles n0 + i, i < 4 (waves 0-3)
-          if (ROT) {
-            const float* tr = CSt + tt * CST;
-            const f4 c01 = *reinterpret_cast<const f4*>(tr + 2 * n0);
-            const f4 c23 = *reinterpret_cast<const f4*>(tr + 2 * n0 + 4);
-#pragma unroll
-            for (int pp = 0; pp < 4; ++pp) {
-              const f4& cv = pp < 2 ? c01 : c23;
-              const float cc = cv[2 * (pp & 1)], ss = cv[2 * (pp & 1) + 1];
-              const float q0 = q[pp], q1 = q[pp + 4];
-              const float k0 = k[pp], k1 = k[pp + 4];
-              q[pp] = fmaf(q0, cc, -(q1 * ss));
-              q[pp + 4] = fmaf(q0, ss, q1 * cc);
-              k[pp] = fmaf(k0, cc, -(k1 * ss));
-              k[pp + 4] = fmaf(k0, ss, k1 * cc);
-            }
-          }
-        } else if constexpr (SPLIT) {
-          // pairs (2j, 2j+1), j = n0/2 .. n0/2+3: the rotated columns are waves 0-3's (SHAPE:
-          // when the call rotates)
-          if (ROT && (FULL || rotate)) {
-            const float* tr = CSt + tt * CST;
-            const f4 c01 = *reinterpret_cast<const f4*>(tr + 2 * cs_col<true>(n0 >> 1, tt));
-            const f4 c23 = *reinterpret_cast<const f4*>(tr + 2 * cs_col<true>((n0 >> 1) + 2, tt));
-            // c01 = c0 s0 c1 s1, c23 = c2 s2 c3 s3
-#pragma unroll
-            for (int pp = 0; pp < 4; ++pp) {
-              const f4& cv = pp < 2 ? c01 : c23;
-              const float cc = cv[2 * (pp & 1)], ss = cv[2 * (pp & 1) + 1];
-              const float q0 = q[2 * pp], q1 = q[2 * pp + 1];
-              const float k0 = k[2 * pp], k1 = k[2 * pp + 1];
-              q[2 * pp] = fmaf(q0, cc, -(q1 * ss));
-              q[2 * pp + 1] = fmaf(q0, ss, q1 * cc);
-              k[2 * pp] = fmaf(k0, cc, -(k1 * ss));
-              k[2 * pp + 1] = fmaf(k0, ss, k1 * cc);
-            }
-          }
-        } else if (rotate) {
+        if (rotate) {
           // x' = x cos + sgn partner sin: SISO pairs (2j, 2j+1), MIMO pairs (n, n + N/2)
           float qp[8], kp[8];
 #pragma unroll
@@ -1638,22 +1151,8 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
             k[i] = fmaf(kp[i], ss, k[i] * cc);
           }
         }
-        if (MSPLIT && ROT) {
-          f4 lo, hi;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) { lo[i] = q[i]; hi[i] = q[i + 4]; }
-          if constexpr (!SO) {
-            st_quad<T>(Qs + row * LQ + n0, lo);
-            st_quad<T>(Qs + row * LQ + n0 + 64, hi);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) { lo[i] = k[i]; hi[i] = k[i + 4]; }
-          st_quad<T>(Ks + row * LQ + ks_col<!KSW>(row, n0), lo);
-          st_quad<T>(Ks + row * LQ + ks_col<!KSW>(row, n0 + 64), hi);
-        } else {
-          if constexpr (!SO) st_row8<T>(Qs + row * LQ + n0, q);
-          st_row8<T>(Ks + row * LQ + ks_col<!KSW>(row, n0), k);
-        }
+        st_row8<T>(Qs + row * LQ + n0, q);
+        st_row8<T>(Ks + row * LQ + n0, k);
 #pragma unroll
         for (int i = 0; i < 8; ++i) kt[j][i] = k[i];
       }
@@ -1666,21 +1165,12 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         const float e1 = SC[SB_::SCL + r1] * __expf(cl - SC[SB_::CUM + r1]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const int n = col_of(i);
+          const int n = n0 + i;
           if (FIX || n < N) {
             st_pair<T>(KT + n * LR + swz<ROWS>(2 * rp, n >> KSH), kt[0][i] * e0, kt[1][i] * e1);
           }
         }
       }
-    };
-    if constexpr (SPLIT || MSPLIT) {
-      if (w < 4) {
-        stage_qk(std::true_type{});
-      } else {
-        stage_qk(std::false_type{});
-      }
-    } else if (qk_on) {
-      stage_qk(std::false_type{});
     }
     // value / gate of tokens 2vp, 2vp+1, columns p0 .. p0+3: rank values v mx_r -> VR
     // (row-major; 16-bit also VS, scaled; FP32 VT, transposed and swizzled), rank gates z mz_r
@@ -1713,7 +1203,6 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
           for (int i = 0; i < 4; ++i) sv[i] = v[j][i] * (j ? ev1 : ev0);
           st_quad<T>(VS + (2 * vp + j) * LP + p0, sv);
-          if constexpr (SO) continue;
           *reinterpret_cast<u32x2*>(VR + (2 * vp + j) * LP + p0) = (u32x2){rv[j][0], rv[j][1]};
           *reinterpret_cast<u32x2*>(ZR + (2 * vp + j) * LP + p0) = (u32x2){rz[j][0], rz[j][1]};
         }
@@ -1725,7 +1214,6 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          if constexpr (SO) break;
           f4 vq, zq;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -1748,10 +1236,8 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
             vq[jr][i] = mul_r<T>(v[0][i], mxl[jr][i]);
             zq[i] = mul_r<T>(z[0][i], mzl[jr][i]);
           }
-          if constexpr (!SO) {
-            st_quad<T>(VR + row * LP + p0, vq[jr]);
-            st_quad<T>(ZR + row * LP + p0, zq);
-          }
+          st_quad<T>(VR + row * LP + p0, vq[jr]);
+          st_quad<T>(ZR + row * LP + p0, zq);
         }
         if constexpr (KTR) {
 #pragma unroll
@@ -1774,7 +1260,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
     for (int k = 0; k < kTiles; ++k) {
       const int u = w + kWaves * k;
-      if (!SO && (all_tiles || u < n_tiles)) {
+      if (all_tiles || u < n_tiles) {
         const int ni = u / kPT, pj = u - ni * kPT;
         st_quad<T>(Sb + (16 * pj + l16) * LQ + 16 * ni + 4 * lg, st[k]);
       }
@@ -1830,7 +1316,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     const int tq = trow / R;
     // 16-bit: the query rows of this tile, B operand of the scores and A operand of inter
     typename M::v8 qv[F32 ? 1 : NP / 32];
-    if constexpr (!F32 && !SO) {
+    if constexpr (!F32) {
 #pragma unroll
       for (int kk = 0; kk < NP / 32; ++kk) {
         qv[kk] = *reinterpret_cast<const typename M::v8*>(Qs + trow * LQ + 32 * kk + 8 * lg);
@@ -1841,12 +1327,12 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
     for (int sj = 0; sj < RT; ++sj) {
       acc[sj] = zero4();
-      if (SO || sj > it) continue;
+      if (sj > it) continue;
       if constexpr (!F32) {
 #pragma unroll
         for (int kk = 0; kk < NP / 32; ++kk) {
           const typename M::v8 av = *reinterpret_cast<const typename M::v8*>(
-              Ks + (16 * sj + l16) * LQ + ks_col<!KSW>(l16, 32 * kk + 8 * lg));
+              Ks + (16 * sj + l16) * LQ + 32 * kk + 8 * lg);
           acc[sj] = M::mma(av, qv[kk], acc[sj]);
         }
       } else {
@@ -1868,7 +1354,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         // A: 8 tokens of column nrow from the row-major Ks, two transposing reads of 4 tokens
         // (in each 16-lane group, lane 4a + b receives element b of the 8-byte vectors of lanes
         // a, a + 4, a + 8, a + 12: lane x addresses token x / 4, columns 4 (x % 4) ..)
-        const T* kc = Ks + (l16 >> 2) * LQ + ks_col<!KSW>(l16 >> 2, 16 * ni + 4 * (l16 & 3));
+        const T* kc = Ks + (l16 >> 2) * LQ + 16 * ni + 4 * (l16 & 3);
         const T* vc = VS + (l16 >> 2) * LP + 16 * pj + 4 * (l16 & 3);  // B: the same from VS
 #pragma unroll
         for (int kk = 0; kk < ROWS; kk += 32) {
@@ -1901,15 +1387,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     if (ph_on && c + 1 < nsub) {
       float pa[TPL];
       angles_of(pa);
-      phase_stage<PG, TPL, CST, SPLIT, F32>(csb(c + 1), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
+      phase_stage<PG, TPL, CST, false, F32>(csb(c + 1), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
                                        scb(c + 1) + SB_::DTV, t0 + TOK, L, pg, lane, angles, pa,
                                        fph, fblk, blk_stride);
     }
     if constexpr (FULL || SHAPE) loads_side();
-    if constexpr (SO) {
-      __syncthreads();
-      continue;
-    }
     // decayed scores W[t, s] = Sc[t, s] d[t, s] in FP32
     const float cum_t = SC[SB_::CUM + tq];
     const float gam_t = SC[SB_::GAM + tq];
@@ -2085,7 +1567,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       const int r = i / N, n = i - r * N;
       static_cast<T*>(a.final_k.ptr)[b * a.final_k.stride[0] + h * a.final_k.stride[1] +
                                      r * a.final_k.stride[2] + n] =
-          Ks[(tl * R + r) * LQ + ks_col<!KSW>(tl * R + r, n)];
+          Ks[(tl * R + r) * LQ + n];
     }
   }
 
@@ -2123,653 +1605,6 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   }
 }
 
-
-// ------------------------------------------------------------ 16-wave SISO scan
-
-// scan16_kernel<T, R, SO>: the model's shape in projection form (ranks 1 and 4, N = 128, P = 64,
-// 32 angles, one group, 16-bit activations; forwards or backwards) with 1024 threads, so that
-// four waves share each SIMD to hide one another's LDS, MFMA and transcendental latency. A
-// sub-chunk is 64 rows (token, rank), rank minor: 64 tokens at rank 1, 16 at rank 4, whose
-// decay weights, phases and scalars are per token and whose output sums the token's R rows
-// (times mimo_out). Per sub-chunk, three intervals between workgroup barriers:
-//   A  staging (every wave): row qt's q / k (bias and rotation on prep's normalized rows; waves
-//      0-7 the rotated columns, waves 8-15 the others) -> Qs, Ks; row vt's value / gate (times
-//      the rounded mimo_x / mimo_z at rank 4) -> VR, ZR and the carry's scaled values -> VS; the
-//      state, rounded -> Sb; the side block and angle tile of the next sub-chunk -> LDS;
-//   B  waves 0-9 one causal score tile each (Sc^T = K Q^T) and its decay weights W -> WS;
-//      every wave the carry products of its two state tiles; the next sub-chunk's global loads
-//      are issued here;
-//   C  wave w the output tile (row tile w / 4, P tile w % 4): intra V^T W^T from WS, inter
-//      rnd(S) Q^T, epilogue, store; waves 0-7, whose row tiles 0 and 1 have the shortest intra
-//      products, also the phases of the next sub-chunk (a long dependent chain per wave).
-// Same mathematics and rounding points as scan_kernel<T, R, true> (whose header lists them), but
-// for q / k, which start from prep's rows rounded after the RMSNorm (the reference's rounding
-// point, model.py:48-55).
-
-constexpr int k16Threads = 1024;
-
-// LDS layout, 16-bit elements unless noted. The strides and swizzles make every access pattern
-// of the kernel conflict-free under the measured gfx950 LDS behaviour: 16-byte reads of 16 rows
-// at one 16-byte chunk (the MFMA operands) with 288-byte rows or an XOR swizzle of 256-byte rows;
-// 8-byte accesses (stores, transposing reads) 32 lanes at a time over 64 banks of 4 bytes, so
-// the 32 lanes' 8-byte pieces must cover 256 distinct bytes.
-//   Qs, Ks  [64 tokens][144]: 288-byte rows
-//   Sb      [64 p][128]: 256-byte rows, 16-byte chunk c of row p at c ^ (p % 16) (sb_off)
-//   VR, ZR, VS [64 tokens][64]: 128-byte rows, 32-byte pair and chunk half swizzled (v_off)
-//   WS      [64 t][80]: 160-byte rows
-struct Lay16 {
-  static constexpr int ROWS = 64, LQ = kNPad + 16, LS = kNPad, LV = kPPad, LW = kPPad + 16, ES = 2;
-  static constexpr int QS = 0;
-  static constexpr int KS = QS + ROWS * LQ * ES;
-  static constexpr int VR = KS + ROWS * LQ * ES;
-  static constexpr int ZR = VR + ROWS * LV * ES;
-  static constexpr int VS = ZR + ROWS * LV * ES;
-  static constexpr int SB = VS + ROWS * LV * ES;
-  static constexpr int WS = SB + kPPad * LS * ES;  // decay weights [t][s'] (s' permuted, below)
-  static constexpr int FB = WS + ROWS * LW * ES;
-  // floats from FB: two side blocks (scalar blocks), the angle tile, two cos / sin tables, the
-  // phase block sum and carry per angle
-  static constexpr int SCB = 5 * ROWS + 8, SC0 = 0;
-  static constexpr int ANG = SC0 + 2 * SCB;
-  static constexpr int CST = 2 * kSMax + 4, CSB = ROWS * CST;
-  static constexpr int CS0 = ANG + ROWS * kSMax, PBASE = CS0 + 2 * CSB, POFF = PBASE + kSMax;
-  // rank 4: the rounded mimo_x, mimo_z and mimo_out [R][P]
-  static constexpr int MX = POFF + kSMax, MZ = MX + 4 * kPPad, MO = MZ + 4 * kPPad;
-  static constexpr int BYTES = FB + 4 * (MO + 4 * kPPad);
-};
-static_assert(Lay16::BYTES <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
-static_assert(Lay16::FB % 16 == 0 && Lay16::WS % 16 == 0 && Lay16::SB % 16 == 0 &&
-              (Lay16::ANG * 4) % 16 == 0 && (Lay16::CS0 * 4) % 16 == 0, "alignment");
-
-// Element offset of column `col` of state row p in Sb (16-byte chunks XOR-swizzled by row).
-__device__ __forceinline__ int sb_off(int p, int col) {
-  return p * Lay16::LS + 8 * ((col >> 3) ^ (p & 15)) + (col & 7);
-}
-
-// Element offset of column `col` of token row r in VR, ZR, VS: the row's 32-byte pair
-// (col / 16) XOR (r / 2) % 4 and the chunk within it flipped by (r / 8) % 2. Eight consecutive
-// rows then place one pair in eight distinct 32-byte bank groups (the transposing reads), and
-// sixteen consecutive rows one chunk in sixteen distinct 16-byte groups (the epilogue reads).
-__device__ __forceinline__ int v_off(int r, int col) {
-  const int c = col >> 3;
-  const int pc = 2 * ((c >> 1) ^ ((r >> 1) & 3)) + ((c & 1) ^ ((r >> 3) & 1));
-  return r * Lay16::LV + 8 * pc + (col & 7);
-}
-
-// The causal score tiles (row tile it, column tile sj <= it) of waves 0-9: the diagonal tiles,
-// whose decay weights take the most arithmetic, on waves 0-3 (one per SIMD).
-__device__ __forceinline__ void score_tile16(int w, int& it, int& sj) {
-  // w: 0 1 2 3 | 4 5 6 7 8 9  ->  (0,0) (1,1) (2,2) (3,3) | (1,0) (2,0) (2,1) (3,0) (3,1) (3,2)
-  const int k = w - 4;
-  it = w < 4 ? w : (k < 1 ? 1 : (k < 3 ? 2 : 3));
-  sj = w < 4 ? w : (k < 1 ? 0 : (k < 3 ? k - 1 : k - 3));
-}
-
-template <typename T, int R, bool SO>
-__global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a,
-                                                            const ScanGeom g,
-                                                            const float* __restrict__ prep) {
-  static_assert(R == 1 || R == 4, "scan16_kernel: ranks 1 and 4");
-  using M = Mma<T>;
-  using Ly = Lay16;
-  constexpr int TOK = 64 / R;  // tokens per 64-row sub-chunk (rows (token, rank), rank minor)
-  using SB_ = ScBlk<TOK>;
-  constexpr int LQ = Ly::LQ, LW = Ly::LW, CST = Ly::CST, ES = 2, S = kSMax;
-  // phase: 16 lanes per angle, TPL tokens per lane (waves 0-7)
-  constexpr int PG = 16, TPL = TOK / 16;
-  const int H = a.heads, L = a.length;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l16 = lane & 15, lg = lane >> 4;
-
-  int bid = blockIdx.x;
-  if (g.xcd_map) {
-    const int per = gridDim.x >> 3;
-    bid = (bid & 7) * per + (bid >> 3);
-  }
-  const int b = bid / H, h = bid - b * H;
-
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  T* Qs = lds_t<T>(smem, Ly::QS);
-  T* Ks = lds_t<T>(smem, Ly::KS);
-  T* VR = lds_t<T>(smem, Ly::VR);
-  T* ZR = lds_t<T>(smem, Ly::ZR);
-  T* VS = lds_t<T>(smem, Ly::VS);
-  T* Sb = lds_t<T>(smem, Ly::SB);
-  T* WS = lds_t<T>(smem, Ly::WS);
-  float* F = lds_t<float>(smem, Ly::FB);
-  const float Dh = ldx(a.D.ptr, a.D.dtype, h * a.D.stride[0]);
-
-  // ---- lane roles
-  // q / k: rows qt and qt + 32 (rank qr), four columns. Rank 1: n0 .. n0+3, waves 0-7 the
-  // rotated columns 0-63 (pairs (2j, 2j+1)). Rank 4 (the MIMO rotation pairs column n with
-  // n + 64, n < 32): waves 0-7 columns n0, n0+1, n0+64, n0+65 (n0 = 2 (tid % 16)), waves 8-15
-  // four of the unrotated columns 32-63 and 96-127.
-  const bool rot = w < 8;
-  const int qt = (tid & 511) >> 4, qr = qt & (R - 1);
-  const int n0 = R == 1 ? 64 * (tid >> 9) + 4 * (tid & 15)
-                        : (rot ? 2 * (tid & 15) : ((tid & 15) < 8 ? 32 : 64) + 4 * (tid & 15));
-  auto qcol = [&](int i) { return R > 1 && rot ? n0 + (i & 1) + 64 * (i >> 1) : n0 + i; };
-  // value / gate: row vt (token vt / R, rank vt % R), columns p0 .. p0+3
-  const int vt = tid >> 4, p0 = 4 * (tid & 15);
-  // phase (waves 0-7): angle ps, tokens TPL pg .. TPL pg + 3
-  const int ps = tid >> 4, pg = tid & 15;
-  const bool ph_wave = w < 8;
-  // state tiles (ni, pj), k = 0, 1: ni = w / 2, pj = 2 (w % 2) + k; lane holds
-  // n = 16 ni + 4 lg + i, p = 16 pj + l16 (S^T in MFMA accumulator layout)
-  const int sni = w >> 1, spj0 = 2 * (w & 1);
-
-  for (int s = tid; s < S; s += k16Threads) {
-    F[Ly::PBASE + s] = 0.f;
-    F[Ly::POFF + s] = a.initial_phase.ptr != nullptr
-                          ? static_cast<const float*>(a.initial_phase.ptr)
-                                [b * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
-                                 s * a.initial_phase.stride[2]]
-                          : 0.f;
-  }
-
-  // rounded biases of the lane's 4 columns, rank qr (the rows come normalized from prep)
-  float bq[4], bk[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int n = qcol(i);
-    bq[i] = rnd<T>(ldx(a.q_bias.ptr, a.q_bias.dtype,
-                       h * a.q_bias.stride[0] + qr * a.q_bias.stride[1] + n));
-    bk[i] = rnd<T>(ldx(a.k_bias.ptr, a.k_bias.dtype,
-                       h * a.k_bias.stride[0] + qr * a.k_bias.stride[1] + n));
-  }
-  if constexpr (R > 1) {
-    // the rounded mimo_x / mimo_z and mimo_out of this head (ops.py:700-714, 869-877)
-    for (int i = tid; i < R * kPPad; i += k16Threads) {
-      const int r = i / kPPad, p = i - r * kPPad;
-      F[Ly::MX + i] = rnd<T>(ldx(a.mimo_x.ptr, a.mimo_x.dtype,
-                                 h * a.mimo_x.stride[0] + r * a.mimo_x.stride[1] + p));
-      F[Ly::MZ + i] = rnd<T>(ldx(a.mimo_z.ptr, a.mimo_z.dtype,
-                                 h * a.mimo_z.stride[0] + r * a.mimo_z.stride[1] + p));
-      F[Ly::MO + i] = ldx(a.mimo_out.ptr, a.mimo_out.dtype,
-                          h * a.mimo_out.stride[0] + r * a.mimo_out.stride[1] + p);
-    }
-  }
-
-  f4 st[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    st[k] = zero4();
-    if (a.initial_state.ptr != nullptr) {
-      const int p = 16 * (spj0 + k) + l16;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = 16 * sni + 4 * lg + i;
-        st[k][i] = static_cast<const float*>(a.initial_state.ptr)
-            [b * a.initial_state.stride[0] + h * a.initial_state.stride[1] +
-             p * a.initial_state.stride[2] + n];
-      }
-    }
-  }
-  // Endpoint continuation (ops.py:681-686): S += dt_0 (1 - trap_0) sum_r (v_prev mx_r) k_prev_r^T.
-  if (a.initial_k.ptr != nullptr && L > 0) {
-    float dt0, adt0;
-    dt_adt(true, ldx(a.dt.ptr, a.dt.dtype, b * a.dt.stride[0] + h * a.dt.stride[2]),
-           ldx(a.a.ptr, a.a.dtype, b * a.a.stride[0] + h * a.a.stride[2]),
-           ldx(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0]), dt0, adt0);
-    const float tr0 = sigmoidf(ldx(a.trap.ptr, a.trap.dtype,
-                                   b * a.trap.stride[0] + h * a.trap.stride[2]));
-    const float c0 = dt0 * (1.f - tr0);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int p = 16 * (spj0 + k) + l16;
-      const float v0 = to_f(static_cast<const T*>(a.initial_value.ptr)
-                                [b * a.initial_value.stride[0] + h * a.initial_value.stride[1] + p]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int n = 16 * sni + 4 * lg + i;
-        float outer = 0.f;
-        for (int r = 0; r < R; ++r) {
-          const float pv = R > 1 ? mul_r<T>(v0, rnd<T>(ldx(a.mimo_x.ptr, a.mimo_x.dtype,
-                                                             h * a.mimo_x.stride[0] +
-                                                                 r * a.mimo_x.stride[1] + p)))
-                                 : v0;
-          const float k0 = to_f(static_cast<const T*>(a.initial_k.ptr)
-                                    [b * a.initial_k.stride[0] + h * a.initial_k.stride[1] +
-                                     r * a.initial_k.stride[2] + n]);
-          outer += pv * k0;
-        }
-        st[k][i] += c0 * outer;
-      }
-    }
-  }
-
-  // ---- global reads: one buffer resource over the batch row of the projection (its extent
-  // ends at token L: rows past it read zero, stores past it are dropped) and one over the
-  // workspace; per-lane byte offsets at token 0
-  const int tok_b = g.tok_b;
-  const __amdgpu_buffer_rsrc_t rs_p =
-      make_rsrc(g.proj + b * g.proj_b, L * (tok_b < 0 ? -tok_b : tok_b));
-  const __amdgpu_buffer_rsrc_t rs_w = make_rsrc(prep, g.ws_bytes);
-  // the normalized q / k rows of batch row b: row (token, rank) at 2 N elements, k after q (rows
-  // past token L read zero)
-  const __amdgpu_buffer_rsrc_t rs_qk =
-      make_rsrc(reinterpret_cast<const char*>(prep) + g.ws_qk +
-                    static_cast<int64_t>(b) * L * R * 4 * kNPad,
-                L * R * 4 * kNPad);
-  const int o_qk = qt * 4 * kNPad + n0 * ES;  // row qt (forward order), column n0 of q
-  const int o_vz = g.o_v + h * g.vz_h + (vt / R) * tok_b + p0 * ES, d_z = g.o_z - g.o_v;
-  const int nsub = g.nsub, scw = g.scw;
-  // side words (waves 0-3, one float pair per lane): the scalar block
-  const int q2 = 2 * tid;
-  const bool side_on = q2 < scw;
-  const int side_o =
-      side_on ? static_cast<int>(g.ws_sc + static_cast<int64_t>(b * H + h) * nsub * scw + q2) * 4
-              : 0;
-  const int side_s = scw * 4;
-  // angle words (waves 0-7): 4 tokens of one angle each, in the tile order [TOK / 4][S][4]
-  const int ang_o = static_cast<int>(g.ws_ang + static_cast<int64_t>(b) * g.L4 * S * 4 + 4 * tid) * 4;
-  const int ang_s = (TOK / 4) * S * 16;
-  const bool ang_on = tid < TOK * S / 4;
-
-  float* fph = a.final_phase.ptr != nullptr && ph_wave
-                   ? static_cast<float*>(a.final_phase.ptr) + b * a.final_phase.stride[0] +
-                         h * a.final_phase.stride[1] + ps * a.final_phase.stride[2]
-                   : nullptr;
-  float* fblk = a.block_phase.ptr != nullptr && ph_wave
-                    ? static_cast<float*>(a.block_phase.ptr) + b * a.block_phase.stride[0] +
-                          h * a.block_phase.stride[1] + ps * a.block_phase.stride[3]
-                    : nullptr;
-  const int64_t blk_stride = a.block_phase.stride[2];
-  const __amdgpu_buffer_rsrc_t rs_o =
-      make_rsrc(const_cast<char*>(g.out_base) + b * g.out_b, L * (g.out_t < 0 ? -g.out_t : g.out_t));
-  const int out_t = g.out_t, o_out = h * g.out_h + g.out_o0;
-
-  // q / k words: [token qt, qt + 32][q, k] 4 elements each
-  uint32_t rq[2][2], rk[2][2], rv[2], rz[2];
-  float2 side = make_float2(0.f, 0.f);
-  float4 ang = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto load_qk = [&](int t0) {
-    // the rows are stored in the call's token order: logical token t at rows t R .. t R + R - 1
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int o = o_qk + (t0 * R + 32 * j) * 4 * kNPad;
-      if (R > 1 && rot) {
-        // columns n0, n0 + 1 and their rotation partners n0 + 64, n0 + 65
-        rq[j][0] = __builtin_amdgcn_raw_buffer_load_b32(rs_qk, o, 0, 0);
-        rq[j][1] = __builtin_amdgcn_raw_buffer_load_b32(rs_qk, o + 128, 0, 0);
-        rk[j][0] = __builtin_amdgcn_raw_buffer_load_b32(rs_qk, o + 2 * kNPad, 0, 0);
-        rk[j][1] = __builtin_amdgcn_raw_buffer_load_b32(rs_qk, o + 2 * kNPad + 128, 0, 0);
-      } else {
-        bload_words<2>(rq[j], rs_qk, o);
-        bload_words<2>(rk[j], rs_qk, o + 2 * kNPad);
-      }
-    }
-  };
-  auto load_vz = [&](int t0) {
-    bload_words<2>(rv, rs_p, o_vz + t0 * tok_b);
-    bload_words<2>(rz, rs_p, o_vz + t0 * tok_b + d_z);
-  };
-  auto load_side = [&](int c) {
-    if (w < 4) {
-      const u32x2 v = __builtin_bit_cast(
-          u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, side_o + c * side_s, 0, 0));
-      side = make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
-    }
-    if (w < 8) {
-      const u32x4 v = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_w, ang_o + c * ang_s, 0, 0));
-      ang = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-                        __uint_as_float(v[3]));
-    }
-  };
-  float* ANG = F + Ly::ANG;
-  // angle tile slot of 4-token group gq and angle s (XOR-keyed by the group's phase lane)
-  auto ang_slot = [&](int gq, int s) { return gq * kSMax + (s ^ gq); };
-  auto put_side = [&](int c) {
-    if (w < 4 && side_on) *reinterpret_cast<float2*>(F + Ly::SC0 + (c & 1) * Ly::SCB + q2) = side;
-    if (w < 8 && ang_on) {
-      const int gq = tid / S;
-      *reinterpret_cast<float4*>(ANG + 4 * ang_slot(gq, tid - gq * S)) = ang;
-    }
-  };
-  auto scb = [&](int c) { return F + Ly::SC0 + (c & 1) * Ly::SCB; };
-  auto csb = [&](int c) { return F + Ly::CS0 + (c & 1) * Ly::CSB; };
-  auto phases = [&](int c) {
-    // phases of sub-chunk c (waves 0-7), from the angle tile and the dt of its side block
-    if (ph_wave && c < nsub) {
-      float pa[TPL];
-      if constexpr (TPL == 4) {
-        const float4 v = *reinterpret_cast<const float4*>(ANG + 4 * ang_slot(pg, ps));
-        pa[0] = v.x;
-        pa[1] = v.y;
-        pa[2] = v.z;
-        pa[3] = v.w;
-      } else {
-        pa[0] = ANG[4 * ang_slot(pg >> 2, ps) + (pg & 3)];  // token pg of its 4-token group
-      }
-      phase_stage<PG, TPL, CST, true, false>(csb(c), ps, F + Ly::PBASE + ps, F + Ly::POFF + ps,
-                                             scb(c) + SB_::DTV, c * TOK, L, pg, lane, true, pa,
-                                             fph, fblk, blk_stride);
-    }
-  };
-
-  // prologue: side block and angle tile of sub-chunk 0, its phases; the loads of 0 and 1
-  load_side(0);
-  load_qk(0);
-  load_vz(0);
-  put_side(0);
-  load_side(1);
-  __syncthreads();
-  phases(0);
-  __syncthreads();
-
-  float log_decay = 0.f;
-  for (int c = 0; c < nsub; ++c) {
-    const int t0 = c * TOK;
-    const float* SC = scb(c);
-    const float* CSt = csb(c);
-
-    // ---- A: staging
-    if (c + 1 < nsub) put_side(c + 1);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      // row rw (token tt): q = q^ + bias, k = k^ + bias, rotated. Rank 1: pairs (n0, n0+1),
-      // (n0+2, n0+3), angles n0 / 2 and n0 / 2 + 1; rank 4: pairs (n0 + e, n0 + 64 + e), angles
-      // n0 + e (e < 2). Both angle pairs are adjacent in the cos / sin table row.
-      const int rw = qt + 32 * j, tt = rw / R;
-      f4 q, k;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        q[i] = raw_get<T>(rq[j], i) + bq[i];
-        k[i] = raw_get<T>(rk[j], i) + bk[i];
-      }
-      if (rot) {
-        const f4 cv = *reinterpret_cast<const f4*>(
-            CSt + tt * CST + 2 * cs_col<true>(R == 1 ? n0 >> 1 : n0, tt));
-#pragma unroll
-        for (int pp = 0; pp < 2; ++pp) {
-          // the pair's two columns: (2 pp, 2 pp + 1) for rank 1, (pp, pp + 2) for rank 4
-          const int u0 = R == 1 ? 2 * pp : pp, u1 = R == 1 ? 2 * pp + 1 : pp + 2;
-          const float cc = cv[2 * pp], ss = cv[2 * pp + 1];
-          const float q0 = q[u0], q1 = q[u1];
-          const float k0 = k[u0], k1 = k[u1];
-          q[u0] = fmaf(q0, cc, -(q1 * ss));
-          q[u1] = fmaf(q0, ss, q1 * cc);
-          k[u0] = fmaf(k0, cc, -(k1 * ss));
-          k[u1] = fmaf(k0, ss, k1 * cc);
-        }
-      }
-      if (R > 1 && rot) {
-        if constexpr (!SO) {
-          st_pair<T>(Qs + rw * LQ + n0, q[0], q[1]);
-          st_pair<T>(Qs + rw * LQ + n0 + 64, q[2], q[3]);
-        }
-        st_pair<T>(Ks + rw * LQ + n0, k[0], k[1]);
-        st_pair<T>(Ks + rw * LQ + n0 + 64, k[2], k[3]);
-      } else {
-        if constexpr (!SO) st_quad<T>(Qs + rw * LQ + n0, q);
-        st_quad<T>(Ks + rw * LQ + n0, k);
-      }
-    }
-    {
-      // value / gate of row vt (token tv): VR / ZR = v, z (rank 1 as loaded; rank 4 times the
-      // rounded mimo_x / mimo_z of the row's rank, rounded), VS = VR * scale * exp(cum_last - cum)
-      const int tv = vt / R;
-      const float ev = SC[SB_::SCL + tv] * __expf(SC[SB_::CL] - SC[SB_::CUM + tv]);
-      f4 sv;
-      if constexpr (R == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sv[i] = raw_get<T>(rv, i) * ev;
-        if constexpr (!SO) {
-          *reinterpret_cast<u32x2*>(VR + v_off(vt, p0)) = (u32x2){rv[0], rv[1]};
-          *reinterpret_cast<u32x2*>(ZR + v_off(vt, p0)) = (u32x2){rz[0], rz[1]};
-        }
-      } else {
-        const int mo = (vt & (R - 1)) * kPPad + p0;
-        const f4 mx = *reinterpret_cast<const f4*>(F + Ly::MX + mo);
-        f4 vq;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          vq[i] = mul_r<T>(raw_get<T>(rv, i), mx[i]);
-          sv[i] = vq[i] * ev;
-        }
-        if constexpr (!SO) {
-          const f4 mz = *reinterpret_cast<const f4*>(F + Ly::MZ + mo);
-          f4 zq;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) zq[i] = mul_r<T>(raw_get<T>(rz, i), mz[i]);
-          st_quad<T>(VR + v_off(vt, p0), vq);
-          st_quad<T>(ZR + v_off(vt, p0), zq);
-        }
-      }
-      st_quad<T>(VS + v_off(vt, p0), sv);
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if constexpr (!SO) st_quad<T>(Sb + sb_off(16 * (spj0 + k) + l16, 16 * sni + 4 * lg), st[k]);
-    }
-    {
-      const float ecl = SC[SB_::ECL];
-      log_decay += SC[SB_::CL];
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) st[k][i] *= ecl;
-      }
-    }
-    __syncthreads();
-
-    // ---- B: score tiles and decay weights, carry products, phases of c + 1; loads of c + 1
-    __builtin_amdgcn_sched_barrier(0);
-    load_qk(t0 + TOK);
-    __builtin_amdgcn_sched_barrier(0);
-    if (!SO && w < 10) {
-      int it, sj;
-      score_tile16(w, it, sj);
-      const int tq = 16 * it + l16;
-      f4 acc = zero4();
-      // (four waves per SIMD hide the operand latency: one k-step's operands in registers at a
-      // time keeps the kernel within 128 VGPRs)
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const typename M::v8 av = *reinterpret_cast<const typename M::v8*>(
-            Ks + (16 * sj + l16) * LQ + 32 * kk + 8 * lg);
-        const typename M::v8 bv =
-            *reinterpret_cast<const typename M::v8*>(Qs + tq * LQ + 32 * kk + 8 * lg);
-        acc = M::mma(av, bv, acc);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // decay weights by token: row tq is token tq / R, column rows 16 sj + 4 lg + i are
-      // tokens (16 sj + 4 lg + i) / R (rank 4: the one token 4 sj + lg)
-      const int tqt = tq / R;
-      const float cum_t = SC[SB_::CUM + tqt];
-      f4 wv;
-      if (sj < it) {
-        // d = exp(cum_t - cend) * (scale_s exp(cend - cum_s)), both factors <= 1
-        const float at = __expf(cum_t - SC[SB_::CEND + sj]);
-        if constexpr (R == 1) {
-          const f4 bs = *reinterpret_cast<const f4*>(SC + SB_::BSC + 16 * sj + 4 * lg);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) wv[i] = acc[i] * (at * bs[i]);
-        } else {
-          const float bs = SC[SB_::BSC + 4 * sj + lg];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) wv[i] = acc[i] * (at * bs);
-        }
-      } else {
-        const float gam_t = SC[SB_::GAM + tqt];
-        int tq_m = tqt;
-        __asm__ volatile("" : "+v"(tq_m));
-        if constexpr (R == 1) {
-          const f4 c4 = *reinterpret_cast<const f4*>(SC + SB_::CUM + 16 * sj + 4 * lg);
-          const f4 s4 = *reinterpret_cast<const f4*>(SC + SB_::SCL + 16 * sj + 4 * lg);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int ts = 16 * sj + 4 * lg + i;
-            const float lower = s4[i] * __expf(cum_t - c4[i]);
-            const float d = tq_m > ts ? lower : (tq_m == ts ? gam_t : 0.f);
-            wv[i] = acc[i] * d;
-          }
-        } else {
-          // same token (every rank pair): gamma; an earlier token: the decayed scale
-          const int ts = 4 * sj + lg;
-          const float lower = SC[SB_::SCL + ts] * __expf(cum_t - SC[SB_::CUM + ts]);
-          const float d = tq_m > ts ? lower : (tq_m == ts ? gam_t : 0.f);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) wv[i] = acc[i] * d;
-        }
-      }
-      // W[t][s], s = 16 sj + 4 lg + i, at s' = 32 (sj / 2) + 8 lg + 4 (sj % 2) + i: the order of
-      // the intra product's K axis (below)
-      st_quad<T>(WS + tq * LW + 32 * (sj >> 1) + 8 * lg + 4 * (sj & 1), wv);
-    }
-    {
-      // carry: S^T(ni, pj) += K~^T V~ over the 64 tokens. A: 8 tokens of column n from the
-      // row-major Ks by two transposing reads (in each 16-lane group, lane 4a + b receives
-      // element b of the 8-byte vectors of lanes a, a + 4, a + 8, a + 12); B: the same from VS.
-      // The K axis of k-step kk, lane group lg: tokens kk + 4 lg + j (slots j) and
-      // kk + 16 + 4 lg + j (slots 4 + j), so the 32 lanes of each read take 8 consecutive tokens
-      const int xr = l16 >> 2, xc = 4 * (l16 & 3);
-#pragma unroll
-      for (int kk = 0; kk < 64; kk += 32) {  // the 64 rows
-        const int r0 = kk + 4 * lg + xr;
-        const T* k0 = Ks + r0 * LQ + 16 * sni + xc;
-        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(k0));
-        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) i16x4*)(k0 + 16 * LQ));
-        const typename M::v8 av = __builtin_bit_cast(
-            typename M::v8, (i16x8){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int vc = 16 * (spj0 + k) + xc;
-          const i16x4 vlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(VS + v_off(r0, vc)));
-          const i16x4 vhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(VS + v_off(r0 + 16, vc)));
-          const typename M::v8 bv = __builtin_bit_cast(
-              typename M::v8,
-              (i16x8){vlo[0], vlo[1], vlo[2], vlo[3], vhi[0], vhi[1], vhi[2], vhi[3]});
-          st[k] = M::mma(av, bv, st[k]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    load_vz(t0 + TOK);
-    __builtin_amdgcn_sched_barrier(0);
-    load_side(c + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-
-    // ---- C: output tile (row tile it, P tile pj)
-    if constexpr (!SO) {
-      const int it = w >> 2, pj = w & 3;
-      const int tq = 16 * it + l16;
-      f4 yi = zero4(), ye = zero4();
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        if (2 * m > it) continue;
-        // intra: V^T W^T over tokens s = 32 m + 4 lg + i and 32 m + 16 + 4 lg + i
-        const int vrow = 32 * m + 4 * lg + (l16 >> 2), vcol = 16 * pj + 4 * (l16 & 3);
-        const typename M::v4 b0 = __builtin_bit_cast(
-            typename M::v4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                (__attribute__((address_space(3))) i16x4*)(VR + v_off(vrow, vcol))));
-        const typename M::v4 b1 = __builtin_bit_cast(
-            typename M::v4,
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) i16x4*)(VR + v_off(vrow + 16, vcol))));
-        typename M::v8 av, bv = *reinterpret_cast<const typename M::v8*>(WS + tq * LW + 32 * m + 8 * lg);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          av[i] = b0[i];
-          av[4 + i] = b1[i];
-        }
-        if (2 * m + 1 > it) {
-          // column tile 2m + 1 lies above it: the operand's upper half (two words) is zero
-          // (element-wise 16-bit zeroing took a select and a permute per element)
-          u32x4 bw = __builtin_bit_cast(u32x4, bv);
-          bw[2] = 0u;
-          bw[3] = 0u;
-          bv = __builtin_bit_cast(typename M::v8, bw);
-        }
-        yi = M::mma(av, bv, yi);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        // inter: rnd(S) Q^T
-        const typename M::v8 av = *reinterpret_cast<const typename M::v8*>(
-            Sb + sb_off(16 * pj + l16, 32 * kk + 8 * lg));
-        const typename M::v8 bv =
-            *reinterpret_cast<const typename M::v8*>(Qs + tq * LQ + 32 * kk + 8 * lg);
-        ye = M::mma(av, bv, ye);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // epilogue: row tq (token tq / R), columns pb .. pb+3
-      const int pb = 16 * pj + 4 * lg, tqt = tq / R;
-      const float ecum_t = __expf(SC[SB_::CUM + tqt]);
-      const typename M::v4 v4 = *reinterpret_cast<const typename M::v4*>(VR + v_off(tq, pb));
-      const typename M::v4 z4 = *reinterpret_cast<const typename M::v4*>(ZR + v_off(tq, pb));
-      f4 y;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * to_f(v4[i])) * silu_fast(to_f(z4[i]));
-      }
-      if constexpr (R > 1) {
-        // times mimo_out of the row's rank, summed over the token's R rows: lanes 4m .. 4m+3
-        // of the 16-lane group (DPP quad permutes lane ^ 1 and lane ^ 2)
-        const f4 mo = *reinterpret_cast<const f4*>(F + Ly::MO + (tq & (R - 1)) * kPPad + pb);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float t = y[i] * mo[i];
-          t += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                             0, __builtin_bit_cast(int, t), 0xb1, 0xf, 0xf, false));
-          t += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                             0, __builtin_bit_cast(int, t), 0x4e, 0xf, 0xf, false));
-          y[i] = t;
-        }
-      }
-      if (R == 1 || (tq & (R - 1)) == 0) {
-        bstore_quad<T>(y, rs_o, (tqt * out_t + o_out + pb * ES) +
-                                    __builtin_amdgcn_readfirstlane(t0 * out_t));
-      }
-    }
-    // phases of c + 1: its angle tile and side block came to LDS in A; its cos / sin table is
-    // the other buffer than the one A read
-    phases(c + 1);
-    __syncthreads();
-  }
-
-  // ---- final k: the biased, rotated k rows of token L-1, still in Ks from the last sub-chunk
-  if (a.final_k.ptr != nullptr && L > 0) {
-    const int tl = (L - 1) - (nsub - 1) * TOK;
-    for (int i = tid; i < R * kNPad; i += k16Threads) {
-      const int r = i / kNPad, n = i - r * kNPad;
-      static_cast<T*>(a.final_k.ptr)[b * a.final_k.stride[0] + h * a.final_k.stride[1] +
-                                     r * a.final_k.stride[2] + n] = Ks[(tl * R + r) * LQ + n];
-    }
-  }
-  if (a.final_decay.ptr != nullptr && tid == 0) {
-    static_cast<float*>(a.final_decay.ptr)[b * a.final_decay.stride[0] +
-                                           h * a.final_decay.stride[1]] = log_decay;
-  }
-  if (a.block_phase.ptr != nullptr && L > 0) {
-    for (int i = tid; i < S; i += k16Threads) {
-      static_cast<float*>(a.block_phase.ptr)[b * a.block_phase.stride[0] +
-                                             h * a.block_phase.stride[1] +
-                                             ((L - 1) >> 6) * a.block_phase.stride[2] +
-                                             i * a.block_phase.stride[3]] = F[Ly::PBASE + i];
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int p = 16 * (spj0 + k) + l16;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = 16 * sni + 4 * lg + i;
-      static_cast<float*>(a.final_state.ptr)[b * a.final_state.stride[0] +
-                                             h * a.final_state.stride[1] +
-                                             p * a.final_state.stride[2] + n] = st[k][i];
-    }
-  }
-}
 
 // ------------------------------------------------------------ segmented scan (composition)
 
@@ -3189,22 +2024,105 @@ __global__ __launch_bounds__(kCompThreads) void gather_kernel(const m3_scan_args
 
 // ------------------------------------------------------------------ host side
 
+static bool pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// A call scan16_kernel may serve (the projection form is checked later, at launch): the model's
-// SISO shape in a 16-bit activation dtype with RMSNorm, head biases, raw dt and angle phases.
-static bool scan16_candidate(const m3_scan_args& a) {
-  return (a.act_dtype == M3_BF16 || a.act_dtype == M3_F16) &&
-         (a.rank == 1 || a.rank == 4) && a.groups == 1 &&
-         a.d_state == kNPad && a.head_dim == kPPad && a.num_angles == kSMax &&
-         a.q_norm_w.ptr != nullptr && a.k_norm_w.ptr != nullptr && a.q_bias.ptr != nullptr &&
-         a.k_bias.ptr != nullptr && a.raw_dt != 0 && a.phase_mode == M3_PHASE_ANGLES &&
-         (a.mimo_rotation != 0) == (a.rank > 1);
+// The form in which scan16_kernel takes a call (Form16), -1 when it does not: a 16-bit call of up
+// to 128 columns, 64 values and 32 angles at ranks 1, 2, 4 and 8, whose q / k / value / gate /
+// out rows can be read and written 4 elements at a time, each token's row (of one group, rank or
+// head) below the next token's, and whose offsets within a batch row fit 32 bits (the loads run
+// up to two sub-chunks, 128 tokens, and a token group ahead). Projection form: norm weights,
+// biases, raw dt, angle increments; hook form: none of the norms, phases given or none.
+// Every such call is faster on it than on the kernel it took before (per call, scan_kernel then
+// scan16_kernel, 8 x 1024 tokens, 32 heads): hook form rank 1 80 -> 72 us, rank 2 184 -> 118,
+// rank 4 332 -> 207, rank 8 628 -> 392; projection form rank 2 140 -> 121, rank 8 487 -> 391,
+// d_state 64 rank 1 114 -> 67; the recurrent scan at d_state 96, 4 x 1500 tokens, 16 heads:
+// 21.6 ms -> 86 us.
+static int form16_of(const m3_scan_args& a) {
+  if (a.act_dtype != M3_BF16 && a.act_dtype != M3_F16) return -1;
+  if (a.rank != 1 && a.rank != 2 && a.rank != 4 && a.rank != 8) return -1;
+  const int N = a.d_state, P = a.head_dim, S = a.num_angles;
+  if (N < 4 || N > kNPad || N % 4 != 0 || P <= 0 || P > kPPad || P % 4 != 0 || S > kSMax ||
+      a.length <= 0 || a.batch <= 0 || a.groups <= 0 || a.heads % a.groups != 0) {
+    return -1;
+  }
+  const bool rotates = a.phase_mode != M3_PHASE_NONE;
+  // the MIMO pairs' columns come in chunks of 4 (4 S == N there, 2 S <= N otherwise: validated)
+  if (rotates && (a.mimo_rotation ? S % 4 != 0 || 4 * S != N : 2 * S > N)) return -1;
+  if (rotates && S <= 0) return -1;
+  const bool norm = a.q_norm_w.ptr != nullptr && a.k_norm_w.ptr != nullptr;
+  const bool proj = norm && a.q_bias.ptr != nullptr && a.k_bias.ptr != nullptr &&
+                    a.raw_dt != 0 && a.dt_bias.ptr != nullptr && a.phase_mode == M3_PHASE_ANGLES;
+  const bool hook = a.q_norm_w.ptr == nullptr && a.k_norm_w.ptr == nullptr && a.raw_dt == 0 &&
+                    a.phase_mode != M3_PHASE_ANGLES;
+  if (!proj && !hook) return -1;
+  const int64_t len = a.length, ahead = len + 256;
+  // rows of `dims` outer axes (extents in `ext`) read `span` elements at a time
+  auto rows_ok = [&](const m3_tensor& t, std::initializer_list<int64_t> ext, int64_t span) {
+    if (t.ptr == nullptr || reinterpret_cast<uintptr_t>(t.ptr) % 8 != 0) return false;
+    int i = 0;
+    for (int64_t e : ext) {
+      if (e > 1 && t.stride[i] % 4 != 0) return false;
+      ++i;
+    }
+    const int64_t s1 = t.stride[1] < 0 ? -t.stride[1] : t.stride[1];
+    return (len == 1 || s1 >= span) && ahead * s1 * 2 < INT32_MAX;
+  };
+  if (!rows_ok(a.q, {a.batch, len, a.groups, a.rank}, N) ||
+      !rows_ok(a.k, {a.batch, len, a.groups, a.rank}, N) ||
+      !rows_ok(a.value, {a.batch, len, a.heads}, P) || !rows_ok(a.gate, {a.batch, len, a.heads}, P) ||
+      !rows_ok(a.out, {a.batch, len, a.heads}, P)) {
+    return -1;
+  }
+  // one token: its stride is never used to reach another, and must not take the offsets out of
+  // range or make a second token alias the first
+  if (len == 1) {
+    for (const m3_tensor* t : {&a.value, &a.gate, &a.out}) {
+      if ((t->stride[1] < 0 ? -t->stride[1] : t->stride[1]) < P) return -1;
+    }
+  }
+  const int64_t tok = 64 / a.rank, nsub = (len + tok - 1) / tok;
+  if (ahead * a.groups * a.rank * 2 * kNPad * 4 >= INT32_MAX ||
+      (nsub + 3) * (5 * tok + 8) * 4 >= INT32_MAX) {
+    return -1;
+  }
+  if (a.phase_mode == M3_PHASE_ANGLES && ahead * S * 4 >= (int64_t{1} << 30)) return -1;
+  if (a.phase_mode == M3_PHASE_GIVEN) {
+    const int64_t s1 = a.phase.stride[1] < 0 ? -a.phase.stride[1] : a.phase.stride[1];
+    const int64_t span = (S - 1) * a.phase.stride[3] + 1;
+    if (a.phase.ptr == nullptr || a.phase.stride[3] < 0 || s1 < span ||
+        ahead * s1 * 4 >= (int64_t{1} << 30)) {
+      return -1;
+    }
+  }
+  // offsets within one (batch, head) of the states and within one head of the parameters, in
+  // 32 bits
+  for (const m3_tensor* t : {&a.initial_state, &a.final_state}) {
+    if (t->ptr != nullptr && (t->stride[2] < 0 || (P * t->stride[2] + N) * 4 >= (int64_t{1} << 30))) {
+      return -1;
+    }
+  }
+  for (const m3_tensor* t : {&a.q_bias, &a.k_bias, &a.mimo_x, &a.mimo_z, &a.mimo_out}) {
+    if (t->ptr != nullptr && (t->stride[1] < 0 || (a.rank * t->stride[1] + N) * 4 >= (int64_t{1} << 30))) {
+      return -1;
+    }
+  }
+  if (a.initial_k.ptr != nullptr &&
+      (a.initial_k.stride[2] < 0 || (a.rank * a.initial_k.stride[2] + N) * 2 >= (int64_t{1} << 30))) {
+    return -1;
+  }
+  if (!proj) return kHook;
+  return N == kNPad && P == kPPad && S == kSMax && a.groups == 1 && (a.rank == 1 || a.rank == 4) &&
+                 (a.mimo_rotation != 0) == (a.rank > 1)
+             ? kModel
+             : kProj;
 }
 
 // Prep workspace regions (floats, each 16-byte aligned) and the sub-chunk geometry; returns the
-// workspace size in bytes.
-static size_t ws_layout(const m3_scan_args& a, ScanGeom& g) {
+// workspace size in bytes. `form16`: form16_of(a), or -1 for a layout without the 16-wave scan's
+// rows.
+static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   const int rows = a.act_dtype == M3_F32 ? Mma<float>::ROWS : Mma<__bf16>::ROWS;
   const int rank = a.rank > 0 ? a.rank : 1;
   g.tok = rows / rank > 0 ? rows / rank : 1;
@@ -3212,7 +2130,10 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g) {
   g.nsub = static_cast<int>((len + g.tok - 1) / g.tok);
   g.scw = 5 * g.tok + 8;  // ScBlk<tok>::SIZE
   g.L4 = static_cast<int>((len + 3) / 4);
-  const bool norm = a.q_norm_w.ptr != nullptr;
+  g.form16 = form16;
+  g.perm = a.phase_mode != M3_PHASE_NONE && a.mimo_rotation != 0;
+  g.wlo = !pow2(a.d_state);
+  const bool norm = a.q_norm_w.ptr != nullptr && form16 < 0;
   const bool angles = a.phase_mode == M3_PHASE_ANGLES;
   const int64_t batch = a.batch > 0 ? a.batch : 0;
   int64_t off = 0;
@@ -3228,20 +2149,14 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g) {
   // the projection form's 32-bit offsets run up to two sub-chunk strides past the end
   g.ws_bytes = bytes < (int64_t{1} << 30) ? static_cast<int>(bytes) : -1;
   g.ws_qk = -1;
-  g.qk_bytes = -1;
-  const int64_t qk = batch * len * (a.rank > 0 ? a.rank : 1) * 2 * a.d_state * 2;
-  if (scan16_candidate(a) && qk < (int64_t{1} << 30)) {
-    // 256-byte aligned, addressed in 32 bits (the rows' offsets run up to two sub-chunks past
-    // the end); larger calls take scan_kernel, which reads the raw rows
-    g.ws_qk = (bytes + 255) / 256 * 256;
-    g.qk_bytes = static_cast<int>(qk);
-    return static_cast<size_t>(g.ws_qk + qk);
-  }
-  return static_cast<size_t>(bytes);
+  if (form16 < 0) return static_cast<size_t>(bytes);
+  g.ws_qk = (bytes + 255) / 256 * 256;  // 256-byte aligned
+  return static_cast<size_t>(g.ws_qk + batch * len * a.groups * a.rank * 2 * kNPad *
+                                           (form16 == kProj ? 4 : 2));
 }
 
 template <typename T>
-static ScanGeom make_geom(const m3_scan_args& a) {
+static ScanGeom make_geom(const m3_scan_args& a, int form16) {
   ScanGeom g{};
   const int es = sizeof(T);
   const int total = a.batch * a.heads;
@@ -3261,7 +2176,7 @@ static ScanGeom make_geom(const m3_scan_args& a) {
   g.vec_nw = (a.d_state % 8 == 0) && nw_ok(a.q_norm_w) && nw_ok(a.k_norm_w);
   const int vneed = es * 4;  // 4 elements per v / z load
   g.vec_vz = (a.head_dim % 4 == 0) && vec_ok(a.value, 4, vneed) && vec_ok(a.gate, 4, vneed);
-  ws_layout(a, g);
+  ws_layout(a, g, form16);
   return g;
 }
 
@@ -3389,12 +2304,12 @@ static bool model_shape(const m3_scan_args& a, ScanGeom& g, int es) {
   return true;
 }
 
-template <typename T, int R, bool FULL, bool SO = false, bool SHAPE = false>
+template <typename T, int R, bool FULL, bool SHAPE = false>
 static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* prep, dim3 grid,
                          dim3 block, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SO, SHAPE>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SHAPE>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                        Layout<T>::BYTES);
     if (e != hipSuccess) {
@@ -3402,25 +2317,8 @@ static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* 
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SO, SHAPE>), grid, block, Layout<T>::BYTES, stream,
+  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SHAPE>), grid, block, Layout<T>::BYTES, stream,
                      a, g, prep);
-  return check_launch("m3_scan_fwd");
-}
-
-template <typename T, int R, bool SO>
-static int launch_kernel16(const m3_scan_args& a, const ScanGeom& g, const float* prep,
-                           dim3 grid, hipStream_t stream) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan16_kernel<T, R, SO>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, Lay16::BYTES);
-    if (e != hipSuccess) {
-      return fail(M3_ELAUNCH, "m3_scan_fwd: hipFuncSetAttribute: %s", hipGetErrorString(e));
-    }
-    attr_set = true;
-  }
-  hipLaunchKernelGGL((scan16_kernel<T, R, SO>), grid, dim3(k16Threads), Lay16::BYTES, stream, a, g,
-                     prep);
   return check_launch("m3_scan_fwd");
 }
 
@@ -3429,12 +2327,12 @@ static int launch_kernel16(const m3_scan_args& a, const ScanGeom& g, const float
 // `state_only`: the caller needs only the end state, decay, last k and phase block sums (the
 // outputs are not written where the state-only kernel form applies: the model's shape, 16-bit).
 template <typename T, int R>
-static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
+static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep, bool rows,
                        bool state_only = false) {
-  ScanGeom g = make_geom<T>(a);
+  ScanGeom g = make_geom<T>(a, rows ? form16_of(a) : -1);
   static_assert(Layout<T>::BYTES <= 160 * 1024, "LDS layout exceeds 160 KiB");
   const float* prep = nullptr;
-  const size_t need = ws_layout(a, g);
+  const size_t need = ws_layout(a, g, g.form16);
   if (need > 0) {
     if (a.workspace == nullptr || a.workspace_bytes < need || !aligned16(a.workspace)) {
       return fail(M3_EWORKSPACE, "m3_scan_fwd: needs a 16-byte aligned workspace of %zu bytes",
@@ -3442,19 +2340,14 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
     }
     prep = static_cast<const float*>(a.workspace);
     const int64_t tokens = static_cast<int64_t>(a.batch) * a.length;
-    const int64_t rows = g.ws_norm >= 0 ? tokens * 2 * a.groups * a.rank : 0;
+    const int64_t nrow = g.ws_norm >= 0 || g.form16 >= 0 ? tokens * 2 * a.groups * a.rank : 0;
     const int64_t ang = g.ws_ang >= 0 ? static_cast<int64_t>(a.batch) * g.L4 * a.num_angles * 4 : 0;
     const int64_t blocks = static_cast<int64_t>(a.batch) * g.nsub;  // scalar-block workgroups
-    if (rows >= INT32_MAX || ang >= INT32_MAX || blocks >= INT32_MAX || tokens >= INT32_MAX) {
+    if (nrow >= INT32_MAX || ang >= INT32_MAX || blocks >= INT32_MAX || tokens >= INT32_MAX) {
       return fail(M3_EUNSUPPORTED, "m3_scan_fwd: too many tokens for one launch");
     }
-    // the 16-wave kernel (below) reads prep's normalized rows, not the factors: their 4-byte
-    // stores, one per row, would only add partial-line writes
-    const bool k16 = sizeof(T) == 2 && (R == 1 || R == 4) && g.ws_qk >= 0 && g.qk_bytes > 0 &&
-                     full_shape(a, g, R);
-    g.norm_factors = k16 ? 0 : 1;
     constexpr int kNormRows = norm_rows<T, R>();
-    const int64_t nb_norm = (rows + 16 * kNormRows - 1) / (16 * kNormRows);
+    const int64_t nb_norm = (nrow + 16 * kNormRows - 1) / (16 * kNormRows);
     const int64_t nb_ang = (ang / 4 + 256 * kAngQuads - 1) / (256 * kAngQuads), nb_sc = blocks;
     if (run_prep && nb_norm + nb_ang + nb_sc > 0) {
       const dim3 pgrid(static_cast<unsigned>(nb_norm + nb_ang + nb_sc)), pblock(256);
@@ -3465,23 +2358,17 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
       if (rc != M3_OK) return rc;
     }
   }
-  const dim3 grid(static_cast<unsigned>(a.batch) * a.heads), block(kThreads);
-  if (full_shape(a, g, R) && prep != nullptr) {
-    if constexpr (sizeof(T) == 2 && (R == 1 || R == 4)) {
-      // the model's shape at ranks 1 and 4: the 16-wave kernel, when prep wrote the normalized
-      // rows (below 2^30 bytes of them)
-      if (g.ws_qk >= 0 && g.qk_bytes > 0) {
-        if (state_only) return launch_kernel16<T, R, true>(a, g, prep, grid, stream);
-        return launch_kernel16<T, R, false>(a, g, prep, grid, stream);
-      }
-    }
-    if constexpr (sizeof(T) == 2) {
-      if (state_only) return launch_kernel<T, R, true, true>(a, g, prep, grid, block, stream);
-    }
-    return launch_kernel<T, R, true>(a, g, prep, grid, block, stream);
+  if constexpr (sizeof(T) == 2) {
+    if (g.form16 >= 0) return launch_scan16<T>(a, g, prep, state_only, stream);
   }
-  if (prep != nullptr && model_shape(a, g, static_cast<int>(sizeof(T)))) {
-    return launch_kernel<T, R, false, false, true>(a, g, prep, grid, block, stream);
+  const dim3 grid(static_cast<unsigned>(a.batch) * a.heads), block(kThreads);
+  if constexpr (sizeof(T) == 4) {
+    if (full_shape(a, g, R) && prep != nullptr) {
+      return launch_kernel<T, R, true>(a, g, prep, grid, block, stream);
+    }
+    if (prep != nullptr && model_shape(a, g, static_cast<int>(sizeof(T)))) {
+      return launch_kernel<T, R, false, true>(a, g, prep, grid, block, stream);
+    }
   }
   return launch_kernel<T, R, false>(a, g, prep, grid, block, stream);
 }
@@ -3489,7 +2376,7 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
 // Sub-chunk length of a call's geometry.
 static int sub_chunk_tokens(const m3_scan_args& a) {
   ScanGeom g{};
-  ws_layout(a, g);
+  ws_layout(a, g, -1);
   return g.tok;
 }
 
@@ -3518,22 +2405,24 @@ static bool segmentable(const m3_scan_args& a) {
 // and composition cost 0.37 of its second pass (config 5 long); ties go to the smaller G. At
 // config 5 long (24 (b, h) pairs) that is G = 32 alone (3 full rounds; 622 us per call against
 // 689 at G = 8) and G = 16 for its two concurrent directions (1,070 against 1,100 us).
-static bool pow2(int x) { return x > 0 && (x & (x - 1)) == 0; }
-
 static double split_cost(int64_t bhc, int G) {
   const double rounds = static_cast<double>((bhc * G + 255) / 256);
   return G == 1 ? rounds : 1.37 * rounds / G;
 }
 
-// The shapes the chunked MFMA kernel tiles: d_state a power of 2 up to 128, head_dim up to 64,
-// up to 32 angles, ranks 1, 2, 4 and 8. Others take the recurrent scan (rscan.hip).
-static bool tiled_shape(const m3_scan_args& a) {
+// The shapes the chunked MFMA kernels tile: d_state a power of 2 up to 128, head_dim up to 64,
+// up to 32 angles, ranks 1, 2, 4 and 8, and the 16-wave kernel's calls at every d_state it takes
+// (`rows`: its workspace rows are allowed). Others take the recurrent scan (rscan.hip).
+static bool pow2_shape(const m3_scan_args& a) {
   return pow2(a.d_state) && a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
          a.num_angles <= kSMax && (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8);
 }
+static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
+  return pow2_shape(a) || (rows && form16_of(a) >= 0);
+}
 
 static int segments_for(const m3_scan_args& a, int concurrent = 1) {
-  if (!tiled_shape(a)) return a.segments > 1 ? -1 : 1;
+  if (!pow2_shape(a)) return a.segments > 1 ? -1 : 1;
   if (a.segments == 1 || a.length <= 0 || a.batch <= 0) return 1;
   if (a.segments < 0) return -1;
   if (!segmentable(a)) return a.segments > 1 ? -1 : 1;
@@ -3582,7 +2471,7 @@ struct SegPlan {
   size_t o_state, o_decay, o_blk, o_phase, o_k, o_in_state, o_in_phase, o_in_k, o_in_v;
 };
 
-static SegPlan plan_segments(const m3_scan_args& a, int G) {
+static SegPlan plan_segments(const m3_scan_args& a, int G, bool rows) {
   SegPlan sp{};
   m3_scan_args& a1 = sp.a1;
   a1 = a;
@@ -3600,9 +2489,9 @@ static SegPlan plan_segments(const m3_scan_args& a, int G) {
   a1.initial_value = m3_tensor{};
   ScanGeom g1{};
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-  sp.prep_bytes = up(ws_layout(a1, g1));
+  sp.prep_bytes = up(ws_layout(a1, g1, rows ? form16_of(a1) : -1));
   const size_t es = a.act_dtype == M3_F32 ? 4 : 2;
-  const size_t rows = static_cast<size_t>(a1.batch) * a.heads;
+  const size_t pairs = static_cast<size_t>(a1.batch) * a.heads;
   size_t off = sp.prep_bytes;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -3610,15 +2499,15 @@ static SegPlan plan_segments(const m3_scan_args& a, int G) {
     return o;
   };
   const size_t PN = static_cast<size_t>(a.head_dim) * a.d_state;
-  sp.o_state = take(rows * PN * 4);
-  sp.o_decay = take(rows * 4);
-  sp.o_blk = take(rows * ((a1.length + 63) / 64) * a.num_angles * 4);
-  sp.o_phase = take(rows * a.num_angles * 4);
-  sp.o_k = take(rows * a.rank * a.d_state * es);
-  sp.o_in_state = take(rows * PN * 4);
-  sp.o_in_phase = take(rows * a.num_angles * 4);
-  sp.o_in_k = take(rows * a.rank * a.d_state * es);
-  sp.o_in_v = take(rows * a.head_dim * es);
+  sp.o_state = take(pairs * PN * 4);
+  sp.o_decay = take(pairs * 4);
+  sp.o_blk = take(pairs * ((a1.length + 63) / 64) * a.num_angles * 4);
+  sp.o_phase = take(pairs * a.num_angles * 4);
+  sp.o_k = take(pairs * a.rank * a.d_state * es);
+  sp.o_in_state = take(pairs * PN * 4);
+  sp.o_in_phase = take(pairs * a.num_angles * 4);
+  sp.o_in_k = take(pairs * a.rank * a.d_state * es);
+  sp.o_in_v = take(pairs * a.head_dim * es);
   sp.total_bytes = off;
   return sp;
 }
@@ -3626,8 +2515,8 @@ static SegPlan plan_segments(const m3_scan_args& a, int G) {
 // The segmented scan: pass 1 (prep + scan of every segment from zero), the composition, pass 2
 // (scan of every segment from its true start; prep's results are the same and are reused).
 template <typename T, int R>
-static int launch_segmented(const m3_scan_args& a, int G, hipStream_t stream) {
-  SegPlan sp = plan_segments(a, G);
+static int launch_segmented(const m3_scan_args& a, int G, bool rows, hipStream_t stream) {
+  SegPlan sp = plan_segments(a, G, rows);
   if (a.workspace == nullptr || a.workspace_bytes < sp.total_bytes || !aligned16(a.workspace)) {
     return fail(M3_EWORKSPACE, "m3_scan_fwd: needs a 16-byte aligned workspace of %zu bytes",
                 sp.total_bytes);
@@ -3657,7 +2546,7 @@ static int launch_segmented(const m3_scan_args& a, int G, hipStream_t stream) {
   a1.final_phase = m3_tensor{};
   a1.block_phase = angles ? contiguous(sg.seg_blk, M3_F32, {BG, H, sg.nbs, S}) : m3_tensor{};
   a1.final_k = contiguous(sg.seg_k, a.act_dtype, {BG, H, R, N});
-  int rc = launch_pass<T, R>(a1, stream, true, /*state_only=*/true);
+  int rc = launch_pass<T, R>(a1, stream, true, rows, /*state_only=*/true);
   if (rc != M3_OK) return rc;
 
   // at most kMaxSegments x kSMax + 3 kMaxSegments floats: within the default 64 KiB
@@ -3681,7 +2570,7 @@ static int launch_segmented(const m3_scan_args& a, int G, hipStream_t stream) {
   a2.final_k = a1.final_k;
   a2.final_decay = m3_tensor{};
   a2.block_phase = m3_tensor{};
-  rc = launch_pass<T, R>(a2, stream, false);
+  rc = launch_pass<T, R>(a2, stream, false, rows);
   if (rc != M3_OK) return rc;
   hipLaunchKernelGGL((gather_kernel<T, R>), dim3(static_cast<unsigned>(a.batch) * a.heads),
                      dim3(kCompThreads), 0, stream, a, sg);
@@ -3689,7 +2578,7 @@ static int launch_segmented(const m3_scan_args& a, int G, hipStream_t stream) {
 }
 
 template <typename T, int R>
-static int launch_scan_r(const m3_scan_args& a, hipStream_t stream) {
+static int launch_scan_r(const m3_scan_args& a, bool rows, hipStream_t stream) {
   const int G = segments_for(a);
   if (G < 0) {
     return fail(M3_EUNSUPPORTED,
@@ -3697,17 +2586,17 @@ static int launch_scan_r(const m3_scan_args& a, hipStream_t stream) {
                 "64-token blocks (angle phases), and token-major batch rows",
                 a.segments);
   }
-  if (G > 1) return launch_segmented<T, R>(a, G, stream);
-  return launch_pass<T, R>(a, stream, true);
+  if (G > 1) return launch_segmented<T, R>(a, G, rows, stream);
+  return launch_pass<T, R>(a, stream, true, rows);
 }
 
 template <typename T>
-static int launch_scan(const m3_scan_args& a, hipStream_t stream) {
+static int launch_scan(const m3_scan_args& a, bool rows, hipStream_t stream) {
   switch (a.rank) {
-    case 1: return launch_scan_r<T, 1>(a, stream);
-    case 2: return launch_scan_r<T, 2>(a, stream);
-    case 4: return launch_scan_r<T, 4>(a, stream);
-    case 8: return launch_scan_r<T, 8>(a, stream);
+    case 1: return launch_scan_r<T, 1>(a, rows, stream);
+    case 2: return launch_scan_r<T, 2>(a, rows, stream);
+    case 4: return launch_scan_r<T, 4>(a, rows, stream);
+    case 8: return launch_scan_r<T, 8>(a, rows, stream);
     default: return fail(M3_EUNSUPPORTED, "m3_scan_fwd: rank %d not in {1, 2, 4, 8}", a.rank);
   }
 }
@@ -3816,6 +2705,26 @@ static int validate_scan(const m3_scan_args& a) {
   return M3_OK;
 }
 
+size_t scan_need(const m3_scan_args& a, bool rows) {
+  if (!tiled_shape(a, rows)) return 0;  // the recurrent scan needs no workspace
+  const int G = segments_for(a);
+  if (G > 1) return plan_segments(a, G, rows).total_bytes;
+  ScanGeom g{};
+  return ws_layout(a, g, rows ? form16_of(a) : -1);
+}
+
+int scan_run(const m3_scan_args& a, bool rows, hipStream_t stream) {
+  int rc = validate_scan(a);
+  if (rc != M3_OK) return rc;
+  if (a.batch == 0) return M3_OK;
+  if (!tiled_shape(a, rows)) return launch_recurrent_scan(a, stream);
+  switch (a.act_dtype) {
+    case M3_F32: return launch_scan<float>(a, rows, stream);
+    case M3_BF16: return launch_scan<__bf16>(a, rows, stream);
+    default: return launch_scan<_Float16>(a, rows, stream);
+  }
+}
+
 }  // namespace m3
 
 extern "C" int m3_scan_workspace_size(const m3_scan_args* args, size_t* bytes) {
@@ -3823,13 +2732,7 @@ extern "C" int m3_scan_workspace_size(const m3_scan_args* args, size_t* bytes) {
   if (args == nullptr || bytes == nullptr) {
     return m3::fail(M3_EINVAL, "m3_scan_workspace_size: NULL argument");
   }
-  m3::ScanGeom g{};
-  if (!m3::tiled_shape(*args)) {  // the recurrent scan needs no workspace
-    *bytes = 0;
-    return M3_OK;
-  }
-  const int G = m3::segments_for(*args);
-  *bytes = G > 1 ? m3::plan_segments(*args, G).total_bytes : m3::ws_layout(*args, g);
+  *bytes = m3::scan_need(*args, true);
   return M3_OK;
 }
 
@@ -3852,17 +2755,7 @@ extern "C" int m3_scan_segments(const m3_scan_args* args, int concurrent_calls,
 }
 
 extern "C" int m3_scan_fwd(const m3_scan_args* args, hipStream_t stream) {
-  using namespace m3;
-  clear_error();
-  if (args == nullptr) return fail(M3_EINVAL, "m3_scan_fwd: args is NULL");
-  const m3_scan_args& a = *args;
-  int rc = validate_scan(a);
-  if (rc != M3_OK) return rc;
-  if (a.batch == 0) return M3_OK;
-  if (!tiled_shape(a)) return launch_recurrent_scan(a, stream);
-  switch (a.act_dtype) {
-    case M3_F32: return launch_scan<float>(a, stream);
-    case M3_BF16: return launch_scan<__bf16>(a, stream);
-    default: return launch_scan<_Float16>(a, stream);
-  }
+  m3::clear_error();
+  if (args == nullptr) return m3::fail(M3_EINVAL, "m3_scan_fwd: args is NULL");
+  return m3::scan_run(*args, true, stream);
 }

@@ -1,0 +1,169 @@
+"""The 16-wave scan (16-bit activations) at the shapes and layouts it takes beyond the model's
+own: other d_state, head_dim and angle counts, every rank, groups, padded and reversed token
+strides, calls without phases, biases or a start, and the calls at the edges of a sub-chunk.
+
+Each is compared with the oracle run in FP32 on the same 16-bit values. The bar is 2-norm
+relative: the kernel rounds q / k, the decayed weights, the scaled values, the state and the
+output once each to the activation dtype, six roundings of at most u = 2^-9 (bf16) or 2^-12 (f16)
+relative each, and as root of the sum of squares of uniform errors (u / sqrt 3) that is 1.5 u;
+asserted at 3 u for the output and the state.
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from mamba3_amd import Mamba3, _hip, ops
+from oracle import portable as op
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+BAR = {torch.bfloat16: 3 * 2.0 ** -9, torch.float16: 3 * 2.0 ** -12}
+
+
+def _close(got, want, dtype):
+    got, want = got.double().cpu(), want.double()
+    assert got.shape == want.shape
+    err = ((got - want).norm() / want.norm()).item()
+    assert err <= BAR[dtype], f"relative error {err:.3e}"
+
+
+def _inputs(rank, dtype, *, batch, length, heads, groups, head_dim, d_state, angles, bias,
+            initial, seed):
+    g = torch.Generator().manual_seed(seed)
+
+    def rand(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=g) * scale).to(dtype)
+
+    inp = dict(q=rand(batch, length, groups, rank, d_state), k=rand(batch, length, groups, rank, d_state),
+               value=rand(batch, length, heads, head_dim), gate=rand(batch, length, heads, head_dim),
+               dt=torch.rand(batch, length, heads, generator=g) * 0.1 + 0.001,
+               trap_logits=rand(batch, length, heads), D=torch.randn(heads, generator=g))
+    inp["adt"] = -torch.rand(batch, length, heads, generator=g) * inp["dt"] * 3
+    if rank > 1:
+        for name in ("mimo_x", "mimo_z", "mimo_out"):
+            # values of the activation dtype: the kernel rounds mimo_x and mimo_z to it
+            inp[name] = rand(heads, rank, head_dim, scale=0.5).float()
+    if angles:
+        inp["phase"] = (torch.rand(batch, length, heads, angles, generator=g) * 2 - 1) * 6
+        inp["mimo_rotation"] = rank > 1
+    if bias:
+        inp["q_bias"] = (1 + 0.1 * torch.randn(heads, rank, d_state, generator=g)).to(dtype).float()
+        inp["k_bias"] = (1 + 0.1 * torch.randn(heads, rank, d_state, generator=g)).to(dtype).float()
+    if initial:
+        inp["initial_state"] = torch.randn(batch, heads, head_dim, d_state, generator=g) * 0.3
+        inp["initial_k"] = rand(batch, heads, rank, d_state)
+        inp["initial_value"] = rand(batch, heads, head_dim)
+    return inp
+
+
+def _oracle32(inp):
+    return op.ssd_scan(**{n: (t.float() if isinstance(t, torch.Tensor) else t)
+                          for n, t in inp.items()}, chunk_size=16)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank,groups,head_dim,d_state,angles,length,bias,initial", [
+    (1, 1, 64, 128, 32, 64, True, True),     # the model's shape, one full sub-chunk
+    (1, 1, 64, 128, 32, 1, True, True),      # one token
+    (1, 2, 36, 96, 24, 65, True, True),      # odd widths, two groups, one token over
+    (1, 1, 64, 100, 13, 130, True, False),   # d_state no multiple of 8, few angles
+    (1, 1, 4, 4, 1, 63, False, True),        # the narrowest rows
+    (1, 1, 64, 128, 0, 200, False, False),   # no rotation at all
+    (2, 1, 64, 128, 32, 33, True, True),
+    (2, 3, 20, 48, 12, 95, True, True),
+    (4, 1, 64, 64, 16, 17, True, False),
+    (4, 2, 32, 112, 28, 81, False, True),
+    (8, 1, 64, 128, 32, 9, True, True),
+    (8, 1, 16, 16, 4, 40, True, True),
+    (8, 1, 64, 80, 0, 23, True, False),
+])
+def test_hook_form_shapes(rank, groups, head_dim, d_state, angles, length, bias, initial, dtype):
+    inp = _inputs(rank, dtype, batch=2, length=length, heads=6, groups=groups, head_dim=head_dim,
+                  d_state=d_state, angles=angles, bias=bias, initial=initial, seed=length)
+    want, want_state = _oracle32(inp)
+    got, state = ops.mamba3_scan(**{n: (t.to(DEV) if isinstance(t, torch.Tensor) else t)
+                                    for n, t in inp.items()})
+    _close(got, want, dtype)
+    _close(state, want_state, dtype)
+
+
+@pytest.mark.parametrize("layout", ["padded", "head_major", "unaligned"])
+def test_hook_form_layouts(layout):
+    """Rows padded to a longer token stride, q / k and value / gate as slices of one buffer,
+    head-major values (a token stride below the head stride), and rows that start on odd
+    elements (those take the kernel that reads element by element): the same result."""
+    inp = _inputs(2, torch.bfloat16, batch=2, length=70, heads=4, groups=1, head_dim=64,
+                  d_state=128, angles=32, bias=True, initial=True, seed=7)
+    dev = {n: (t.to(DEV) if isinstance(t, torch.Tensor) else t) for n, t in inp.items()}
+    want, want_state = ops.mamba3_scan(**dev)
+
+    def relayout(t, name):
+        if layout == "head_major" and name in ("value", "gate"):
+            return t.transpose(1, 2).contiguous().transpose(1, 2)
+        lead, last = t.shape[:-1], t.shape[-1]
+        off = 1 if layout == "unaligned" else 8
+        wide = torch.full((*lead, last + 16), float("nan"), dtype=t.dtype, device=DEV)
+        wide[..., off:off + last] = t
+        return wide[..., off:off + last]
+
+    for name in ("q", "k", "value", "gate"):
+        dev[name] = relayout(dev[name], name)
+    got, state = ops.mamba3_scan(**dev)
+    _close(got, want.cpu(), torch.bfloat16)
+    _close(state, want_state.cpu(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("rank,d_model,d_state,length,reverse", [
+    (1, 96, 96, 70, False), (1, 40, 96, 129, True), (2, 64, 128, 40, False),
+    (4, 64, 96, 33, True), (8, 96, 128, 20, False), (4, 128, 128, 1, False),
+])
+def test_projection_form_shapes(rank, d_model, d_state, length, reverse):
+    """The model's mixer at widths other than its own: outputs (both directions) and the cache
+    against the oracle's mixer in FP32 on the same bf16 projection."""
+    torch.manual_seed(length)
+    model = Mamba3(d_model, d_state=d_state, depth=1, mimo_rank=rank).eval()
+    params = {n: w.detach().to(torch.bfloat16).float() for n, w in model.state_dict().items()}
+    model.load_state_dict(params)
+    mixer = model.to(DEV).layers[0].mixer
+    width = mixer.in_proj.weight.shape[0]
+    proj = torch.randn(2, length, width).to(torch.bfloat16)
+    src = proj.flip(1) if reverse else proj
+    want, cache = op.mixer_scan(params, "layers.0.mixer.", src.float(),
+                                op.Dims(d_model, d_state, rank), chunk=16)
+    with torch.inference_mode():
+        got, state, phase, k = ops.scan_projection(proj.to(DEV), mixer, want_cache=not reverse,
+                                                   reverse=reverse)
+    _close(got, want.flip(1) if reverse else want, torch.bfloat16)
+    _close(state, cache[1], torch.bfloat16)
+    if not reverse:
+        _close(k, cache[2], torch.bfloat16)
+        turns = (phase.cpu() - cache[0]) / (2 * math.pi)  # whole turns are the same phase
+        assert (turns - turns.round()).abs().max() < 1e-4
+
+
+def test_scan_without_room_for_rows():
+    """m3_scan_fwd_noalloc's calls too large for the q / k rows run on the kernels that keep
+    none: the same result as the workspace call."""
+    torch.manual_seed(3)
+    b, l, h, n, p, r = 20, 1024, 2, 64, 16, 8  # 20 x 1024 x 8 x 2 x 128 x 2 B = 84 MB of rows
+    mk = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)
+    q, k, v, z, tr = mk(b, l, 1, r, n), mk(b, l, 1, r, n), mk(b, l, h, p), mk(b, l, h, p), mk(b, l, h)
+    dt = torch.rand(b, l, h, device=DEV) * 0.1
+    adt, D = -dt, torch.ones(h, device=DEV)
+    mimo = [torch.rand(h, r, p, device=DEV) for _ in range(3)]
+    want, want_state = ops.mamba3_scan(q, k, v, z, adt, dt, tr, D, mimo_x=mimo[0], mimo_z=mimo[1],
+                                       mimo_out=mimo[2])
+    out, state = torch.empty_like(want), torch.empty_like(want_state)
+    args = _hip.ScanArgs(batch=b, length=l, heads=h, groups=1, rank=r, d_state=n, head_dim=p,
+                         chunk=64, act_dtype=_hip.BF16, phase_mode=_hip.PHASE_NONE, segments=1,
+                         norm_eps=1e-5)
+    for name, t in dict(q=q, k=k, value=v, gate=z, dt=dt, a=adt, trap=tr, D=D, mimo_x=mimo[0],
+                        mimo_z=mimo[1], mimo_out=mimo[2], out=out, final_state=state).items():
+        setattr(args, name, _hip.tensor(t))
+    _hip.call("m3_scan_fwd_noalloc", args, DEV)
+    _close(out, want.cpu(), torch.bfloat16)
+    _close(state, want_state.cpu(), torch.bfloat16)
