@@ -334,19 +334,20 @@ struct Feed {
 
 // The scalar block of sub-chunk c of (batch, head) bh (one wave, lane = token): dt, adt, trap
 // from the raw projection or given (model.py:195-198), gamma = dt sigmoid(trap), scale = gamma +
-// dt' (1 - sigmoid(trap')) of the next token, 0 at the last token (ops.py:659-671), the
-// within-chunk cumsum of adt by a wave scan, and the decay products the scan uses.
+// dt' (1 - sigmoid(trap')) of the next token, 0 at the last token (ops.py:659-671) and, `cut`, at
+// the last of a segment (the next segment starts with it as its endpoint term), the within-chunk
+// cumsum of adt by a wave scan, and the decay products the scan uses.
 template <int TOK, int TPT>
 __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __restrict__ o,
                                              int c, int lane, float dt_bias, float dt_in,
                                              float a_in, float tr_in, float dtn_in,
-                                             float trn_in) {
+                                             float trn_in, bool cut) {
   using B = ScBlk<TOK>;
   const int L = a.length;
   const int tb = c * TOK, t = tb + lane;
   const int wn = min(TOK, L - tb);
   const bool tv = lane < wn;
-  const bool nv = lane < TOK && t + 1 < L;
+  const bool nv = lane < TOK && t + 1 < L && !(cut && lane == TOK - 1);
   const bool raw_dt = a.raw_dt != 0;
   float dt = 0.f, adt = 0.f, tr = 0.f;
   if (tv) {
@@ -400,7 +401,7 @@ template <int TOK, int TPT>
 __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* __restrict__ o,
                                                  int c, int lane, bool live, float dt_bias,
                                                  float dt_in, float a_in, float tr_in,
-                                                 float dtn_in, float trn_in) {
+                                                 float dtn_in, float trn_in, bool cut) {
   static_assert(TOK <= 16 && (TOK & (TOK - 1)) == 0, "segments of at most 16 lanes");
   using B = ScBlk<TOK>;
   const int L = a.length;
@@ -408,7 +409,7 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
   const int tb = c * TOK, t = tb + j;
   const int wn = min(TOK, L - tb);
   const bool tv = j < wn;
-  const bool nv = t + 1 < L;
+  const bool nv = t + 1 < L && !(cut && j == TOK - 1);
   const bool raw_dt = a.raw_dt != 0;
   float dt = 0.f, adt = 0.f, tr = 0.f;
   if (tv) {
@@ -713,6 +714,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     const int bc = blk - nb_norm - nb_ang;
     if (bc >= a.batch * g.nsub) return;  // whole workgroups leave together
     const int b = bc / g.nsub, c = bc - b * g.nsub;
+    const bool cut = (c + 1) * TOK % g.seg_len == 0;  // the sub-chunk ends a segment
     constexpr int HG = 32, NE = (TOK + 1) * HG, NIT = (NE + 255) / 256;
     __shared__ float s_in[3][TOK + 1][HG + 1];
     __shared__ float s_db[HG];  // dt_bias of the group's heads
@@ -764,7 +766,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
           scalar_block_seg<TOK, TPT>(
               a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
               c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
-              s_in[0][TOK][hc], s_in[2][TOK][hc]);
+              s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
         }
       } else {
         for (int hh = w; hh < hn; hh += 4) {
@@ -772,7 +774,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
           scalar_block<TOK, TPT>(
               a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
               lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
-              s_in[2][TOK][hh]);
+              s_in[2][TOK][hh], cut);
         }
       }
       __syncthreads();
@@ -817,7 +819,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   const bool angles = FULL || a.phase_mode == M3_PHASE_ANGLES;
   const bool raw_dt = FULL || a.raw_dt != 0;
   const bool mimo_rot = FULL ? (R > 1) : (a.mimo_rotation != 0);
-  const int H = a.heads, L = a.length;
+  const int H = a.heads;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index (wave-uniform)
   const int l16 = lane & 15, lg = lane >> 4;
@@ -829,7 +831,15 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     const int per = gridDim.x >> 3;
     bid = (bid & 7) * per + (bid >> 3);
   }
-  const int b = bid / H, h = bid - b * H;
+  // segment sgi of batch row b (one unless the call is split): tokens tok0 .. tok0 + L - 1, the
+  // row's sub-chunks c0 .. c0 + nsub - 1
+  const int bs = bid / H, h = bid - bs * H;
+  const int b = g.segs > 1 ? bs / g.segs : bs, sgi = bs - b * g.segs;
+  const int tok0 = sgi * g.seg_len, c0 = tok0 / TOK;
+  const int L = min(g.seg_len, a.length - tok0);
+  const int nsub = (L + TOK - 1) / TOK;
+  const bool fin = !g.last_only || sgi == g.segs - 1;
+  const int bo = g.last_only ? b : bs;
   const int grp = h / (H / a.groups);
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -878,7 +888,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     F[Lay::PBASE + s] = 0.f;
     F[Lay::POFF + s] = a.initial_phase.ptr != nullptr
                            ? static_cast<const float*>(a.initial_phase.ptr)
-                                 [b * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
+                                 [bs * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
                                   s * a.initial_phase.stride[2]]
                            : 0.f;
   }
@@ -943,7 +953,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         const int n = 16 * ni + 4 * lg + i;
         if (p < P && n < N) {
           st[k][i] = static_cast<const float*>(a.initial_state.ptr)
-              [b * a.initial_state.stride[0] + h * a.initial_state.stride[1] +
+              [bs * a.initial_state.stride[0] + h * a.initial_state.stride[1] +
                p * a.initial_state.stride[2] + n];
         }
       }
@@ -952,13 +962,16 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   // Endpoint continuation (ops.py:681-686): S += dt_0 (1 - trap_0) sum_r (v_prev mx_r) k_prev_r.
   if (a.initial_k.ptr != nullptr && L > 0) {
     float dt0, adt0;
-    dt_adt(raw_dt, ldx(a.dt.ptr, a.dt.dtype, b * a.dt.stride[0] + h * a.dt.stride[2]),
-           ldx(a.a.ptr, a.a.dtype, b * a.a.stride[0] + h * a.a.stride[2]),
+    dt_adt(raw_dt,
+           ldx(a.dt.ptr, a.dt.dtype,
+               b * a.dt.stride[0] + tok0 * a.dt.stride[1] + h * a.dt.stride[2]),
+           ldx(a.a.ptr, a.a.dtype, b * a.a.stride[0] + tok0 * a.a.stride[1] + h * a.a.stride[2]),
            raw_dt ? ldx(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0]) : 0.f, dt0,
            adt0);
     const float tr0 = sigmoidf(ldx(a.trap.ptr, a.trap.dtype,
-                                   b * a.trap.stride[0] + h * a.trap.stride[2]));
-    const float c0 = dt0 * (1.f - tr0);
+                                   b * a.trap.stride[0] + tok0 * a.trap.stride[1] +
+                                       h * a.trap.stride[2]));
+    const float ce = dt0 * (1.f - tr0);
 #pragma unroll
     for (int k = 0; k < kTiles; ++k) {
       const int u = w + kWaves * k;
@@ -967,7 +980,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       const int p = 16 * pj + l16;
       if (p >= P) continue;
       const float v0 = to_f(static_cast<const T*>(a.initial_value.ptr)
-                                [b * a.initial_value.stride[0] + h * a.initial_value.stride[1] + p]);
+                                [bs * a.initial_value.stride[0] + h * a.initial_value.stride[1] + p]);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int n = 16 * ni + 4 * lg + i;
@@ -979,11 +992,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
                                                                  r * a.mimo_x.stride[1] + p)))
                                  : v0;
           const float k0 = to_f(static_cast<const T*>(a.initial_k.ptr)
-                                    [b * a.initial_k.stride[0] + h * a.initial_k.stride[1] +
+                                    [bs * a.initial_k.stride[0] + h * a.initial_k.stride[1] +
                                      r * a.initial_k.stride[2] + n]);
           outer += pv * k0;
         }
-        st[k][i] += c0 * outer;
+        st[k][i] += ce * outer;
       }
     }
   }
@@ -991,18 +1004,19 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   // ---- per-token reads
   Feed<T, R, FULL, SHAPE> fd;
   fd.init(a, g, prep, b, h, grp, rp, n0, vp, p0, N, P, norm);
-  float* fph = a.final_phase.ptr != nullptr
-                   ? static_cast<float*>(a.final_phase.ptr) + b * a.final_phase.stride[0] +
+  float* fph = a.final_phase.ptr != nullptr && fin
+                   ? static_cast<float*>(a.final_phase.ptr) + bo * a.final_phase.stride[0] +
                          h * a.final_phase.stride[1] + ps * a.final_phase.stride[2]
                    : nullptr;
   float* fblk = a.block_phase.ptr != nullptr
                     ? static_cast<float*>(a.block_phase.ptr) + b * a.block_phase.stride[0] +
-                          h * a.block_phase.stride[1] + ps * a.block_phase.stride[3]
+                          h * a.block_phase.stride[1] + (tok0 >> 6) * a.block_phase.stride[2] +
+                          ps * a.block_phase.stride[3]
                     : nullptr;
   const int64_t blk_stride = a.block_phase.stride[2];
   const __amdgpu_buffer_rsrc_t rs_o =
       make_rsrc(FIX ? const_cast<char*>(g.out_base) + b * g.out_b : nullptr,
-                FIX ? L * (g.out_t < 0 ? -g.out_t : g.out_t) : 0);
+                FIX ? a.length * (g.out_t < 0 ? -g.out_t : g.out_t) : 0);
   T* out_row = nullptr;
   int out_t = 0, o_out = 0;
   if constexpr (FIX) {
@@ -1036,7 +1050,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   uint32_t rq[2][W8], rk[2][W8], rv[2][W4], rz[2][W4];
   float2 side;   // this lane's side word of a coming sub-chunk
   float4 ang;    // this lane's angle word of a coming sub-chunk
-  const int nsub = g.nsub, scw = g.scw;
+  const int scw = g.scw;
   const int side_n = scw + 2 * ROWS;  // floats of a side block
   float* ANG = F + Lay::ANG;
   // angle tile slot (16 bytes) of 4-token group g and angle s: rows of kSMax slots, the angle
@@ -1069,13 +1083,13 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   // c + 1 are computed and the loads of c + 1 (words) and c + 2 (side, angles) are in flight
   // (interval 2). Side blocks and cos / sin tables alternate between two LDS buffers each.
   // prologue: side block and angle tile of 0 to LDS, phases of 0
-  side = fd.side_in(0);
-  ang = fd.ang_in(0);
-  fd.words(0, min(TOK, L), qk_on, vz_on, rq, rk, rv, rz);
+  side = fd.side_in(c0);
+  ang = fd.ang_in(c0);
+  fd.words(tok0, min(TOK, L), qk_on, vz_on, rq, rk, rv, rz);
   if (2 * tid < side_n) *reinterpret_cast<float2*>(scb(0) + 2 * tid) = side;
   ang_store(ang);
-  side = fd.side_in(1);
-  ang = fd.ang_in(1);
+  side = fd.side_in(c0 + 1);
+  ang = fd.ang_in(c0 + 1);
   __syncthreads();
   if (ph_on && nsub > 0) {
     float pa[TPL];
@@ -1287,24 +1301,24 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     // eight waves do not queue all their loads at once.
     auto loads_qk = [&] {
       __builtin_amdgcn_sched_barrier(0);
-      fd.words_qk(t0 + TOK, min(TOK, L - t0 - TOK), qk_on, rq, rk);
+      fd.words_qk(tok0 + t0 + TOK, min(TOK, L - t0 - TOK), qk_on, rq, rk);
       __builtin_amdgcn_sched_barrier(0);
     };
     auto loads_vz = [&] {
       __builtin_amdgcn_sched_barrier(0);
-      fd.words_vz(t0 + TOK, min(TOK, L - t0 - TOK), vz_on, rv, rz);
+      fd.words_vz(tok0 + t0 + TOK, min(TOK, L - t0 - TOK), vz_on, rv, rz);
       __builtin_amdgcn_sched_barrier(0);
     };
     auto loads_side = [&] {
       __builtin_amdgcn_sched_barrier(0);
-      side = fd.side_in(c + 2);
-      ang = fd.ang_in(c + 2);
+      side = fd.side_in(c0 + c + 2);
+      ang = fd.ang_in(c0 + c + 2);
       __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (!FULL && !SHAPE) {
-      if (c + 1 < nsub) fd.words(t0 + TOK, min(TOK, L - t0 - TOK), qk_on, vz_on, rq, rk, rv, rz);
-      side = fd.side_in(c + 2);
-      ang = fd.ang_in(c + 2);
+      if (c + 1 < nsub) fd.words(tok0 + t0 + TOK, min(TOK, L - t0 - TOK), qk_on, vz_on, rq, rk, rv, rz);
+      side = fd.side_in(c0 + c + 2);
+      ang = fd.ang_in(c0 + c + 2);
     }
 
     // (q / k words first: they are waited for first, at the top of the next iteration)
@@ -1544,12 +1558,12 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           // rows of tokens >= L fall outside the buffer extent: the store is dropped
           bstore_quad<T>(y, rs_o,
                          (tq * out_t + o_out + pb * ES) +
-                             __builtin_amdgcn_readfirstlane(t0 * out_t));
+                             __builtin_amdgcn_readfirstlane((tok0 + t0) * out_t));
         } else {
           if (tq < width) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              if (pb + i < P) out_row[(t0 + tq) * out_t + pb + i] = from_f<T>(y[i]);
+              if (pb + i < P) out_row[(tok0 + t0 + tq) * out_t + pb + i] = from_f<T>(y[i]);
             }
           }
         }
@@ -1561,26 +1575,26 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   }
 
   // ---- final k: the biased, rotated k of token L-1, still in Ks from the last sub-chunk
-  if (a.final_k.ptr != nullptr && L > 0) {
+  if (a.final_k.ptr != nullptr && fin) {
     const int tl = (L - 1) - (nsub - 1) * TOK;  // its row in the last sub-chunk
     for (int i = tid; i < R * N; i += kThreads) {
       const int r = i / N, n = i - r * N;
-      static_cast<T*>(a.final_k.ptr)[b * a.final_k.stride[0] + h * a.final_k.stride[1] +
+      static_cast<T*>(a.final_k.ptr)[bo * a.final_k.stride[0] + h * a.final_k.stride[1] +
                                      r * a.final_k.stride[2] + n] =
           Ks[(tl * R + r) * LQ + n];
     }
   }
 
   if (a.final_decay.ptr != nullptr && tid == 0) {
-    static_cast<float*>(a.final_decay.ptr)[b * a.final_decay.stride[0] +
+    static_cast<float*>(a.final_decay.ptr)[bo * a.final_decay.stride[0] +
                                            h * a.final_decay.stride[1]] = log_decay;
   }
   // the last block's increment sum (the earlier blocks' were written as each one ended)
-  if (a.block_phase.ptr != nullptr && rotate && angles && L > 0) {
+  if (a.block_phase.ptr != nullptr && rotate && angles) {
     for (int i = tid; i < S; i += kThreads) {
       static_cast<float*>(a.block_phase.ptr)[b * a.block_phase.stride[0] +
                                              h * a.block_phase.stride[1] +
-                                             ((L - 1) >> 6) * a.block_phase.stride[2] +
+                                             ((tok0 + L - 1) >> 6) * a.block_phase.stride[2] +
                                              i * a.block_phase.stride[3]] = F[Lay::PBASE + i];
     }
   }
@@ -1589,7 +1603,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
   for (int k = 0; k < kTiles; ++k) {
     const int u = w + kWaves * k;
-    if (u >= n_tiles) continue;
+    if (u >= n_tiles || !fin) continue;
     const int ni = u / kPT, pj = u - ni * kPT;
     const int p = 16 * pj + l16;
     if (p >= P) continue;
@@ -1597,7 +1611,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     for (int i = 0; i < 4; ++i) {
       const int n = 16 * ni + 4 * lg + i;
       if (n < N) {
-        static_cast<float*>(a.final_state.ptr)[b * a.final_state.stride[0] +
+        static_cast<float*>(a.final_state.ptr)[bo * a.final_state.stride[0] +
                                                h * a.final_state.stride[1] +
                                                p * a.final_state.stride[2] + n] = st[k][i];
       }
@@ -1608,12 +1622,12 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 
 // ------------------------------------------------------------ segmented scan (composition)
 
-// A sequence split into G equal segments is scanned twice (pass 1: every segment from a zero
-// state and zero phase; pass 2: every segment from its true start), both passes viewing the
-// [B, L] tensors as [B*G, L/G]. Between them, compose_kernel walks each (b, h)'s segments in
-// order. The scan is linear in its initial state and a rotation by phi + psi is the rotation by
-// psi followed by phi, so with pass 1's local end state U_g (built from k rotated by local
-// phases), log-decay l_g = sum adt and last k k_g:
+// A sequence split into G segments is scanned twice (pass 1: every segment from a zero state and
+// zero phase; pass 2: every segment from its true start), each segment a workgroup per head over
+// the row's own tensors and prep results (ScanGeom::segs). Between them, compose_kernel walks
+// each (b, h)'s segments in order. The scan is linear in its initial state and a rotation by
+// phi + psi is the rotation by psi followed by phi, so with pass 1's local end state U_g (built
+// from k rotated by local phases), log-decay l_g = sum adt and last k k_g:
 //   S_{g+1} = e^{l_g} (S_g + c_g sum_r (v_prev mx_r) k_prev_r^T) + U_g Rot(phi_g)^T,
 //   k_prev <- Rot(phi_g) k_g,  v_prev <- v at the segment's last token,
 // where c_g = dt (1 - trap) at the segment's first token (the endpoint continuation the kernel
@@ -1621,22 +1635,21 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 // 64-token blocks, off <- fmod(off + block sum) (segments start on block boundaries), redone
 // from pass 1's block sums: bit for bit the carry the unsplit scan reaches there, the fmod
 // representative (sign) included. Pass 2 then starts segment g from (S_g, phi_g, k_prev,
-// v_prev) exactly as a prefill continued from a cache, and its last segment's final state,
-// phase and k are the call's (gather_kernel).
+// v_prev) exactly as a prefill continued from a cache; its last segment writes the call's final
+// state, phase and k, and its block sums, which do not depend on the carry, are the call's.
 struct SegGeom {
-  int G, Ls, nbs;         // segments per batch row, tokens and 64-token phase blocks per segment
-  float* seg_state;       // [B*G][H][P][N] pass-1 end states, then pass 2's
+  int G, Ls, nblk;        // segments per batch row, tokens per segment, 64-token blocks per row
+  float* seg_state;       // [B*G][H][P][N] pass 1's end states
   float* seg_decay;       // [B*G][H]
-  float* seg_blk;         // [B*G][H][nbs][S] pass 1's phase block sums (phase mode ANGLES)
-  float* seg_phase;       // [B*G][H][S] pass 2's final phases
-  void* seg_k;            // [B*G][H][R][N] last k of pass 1, then of pass 2 (activation dtype)
+  float* seg_blk;         // [B][H][nblk][S] pass 1's phase block sums (phase mode ANGLES)
+  void* seg_k;            // [B*G][H][R][N] pass 1's last k (activation dtype)
   float* in_state;        // [B*G][H][P][N] pass-2 initial states
   float* in_phase;        // [B*G][H][S]
   void* in_k;             // [B*G][H][R][N]
   void* in_v;             // [B*G][H][P]
 };
 
-constexpr int kCompThreads = 256;                         // state-row threads (and gather_kernel's)
+constexpr int kCompThreads = 256;                         // state-row threads
 constexpr int kCompBlock = 64 + kCompThreads;             // compose_kernel: phase walker + state rows
 constexpr int kCompRows = 8;                              // state rows per workgroup
 constexpr int kCompPer = kCompRows * kNPad / kCompThreads;  // state elements per thread
@@ -1717,9 +1730,10 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       if (tid == 0) __hip_atomic_store(&s_ready, g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     publish(0);
-    const int nbs = sg.nbs, gend = G - 1;
-    const int64_t seg_stride = static_cast<int64_t>(H) * nbs * S;  // floats from segment to segment
-    const float* blk = sg.seg_blk + row(0) * nbs * S + tid;
+    // (segments 0 .. G - 2 are whole: nbs blocks each)
+    const int nbs = sg.Ls >> 6, gend = G - 1;
+    const int64_t seg_stride = static_cast<int64_t>(nbs) * S;  // floats from segment to segment
+    const float* blk = sg.seg_blk + static_cast<int64_t>(bh) * sg.nblk * S + tid;
     // batches never cross a segment's end; every load is issued (the last one repeated past a
     // short batch's end) so the waits stay exact
     auto load = [&](float (&buf)[kWalkBatch], int g, int k0) __attribute__((always_inline)) {
@@ -1771,9 +1785,11 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
 
   // ---- waves 1-4: this workgroup's state rows, segment by segment
   const int tb = tid - 64;
-  const int lgN = 31 - __builtin_clz(N);  // d_state is a power of 2 dividing kCompThreads
-  const int RN = np << lgN;               // this workgroup's state elements
-  const int n = tb & (N - 1);             // the thread's column: element e = tb + kCompThreads i
+  // thread tb holds column tb % 2^lgN (2^lgN: N rounded up to a power of 2, which divides
+  // kCompThreads; threads past column N do nothing) of the rows (tb + kCompThreads i) >> lgN
+  const int lgN = N > 1 ? 32 - __builtin_clz(N - 1) : 0;
+  const int n = min(tb & ((1 << lgN) - 1), N - 1);
+  const bool col_on = (tb & ((1 << lgN) - 1)) < N;
   // rotation partner of column n (-1: not rotated), whether n is the pair's first element, and
   // the pair's angle: SISO pairs (2j, 2j+1), j < S; MIMO pairs (j, j + 2S), j < S
   const int S2 = 2 * S;
@@ -1798,15 +1814,19 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
   const T* seg_k = static_cast<const T*>(sg.seg_k);
   const T* value = static_cast<const T*>(a.value.ptr);
   int pl[kCompPer];
+  bool on[kCompPer];
 #pragma unroll
-  for (int i = 0; i < kCompPer; ++i) pl[i] = min(tb + kCompThreads * i, RN - 1) >> lgN;
+  for (int i = 0; i < kCompPer; ++i) {
+    const int p = (tb + kCompThreads * i) >> lgN;
+    on[i] = col_on && p < np;
+    pl[i] = min(p, np - 1);
+  }
 
   // the start: the caller's state, k and value (zero without them)
   float st[kCompPer], vp[kCompPer], kp[R], mxr[R][kCompPer];
 #pragma unroll
   for (int i = 0; i < kCompPer; ++i) {
-    const int e = tb + kCompThreads * i;
-    st[i] = (e < RN && a.initial_state.ptr != nullptr)
+    st[i] = (on[i] && a.initial_state.ptr != nullptr)
                 ? static_cast<const float*>(a.initial_state.ptr)
                       [b * a.initial_state.stride[0] + h * a.initial_state.stride[1] +
                        (p0 + pl[i]) * a.initial_state.stride[2] + n]
@@ -1842,15 +1862,15 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
     const float* U = sg.seg_state + (sh * P + p0) * N;
 #pragma unroll
     for (int i = 0; i < kCompPer; ++i) {
-      ru[d][i] = U[(pl[i] << lgN) + n];
-      rup[d][i] = U[(pl[i] << lgN) + np_n];
+      ru[d][i] = U[pl[i] * N + n];
+      rup[d][i] = U[pl[i] * N + np_n];
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       rk[d][r] = to_f(seg_k[sh * R * N + r * N + n]);
       rkp[d][r] = to_f(seg_k[sh * R * N + r * N + np_n]);
     }
-    const int tl = gc * sg.Ls + sg.Ls - 1;
+    const int tl = min(gc * sg.Ls + sg.Ls, a.length) - 1;
 #pragma unroll
     for (int i = 0; i < kCompPer; ++i) {
       rv[d][i] = to_f(value[b * a.value.stride[0] + tl * a.value.stride[1] +
@@ -1883,8 +1903,7 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       // (1) segment g's start for pass 2
 #pragma unroll
       for (int i = 0; i < kCompPer; ++i) {
-        const int e = tb + kCompThreads * i;
-        if (e < RN) sg.in_state[(sh * P + p0) * N + e] = st[i];
+        if (on[i]) sg.in_state[(sh * P + p0 + pl[i]) * N + n] = st[i];
       }
       if (lead && tb < N) {
 #pragma unroll
@@ -1893,7 +1912,7 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       if (n == 0) {
 #pragma unroll
         for (int i = 0; i < kCompPer; ++i) {
-          if (tb + kCompThreads * i < RN) in_v[sh * P + p0 + pl[i]] = from_f<T>(vp[i]);
+          if (on[i]) in_v[sh * P + p0 + pl[i]] = from_f<T>(vp[i]);
         }
       }
       // the carry at segment g's start, once the walker has published it. The walker is a wave
@@ -1918,7 +1937,7 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       const float c0 = s_c0g[g], dec = s_decg[g];
 #pragma unroll
       for (int i = 0; i < kCompPer; ++i) {
-        if (tb + kCompThreads * i >= RN) continue;
+        if (!on[i]) continue;
         float endpoint = 0.f;
 #pragma unroll
         for (int r = 0; r < R; ++r) endpoint += (R > 1 ? mul_r<T>(vp[i], mxr[r][i]) : vp[i]) * kp[r];
@@ -1935,90 +1954,12 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
     }
   }
 
-  // the call's decay (its final state, phase and k come from pass 2: gather_kernel)
+  // the call's decay (its final state, phase and k come from pass 2)
   if (lead && tb == 0 && a.final_decay.ptr != nullptr) {
     float decay_sum = 0.f;
     for (int g = 0; g < G; ++g) decay_sum += s_draw[g];
     static_cast<float*>(a.final_decay.ptr)[b * a.final_decay.stride[0] +
                                            h * a.final_decay.stride[1]] = decay_sum;
-  }
-}
-
-// The call's final state, phase and k: pass 2's of each batch row's last segment.
-template <typename T, int R>
-__global__ __launch_bounds__(kCompThreads) void gather_kernel(const m3_scan_args a,
-                                                              const SegGeom sg) {
-  const int H = a.heads, N = a.d_state, P = a.head_dim, S = a.num_angles;
-  const int b = blockIdx.x / H, h = blockIdx.x - b * H;
-  const int64_t sh = (static_cast<int64_t>(b) * sg.G + sg.G - 1) * H + h;
-  // the state: every element loaded before any is stored (the compiler cannot tell the two
-  // buffers apart, so a load-store loop would take one round trip per element per thread)
-  {
-    constexpr int kPer = kPPad * kNPad / kCompThreads;
-    const int lgN = 31 - __builtin_clz(N), PN = P * N;
-    const float* src = sg.seg_state + sh * PN;
-    float v[kPer];
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + kCompThreads * u;
-      v[u] = e < PN ? src[e] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + kCompThreads * u;
-      if (e < PN) {
-        static_cast<float*>(a.final_state.ptr)[b * a.final_state.stride[0] +
-                                               h * a.final_state.stride[1] +
-                                               (e >> lgN) * a.final_state.stride[2] +
-                                               (e & (N - 1))] = v[u];
-      }
-    }
-  }
-  if (a.final_phase.ptr != nullptr) {
-    for (int i = threadIdx.x; i < S; i += kCompThreads) {
-      static_cast<float*>(a.final_phase.ptr)[b * a.final_phase.stride[0] +
-                                             h * a.final_phase.stride[1] +
-                                             i * a.final_phase.stride[2]] = sg.seg_phase[sh * S + i];
-    }
-  }
-  if (a.final_k.ptr != nullptr) {
-    for (int i = threadIdx.x; i < R * N; i += kCompThreads) {
-      const int r = i / N, n = i - r * N;
-      static_cast<T*>(a.final_k.ptr)[b * a.final_k.stride[0] + h * a.final_k.stride[1] +
-                                     r * a.final_k.stride[2] + n] =
-          static_cast<const T*>(sg.seg_k)[sh * R * N + i];
-    }
-  }
-  // Segments start on 64-token block boundaries, so block j of segment g is block g * nbs + j
-  // of the sequence, and its increment sum does not depend on the carry: pass 1's sums are the
-  // call's.
-  if (a.block_phase.ptr != nullptr) {
-    // 16 elements per thread loaded, then stored (as the state above)
-    constexpr int kPer = 16;
-    const int nb = sg.G * sg.nbs;
-    for (int e0 = threadIdx.x; e0 < nb * S; e0 += kPer * kCompThreads) {
-      float v[kPer];
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int e = e0 + kCompThreads * u;
-        if (e < nb * S) {
-          const int blk = e / S, i = e - blk * S, g = blk / sg.nbs, j = blk - g * sg.nbs;
-          const int64_t src = ((static_cast<int64_t>(b) * sg.G + g) * H + h) * sg.nbs + j;
-          v[u] = sg.seg_blk[src * S + i];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int e = e0 + kCompThreads * u;
-        if (e < nb * S) {
-          const int blk = e / S, i = e - blk * S;
-          static_cast<float*>(a.block_phase.ptr)[b * a.block_phase.stride[0] +
-                                                 h * a.block_phase.stride[1] +
-                                                 blk * a.block_phase.stride[2] +
-                                                 i * a.block_phase.stride[3]] = v[u];
-        }
-      }
-    }
   }
 }
 
@@ -2131,6 +2072,9 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   g.scw = 5 * g.tok + 8;  // ScBlk<tok>::SIZE
   g.L4 = static_cast<int>((len + 3) / 4);
   g.form16 = form16;
+  g.segs = 1;
+  g.seg_len = static_cast<int>((len + 63) / 64 * 64);
+  g.last_only = 0;
   g.perm = a.phase_mode != M3_PHASE_NONE && a.mimo_rotation != 0;
   g.wlo = !pow2(a.d_state);
   const bool norm = a.q_norm_w.ptr != nullptr && form16 < 0;
@@ -2323,16 +2267,27 @@ static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* 
 }
 
 // One pass: the prep kernel (unless `run_prep` is false: its workspace already holds this
-// geometry's results) and the scan kernel.
-// `state_only`: the caller needs only the end state, decay, last k and phase block sums (the
-// outputs are not written where the state-only kernel form applies: the model's shape, 16-bit).
+// geometry's results) and the scan kernel over `split`'s segments (one per batch row without).
+// `form16`: the call's (form16_of, -1 without the 16-wave kernel; a pass of a split call has the
+// call's own). `state_only`: the caller needs only the end state, decay, last k and phase block sums (the
+// outputs are not written where the kernel has a state-only form).
+struct Split {
+  int segs, seg_len, last_only;
+};
+
 template <typename T, int R>
-static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep, bool rows,
-                       bool state_only = false) {
-  ScanGeom g = make_geom<T>(a, rows ? form16_of(a) : -1);
+static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep, int form16,
+                       const Split* split = nullptr, bool state_only = false) {
+  ScanGeom g = make_geom<T>(a, form16);
+  const size_t need = ws_layout(a, g, g.form16);
+  if (split != nullptr) {
+    g.segs = split->segs;
+    g.seg_len = split->seg_len;
+    g.last_only = split->last_only;
+    g.xcd_map = static_cast<int64_t>(a.batch) * g.segs * a.heads % 8 == 0;
+  }
   static_assert(Layout<T>::BYTES <= 160 * 1024, "LDS layout exceeds 160 KiB");
   const float* prep = nullptr;
-  const size_t need = ws_layout(a, g, g.form16);
   if (need > 0) {
     if (a.workspace == nullptr || a.workspace_bytes < need || !aligned16(a.workspace)) {
       return fail(M3_EWORKSPACE, "m3_scan_fwd: needs a 16-byte aligned workspace of %zu bytes",
@@ -2361,7 +2316,7 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
   if constexpr (sizeof(T) == 2) {
     if (g.form16 >= 0) return launch_scan16<T>(a, g, prep, state_only, stream);
   }
-  const dim3 grid(static_cast<unsigned>(a.batch) * a.heads), block(kThreads);
+  const dim3 grid(static_cast<unsigned>(a.batch) * g.segs * a.heads), block(kThreads);
   if constexpr (sizeof(T) == 4) {
     if (full_shape(a, g, R) && prep != nullptr) {
       return launch_kernel<T, R, true>(a, g, prep, grid, block, stream);
@@ -2380,74 +2335,79 @@ static int sub_chunk_tokens(const m3_scan_args& a) {
   return g.tok;
 }
 
-// Whether the [B, L] tensors can be viewed as [B*G, L/G]: each batch row of every per-token
-// tensor is its L tokens at the token stride.
-static bool segmentable(const m3_scan_args& a) {
-  // one batch row: its stride never matters (also for a call running backwards)
-  const bool one = a.batch == 1;
-  const m3_tensor* ts[] = {&a.q, &a.k, &a.value, &a.gate, &a.dt, &a.a, &a.trap, &a.out};
-  for (const m3_tensor* t : ts) {
-    if (!one && t->stride[0] != static_cast<int64_t>(a.length) * t->stride[1]) return false;
-  }
-  if (!one && a.phase_mode != M3_PHASE_NONE &&
-      a.phase.stride[0] != static_cast<int64_t>(a.length) * a.phase.stride[1]) {
-    return false;
-  }
-  return a.head_dim <= kPPad && a.d_state <= kNPad;
+// Segments a call's sequence is split into (-1: an explicit request that cannot be met) and their
+// length: a multiple of the sub-chunk, and of the 64-token phase blocks with angle increments; the
+// last segment may be shorter.
+//
+// Automatic (segments == 0): the G of least estimated time. With one workgroup per (b, h,
+// segment), a pass takes ceil(B H G c / 256) rounds over the 256 CUs (c calls of this shape
+// sharing the GPU, 1 alone), each of the segment's sub-chunks plus a prologue. In units of a
+// sub-chunk (2.7 us): the state-only first pass takes kStateOnly of the second where it has a
+// form of its own, the prologue kPrologue, the split's extra launches and composition kCompose,
+// kPerSeg per segment and kWalk per 64-token block walked. Up to 8 segments may be as short as 4
+// sub-chunks, more need 8 each (every further segment costs the composition a serial step).
+// A split is taken wherever it is estimated 5% faster.
+constexpr double kStateOnly = 0.53, kPrologue = 0.8, kCompose = 4.5, kPerSeg = 0.11, kWalk = 0.02;
+
+struct Segments {
+  int count, len;
+};
+
+static Segments cut(int64_t len, int64_t unit, int64_t count) {
+  const int64_t ls = (len + count * unit - 1) / (count * unit) * unit;
+  return Segments{static_cast<int>((len + ls - 1) / ls), static_cast<int>(ls)};
 }
 
-// Segments a call's sequence is split into: 1 for none, -1 for an explicit request that cannot
-// be met. Automatic (segments == 0): the G of least estimated time among 1 and the powers of 2
-// from 4 up that cut L into equal segments of at least 8 sub-chunks (whole 64-token phase
-// blocks with angle phases). With one workgroup per (b, h, segment), G segments take
-// ceil(B H G c / 256) rounds over the 256 CUs of 1 / G of the unsplit workgroup's time (c calls
-// of this shape sharing the GPU, 1 alone), times 1.37 for a split, whose state-only first pass
-// and composition cost 0.37 of its second pass (config 5 long); ties go to the smaller G. At
-// config 5 long (24 (b, h) pairs) that is G = 32 alone (3 full rounds; 622 us per call against
-// 689 at G = 8) and G = 16 for its two concurrent directions (1,070 against 1,100 us).
-static double split_cost(int64_t bhc, int G) {
-  const double rounds = static_cast<double>((bhc * G + 255) / 256);
-  return G == 1 ? rounds : 1.37 * rounds / G;
+static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurrent) {
+  const int64_t tok = sub_chunk_tokens(a), len = a.length;
+  const int64_t bh = static_cast<int64_t>(a.batch) * a.heads, bhc = bh * concurrent;
+  auto rounds = [&](int64_t n) { return static_cast<double>((bhc * n + 255) / 256); };
+  const double walk = a.phase_mode == M3_PHASE_ANGLES ? kWalk * static_cast<double>(len / 64) : 0.0;
+  const double so = a.act_dtype == M3_F32 ? 1.0 : kStateOnly;
+  Segments best = cut(len, unit, 1);
+  double best_cost = 0.95 * rounds(1) * (kPrologue + static_cast<double>((len + tok - 1) / tok));
+  for (int n = 2; n <= kMaxSegments && bh * n <= INT32_MAX; ++n) {
+    const Segments s = cut(len, unit, n);
+    if (s.len < (n <= 8 ? 4 : 8) * tok) break;
+    if (s.count != n) continue;
+    const double cost = rounds(n) * (2 * kPrologue + (1.0 + so) * static_cast<double>(s.len / tok)) +
+                        kCompose + kPerSeg * n + walk;
+    if (cost < best_cost * (1.0 - 1e-9)) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 // The shapes the chunked MFMA kernels tile: d_state a power of 2 up to 128, head_dim up to 64,
 // up to 32 angles, ranks 1, 2, 4 and 8, and the 16-wave kernel's calls at every d_state it takes
 // (`rows`: its workspace rows are allowed). Others take the recurrent scan (rscan.hip).
-static bool pow2_shape(const m3_scan_args& a) {
-  return pow2(a.d_state) && a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
-         a.num_angles <= kSMax && (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8);
-}
 static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
-  return pow2_shape(a) || (rows && form16_of(a) >= 0);
+  return (pow2(a.d_state) && a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
+          a.num_angles <= kSMax && (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8)) ||
+         (rows && form16_of(a) >= 0);
 }
 
-static int segments_for(const m3_scan_args& a, int concurrent = 1) {
-  if (!pow2_shape(a)) return a.segments > 1 ? -1 : 1;
-  if (a.segments == 1 || a.length <= 0 || a.batch <= 0) return 1;
-  if (a.segments < 0) return -1;
-  if (!segmentable(a)) return a.segments > 1 ? -1 : 1;
-  const int64_t bh = static_cast<int64_t>(a.batch) * a.heads;
-  // segments start on the 64-token phase blocks (counted from the call's start)
-  const int align = a.phase_mode == M3_PHASE_ANGLES ? 64 : 1;
-  if (a.segments > 1) {
-    const bool ok = a.segments <= kMaxSegments &&
-                    a.length % (static_cast<int64_t>(a.segments) * align) == 0 &&
-                    bh * a.segments <= INT32_MAX;
-    return ok ? a.segments : -1;
-  }
-  const int tok = sub_chunk_tokens(a);
-  const int64_t bhc = bh * (concurrent > 1 ? concurrent : 1);
-  int best = 1;
-  double best_cost = split_cost(bhc, 1);
-  for (int G = 4; G <= kMaxSegments && bh * G <= INT32_MAX; G *= 2) {
-    if (a.length % (static_cast<int64_t>(G) * align) != 0 || a.length / G < 8 * tok) break;
-    const double c = split_cost(bhc, G);
-    if (c < best_cost * (1.0 - 1e-9)) {
-      best = G;
-      best_cost = c;
+static Segments segments_for(const m3_scan_args& a, int concurrent = 1) {
+  const int64_t len = a.length;
+  const Segments one{1, static_cast<int>((len > 0 ? len + 63 : 64) / 64 * 64)};
+  if (!tiled_shape(a)) return a.segments > 1 ? Segments{-1, 0} : one;
+  if (a.segments == 1 || len <= 0 || a.batch <= 0) return one;
+  if (a.segments < 0) return Segments{-1, 0};
+  const int64_t unit = a.phase_mode == M3_PHASE_ANGLES ? 64 : sub_chunk_tokens(a);
+  if (a.segments == 0) return auto_segments(a, unit, concurrent > 1 ? concurrent : 1);
+  // an explicit count divides the sequence (into whole phase blocks), or is the library's own
+  // choice for a few concurrent calls (m3_scan_segments), whose last segment may be shorter
+  const int64_t align = a.phase_mode == M3_PHASE_ANGLES ? 64 : 1;
+  if (a.segments <= kMaxSegments && static_cast<int64_t>(a.batch) * a.heads * a.segments <= INT32_MAX) {
+    if (len % (a.segments * align) == 0) return cut(len, unit, a.segments);
+    for (int c = 1; c <= 4; ++c) {
+      const Segments s = auto_segments(a, unit, c);
+      if (s.count == a.segments) return s;
     }
   }
-  return best;
+  return Segments{-1, 0};
 }
 
 static m3_tensor contiguous(void* p, int dtype, std::initializer_list<int64_t> dims) {
@@ -2463,35 +2423,19 @@ static m3_tensor contiguous(void* p, int dtype, std::initializer_list<int64_t> d
   return t;
 }
 
-// Pass-1 argument block (pointers into the workspace filled in at launch) and the byte offsets
-// of the segment buffers, after the prep region.
+// Byte offsets of the segment buffers, after the prep region.
 struct SegPlan {
-  m3_scan_args a1;
   size_t prep_bytes, total_bytes;
-  size_t o_state, o_decay, o_blk, o_phase, o_k, o_in_state, o_in_phase, o_in_k, o_in_v;
+  size_t o_state, o_decay, o_blk, o_k, o_in_state, o_in_phase, o_in_k, o_in_v;
 };
 
-static SegPlan plan_segments(const m3_scan_args& a, int G, bool rows) {
+static SegPlan plan_segments(const m3_scan_args& a, const Segments& s, bool rows) {
   SegPlan sp{};
-  m3_scan_args& a1 = sp.a1;
-  a1 = a;
-  const int Ls = a.length / G;
-  a1.batch = a.batch * G;
-  a1.length = Ls;
-  a1.segments = 1;
-  for (m3_tensor* t : {&a1.q, &a1.k, &a1.value, &a1.gate, &a1.dt, &a1.a, &a1.trap, &a1.out}) {
-    t->stride[0] = t->stride[1] * Ls;
-  }
-  if (a.phase_mode != M3_PHASE_NONE) a1.phase.stride[0] = a1.phase.stride[1] * Ls;
-  a1.initial_state = m3_tensor{};
-  a1.initial_phase = m3_tensor{};
-  a1.initial_k = m3_tensor{};
-  a1.initial_value = m3_tensor{};
-  ScanGeom g1{};
+  ScanGeom g{};
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-  sp.prep_bytes = up(ws_layout(a1, g1, rows ? form16_of(a1) : -1));
+  sp.prep_bytes = up(ws_layout(a, g, rows ? form16_of(a) : -1));
   const size_t es = a.act_dtype == M3_F32 ? 4 : 2;
-  const size_t pairs = static_cast<size_t>(a1.batch) * a.heads;
+  const size_t pairs = static_cast<size_t>(a.batch) * a.heads, segs = pairs * s.count;
   size_t off = sp.prep_bytes;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -2499,15 +2443,14 @@ static SegPlan plan_segments(const m3_scan_args& a, int G, bool rows) {
     return o;
   };
   const size_t PN = static_cast<size_t>(a.head_dim) * a.d_state;
-  sp.o_state = take(pairs * PN * 4);
-  sp.o_decay = take(pairs * 4);
-  sp.o_blk = take(pairs * ((a1.length + 63) / 64) * a.num_angles * 4);
-  sp.o_phase = take(pairs * a.num_angles * 4);
-  sp.o_k = take(pairs * a.rank * a.d_state * es);
-  sp.o_in_state = take(pairs * PN * 4);
-  sp.o_in_phase = take(pairs * a.num_angles * 4);
-  sp.o_in_k = take(pairs * a.rank * a.d_state * es);
-  sp.o_in_v = take(pairs * a.head_dim * es);
+  sp.o_state = take(segs * PN * 4);
+  sp.o_decay = take(segs * 4);
+  sp.o_blk = take(pairs * ((a.length + 63) / 64) * a.num_angles * 4);
+  sp.o_k = take(segs * a.rank * a.d_state * es);
+  sp.o_in_state = take(segs * PN * 4);
+  sp.o_in_phase = take(segs * a.num_angles * 4);
+  sp.o_in_k = take(segs * a.rank * a.d_state * es);
+  sp.o_in_v = take(segs * a.head_dim * es);
   sp.total_bytes = off;
   return sp;
 }
@@ -2515,42 +2458,49 @@ static SegPlan plan_segments(const m3_scan_args& a, int G, bool rows) {
 // The segmented scan: pass 1 (prep + scan of every segment from zero), the composition, pass 2
 // (scan of every segment from its true start; prep's results are the same and are reused).
 template <typename T, int R>
-static int launch_segmented(const m3_scan_args& a, int G, bool rows, hipStream_t stream) {
-  SegPlan sp = plan_segments(a, G, rows);
+static int launch_segmented(const m3_scan_args& a, const Segments& s, bool rows,
+                            hipStream_t stream) {
+  const SegPlan sp = plan_segments(a, s, rows);
   if (a.workspace == nullptr || a.workspace_bytes < sp.total_bytes || !aligned16(a.workspace)) {
     return fail(M3_EWORKSPACE, "m3_scan_fwd: needs a 16-byte aligned workspace of %zu bytes",
                 sp.total_bytes);
   }
   char* ws = static_cast<char*>(a.workspace);
-  const int64_t BG = sp.a1.batch, H = a.heads, P = a.head_dim, N = a.d_state, S = a.num_angles;
+  const int G = s.count;
+  const int64_t B = a.batch, BG = B * G, H = a.heads, P = a.head_dim, N = a.d_state;
+  const int64_t S = a.num_angles;
   const bool angles = a.phase_mode == M3_PHASE_ANGLES;
   SegGeom sg{};
   sg.G = G;
-  sg.Ls = sp.a1.length;
-  sg.nbs = (sg.Ls + 63) / 64;
+  sg.Ls = s.len;
+  sg.nblk = (a.length + 63) / 64;
   sg.seg_state = reinterpret_cast<float*>(ws + sp.o_state);
   sg.seg_decay = reinterpret_cast<float*>(ws + sp.o_decay);
   sg.seg_blk = reinterpret_cast<float*>(ws + sp.o_blk);
-  sg.seg_phase = reinterpret_cast<float*>(ws + sp.o_phase);
   sg.seg_k = ws + sp.o_k;
   sg.in_state = reinterpret_cast<float*>(ws + sp.o_in_state);
   sg.in_phase = reinterpret_cast<float*>(ws + sp.o_in_phase);
   sg.in_k = ws + sp.o_in_k;
   sg.in_v = ws + sp.o_in_v;
 
-  m3_scan_args a1 = sp.a1;
-  a1.workspace = ws;
+  m3_scan_args a1 = a;
   a1.workspace_bytes = sp.prep_bytes;
+  a1.initial_state = m3_tensor{};
+  a1.initial_phase = m3_tensor{};
+  a1.initial_k = m3_tensor{};
+  a1.initial_value = m3_tensor{};
   a1.final_state = contiguous(sg.seg_state, M3_F32, {BG, H, P, N});
   a1.final_decay = contiguous(sg.seg_decay, M3_F32, {BG, H});
   a1.final_phase = m3_tensor{};
-  a1.block_phase = angles ? contiguous(sg.seg_blk, M3_F32, {BG, H, sg.nbs, S}) : m3_tensor{};
+  a1.block_phase = angles ? contiguous(sg.seg_blk, M3_F32, {B, H, sg.nblk, S}) : m3_tensor{};
   a1.final_k = contiguous(sg.seg_k, a.act_dtype, {BG, H, R, N});
-  int rc = launch_pass<T, R>(a1, stream, true, rows, /*state_only=*/true);
+  const Split first{G, s.len, 0}, second{G, s.len, 1};
+  const int form16 = rows ? form16_of(a) : -1;
+  int rc = launch_pass<T, R>(a1, stream, true, form16, &first, /*state_only=*/true);
   if (rc != M3_OK) return rc;
 
   // at most kMaxSegments x kSMax + 3 kMaxSegments floats: within the default 64 KiB
-  const size_t clds = compose_lds_bytes(G, S);
+  const size_t clds = compose_lds_bytes(G, a.num_angles);
   static_assert(sizeof(float) * (kMaxSegments * kSMax + 3 * kMaxSegments) <= 65536,
                 "compose_kernel's LDS fits the default limit");
   const unsigned row_groups = static_cast<unsigned>((P + kCompRows - 1) / kCompRows);
@@ -2560,34 +2510,27 @@ static int launch_segmented(const m3_scan_args& a, int G, bool rows, hipStream_t
   rc = check_launch("m3_scan_fwd (compose)");
   if (rc != M3_OK) return rc;
 
-  m3_scan_args a2 = a1;
+  m3_scan_args a2 = a;
+  a2.workspace_bytes = sp.prep_bytes;
   a2.initial_state = contiguous(sg.in_state, M3_F32, {BG, H, P, N});
   a2.initial_phase = angles ? contiguous(sg.in_phase, M3_F32, {BG, H, S}) : m3_tensor{};
   a2.initial_k = contiguous(sg.in_k, a.act_dtype, {BG, H, R, N});
   a2.initial_value = contiguous(sg.in_v, a.act_dtype, {BG, H, P});
-  a2.final_state = a1.final_state;
-  a2.final_phase = angles ? contiguous(sg.seg_phase, M3_F32, {BG, H, S}) : m3_tensor{};
-  a2.final_k = a1.final_k;
-  a2.final_decay = m3_tensor{};
-  a2.block_phase = m3_tensor{};
-  rc = launch_pass<T, R>(a2, stream, false, rows);
-  if (rc != M3_OK) return rc;
-  hipLaunchKernelGGL((gather_kernel<T, R>), dim3(static_cast<unsigned>(a.batch) * a.heads),
-                     dim3(kCompThreads), 0, stream, a, sg);
-  return check_launch("m3_scan_fwd (gather)");
+  a2.final_decay = m3_tensor{};  // compose_kernel's
+  return launch_pass<T, R>(a2, stream, false, form16, &second);
 }
 
 template <typename T, int R>
 static int launch_scan_r(const m3_scan_args& a, bool rows, hipStream_t stream) {
-  const int G = segments_for(a);
-  if (G < 0) {
+  const Segments s = segments_for(a);
+  if (s.count < 0) {
     return fail(M3_EUNSUPPORTED,
                 "m3_scan_fwd: %d segments need 1 < segments <= 256 dividing L into whole "
-                "64-token blocks (angle phases), and token-major batch rows",
+                "64-token blocks (angle phases)",
                 a.segments);
   }
-  if (G > 1) return launch_segmented<T, R>(a, G, rows, stream);
-  return launch_pass<T, R>(a, stream, true, rows);
+  if (s.count > 1) return launch_segmented<T, R>(a, s, rows, stream);
+  return launch_pass<T, R>(a, stream, true, rows ? form16_of(a) : -1);
 }
 
 template <typename T>
@@ -2707,8 +2650,8 @@ static int validate_scan(const m3_scan_args& a) {
 
 size_t scan_need(const m3_scan_args& a, bool rows) {
   if (!tiled_shape(a, rows)) return 0;  // the recurrent scan needs no workspace
-  const int G = segments_for(a);
-  if (G > 1) return plan_segments(a, G, rows).total_bytes;
+  const Segments s = segments_for(a);
+  if (s.count > 1) return plan_segments(a, s, rows).total_bytes;
   ScanGeom g{};
   return ws_layout(a, g, rows ? form16_of(a) : -1);
 }
@@ -2745,7 +2688,7 @@ extern "C" int m3_scan_segments(const m3_scan_args* args, int concurrent_calls,
   if (concurrent_calls < 1) {
     return m3::fail(M3_EINVAL, "m3_scan_segments: concurrent_calls must be at least 1");
   }
-  const int G = m3::segments_for(*args, concurrent_calls);
+  const int G = m3::segments_for(*args, concurrent_calls).count;
   if (G < 0) {
     return m3::fail(M3_EUNSUPPORTED, "m3_scan_segments: the requested %d segments cannot be met",
                     args->segments);

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   // phase: PG lanes per angle, TPL tokens per lane, on the first PG / 2 waves (32 angles)
   constexpr int TPL = F == kModel && R == 4 ? 1 : 4;
   constexpr int PG = TOK / TPL, PW = PG * kSMax / 64;
-  const int H = a.heads, L = a.length;
+  const int H = a.heads;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
@@ -129,7 +129,13 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     const int per = gridDim.x >> 3;
     bid = (bid & 7) * per + (bid >> 3);
   }
-  const int b = bid / H, h = bid - b * H;
+  // segment sgi of batch row b (one unless the call is split): tokens tok0 .. tok0 + L - 1, its
+  // sub-chunks from the row's sub-chunk c0 on
+  const int bs = bid / H, h = bid - bs * H;
+  const int b = g.segs > 1 ? bs / g.segs : bs, sgi = bs - b * g.segs;
+  const int tok0 = sgi * g.seg_len, c0 = tok0 / TOK;
+  const int L = min(g.seg_len, a.length - tok0);
+  const int nsub = (L + TOK - 1) / TOK;
   const int GRP = F == kModel ? 1 : a.groups;
   const int grp = F == kModel ? 0 : h / (H / GRP);
   const int perm = F == kModel ? (R > 1 ? 1 : 0) : g.perm;
@@ -173,7 +179,8 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     const int64_t s1 = t.stride[1];
     const int64_t back = s1 < 0 ? (L - 1) * s1 : 0;
     Rows r;
-    r.rs = make_rsrc(static_cast<const char*>(t.ptr) + (b * t.stride[0] + head_off + back) * es,
+    r.rs = make_rsrc(static_cast<const char*>(t.ptr) +
+                         (b * t.stride[0] + tok0 * s1 + head_off + back) * es,
                      static_cast<int>(((L - 1) * (s1 < 0 ? -s1 : s1) + span) * es));
     r.step = static_cast<int>(s1) * es;
     r.o0 = static_cast<int>(-back) * es;
@@ -190,16 +197,17 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   // prep's q / k rows of batch row b: row (token, group, rank) at 2 RB bytes, k after q
   const int tok_qk = GRP * R * 2 * RB;
   const __amdgpu_buffer_rsrc_t rs_qk = make_rsrc(
-      reinterpret_cast<const char*>(prep) + g.ws_qk + static_cast<int64_t>(b) * L * tok_qk,
+      reinterpret_cast<const char*>(prep) + g.ws_qk +
+          (static_cast<int64_t>(b) * a.length + tok0) * tok_qk,
       L * tok_qk);
   // row (token qt / R, rank qt % R) of this group, slot n0 of q; 32 rows on: 32 / R tokens
   const int o_qk = (qt / R) * tok_qk + (grp * R + qr) * 2 * RB + n0 * (ROWF ? 4 : 2);
-  const int nsub = g.nsub, scw = g.scw;
+  const int scw = g.scw;
   // side words (waves 0-3, one float pair per lane): the scalar block
   const int q2 = 2 * tid;
   const bool side_on = q2 < scw;
   const __amdgpu_buffer_rsrc_t rs_s =
-      make_rsrc(prep + g.ws_sc + static_cast<int64_t>(b * H + h) * nsub * scw, nsub * scw * 4);
+      make_rsrc(prep + g.ws_sc + (static_cast<int64_t>(b * H + h) * g.nsub + c0) * scw, nsub * scw * 4);
   const int side_o = side_on ? q2 * 4 : 0;
   const int side_s = scw * 4;
   // angle words: 4 tokens of angle tid % 32 each, in the tile order [TOK / 4][32][4]; prep's
@@ -209,7 +217,8 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   constexpr int kPast = 0x40000000;  // beyond every extent (below 2^30 bytes), also advanced
   const __amdgpu_buffer_rsrc_t rs_a =
       GIVEN ? make_rsrc(nullptr, 0)
-            : make_rsrc(prep + g.ws_ang + static_cast<int64_t>(b) * g.L4 * S * 4, g.L4 * S * 16);
+            : make_rsrc(prep + g.ws_ang + (static_cast<int64_t>(b) * g.L4 + tok0 / 4) * S * 4,
+                        (L + 3) / 4 * S * 16);
   const int ang_o = asl < S ? (agq * S + asl) * 16 : kPast;
   const int ang_s = (TOK / 4) * S * 16;
   const bool phases_in = GIVEN && a.phase_mode == M3_PHASE_GIVEN;
@@ -220,13 +229,18 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
                       ? gx.o0 + 4 * agq * gx.step + asl * static_cast<int>(a.phase.stride[3]) * 4
                       : kPast;
 
-  float* fph = a.final_phase.ptr != nullptr && ph_wave && ps < S
-                   ? static_cast<float*>(a.final_phase.ptr) + b * a.final_phase.stride[0] +
+  // where the end state, phase and k go: the segment's own slots (pass 1 of a split call), or the
+  // call's outputs, written by the last segment alone
+  const bool fin = !g.last_only || sgi == g.segs - 1;
+  const int bo = g.last_only ? b : bs;
+  float* fph = a.final_phase.ptr != nullptr && fin && ph_wave && ps < S
+                   ? static_cast<float*>(a.final_phase.ptr) + bo * a.final_phase.stride[0] +
                          h * a.final_phase.stride[1] + ps * a.final_phase.stride[2]
                    : nullptr;
   float* fblk = a.block_phase.ptr != nullptr && ph_wave && ps < S
                     ? static_cast<float*>(a.block_phase.ptr) + b * a.block_phase.stride[0] +
-                          h * a.block_phase.stride[1] + ps * a.block_phase.stride[3]
+                          h * a.block_phase.stride[1] + (tok0 >> 6) * a.block_phase.stride[2] +
+                          ps * a.block_phase.stride[3]
                     : nullptr;
   const int64_t blk_stride = a.block_phase.stride[2];
 
@@ -364,14 +378,14 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   float po = 0.f;  // the phase carry of angle tid
   if (a.initial_phase.ptr != nullptr && tid < S) {
     po = static_cast<const float*>(a.initial_phase.ptr)
-        [b * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
+        [bs * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
          tid * a.initial_phase.stride[2]];
   }
   // the lane's state elements: offsets of (p, column) in floats, row stride `sp`, and its [P, N]
   // slice's resource (the final state is stored the same way)
-  auto state_rs = [&](const m3_tensor& t) {
+  auto state_rs = [&](const m3_tensor& t, int row) {
     const int sp = static_cast<int>(t.stride[2]);
-    return make_rsrc(static_cast<const float*>(t.ptr) + b * t.stride[0] + h * t.stride[1],
+    return make_rsrc(static_cast<const float*>(t.ptr) + row * t.stride[0] + h * t.stride[1],
                      ((P - 1) * sp + N) * 4);
   };
   auto state_off = [&](int k, int i, int sp) {
@@ -380,7 +394,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   };
   f4 st[2] = {zero4(), zero4()};
   if (a.initial_state.ptr != nullptr) {
-    const __amdgpu_buffer_rsrc_t rs = state_rs(a.initial_state);
+    const __amdgpu_buffer_rsrc_t rs = state_rs(a.initial_state, bs);
     const int sp = static_cast<int>(a.initial_state.stride[2]);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -390,17 +404,19 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   }
   // Endpoint continuation (ops.py:681-686): S += dt_0 (1 - trap_0) sum_r (v_prev mx_r) k_prev_r^T.
   if (a.initial_k.ptr != nullptr) {
-    const RawX dt_r = ldraw(a.dt.ptr, a.dt.dtype, b * a.dt.stride[0] + h * a.dt.stride[2]);
-    const RawX tr_r = ldraw(a.trap.ptr, a.trap.dtype, b * a.trap.stride[0] + h * a.trap.stride[2]);
+    const RawX dt_r = ldraw(a.dt.ptr, a.dt.dtype,
+                            b * a.dt.stride[0] + tok0 * a.dt.stride[1] + h * a.dt.stride[2]);
+    const RawX tr_r = ldraw(a.trap.ptr, a.trap.dtype,
+                            b * a.trap.stride[0] + tok0 * a.trap.stride[1] + h * a.trap.stride[2]);
     const RawX db_r = F == kHook ? RawX{0u, 0u}
                                  : ldraw(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0]);
     const int kr_s = static_cast<int>(a.initial_k.stride[2]);
     const __amdgpu_buffer_rsrc_t rs_v =
-        make_rsrc(static_cast<const T*>(a.initial_value.ptr) + b * a.initial_value.stride[0] +
+        make_rsrc(static_cast<const T*>(a.initial_value.ptr) + bs * a.initial_value.stride[0] +
                       h * a.initial_value.stride[1],
                   P * ES);
     const __amdgpu_buffer_rsrc_t rs_k =
-        make_rsrc(static_cast<const T*>(a.initial_k.ptr) + b * a.initial_k.stride[0] +
+        make_rsrc(static_cast<const T*>(a.initial_k.ptr) + bs * a.initial_k.stride[0] +
                       h * a.initial_k.stride[1],
                   ((R - 1) * kr_s + N) * ES);
     auto b16 = [&](__amdgpu_buffer_rsrc_t r, int i) {
@@ -767,31 +783,31 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   }
 
   // ---- final k: the biased, rotated k rows of token L-1, still in Ks from the last sub-chunk
-  if (a.final_k.ptr != nullptr && L > 0) {
+  if (a.final_k.ptr != nullptr && fin) {
     const int tl = (L - 1) - (nsub - 1) * TOK;
     for (int i = tid; i < R * kNPad; i += k16Threads) {
       const int r = i / kNPad, sl = i - r * kNPad;
       if (sl < N) {
-        static_cast<T*>(a.final_k.ptr)[b * a.final_k.stride[0] + h * a.final_k.stride[1] +
+        static_cast<T*>(a.final_k.ptr)[bo * a.final_k.stride[0] + h * a.final_k.stride[1] +
                                        r * a.final_k.stride[2] + col(sl)] =
             Ks[(tl * R + r) * LQ + sl];
       }
     }
   }
   if (a.final_decay.ptr != nullptr && tid == 0) {
-    static_cast<float*>(a.final_decay.ptr)[b * a.final_decay.stride[0] +
+    static_cast<float*>(a.final_decay.ptr)[bo * a.final_decay.stride[0] +
                                            h * a.final_decay.stride[1]] = log_decay;
   }
-  if (a.block_phase.ptr != nullptr && L > 0) {
+  if (a.block_phase.ptr != nullptr) {
     for (int i = tid; i < S; i += k16Threads) {
       static_cast<float*>(a.block_phase.ptr)[b * a.block_phase.stride[0] +
                                              h * a.block_phase.stride[1] +
-                                             ((L - 1) >> 6) * a.block_phase.stride[2] +
+                                             ((tok0 + L - 1) >> 6) * a.block_phase.stride[2] +
                                              i * a.block_phase.stride[3]] = F_[Ly::PBASE + i];
     }
   }
-  {
-    const __amdgpu_buffer_rsrc_t rs = state_rs(a.final_state);
+  if (fin) {
+    const __amdgpu_buffer_rsrc_t rs = state_rs(a.final_state, bo);
     const int sp = static_cast<int>(a.final_state.stride[2]);
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -843,7 +859,7 @@ static int launch_rank16(const m3_scan_args& a, const ScanGeom& g, const float* 
 template <typename T>
 int launch_scan16(const m3_scan_args& a, const ScanGeom& g, const float* prep, bool state_only,
                   hipStream_t stream) {
-  const unsigned grid = static_cast<unsigned>(a.batch) * a.heads;
+  const unsigned grid = static_cast<unsigned>(a.batch) * g.segs * a.heads;
   switch (a.rank) {
     case 1: return launch_rank16<T, 1>(a, g, prep, state_only, grid, stream);
     case 2: return launch_rank16<T, 2>(a, g, prep, state_only, grid, stream);

@@ -108,6 +108,12 @@ struct ScanGeom {
   // ceil(L / 4)), scalar blocks [B*H][nsub][scw] of `tok`-token sub-chunks
   int64_t ws_norm, ws_ang, ws_sc;
   int L4, tok, nsub, scw;
+  // the call's split: segments per batch row and tokens per segment (the last may be shorter; a
+  // multiple of `tok`, and of 64 with angle increments). One workgroup per (batch, segment,
+  // head); the per-token tensors and prep's results stay the whole row's, the initial_* tensors
+  // are per segment. last_only: the final_* outputs are per batch row and the last segment's
+  // alone (pass 2), else per segment (pass 1).
+  int segs, seg_len, last_only;
   int ws_bytes;  // workspace bytes when below 2^31 (the projection form addresses it in 32 bits)
   // the 16-wave kernel (scan16_kernel): its form (Form16, -1: the call takes another kernel),
   // whether the columns are permuted into slots (the MIMO rotation), and the q / k rows
