@@ -453,9 +453,9 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
 // The first two give each workgroup several rows' loads in flight: with one round trip per
 // workgroup they were bound by workgroup turnover (the scalar blocks' LDS allows 6 workgroups per
 // CU). The scalar blocks, the longest workgroups, are dispatched first.
-//  [.., +nb_sc)  one workgroup per (batch, sub-chunk): the dt / a / trap of its TOK tokens and
-//                the next sub-chunk's first, every head, loaded with consecutive lanes on
-//                consecutive heads (32 heads per pass) into LDS; then one wave per head computes
+//  [.., +nb_sc)  one workgroup per (batch, sub-chunk, head group): the dt / a / trap of its TOK
+//                tokens and the next sub-chunk's first, loaded with consecutive lanes on
+//                consecutive heads (32 heads per pass, or 8 in groups that small) into LDS; then one wave per head computes
 //                that head's scalar block (sub-chunks of 16 tokens or fewer: one 16- or 8-lane
 //                segment per head, 4 or 8 heads per wave).
 // q / k rows per 16-lane group of prep_kernel: 16 for the 16-bit single-rank rows (their fewer,
@@ -470,13 +470,13 @@ constexpr int kAngQuads = 4;  // (4-token group, angle) pairs per lane of prep_k
 template <typename T, int R>
 __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const ScanGeom g,
                                                    float* __restrict__ ws, int nb_norm,
-                                                   int nb_ang) {
+                                                   int nb_ang, int head_groups) {
   // every index below fits 31 bits (checked by the host)
   constexpr int TOK = Mma<T>::ROWS / R, TPT = 16 / R;
   constexpr int kNormRows = norm_rows<T, R>();
   // the longest-running range (scalar blocks) is dispatched first: block ids [0, nb_sc) map to
   // it, the rest to the norm and angle ranges in order
-  const int nb_sc = a.batch * g.nsub;
+  const int nb_sc = a.batch * g.nsub * head_groups;
   const int tid = threadIdx.x;
   const int blk = static_cast<int>(blockIdx.x) < nb_sc ? static_cast<int>(blockIdx.x) + nb_norm + nb_ang
                                                        : static_cast<int>(blockIdx.x) - nb_sc;
@@ -711,13 +711,15 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
       *reinterpret_cast<float4*>(ws + g.ws_ang + 4 * static_cast<int64_t>(quad)) = v;
     }
   } else {
-    const int bc = blk - nb_norm - nb_ang;
+    const int hgi = (blk - nb_norm - nb_ang) % head_groups, bc = (blk - nb_norm - nb_ang) / head_groups;
     if (bc >= a.batch * g.nsub) return;  // whole workgroups leave together
     const int b = bc / g.nsub, c = bc - b * g.nsub;
     const bool cut = (c + 1) * TOK % g.seg_len == 0;  // the sub-chunk ends a segment
-    constexpr int HG = 32, NE = (TOK + 1) * HG, NIT = (NE + 255) / 256;
-    __shared__ float s_in[3][TOK + 1][HG + 1];
-    __shared__ float s_db[HG];  // dt_bias of the group's heads
+    const int hpg = (a.heads + head_groups - 1) / head_groups;  // heads of this workgroup
+    const int h_end = min(a.heads, (hgi + 1) * hpg);
+    constexpr int HG_MAX = 32;
+    __shared__ float s_in[3][TOK + 1][HG_MAX + 1];
+    __shared__ float s_db[HG_MAX];  // dt_bias of the group's heads
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const char* base_dt = static_cast<const char*>(offx(a.dt.ptr, a.dt.dtype, b * a.dt.stride[0]));
     const char* base_a = static_cast<const char*>(offx(a.a.ptr, a.a.dtype, b * a.a.stride[0]));
@@ -726,58 +728,66 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     const int s1_dt = static_cast<int>(a.dt.stride[1]), s2_dt = static_cast<int>(a.dt.stride[2]);
     const int s1_a = static_cast<int>(a.a.stride[1]), s2_a = static_cast<int>(a.a.stride[2]);
     const int s1_tr = static_cast<int>(a.trap.stride[1]), s2_tr = static_cast<int>(a.trap.stride[2]);
-    for (int h0 = 0; h0 < a.heads; h0 += HG) {
-      const int hn = min(HG, a.heads - h0);
-      // raw loads of every element first (clamped to valid tokens / heads), then decode and store
-      RawX rd[NIT], ra[NIT], rt[NIT];
-      // dt_bias with the batch (inside the per-head loop below, after its stores, each head's
-      // load would be a round trip of its own)
-      const RawX rdb = a.raw_dt != 0
-                           ? ldraw(a.dt_bias.ptr, a.dt_bias.dtype,
-                                   (h0 + min(tid & (HG - 1), hn - 1)) * a.dt_bias.stride[0])
-                           : RawX{0u, 0u};
+    auto heads_of = [&](auto hg) {
+      constexpr int HG = decltype(hg)::value, NE = (TOK + 1) * HG, NIT = (NE + 255) / 256;
+      for (int h0 = hgi * hpg; h0 < h_end; h0 += HG) {
+        const int hn = min(HG, h_end - h0);
+        // raw loads of every element first (clamped to valid tokens / heads), then decode and store
+        RawX rd[NIT], ra[NIT], rt[NIT];
+        // dt_bias with the batch (inside the per-head loop below, after its stores, each head's
+        // load would be a round trip of its own)
+        const RawX rdb = a.raw_dt != 0
+                             ? ldraw(a.dt_bias.ptr, a.dt_bias.dtype,
+                                     (h0 + min(tid & (HG - 1), hn - 1)) * a.dt_bias.stride[0])
+                             : RawX{0u, 0u};
 #pragma unroll
-      for (int k = 0; k < NIT; ++k) {
-        const int e = min(tid + 256 * k, NE - 1);
-        const int j = e / HG, hh = e - j * HG;
-        const int t = min(c * TOK + j, L - 1), h = h0 + min(hh, hn - 1);
-        rd[k] = ldraw(base_dt, a.dt.dtype, t * s1_dt + h * s2_dt);
-        ra[k] = ldraw(base_a, a.a.dtype, t * s1_a + h * s2_a);
-        rt[k] = ldraw(base_tr, a.trap.dtype, t * s1_tr + h * s2_tr);
-      }
-#pragma unroll
-      for (int k = 0; k < NIT; ++k) {
-        const int e = tid + 256 * k;
-        if (e < NE) {
+        for (int k = 0; k < NIT; ++k) {
+          const int e = min(tid + 256 * k, NE - 1);
           const int j = e / HG, hh = e - j * HG;
-          s_in[0][j][hh] = decode(rd[k], a.dt.dtype);
-          s_in[1][j][hh] = decode(ra[k], a.a.dtype);
-          s_in[2][j][hh] = decode(rt[k], a.trap.dtype);
+          const int t = min(c * TOK + j, L - 1), h = h0 + min(hh, hn - 1);
+          rd[k] = ldraw(base_dt, a.dt.dtype, t * s1_dt + h * s2_dt);
+          ra[k] = ldraw(base_a, a.a.dtype, t * s1_a + h * s2_a);
+          rt[k] = ldraw(base_tr, a.trap.dtype, t * s1_tr + h * s2_tr);
         }
+#pragma unroll
+        for (int k = 0; k < NIT; ++k) {
+          const int e = tid + 256 * k;
+          if (e < NE) {
+            const int j = e / HG, hh = e - j * HG;
+            s_in[0][j][hh] = decode(rd[k], a.dt.dtype);
+            s_in[1][j][hh] = decode(ra[k], a.a.dtype);
+            s_in[2][j][hh] = decode(rt[k], a.trap.dtype);
+          }
+        }
+        if (tid < HG) s_db[tid] = a.raw_dt != 0 ? decode(rdb, a.dt_bias.dtype) : 0.f;
+        __syncthreads();
+        if constexpr (TOK <= 16) {
+          // 64 / TOK heads per wave (one wave per head would leave most lanes idle)
+          constexpr int HPW = 64 / TOK;
+          const int j = lane & (TOK - 1);
+          for (int hb = w * HPW; hb < hn; hb += 4 * HPW) {
+            const int hh = hb + lane / TOK, hc = min(hh, hn - 1);
+            scalar_block_seg<TOK, TPT>(
+                a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
+                c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
+                s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
+          }
+        } else {
+          for (int hh = w; hh < hn; hh += 4) {
+            const int h = h0 + hh, j = min(lane, TOK - 1);
+            scalar_block<TOK, TPT>(
+                a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
+                lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
+                s_in[2][TOK][hh], cut);
+          }
+        }
+        __syncthreads();
       }
-      if (tid < HG) s_db[tid] = a.raw_dt != 0 ? decode(rdb, a.dt_bias.dtype) : 0.f;
-      __syncthreads();
-      if constexpr (TOK <= 16) {
-        // 64 / TOK heads per wave (one wave per head would leave most lanes idle)
-        constexpr int HPW = 64 / TOK;
-        const int j = lane & (TOK - 1);
-        for (int hb = w * HPW; hb < hn; hb += 4 * HPW) {
-          const int hh = hb + lane / TOK, hc = min(hh, hn - 1);
-          scalar_block_seg<TOK, TPT>(
-              a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
-              c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
-              s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
-        }
-      } else {
-        for (int hh = w; hh < hn; hh += 4) {
-          const int h = h0 + hh, j = min(lane, TOK - 1);
-          scalar_block<TOK, TPT>(
-              a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
-              lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
-              s_in[2][TOK][hh], cut);
-        }
-      }
-      __syncthreads();
+    };
+    if (hpg <= 8) {
+      heads_of(std::integral_constant<int, 8>{});
+    } else {
+      heads_of(std::integral_constant<int, HG_MAX>{});
     }
   }
 }
@@ -1631,11 +1641,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 //   S_{g+1} = e^{l_g} (S_g + c_g sum_r (v_prev mx_r) k_prev_r^T) + U_g Rot(phi_g)^T,
 //   k_prev <- Rot(phi_g) k_g,  v_prev <- v at the segment's last token,
 // where c_g = dt (1 - trap) at the segment's first token (the endpoint continuation the kernel
-// applies to initial_k / initial_value). The phase carry phi is the kernel's own walk over
+// applies to initial_k / initial_value; here it is part of the state pass 2 starts from, whose
+// workgroups then skip it). The phase carry phi is the kernel's own walk over
 // 64-token blocks, off <- fmod(off + block sum) (segments start on block boundaries), redone
 // from pass 1's block sums: bit for bit the carry the unsplit scan reaches there, the fmod
-// representative (sign) included. Pass 2 then starts segment g from (S_g, phi_g, k_prev,
-// v_prev) exactly as a prefill continued from a cache; its last segment writes the call's final
+// representative (sign) included. Pass 2 then starts segment g from S_g and phi_g; its last segment writes the call's final
 // state, phase and k, and its block sums, which do not depend on the carry, are the call's.
 struct SegGeom {
   int G, Ls, nblk;        // segments per batch row, tokens per segment, 64-token blocks per row
@@ -1645,8 +1655,6 @@ struct SegGeom {
   void* seg_k;            // [B*G][H][R][N] pass 1's last k (activation dtype)
   float* in_state;        // [B*G][H][P][N] pass-2 initial states
   float* in_phase;        // [B*G][H][S]
-  void* in_k;             // [B*G][H][R][N]
-  void* in_v;             // [B*G][H][P]
 };
 
 constexpr int kCompThreads = 256;                         // state-row threads
@@ -1691,37 +1699,42 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
   __shared__ int s_ready;          // segments whose starting carry is in s_phig
   auto row = [&](int g) { return (static_cast<int64_t>(b) * G + g) * H + h; };
 
-  // per segment, in parallel: the endpoint coefficient and the decay
-  {
-    const float dtb = raw_dt ? ldx(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0]) : 0.f;
-    for (int g = tid; g < G; g += kCompBlock) {
-      const int t0 = g * sg.Ls;
+  // per segment, in parallel: the endpoint coefficient and the decay (raw loads of segment tid,
+  // decoded after the other loads are out)
+  const int gc0 = min(tid, G - 1);
+  const int64_t tc0 = static_cast<int64_t>(gc0) * sg.Ls;
+  const RawX dt_r = ldraw(a.dt.ptr, a.dt.dtype,
+                          b * a.dt.stride[0] + tc0 * a.dt.stride[1] + h * a.dt.stride[2]);
+  const RawX tr_r = ldraw(a.trap.ptr, a.trap.dtype,
+                          b * a.trap.stride[0] + tc0 * a.trap.stride[1] + h * a.trap.stride[2]);
+  const RawX db_r = raw_dt ? ldraw(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0])
+                           : RawX{0u, 0u};
+  const float lg_dec = sg.seg_decay[row(gc0)];
+  static_assert(kMaxSegments <= kCompBlock, "a thread per segment");
+  auto coefficients = [&]() __attribute__((always_inline)) {
+    if (tid < G) {
       float dt0, adt0;
-      dt_adt(raw_dt, ldx(a.dt.ptr, a.dt.dtype,
-                         b * a.dt.stride[0] + t0 * a.dt.stride[1] + h * a.dt.stride[2]),
-             ldx(a.a.ptr, a.a.dtype, b * a.a.stride[0] + t0 * a.a.stride[1] + h * a.a.stride[2]),
-             dtb, dt0, adt0);
-      s_c0g[g] = dt0 * (1.f - sigmoidf(ldx(a.trap.ptr, a.trap.dtype,
-                                           b * a.trap.stride[0] + t0 * a.trap.stride[1] +
-                                               h * a.trap.stride[2])));
-      const float l = sg.seg_decay[row(g)];
-      s_draw[g] = l;
-      s_decg[g] = expf(l);
+      dt_adt(raw_dt, decode(dt_r, a.dt.dtype), 0.f, raw_dt ? decode(db_r, a.dt_bias.dtype) : 0.f, dt0,
+             adt0);
+      s_c0g[tid] = dt0 * (1.f - sigmoidf(decode(tr_r, a.trap.dtype)));
+      s_draw[tid] = lg_dec;
+      s_decg[tid] = expf(lg_dec);
     }
-  }
-  if (tid == 0) s_ready = walk ? 0 : G;
-  __syncthreads();
+    if (tid == 0) s_ready = walk ? 0 : G;
+    __syncthreads();
+  };
 
   if (tid < 64) {
     // ---- wave 0: the phase carry, the kernel's own recurrence off <- fmod(off + block sum)
     // over the blocks of segments 0 .. G-2 in order, published at each segment's start. Lanes
     // s < S walk angle s; block sums are loaded a batch ahead of the fmod chain.
-    if (!walk || tid >= S) return;
+    const bool walker = walk && tid < S;
+    const int tw = walker ? tid : 0;  // lanes without an angle load angle 0 and do nothing else
     float off = 0.f;
-    if (a.initial_phase.ptr != nullptr) {
+    if (a.initial_phase.ptr != nullptr && walk) {
       off = static_cast<const float*>(a.initial_phase.ptr)
           [b * a.initial_phase.stride[0] + h * a.initial_phase.stride[1] +
-           tid * a.initial_phase.stride[2]];
+           tw * a.initial_phase.stride[2]];
     }
     auto publish = [&](int g) __attribute__((always_inline)) {
       s_phig[g * S + tid] = off;
@@ -1729,11 +1742,10 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       __atomic_signal_fence(__ATOMIC_SEQ_CST);
       if (tid == 0) __hip_atomic_store(&s_ready, g + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
-    publish(0);
     // (segments 0 .. G - 2 are whole: nbs blocks each)
     const int nbs = sg.Ls >> 6, gend = G - 1;
     const int64_t seg_stride = static_cast<int64_t>(nbs) * S;  // floats from segment to segment
-    const float* blk = sg.seg_blk + static_cast<int64_t>(bh) * sg.nblk * S + tid;
+    const float* blk = sg.seg_blk + static_cast<int64_t>(bh) * sg.nblk * S + tw;
     // batches never cross a segment's end; every load is issued (the last one repeated past a
     // short batch's end) so the waits stay exact
     auto load = [&](float (&buf)[kWalkBatch], int g, int k0) __attribute__((always_inline)) {
@@ -1759,10 +1771,13 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       }
       if (k0 + n == nbs) publish(g + 1);  // segment g walked: the carry at segment g + 1's start
     };
+    float bufA[kWalkBatch], bufB[kWalkBatch];
+    int gA = 0, kA = 0;
+    if (walk && gend > 0) load(bufA, gA, kA);
+    coefficients();
+    if (!walker) return;
+    publish(0);
     if (gend > 0) {
-      float bufA[kWalkBatch], bufB[kWalkBatch];
-      int gA = 0, kA = 0;
-      load(bufA, gA, kA);
       for (;;) {
         int gB = gA, kB = kA;
         advance(gB, kB);
@@ -1809,8 +1824,6 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
   auto rot = [&](float x, float xp, float c, float sn) {
     return lo ? x * c - xp * sn : xp * sn + x * c;
   };
-  T* in_k = static_cast<T*>(sg.in_k);
-  T* in_v = static_cast<T*>(sg.in_v);
   const T* seg_k = static_cast<const T*>(sg.seg_k);
   const T* value = static_cast<const T*>(a.value.ptr);
   int pl[kCompPer];
@@ -1879,6 +1892,7 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) fetch(d, d);
+  coefficients();
 
   for (int g0 = 0; g0 < G; g0 += D) {
 #pragma unroll
@@ -1900,20 +1914,15 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
       }
       fetch(d, g + D);
 
-      // (1) segment g's start for pass 2
+      // (1) segment g's start for pass 2: the state with the endpoint term (ops.py:681-686)
+      const float c0 = s_c0g[g], dec = s_decg[g];
 #pragma unroll
       for (int i = 0; i < kCompPer; ++i) {
+        float endpoint = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) endpoint += (R > 1 ? mul_r<T>(vp[i], mxr[r][i]) : vp[i]) * kp[r];
+        st[i] += c0 * endpoint;
         if (on[i]) sg.in_state[(sh * P + p0 + pl[i]) * N + n] = st[i];
-      }
-      if (lead && tb < N) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) in_k[sh * R * N + r * N + n] = from_f<T>(kp[r]);
-      }
-      if (n == 0) {
-#pragma unroll
-        for (int i = 0; i < kCompPer; ++i) {
-          if (on[i]) in_v[sh * P + p0 + pl[i]] = from_f<T>(vp[i]);
-        }
       }
       // the carry at segment g's start, once the walker has published it. The walker is a wave
       // of this workgroup (resident with it) and publishes every segment without waiting on
@@ -1933,16 +1942,10 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
         if (lead && tb < S) sg.in_phase[sh * S + tb] = s_phig[g * S + tb];
       }
 
-      // (2) the state at the segment's end: e^l (S + c0 sum_r (v_prev mx_r) k_prev_r^T) + Rot U
-      const float c0 = s_c0g[g], dec = s_decg[g];
+      // (2) the state at the segment's end: e^l S + Rot U
 #pragma unroll
       for (int i = 0; i < kCompPer; ++i) {
-        if (!on[i]) continue;
-        float endpoint = 0.f;
-#pragma unroll
-        for (int r = 0; r < R; ++r) endpoint += (R > 1 ? mul_r<T>(vp[i], mxr[r][i]) : vp[i]) * kp[r];
-        const float uu = part >= 0 ? rot(u[i], up[i], cs, sn) : u[i];
-        st[i] = dec * (st[i] + c0 * endpoint) + uu;
+        if (on[i]) st[i] = dec * st[i] + (part >= 0 ? rot(u[i], up[i], cs, sn) : u[i]);
       }
       // (3) the next segment's endpoint: this segment's last k, rotated by its carry, and value
 #pragma unroll
@@ -2297,7 +2300,13 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
     const int64_t tokens = static_cast<int64_t>(a.batch) * a.length;
     const int64_t nrow = g.ws_norm >= 0 || g.form16 >= 0 ? tokens * 2 * a.groups * a.rank : 0;
     const int64_t ang = g.ws_ang >= 0 ? static_cast<int64_t>(a.batch) * g.L4 * a.num_angles * 4 : 0;
-    const int64_t blocks = static_cast<int64_t>(a.batch) * g.nsub;  // scalar-block workgroups
+    // scalar-block workgroups: one per sub-chunk and group of heads. A call of many sub-chunks
+    // fills the GPU with all its heads in one group (8 heads each there, 4 times the workgroups,
+    // took 33 -> 44 us at 1024 sub-chunks); one of few is a chain of one workgroup's loads and
+    // scans, which groups of 8 heads shorten (28 sub-chunks of 64 heads: prep 15.5 -> 13.0 us)
+    const int64_t subs = static_cast<int64_t>(a.batch) * g.nsub;
+    const int head_groups = (a.heads + 31) / 32 * subs < 256 ? (a.heads + 7) / 8 : 1;
+    const int64_t blocks = subs * head_groups;
     if (nrow >= INT32_MAX || ang >= INT32_MAX || blocks >= INT32_MAX || tokens >= INT32_MAX) {
       return fail(M3_EUNSUPPORTED, "m3_scan_fwd: too many tokens for one launch");
     }
@@ -2308,7 +2317,7 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
       const dim3 pgrid(static_cast<unsigned>(nb_norm + nb_ang + nb_sc)), pblock(256);
       hipLaunchKernelGGL((prep_kernel<T, R>), pgrid, pblock, 0, stream, a, g,
                          static_cast<float*>(a.workspace), static_cast<int>(nb_norm),
-                         static_cast<int>(nb_ang));
+                         static_cast<int>(nb_ang), head_groups);
       int rc = check_launch("m3_scan_fwd (prep)");
       if (rc != M3_OK) return rc;
     }
@@ -2343,11 +2352,16 @@ static int sub_chunk_tokens(const m3_scan_args& a) {
 // segment), a pass takes ceil(B H G c / 256) rounds over the 256 CUs (c calls of this shape
 // sharing the GPU, 1 alone), each of the segment's sub-chunks plus a prologue. In units of a
 // sub-chunk (2.7 us): the state-only first pass takes kStateOnly of the second where it has a
-// form of its own, the prologue kPrologue, the split's extra launches and composition kCompose,
-// kPerSeg per segment and kWalk per 64-token block walked. Up to 8 segments may be as short as 4
-// sub-chunks, more need 8 each (every further segment costs the composition a serial step).
-// A split is taken wherever it is estimated 5% faster.
-constexpr double kStateOnly = 0.53, kPrologue = 0.8, kCompose = 4.5, kPerSeg = 0.11, kWalk = 0.02;
+// form of its own, a workgroup's start kPrologue (with phases; without them less), the split's
+// extra launches and composition kCompose, kPerSeg per segment and kWalk per 64-token block
+// walked. A further segment is a serial step of the composition, so more than a few must be
+// longer: 16-bit segments of 4 sub-chunks up to 8 segments, else 8; FP32's (three times as long a
+// sub-chunk) 2 up to 16, else 4. Measured (bf16, angle increments, graph-timed, us):
+//   1 x 1792, 64 heads:  unsplit 91, G = 2 93, 4 71, 7 87     1 x 1792, 32 heads: 90; 4 67, 7 59, 14 73
+//   1 x 8192, 32 heads:  348; 4 170, 8 110, 16 124            3 x 3072, 24 heads: 144; 2 138, 3 109, 6 122
+//   1 x 61440, 24 heads: 2528; 8 596, 10 500, 16 609, 32 506  4 x 2048, 32 heads: 104; 2 112
+//   1 x 512, 64 heads:   38; 2 52, 4 52                       FP32 2 x 1024, 8 heads: 240; 4 149, 8 100, 16 84
+constexpr double kStateOnly = 0.53, kCompose = 4.5, kPerSeg = 0.11, kWalk = 0.02;
 
 struct Segments {
   int count, len;
@@ -2363,14 +2377,17 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
   const int64_t bh = static_cast<int64_t>(a.batch) * a.heads, bhc = bh * concurrent;
   auto rounds = [&](int64_t n) { return static_cast<double>((bhc * n + 255) / 256); };
   const double walk = a.phase_mode == M3_PHASE_ANGLES ? kWalk * static_cast<double>(len / 64) : 0.0;
-  const double so = a.act_dtype == M3_F32 ? 1.0 : kStateOnly;
+  const bool f32 = a.act_dtype == M3_F32;
+  const double so = f32 ? 1.0 : kStateOnly;
+  const double prologue = a.phase_mode == M3_PHASE_NONE ? 0.8 : 3.0;
   Segments best = cut(len, unit, 1);
-  double best_cost = 0.95 * rounds(1) * (kPrologue + static_cast<double>((len + tok - 1) / tok));
+  double best_cost = 0.95 * rounds(1) * (prologue + static_cast<double>((len + tok - 1) / tok));
   for (int n = 2; n <= kMaxSegments && bh * n <= INT32_MAX; ++n) {
     const Segments s = cut(len, unit, n);
-    if (s.len < (n <= 8 ? 4 : 8) * tok) break;
+    const int shortest = f32 ? (n <= 16 ? 2 : 4) : (n <= 8 ? 4 : 8);
+    if (s.len < shortest * tok) break;
     if (s.count != n) continue;
-    const double cost = rounds(n) * (2 * kPrologue + (1.0 + so) * static_cast<double>(s.len / tok)) +
+    const double cost = rounds(n) * (2 * prologue + (1.0 + so) * static_cast<double>(s.len / tok)) +
                         kCompose + kPerSeg * n + walk;
     if (cost < best_cost * (1.0 - 1e-9)) {
       best = s;
@@ -2426,7 +2443,7 @@ static m3_tensor contiguous(void* p, int dtype, std::initializer_list<int64_t> d
 // Byte offsets of the segment buffers, after the prep region.
 struct SegPlan {
   size_t prep_bytes, total_bytes;
-  size_t o_state, o_decay, o_blk, o_k, o_in_state, o_in_phase, o_in_k, o_in_v;
+  size_t o_state, o_decay, o_blk, o_k, o_in_state, o_in_phase;
 };
 
 static SegPlan plan_segments(const m3_scan_args& a, const Segments& s, bool rows) {
@@ -2449,8 +2466,6 @@ static SegPlan plan_segments(const m3_scan_args& a, const Segments& s, bool rows
   sp.o_k = take(segs * a.rank * a.d_state * es);
   sp.o_in_state = take(segs * PN * 4);
   sp.o_in_phase = take(segs * a.num_angles * 4);
-  sp.o_in_k = take(segs * a.rank * a.d_state * es);
-  sp.o_in_v = take(segs * a.head_dim * es);
   sp.total_bytes = off;
   return sp;
 }
@@ -2480,8 +2495,6 @@ static int launch_segmented(const m3_scan_args& a, const Segments& s, bool rows,
   sg.seg_k = ws + sp.o_k;
   sg.in_state = reinterpret_cast<float*>(ws + sp.o_in_state);
   sg.in_phase = reinterpret_cast<float*>(ws + sp.o_in_phase);
-  sg.in_k = ws + sp.o_in_k;
-  sg.in_v = ws + sp.o_in_v;
 
   m3_scan_args a1 = a;
   a1.workspace_bytes = sp.prep_bytes;
@@ -2514,8 +2527,8 @@ static int launch_segmented(const m3_scan_args& a, const Segments& s, bool rows,
   a2.workspace_bytes = sp.prep_bytes;
   a2.initial_state = contiguous(sg.in_state, M3_F32, {BG, H, P, N});
   a2.initial_phase = angles ? contiguous(sg.in_phase, M3_F32, {BG, H, S}) : m3_tensor{};
-  a2.initial_k = contiguous(sg.in_k, a.act_dtype, {BG, H, R, N});
-  a2.initial_value = contiguous(sg.in_v, a.act_dtype, {BG, H, P});
+  a2.initial_k = m3_tensor{};  // (in in_state)
+  a2.initial_value = m3_tensor{};
   a2.final_decay = m3_tensor{};  // compose_kernel's
   return launch_pass<T, R>(a2, stream, false, form16, &second);
 }
