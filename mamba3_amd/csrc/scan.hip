@@ -56,6 +56,7 @@ struct Feed {
   static constexpr int ES = sizeof(T), W8 = Words<T>::W8, W4 = Words<T>::W4;
   static constexpr int ROWS = Mma<T>::ROWS, TOK = ROWS / R;
   static constexpr int VJ = R == 1 ? 2 : 1;  // value / gate tokens per lane
+  static constexpr int kPast = 0x7f000000;   // beyond the workspace (below 2^30 bytes there)
   // FULL
   __amdgpu_buffer_rsrc_t rs_p, rs_w;
   int o_qk, o_vz, d_q1, d_k, d_z, tok_b;  // per-lane byte offsets at token 0, uniform deltas
@@ -71,6 +72,7 @@ struct Feed {
   int64_t side_ps, ang_ps;      // per-sub-chunk strides (floats)
   int q_t, q_r, k_t, k_r, v_t, z_t, ph_t, ph_s, qk_n, vz_n;
   int side_tok, side_lim;       // norm words: token of the word (sub-chunk 0), last valid
+  int ang_grp;                  // angle words: 4-token group of the word (sub-chunk 0)
   bool vec_qk, vec_vz, given;
   int rp, vp, nsub, L, S, L4;
 
@@ -90,6 +92,10 @@ struct Feed {
     const int q2 = 2 * tid;
     const int64_t sc0 = g.ws_sc + static_cast<int64_t>(b * H + h) * nsub * scw + q2;
     const int nrow = (q2 - scw) >> 1;  // norm word: row of the sub-chunk (token nrow / R)
+    // FULL, BUF: the norm word's token at sub-chunk 0 (other words: none) and the angle word's
+    // 4-token group; past the row's end they are not the row's any more and read as zero
+    side_tok = q2 >= scw ? nrow / R : INT32_MIN / 2;
+    ang_grp = tid / max(S, 1);
     if constexpr (FULL) {
       tok_b = g.tok_b;
       rs_p = make_rsrc(g.proj + b * g.proj_b, L * (tok_b < 0 ? -tok_b : tok_b));
@@ -279,8 +285,8 @@ struct Feed {
   // this lane's side word of sub-chunk c (FULL: unconditional; unused words read anything)
   __device__ __forceinline__ float2 side_in(int c) const {
     if constexpr (FULL || BUF) {
-      const u32x2 v = __builtin_bit_cast(
-          u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, side_o + c * side_s, 0, 0));
+      const int o = side_tok + c * TOK < L ? side_o + c * side_s : kPast;
+      const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_w, o, 0, 0));
       return make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
     } else {
       float2 v = make_float2(1.f, 1.f);
@@ -302,8 +308,8 @@ struct Feed {
       }
     }
     if constexpr (FULL || BUF) {
-      const u32x4 v = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_w, ang_o + c * ang_s, 0, 0));
+      const int o = ang_grp + c * (TOK / 4) < L4 ? ang_o + c * ang_s : kPast;
+      const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_w, o, 0, 0));
       return make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
                          __uint_as_float(v[3]));
     } else {
@@ -796,7 +802,12 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
 // model's shape (N = 128, P = 64, 32 angles when rotating, aligned 16-byte rows) with the generic inputs (the hook form): the dimensions and the vector-load
 // choice are compile-time constants, the features stay runtime; every read and the output go
 // through buffer resources at per-lane offsets, issued unconditionally as in the FULL form.
-template <typename T, int R, bool FULL, bool SHAPE = false>
+//
+// SO (state only, FP32): the segmented scan's first pass, which needs the end state, log decay,
+// last k and phase block sums but no outputs: the stores of Qs, VR, ZR, Sb and the output are left
+// out, and with them (dead code) the q math, the scores, the decay weights, the intra and inter
+// products and the epilogue.
+template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, const ScanGeom g,
                                                         const float* __restrict__ prep) {
   using M = Mma<T>;
@@ -806,7 +817,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   constexpr int WPR = kWaves / RT;     // waves sharing one query row tile
   constexpr int TOK = ROWS / R;        // tokens per sub-chunk
   constexpr bool F32 = sizeof(T) == 4;
-  static_assert(F32 || !(FULL || SHAPE), "16-bit calls of the model's shapes take scan16_kernel");
+  static_assert(F32 || !(FULL || SHAPE || SO), "16-bit calls of those forms take scan16_kernel");
   constexpr int ES = sizeof(T);
   constexpr int LQ = Lay::LQ, LR = Lay::LR, LP = Lay::LP, NP = kNPad, CST = Lay::CST;
   using SB_ = ScBlk<TOK>;
@@ -869,8 +880,9 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   const int rp = tid >> 4, n0 = 8 * (tid & 15);
   const bool qk_on = rp < ROWS / 2 && n0 < N;
   // v / z: row pair vp (rows 2vp, 2vp+1; tokens 2vp, 2vp+1 for R = 1), columns p0 .. p0+3
+  // (FP32's 32 rows are 256 lanes' work each: q / k on waves 0-3, value / gate on waves 4-7)
   constexpr int P4 = kPPad / 4;
-  const int vp = tid / P4, p0 = 4 * (tid % P4);
+  const int vp = (F32 ? tid ^ 256 : tid) / P4, p0 = 4 * (tid % P4);
   const bool vz_on = 2 * vp < TOK * R && p0 < P;
   // phase: angle ps, token group pg (tokens TPL pg .. TPL pg + TPL-1)
   const int pg = tid % PG, ps = tid / PG;
@@ -1143,27 +1155,37 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           q[i] = fmaf(raw_get<T>(rq[j], i), fq[j] * wq[i], bq[R == 1 ? 0 : j][i]);
           k[i] = fmaf(raw_get<T>(rk[j], i), fk[j] * wk[i], bk[R == 1 ? 0 : j][i]);
         }
-        if (rotate) {
-          // x' = x cos + sgn partner sin: SISO pairs (2j, 2j+1), MIMO pairs (n, n + N/2)
+        if (rotate && !mimo_rot) {
+          // pairs (2j, 2j+1): one cos / sin per pair (cos 1, sin 0 past the call's angles)
+#pragma unroll
+          for (int pp = 0; pp < 4; ++pp) {
+            const float2 cs = *reinterpret_cast<const float2*>(CSt + tt * CST + 2 * rcol[2 * pp]);
+            const bool on = rsgn[2 * pp] != 0.f;
+            const float cc = on ? cs.x : 1.f, ss = on ? cs.y : 0.f;
+            const float q0 = q[2 * pp], q1 = q[2 * pp + 1], k0 = k[2 * pp], k1 = k[2 * pp + 1];
+            q[2 * pp] = fmaf(q1, -ss, q0 * cc);
+            q[2 * pp + 1] = fmaf(q0, ss, q1 * cc);
+            k[2 * pp] = fmaf(k1, -ss, k0 * cc);
+            k[2 * pp + 1] = fmaf(k0, ss, k1 * cc);
+          }
+        } else if (rotate) {
+          // x' = x cos + sgn partner sin: MIMO pairs (n, n + N/2)
           float qp[8], kp[8];
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            if (!mimo_rot) {
-              qp[i] = q[i ^ 1];
-              kp[i] = k[i ^ 1];
+            const int half = N >> 1;
+            if (FULL) {
+              // N = 128: the partner lane is lane ^ 8, a rotation by 8 in the 16-lane row
+              qp[i] = dpp_shr<0x128>(q[i]);
+              kp[i] = dpp_shr<0x128>(k[i]);
+            } else if (half >= 8) {
+              // (half is a multiple of 8: the host's check)
+              const int l = tid & 15, src = 8 * l < half ? l + (half >> 3) : l - (half >> 3);
+              qp[i] = __shfl(q[i], src, 16);
+              kp[i] = __shfl(k[i], src, 16);
             } else {
-              const int half = N >> 1;
-              if (FULL) {
-                // N = 128: the partner lane is lane ^ 8, a rotation by 8 in the 16-lane row
-                qp[i] = dpp_shr<0x128>(q[i]);
-                kp[i] = dpp_shr<0x128>(k[i]);
-              } else if (half >= 8) {
-                qp[i] = __shfl_xor(q[i], half >> 3, 16);
-                kp[i] = __shfl_xor(k[i], half >> 3, 16);
-              } else {
-                qp[i] = q[i ^ half];
-                kp[i] = k[i ^ half];
-              }
+              qp[i] = q[i ^ half];
+              kp[i] = k[i ^ half];
             }
           }
 #pragma unroll
@@ -1175,7 +1197,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
             k[i] = fmaf(kp[i], ss, k[i] * cc);
           }
         }
-        st_row8<T>(Qs + row * LQ + n0, q);
+        if constexpr (!SO) st_row8<T>(Qs + row * LQ + n0, q);
         st_row8<T>(Ks + row * LQ + n0, k);
 #pragma unroll
         for (int i = 0; i < 8; ++i) kt[j][i] = k[i];
@@ -1238,6 +1260,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
+          if constexpr (SO) break;
           f4 vq, zq;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -1260,8 +1283,10 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
             vq[jr][i] = mul_r<T>(v[0][i], mxl[jr][i]);
             zq[i] = mul_r<T>(z[0][i], mzl[jr][i]);
           }
-          st_quad<T>(VR + row * LP + p0, vq[jr]);
-          st_quad<T>(ZR + row * LP + p0, zq);
+          if constexpr (!SO) {
+            st_quad<T>(VR + row * LP + p0, vq[jr]);
+            st_quad<T>(ZR + row * LP + p0, zq);
+          }
         }
         if constexpr (KTR) {
 #pragma unroll
@@ -1284,7 +1309,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
     for (int k = 0; k < kTiles; ++k) {
       const int u = w + kWaves * k;
-      if (all_tiles || u < n_tiles) {
+      if (!SO && (all_tiles || u < n_tiles)) {
         const int ni = u / kPT, pj = u - ni * kPT;
         st_quad<T>(Sb + (16 * pj + l16) * LQ + 16 * ni + 4 * lg, st[k]);
       }
@@ -1346,12 +1371,23 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         qv[kk] = *reinterpret_cast<const typename M::v8*>(Qs + trow * LQ + 32 * kk + 8 * lg);
       }
     }
+    // FP32 operands are read 4 elements of K per lane (a 16-byte LDS read feeds 4 MFMAs): MFMA i of
+    // a 16-element step takes elements 4 lg + i from both operands, K's own order permuted alike
+    // (2 x 1024 tokens of 8 heads, 256-token segments: 71 us a pass with one 4-byte read per
+    // operand and MFMA, 28 us so; 8 x 1000 tokens, 32 heads 253 -> 225). The query rows serve the scores and inter.
+    f4 qf[F32 ? NP / 16 : 1];
+    if constexpr (F32 && !SO) {
+#pragma unroll
+      for (int kk = 0; kk < NP / 16; ++kk) {
+        qf[kk] = *reinterpret_cast<const f4*>(Qs + trow * LQ + 16 * kk + 4 * lg);
+      }
+    }
     // scores Sc^T tiles (rows s, column t), issued before the phase work below
     f4 acc[RT];
 #pragma unroll
     for (int sj = 0; sj < RT; ++sj) {
       acc[sj] = zero4();
-      if (sj > it) continue;
+      if (SO || sj > it) continue;
       if constexpr (!F32) {
 #pragma unroll
         for (int kk = 0; kk < NP / 32; ++kk) {
@@ -1360,9 +1396,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           acc[sj] = M::mma(av, qv[kk], acc[sj]);
         }
       } else {
-#pragma unroll 8
-        for (int kk = 0; kk < NP; kk += 4) {
-          acc[sj] = M::mma(Ks[(16 * sj + l16) * LQ + kk + lg], Qs[trow * LQ + kk + lg], acc[sj]);
+#pragma unroll
+        for (int kk = 0; kk < NP / 16; ++kk) {
+          const f4 kv = *reinterpret_cast<const f4*>(Ks + (16 * sj + l16) * LQ + 16 * kk + 4 * lg);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[sj] = M::mma(kv[i], qf[kk][i], acc[sj]);
         }
       }
     }
@@ -1400,9 +1438,11 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
         }
       } else {
 #pragma unroll
-        for (int kk = 0; kk < ROWS; kk += 4) {
-          st[k] = M::mma(KT[nrow * LR + swz<ROWS>(kk + lg, nrow >> KSH)],
-                         VT[prow * LR + swz<ROWS>(kk + lg, prow >> VSH)], st[k]);
+        for (int kk = 0; kk < ROWS; kk += 16) {
+          const f4 kv = *reinterpret_cast<const f4*>(KT + nrow * LR + swz<ROWS>(kk + 4 * lg, nrow >> KSH));
+          const f4 vv = *reinterpret_cast<const f4*>(VT + prow * LR + swz<ROWS>(kk + 4 * lg, prow >> VSH));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[k] = M::mma(kv[i], vv[i], st[k]);
         }
       }
     }
@@ -1416,6 +1456,10 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
                                        fph, fblk, blk_stride);
     }
     if constexpr (FULL || SHAPE) loads_side();
+    if constexpr (SO) {
+      __syncthreads();
+      continue;
+    }
     // decayed scores W[t, s] = Sc[t, s] d[t, s] in FP32
     const float cum_t = SC[SB_::CUM + tq];
     const float gam_t = SC[SB_::GAM + tq];
@@ -1508,14 +1552,15 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
         for (int sj = 0; sj < RT; ++sj) {
           if (sj > it) continue;
+          const f4 vv = *reinterpret_cast<const f4*>(VT + pcol * LR + swz<ROWS>(16 * sj + 4 * lg, key));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            yi = M::mma(VT[pcol * LR + swz<ROWS>(16 * sj + 4 * lg + i, key)], wsc[sj][i], yi);
-          }
+          for (int i = 0; i < 4; ++i) yi = M::mma(vv[i], wsc[sj][i], yi);
         }
-#pragma unroll 8
-        for (int kk = 0; kk < NP; kk += 4) {
-          ye = M::mma(Sb[pcol * LQ + kk + lg], Qs[trow * LQ + kk + lg], ye);
+#pragma unroll
+        for (int kk = 0; kk < NP / 16; ++kk) {
+          const f4 sv = *reinterpret_cast<const f4*>(Sb + pcol * LQ + 16 * kk + 4 * lg);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) ye = M::mma(sv[i], qf[kk][i], ye);
         }
       }
       // epilogue: row trow (token tq, rank rr), columns pb .. pb+3
@@ -2251,12 +2296,12 @@ static bool model_shape(const m3_scan_args& a, ScanGeom& g, int es) {
   return true;
 }
 
-template <typename T, int R, bool FULL, bool SHAPE = false>
+template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false>
 static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* prep, dim3 grid,
                          dim3 block, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SHAPE>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SHAPE, SO>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                        Layout<T>::BYTES);
     if (e != hipSuccess) {
@@ -2264,7 +2309,7 @@ static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* 
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SHAPE>), grid, block, Layout<T>::BYTES, stream,
+  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SHAPE, SO>), grid, block, Layout<T>::BYTES, stream,
                      a, g, prep);
   return check_launch("m3_scan_fwd");
 }
@@ -2328,11 +2373,14 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
   const dim3 grid(static_cast<unsigned>(a.batch) * g.segs * a.heads), block(kThreads);
   if constexpr (sizeof(T) == 4) {
     if (full_shape(a, g, R) && prep != nullptr) {
+      if (state_only) return launch_kernel<T, R, true, false, true>(a, g, prep, grid, block, stream);
       return launch_kernel<T, R, true>(a, g, prep, grid, block, stream);
     }
     if (prep != nullptr && model_shape(a, g, static_cast<int>(sizeof(T)))) {
+      if (state_only) return launch_kernel<T, R, false, true, true>(a, g, prep, grid, block, stream);
       return launch_kernel<T, R, false, true>(a, g, prep, grid, block, stream);
     }
+    if (state_only) return launch_kernel<T, R, false, false, true>(a, g, prep, grid, block, stream);
   }
   return launch_kernel<T, R, false>(a, g, prep, grid, block, stream);
 }
@@ -2351,9 +2399,8 @@ static int sub_chunk_tokens(const m3_scan_args& a) {
 // Automatic (segments == 0): the G of least estimated time. With one workgroup per (b, h,
 // segment), a pass takes ceil(B H G c / 256) rounds over the 256 CUs (c calls of this shape
 // sharing the GPU, 1 alone), each of the segment's sub-chunks plus a prologue. In units of a
-// sub-chunk (2.7 us): the state-only first pass takes kStateOnly of the second where it has a
-// form of its own, a workgroup's start kPrologue (with phases; without them less), the split's
-// extra launches and composition kCompose, kPerSeg per segment and kWalk per 64-token block
+// sub-chunk (2.7 us): the state-only first pass takes kStateOnly of the second, a
+// workgroup's start 3 (without phases less), the split's extra launches and composition kCompose, kPerSeg per segment and kWalk per 64-token block
 // walked. A further segment is a serial step of the composition, so more than a few must be
 // longer: 16-bit segments of 4 sub-chunks up to 8 segments, else 8; FP32's (three times as long a
 // sub-chunk) 2 up to 16, else 4. Measured (bf16, angle increments, graph-timed, us):
@@ -2378,7 +2425,6 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
   auto rounds = [&](int64_t n) { return static_cast<double>((bhc * n + 255) / 256); };
   const double walk = a.phase_mode == M3_PHASE_ANGLES ? kWalk * static_cast<double>(len / 64) : 0.0;
   const bool f32 = a.act_dtype == M3_F32;
-  const double so = f32 ? 1.0 : kStateOnly;
   const double prologue = a.phase_mode == M3_PHASE_NONE ? 0.8 : 3.0;
   Segments best = cut(len, unit, 1);
   double best_cost = 0.95 * rounds(1) * (prologue + static_cast<double>((len + tok - 1) / tok));
@@ -2387,7 +2433,7 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
     const int shortest = f32 ? (n <= 16 ? 2 : 4) : (n <= 8 ? 4 : 8);
     if (s.len < shortest * tok) break;
     if (s.count != n) continue;
-    const double cost = rounds(n) * (2 * prologue + (1.0 + so) * static_cast<double>(s.len / tok)) +
+    const double cost = rounds(n) * (2 * prologue + (1.0 + kStateOnly) * static_cast<double>(s.len / tok)) +
                         kCompose + kPerSeg * n + walk;
     if (cost < best_cost * (1.0 - 1e-9)) {
       best = s;
@@ -2397,13 +2443,21 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
   return best;
 }
 
-// The shapes the chunked MFMA kernels tile: d_state a power of 2 up to 128, head_dim up to 64,
-// up to 32 angles, ranks 1, 2, 4 and 8, and the 16-wave kernel's calls at every d_state it takes
+// The shapes the chunked MFMA kernels tile: up to 128 columns, 64 values and 32 angles at ranks 1,
+// 2, 4 and 8, with d_state a power of 2; in FP32 also any other, with the MIMO rotation where its
+// pairs lie whole 8-column lanes apart (d_state 96, 4 x 1500 tokens, 16 heads: 21.7 ms on the
+// recurrent scan, 185 us here); and the 16-wave kernel's calls at every d_state it takes
 // (`rows`: its workspace rows are allowed). Others take the recurrent scan (rscan.hip).
 static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
-  return (pow2(a.d_state) && a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
-          a.num_angles <= kSMax && (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8)) ||
-         (rows && form16_of(a) >= 0);
+  const bool fits = a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
+                    a.num_angles <= kSMax &&
+                    (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8);
+  if (fits && pow2(a.d_state)) return true;
+  if (fits && a.act_dtype == M3_F32 && a.q.ptr != nullptr &&
+      (a.phase_mode == M3_PHASE_NONE || a.mimo_rotation == 0 || a.d_state % 16 == 0)) {
+    return true;
+  }
+  return rows && form16_of(a) >= 0;
 }
 
 static Segments segments_for(const m3_scan_args& a, int concurrent = 1) {

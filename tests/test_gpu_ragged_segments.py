@@ -82,3 +82,23 @@ def test_two_concurrent_calls_take_the_librarys_ragged_count():
         want = ops.scan_projection(proj, mixer)
     _close(call.out, want[0], torch.bfloat16)
     _close(call.final_state, want[1], torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d_model,d_state,rank,length", [
+    (64, 128, 1, 1000), (64, 128, 4, 33), (64, 64, 2, 70), (256, 96, 1, 130)])
+def test_ragged_rows_read_only_their_own(d_model, d_state, rank, length, dtype, monkeypatch):
+    """A last sub-chunk that is not full reads nothing past its row: neither what a workspace held
+    before (all bits set: NaN) nor the next batch row, here all NaN, reaches the first row."""
+    monkeypatch.setattr(ops, "SCAN_SEGMENTS", 1)
+    torch.manual_seed(length)
+    mixer = Mamba3(d_model, d_state=d_state, depth=1, mimo_rank=rank).eval().to(DEV).layers[0].mixer
+    proj = torch.randn(2, length, mixer.in_proj.weight.shape[0], device=DEV).to(dtype)
+    with torch.inference_mode():
+        want = ops.scan_projection(proj[:1].contiguous(), mixer, want_cache=True)
+        proj[1] = float("nan")
+        call = ops.ScanCall(proj, mixer, want_cache=True)
+        call._keep[-1].fill_(255)
+        call.launch()
+    for got, ref in zip((call.out, call.final_state, call.final_phase, call.final_k), want):
+        assert torch.equal(got[:1], ref)
