@@ -9,18 +9,25 @@ namespace m3 {
 // 32 angles, forwards or backwards, with 1024 threads, so that four waves share each SIMD to hide
 // one another's LDS, MFMA and transcendental latency. A sub-chunk is 64 rows (token, rank), rank
 // minor: 64 / R tokens, whose decay weights, phases and scalars are per token and whose output
-// sums the token's R rows (times mimo_out). Per sub-chunk, three intervals between workgroup
-// barriers:
-//   A  staging (every wave): row qt's q / k (bias and rotation on prep's rows; waves 0-7 the
-//      slots that can rotate, waves 8-15 the others) -> Qs, Ks; row vt's value / gate (times the
-//      rounded mimo_x / mimo_z above rank 1) -> VR, ZR and the carry's scaled values -> VS; the
-//      state, rounded -> Sb; the side block and angle tile of the next sub-chunk -> LDS;
-//   B  waves 0-9 one causal score tile each (Sc^T = K Q^T) and its decay weights W -> WS;
-//      every wave the carry products of its two state tiles; the next sub-chunk's global loads
-//      are issued here;
-//   C  wave w the output tile (row tile w / 4, P tile w % 4): intra V^T W^T from WS, inter
-//      rnd(S) Q^T, epilogue, store; waves 0-7, whose row tiles 0 and 1 have the shortest intra
-//      products, also the phases of the next sub-chunk (a long dependent chain per wave).
+// sums the token's R rows (times mimo_out). The work of a sub-chunk c, between workgroup barriers:
+//   staging   every wave: row qt's q / k (bias and rotation on prep's rows; waves 0-7 the slots
+//             that can rotate, waves 8-15 the others) -> Qs, Ks; row vt's values scaled for the
+//             carry -> VS;
+//   start     row vt's gate and value -> ZR, VR; the wave's two state tiles, rounded -> Sb, decayed;
+//   scores    ten waves one causal tile each (Sc^T = K Q^T) and its decay weights W -> WS;
+//   carry     every wave the products of its two state tiles;
+//   output    wave w the output tile (row tile w / 4, P tile w % 4): intra V^T W^T from WS, inter
+//             rnd(S) Q^T, epilogue, store;
+//   phases    of c + 1, on the first waves: a long dependent chain per wave.
+// Rank 1, three intervals: staging and start | scores and carry | output and phases (whose waves
+// 0-7 have the shortest intra products). Above rank 1, two: start, phases, scores (on the waves
+// without phases) and carry of c | staging of c + 1 (Qs has two tiles; Ks and VS were last read in
+// the first interval) and output of c. VALU, LDS and MFMA work then share both intervals, and a
+// sub-chunk's four waves per SIMD overlap them: 8 x 4096 tokens, 32 heads at rank 4 792 -> 686 us
+// per call, the rank-2 hook (4 x 2048) 186 -> 172. Rank 1 in two intervals measured 388 -> 402 (8 x
+// 8192): its phases are four times as long, and no wave is left to hide them. The interval
+// lengths are set by the SIMD's lowest-priority waves (12-15), not by the first to finish: raising
+// the priority of the later waves (s_setprio) measured 2-5% slower.
 // Same mathematics and rounding points as scan_kernel (whose header lists them).
 //
 // Slots. prep writes the q / k rows with their columns in slot order: the rotation's pairs first,
@@ -47,47 +54,61 @@ constexpr int k16Threads = 1024;
 // the 32 lanes' 8-byte pieces must cover 256 distinct bytes.
 //   Qs, Ks  [64 tokens][144]: 288-byte rows
 //   Sb      [64 p][128]: 256-byte rows, 16-byte chunk c of row p at c ^ (p % 16) (sb_off)
-//   VR, ZR, VS [64 tokens][64]: 128-byte rows, 32-byte pair and chunk half swizzled (v_off)
+//   VR, VS  [64 tokens][64]: 128-byte rows, 32-byte pair and chunk half swizzled (v_off)
+//   ZR      rank 1 the same; above it [64 rows][64] FP32: 256-byte rows, 16-byte chunks
+//           XOR-swizzled by row (z_off)
 //   WS      [64 t][80]: 160-byte rows
-struct Lay16 {
+struct Lay16Rows {
   static constexpr int ROWS = 64, LQ = kNPad + 16, LS = kNPad, LV = kPPad, LW = kPPad + 16, ES = 2;
-  static constexpr int QS = 0;
-  static constexpr int KS = QS + ROWS * LQ * ES;
+};
+template <int R>
+struct Lay16 : Lay16Rows {
+  static constexpr bool TWO = R > 1;              // the two-interval schedule
+  static constexpr int QS = 0, QB = ROWS * LQ;    // one or two Qs tiles, QB elements apart
+  static constexpr int KS = QS + (TWO ? 2 : 1) * QB * ES;
   static constexpr int VR = KS + ROWS * LQ * ES;
   static constexpr int ZR = VR + ROWS * LV * ES;
-  static constexpr int VS = ZR + ROWS * LV * ES;
+  static constexpr int VS = ZR + ROWS * LV * (TWO ? 4 : ES);  // (ZR: FP32 above rank 1)
   static constexpr int SB = VS + ROWS * LV * ES;
   static constexpr int WS = SB + kPPad * LS * ES;  // decay weights [t][s'] (s' permuted, below)
   static constexpr int FB = WS + ROWS * LW * ES;
-  // floats from FB: two side blocks (scalar blocks), the angle tile, two cos / sin tables, the
-  // phase block sum and carry per angle
-  static constexpr int SCB = 5 * ROWS + 8, SC0 = 0;
-  static constexpr int ANG = SC0 + 2 * SCB;
-  static constexpr int CST = 2 * kSMax + 4, CSB = ROWS * CST;
-  static constexpr int CS0 = ANG + ROWS * kSMax, PBASE = CS0 + 2 * CSB, POFF = PBASE + kSMax;
+  // floats from FB: the side blocks (scalar blocks) of two or three sub-chunks, the angle tile, the
+  // cos / sin tables (two at rank 1, whose phases run while the staging's table is still needed),
+  // the phase block sum and carry per angle
+  static constexpr int SCB = 5 * ROWS + 8, SC0 = 0, NSC = TWO ? 3 : 2;
+  static constexpr int ANG = SC0 + NSC * SCB;
+  static constexpr int CST = 2 * kSMax + 4, CSB = ROWS * CST, NCS = TWO ? 1 : 2;
+  static constexpr int CS0 = ANG + ROWS * kSMax, PBASE = CS0 + NCS * CSB, POFF = PBASE + kSMax;
   // ranks above 1: the rounded mimo_x, mimo_z and mimo_out [R][P]
-  static constexpr int MX = POFF + kSMax, MZ = MX + kRMax * kPPad, MO = MZ + kRMax * kPPad;
+  static constexpr int MP = TWO ? R * kPPad : 0;
+  static constexpr int MX = POFF + kSMax, MZ = MX + MP, MO = MZ + MP;
   // form kProj: the decay weights' second halves, W - rnd(W) (g.wlo)
-  static constexpr int WL = FB + 4 * (MO + kRMax * kPPad);
+  static constexpr int WL = FB + 4 * (MO + MP);
   static constexpr int bytes(bool wlo) { return wlo ? WL + ROWS * LW * ES : WL; }
+  static_assert(WL + ROWS * LW * ES <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
+  static_assert(FB % 16 == 0 && WS % 16 == 0 && SB % 16 == 0 && WL % 16 == 0 && (ANG * 4) % 16 == 0 &&
+                    (CS0 * 4) % 16 == 0 && (MX * 4) % 16 == 0,
+                "alignment");
 };
-static_assert(Lay16::bytes(true) <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
-static_assert(Lay16::FB % 16 == 0 && Lay16::WS % 16 == 0 && Lay16::SB % 16 == 0 &&
-              (Lay16::ANG * 4) % 16 == 0 && (Lay16::CS0 * 4) % 16 == 0, "alignment");
 
 // Element offset of column `col` of state row p in Sb (16-byte chunks XOR-swizzled by row).
 __device__ __forceinline__ int sb_off(int p, int col) {
-  return p * Lay16::LS + 8 * ((col >> 3) ^ (p & 15)) + (col & 7);
+  return p * Lay16Rows::LS + 8 * ((col >> 3) ^ (p & 15)) + (col & 7);
 }
 
-// Element offset of column `col` of token row r in VR, ZR, VS: the row's 32-byte pair
+// Element offset of column `col` of row r in the FP32 ZR.
+__device__ __forceinline__ int z_off(int r, int col) {
+  return r * Lay16Rows::LV + 4 * ((col >> 2) ^ (r & 15)) + (col & 3);
+}
+
+// Element offset of column `col` of token row r in VR, VS and rank 1's ZR: the row's 32-byte pair
 // (col / 16) XOR (r / 2) % 4 and the chunk within it flipped by (r / 8) % 2. Eight consecutive
 // rows then place one pair in eight distinct 32-byte bank groups (the transposing reads), and
 // sixteen consecutive rows one chunk in sixteen distinct 16-byte groups (the epilogue reads).
 __device__ __forceinline__ int v_off(int r, int col) {
   const int c = col >> 3;
   const int pc = 2 * ((c >> 1) ^ ((r >> 1) & 3)) + ((c & 1) ^ ((r >> 3) & 1));
-  return r * Lay16::LV + 8 * pc + (col & 7);
+  return r * Lay16Rows::LV + 8 * pc + (col & 7);
 }
 
 // The causal score tiles (row tile it, column tile sj <= it) of waves 0-9: the diagonal tiles,
@@ -106,7 +127,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   static_assert(R == 1 || R == 2 || R == 4 || R == 8, "scan16_kernel: ranks 1, 2, 4 and 8");
   static_assert(F != kModel || R == 1 || R == 4, "scan16_kernel: the model's shape");
   using M = Mma<T>;
-  using Ly = Lay16;
+  using Ly = Lay16<R>;
   constexpr int TOK = 64 / R;  // tokens per 64-row sub-chunk (rows (token, rank), rank minor)
   using SB_ = ScBlk<TOK>;
   constexpr int LQ = Ly::LQ, LW = Ly::LW, CST = Ly::CST, ES = 2;
@@ -146,6 +167,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   T* Ks = lds_t<T>(smem, Ly::KS);
   T* VR = lds_t<T>(smem, Ly::VR);
   T* ZR = lds_t<T>(smem, Ly::ZR);
+  float* ZF = lds_t<float>(smem, Ly::ZR);  // above rank 1
   T* VS = lds_t<T>(smem, Ly::VS);
   T* Sb = lds_t<T>(smem, Ly::SB);
   T* WS = lds_t<T>(smem, Ly::WS);
@@ -284,13 +306,14 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   float* ANG = F_ + Ly::ANG;
   // angle tile slot of 4-token group gq and angle s (XOR-keyed by the group's phase lane)
   auto ang_slot = [&](int gq, int s) { return gq * kSMax + (s ^ gq); };
-  auto put_side = [&](int c) {
-    if (w < 4 && side_on) *reinterpret_cast<float2*>(F_ + Ly::SC0 + (c & 1) * Ly::SCB + q2) = side;
+  // side block slots (floats from F_) of sub-chunks c, c + 1 and c + 2, rotated once per sub-chunk
+  int sc0 = Ly::SC0, sc1 = sc0 + Ly::SCB, sc2 = sc1 + Ly::SCB;
+  auto put_side = [&](int slot) {
+    if (w < 4 && side_on) *reinterpret_cast<float2*>(F_ + slot + q2) = side;
     if (w < 8 && ang_on) *reinterpret_cast<float4*>(ANG + 4 * ang_slot(agq, asl)) = ang;
   };
-  auto scb = [&](int c) { return F_ + Ly::SC0 + (c & 1) * Ly::SCB; };
-  auto csb = [&](int c) { return F_ + Ly::CS0 + (c & 1) * Ly::CSB; };
-  auto phases = [&](int c) {
+  auto cst = [&](int c) { return F_ + Ly::CS0 + (Ly::NCS == 2 ? c & 1 : 0) * Ly::CSB; };
+  auto phases = [&](int c, int slot) {
     // phases of sub-chunk c (the phase waves), from the angle tile and the dt of its side block
     if (ph_wave && c < nsub) {
       float pa[TPL];
@@ -303,8 +326,8 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       } else {
         pa[0] = ANG[4 * ang_slot(pg >> 2, ps) + (pg & 3)];  // token pg of its 4-token group
       }
-      phase_stage<PG, TPL, CST, true, false>(csb(c), ps, F_ + Ly::PBASE + ps, F_ + Ly::POFF + ps,
-                                             scb(c) + SB_::DTV, c * TOK, L, pg, lane, !GIVEN, pa,
+      phase_stage<PG, TPL, CST, true, false>(cst(c), ps, F_ + Ly::PBASE + ps, F_ + Ly::POFF + ps,
+                                             F_ + slot + SB_::DTV, c * TOK, L, pg, lane, !GIVEN, pa,
                                              fph, fblk, blk_stride);
     }
   };
@@ -460,7 +483,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     }
   }
   __builtin_amdgcn_sched_barrier(0);
-  put_side(0);
+  put_side(sc0);
   load_side(1);
   if (tid < kSMax) {
     F_[Ly::PBASE + tid] = 0.f;
@@ -486,17 +509,12 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     }
   }
   __syncthreads();
-  phases(0);
-  __syncthreads();
-
-  float log_decay = 0.f;
-  for (int c = 0; c < nsub; ++c) {
-    const int t0 = c * TOK;
-    const float* SC = scb(c);
-    const float* CSt = csb(c);
-
-    // ---- A: staging
-    if (c + 1 < nsub) put_side(c + 1);
+  phases(0, sc0);
+  // q / k of the coming sub-chunk -> its Qs tile and Ks
+  // (`qo`: the Qs tile's element offset). Rank 1 addresses q and k, and the two state tiles, from
+  // one base each, so that two stores are one instruction: 404 -> 390 us at 8 x 8192; at rank 4 the
+  // same measured 686 -> 701 (8 x 4096).
+  auto stage_qk = [&](int qo, const float* CSt) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       // row rw (token tt): q = q^ + bias, k = k^ + bias, rotated: pairs (n0, n0 + 1) and
@@ -521,46 +539,58 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
           k[2 * pp + 1] = fmaf(k0, ss, k1 * cc);
         }
       }
-      if constexpr (!SO) st_quad<T>(Qs + rw * LQ + n0, q);
-      st_quad<T>(Ks + rw * LQ + n0, k);
+      T* qd = R == 1 ? Qs + qt * LQ + n0 + 32 * j * LQ : Qs + rw * LQ + n0;
+      T* kd = R == 1 ? Qs + qt * LQ + n0 + (Ly::KS - Ly::QS) / ES + 32 * j * LQ : Ks + rw * LQ + n0;
+      if constexpr (!SO) st_quad<T>(qd + qo, q);
+      st_quad<T>(kd, k);
     }
-    {
-      // value / gate of row vt (token tv): VR / ZR = v, z (rank 1 as loaded; above it times the
-      // rounded mimo_x / mimo_z of the row's rank, rounded), VS = VR * scale * exp(cum_last - cum)
-      const int tv = vt / R;
-      const float ev = SC[SB_::SCL + tv] * __expf(SC[SB_::CL] - SC[SB_::CUM + tv]);
-      f4 sv;
+  };
+  // its values scaled for the carry -> VS: value (above rank 1 times the rounded mimo_x of the
+  // row's rank, rounded, kept in rv) * scale * exp(cum_last - cum)
+  auto stage_vs = [&](const float* SN) {
+    const int tv = vt / R;
+    const float ev = SN[SB_::SCL + tv] * __expf(SN[SB_::CL] - SN[SB_::CUM + tv]);
+    f4 vq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vq[i] = raw_get<T>(rv, i);
+    if constexpr (R > 1) {
+      const f4 mx = *reinterpret_cast<const f4*>(F_ + Ly::MX + (vt & (R - 1)) * kPPad + p0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vq[i] *= mx[i];
+      rv[0] = pack2<T>(vq[0], vq[1]);
+      rv[1] = pack2<T>(vq[2], vq[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vq[i] = raw_get<T>(rv, i);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) vq[i] *= ev;
+    st_quad<T>(VS + v_off(vt, p0), vq);
+  };
+  // the gate of row vt -> ZR (rank 1 as loaded; above it silu of the rounded z * mimo_z in FP32, so
+  // that the interval with the staging has less of the transcendental work), its values -> VR,
+  // the state at the sub-chunk's start, rounded -> Sb
+  auto stage_out = [&] {
+    if constexpr (!SO) {
       if constexpr (R == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sv[i] = raw_get<T>(rv, i) * ev;
-        if constexpr (!SO) {
-          *reinterpret_cast<u32x2*>(VR + v_off(vt, p0)) = (u32x2){rv[0], rv[1]};
-          *reinterpret_cast<u32x2*>(ZR + v_off(vt, p0)) = (u32x2){rz[0], rz[1]};
-        }
+        *reinterpret_cast<u32x2*>(ZR + v_off(vt, p0)) = (u32x2){rz[0], rz[1]};
       } else {
-        const int mo = (vt & (R - 1)) * kPPad + p0;
-        const f4 mx = *reinterpret_cast<const f4*>(F_ + Ly::MX + mo);
-        f4 vq;
+        const f4 mz = *reinterpret_cast<const f4*>(F_ + Ly::MZ + (vt & (R - 1)) * kPPad + p0);
+        f4 zq;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          vq[i] = mul_r<T>(raw_get<T>(rv, i), mx[i]);
-          sv[i] = vq[i] * ev;
-        }
-        if constexpr (!SO) {
-          const f4 mz = *reinterpret_cast<const f4*>(F_ + Ly::MZ + mo);
-          f4 zq;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) zq[i] = mul_r<T>(raw_get<T>(rz, i), mz[i]);
-          st_quad<T>(VR + v_off(vt, p0), vq);
-          st_quad<T>(ZR + v_off(vt, p0), zq);
-        }
+        for (int i = 0; i < 4; ++i) zq[i] = silu_fast(mul_r<T>(raw_get<T>(rz, i), mz[i]));
+        *reinterpret_cast<f4*>(ZF + z_off(vt, p0)) = zq;
       }
-      st_quad<T>(VS + v_off(vt, p0), sv);
-    }
+      *reinterpret_cast<u32x2*>(VR + v_off(vt, p0)) = (u32x2){rv[0], rv[1]};
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if constexpr (!SO) st_quad<T>(Sb + sb_off(16 * (spj0 + k) + l16, 16 * sni + 4 * lg), st[k]);
+      for (int k = 0; k < 2; ++k) {
+        const int so = R == 1 ? sb_off(16 * spj0 + l16, 16 * sni + 4 * lg) + 16 * k * Ly::LS
+                              : sb_off(16 * (spj0 + k) + l16, 16 * sni + 4 * lg);
+        st_quad<T>(Sb + so, st[k]);
+      }
     }
+  };
+  float log_decay = 0.f;
+  auto decay_state = [&](const float* SC) {
     {
       const float ecl = SC[SB_::ECL];
       log_decay += SC[SB_::CL];
@@ -570,15 +600,12 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         for (int i = 0; i < 4; ++i) st[k][i] *= ecl;
       }
     }
-    __syncthreads();
-
-    // ---- B: score tiles and decay weights, carry products, phases of c + 1; loads of c + 1
-    __builtin_amdgcn_sched_barrier(0);
-    load_qk(t0 + TOK);
-    __builtin_amdgcn_sched_barrier(0);
-    if (!SO && w < 10) {
+  };
+  // causal score tile `tile` (score_tile16) and its decay weights -> WS
+  auto scores = [&](int tile, const T* Qc, const float* SC) {
+    if constexpr (!SO) {
       int it, sj;
-      score_tile16(w, it, sj);
+      score_tile16(tile, it, sj);
       const int tq = 16 * it + l16;
       f4 acc = zero4();
       // (four waves per SIMD hide the operand latency: one k-step's operands in registers at a
@@ -588,7 +615,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         const typename M::v8 av = *reinterpret_cast<const typename M::v8*>(
             Ks + (16 * sj + l16) * LQ + 32 * kk + 8 * lg);
         const typename M::v8 bv =
-            *reinterpret_cast<const typename M::v8*>(Qs + tq * LQ + 32 * kk + 8 * lg);
+            *reinterpret_cast<const typename M::v8*>(Qc + tq * LQ + 32 * kk + 8 * lg);
         acc = M::mma(av, bv, acc);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -649,6 +676,8 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         st_quad<T>(WL + wo, wv);
       }
     }
+  };
+  auto carry = [&] {
     {
       // carry: S^T(ni, pj) += K~^T V~ over the 64 tokens. A: 8 tokens of column n from the
       // row-major Ks by two transposing reads (in each 16-lane group, lane 4a + b receives
@@ -681,14 +710,9 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
-    load_vz(t0 + TOK);
-    __builtin_amdgcn_sched_barrier(0);
-    load_side(c + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-
-    // ---- C: output tile (row tile it, P tile pj)
+  };
+  // output tile (row tile it, P tile pj) of the sub-chunk at token t0
+  auto output = [&](int t0, const T* Qc, const float* SC) {
     if constexpr (!SO) {
       const int it = w >> 2, pj = w & 3;
       const int tq = 16 * it + l16;
@@ -737,7 +761,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         const typename M::v8 av = *reinterpret_cast<const typename M::v8*>(
             Sb + sb_off(16 * pj + l16, 32 * kk + 8 * lg));
         const typename M::v8 bv =
-            *reinterpret_cast<const typename M::v8*>(Qs + tq * LQ + 32 * kk + 8 * lg);
+            *reinterpret_cast<const typename M::v8*>(Qc + tq * LQ + 32 * kk + 8 * lg);
         ye = M::mma(av, bv, ye);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -745,11 +769,18 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       const int pb = 16 * pj + 4 * lg, tqt = tq / R;
       const float ecum_t = __expf(SC[SB_::CUM + tqt]);
       const typename M::v4 v4 = *reinterpret_cast<const typename M::v4*>(VR + v_off(tq, pb));
-      const typename M::v4 z4 = *reinterpret_cast<const typename M::v4*>(ZR + v_off(tq, pb));
+      typename M::v4 z4;
+      f4 sz;
+      if constexpr (R == 1) {
+        z4 = *reinterpret_cast<const typename M::v4*>(ZR + v_off(tq, pb));
+      } else {
+        sz = *reinterpret_cast<const f4*>(ZF + z_off(tq, pb));
+      }
       f4 y;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * to_f(v4[i])) * silu_fast(to_f(z4[i]));
+        const float gate = R == 1 ? silu_fast(to_f(z4[i])) : sz[i];
+        y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * to_f(v4[i])) * gate;
       }
       if constexpr (R > 1) {
         // times mimo_out of the row's rank, summed over the token's R rows, consecutive lanes
@@ -776,10 +807,77 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
                                      __builtin_amdgcn_readfirstlane(t0 * go.step));
       }
     }
-    // phases of c + 1: its angle tile and side block came to LDS in A; its cos / sin table is
-    // the other buffer than the one A read
-    phases(c + 1);
+  };
+  auto pin = [] { __builtin_amdgcn_sched_barrier(0); };
+
+  if constexpr (R == 1) {
+    // three intervals per sub-chunk
     __syncthreads();
+    for (int c = 0; c < nsub; ++c) {
+      const int t0 = c * TOK;
+      const float* SC = F_ + sc0;
+      if (c + 1 < nsub) put_side(sc1);
+      stage_qk(0, cst(c));
+      stage_vs(SC);
+      stage_out();
+      decay_state(SC);
+      __syncthreads();
+      pin();
+      load_qk(t0 + TOK);
+      pin();
+      if (w < 10) scores(w, Qs, SC);
+      carry();
+      pin();
+      load_vz(t0 + TOK);
+      pin();
+      load_side(c + 2);
+      pin();
+      __syncthreads();
+      output(t0, Qs, SC);
+      phases(c + 1, sc1);
+      __syncthreads();
+      const int sct = sc0;
+      sc0 = sc1;
+      sc1 = sct;
+    }
+  } else {
+    // two intervals per sub-chunk; the first sub-chunk's staging ahead of the loop
+    __syncthreads();
+    stage_qk(0, cst(0));
+    stage_vs(F_ + sc0);
+    if (nsub > 1) put_side(sc1);
+    load_qk(TOK);
+    load_side(2);
+    __syncthreads();
+    for (int c = 0; c < nsub; ++c) {
+      const int t0 = c * TOK;
+      const float* SC = F_ + sc0;
+      const T* Qc = Qs + (c & 1) * Ly::QB;
+      stage_out();
+      pin();
+      load_vz(t0 + TOK);
+      pin();
+      decay_state(SC);
+      phases(c + 1, sc1);
+      if (w < 2 || w >= 8) scores((w - 8) & 15, Qc, SC);  // waves 8-15 and 0, 1
+      carry();
+      __syncthreads();
+      if (c + 1 < nsub) {
+        stage_qk(((c + 1) & 1) * Ly::QB, cst(c + 1));
+        stage_vs(F_ + sc1);
+        if (c + 2 < nsub) put_side(sc2);
+      }
+      pin();
+      load_qk(t0 + 2 * TOK);
+      load_side(c + 3);
+      pin();
+      output(t0, Qc, SC);
+      __syncthreads();
+      const int sct = sc0;
+      sc0 = sc1;
+      sc1 = sc2;
+      sc2 = sct;
+    }
   }
 
   // ---- final k: the biased, rotated k rows of token L-1, still in Ks from the last sub-chunk
@@ -823,7 +921,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
 template <typename T, int R, Form16 F, bool SO>
 static int launch_one16(const m3_scan_args& a, const ScanGeom& g, const float* prep,
                         unsigned grid, hipStream_t stream) {
-  constexpr int kBytes = Lay16::bytes(F == kProj && !SO);
+  constexpr int kBytes = Lay16<R>::bytes(F == kProj && !SO);
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan16_kernel<T, R, F, SO>),
