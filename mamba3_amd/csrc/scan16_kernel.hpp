@@ -247,9 +247,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   const Rows gx = phases_in ? rows_of(a.phase, h * a.phase.stride[2],
                                       (S - 1) * static_cast<int>(a.phase.stride[3]) + 1, 4)
                             : Rows{make_rsrc(nullptr, 0), 0, 0};
-  const int o_x = phases_in && asl < S
-                      ? gx.o0 + 4 * agq * gx.step + asl * static_cast<int>(a.phase.stride[3]) * 4
-                      : kPast;
+  const int o_x = gx.o0 + 4 * agq * gx.step + asl * static_cast<int>(a.phase.stride[3]) * 4;
 
   // where the end state, phase and k go: the segment's own slots (pass 1 of a split call), or the
   // call's outputs, written by the last segment alone
@@ -292,7 +290,10 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     }
     if (w < 8) {
       if constexpr (GIVEN) {
-        const int o = o_x + c * TOK * gx.step;
+        // lanes past the call's angles stay at kPast: moved on with the others, backwards (a
+        // negative step) they would come back into an extent above half of 2^30 bytes. The host
+        // keeps 256 tokens between every extent and 2^30, so the 4 steps below stay past it too.
+        const int o = asl < S ? o_x + c * TOK * gx.step : kPast;
         ang = make_float4(bload_f32(gx.rs, o), bload_f32(gx.rs, o + gx.step),
                           bload_f32(gx.rs, o + 2 * gx.step), bload_f32(gx.rs, o + 3 * gx.step));
       } else {

@@ -167,3 +167,42 @@ def test_scan_without_room_for_rows():
     _hip.call("m3_scan_fwd_noalloc", args, DEV)
     _close(out, want.cpu(), torch.bfloat16)
     _close(state, want_state.cpu(), torch.bfloat16)
+
+
+def test_reversed_call_with_far_given_phases():
+    """A reversed call whose phases of one batch row span more than 2^29 bytes, with fewer angles
+    than the kernel's 32: the lanes without an angle read none of them at any token. The same
+    arithmetic as the forward call on flipped inputs, so the same bits."""
+    torch.manual_seed(11)
+    l, h, n, p, s = 40000, 2, 64, 4, 16
+    rows = torch.empty(1, l, 256, s, device=DEV)  # 256 heads' worth: 16 KiB per token, 655 MB
+    rows.uniform_(-3, 3)
+    mk = lambda *shape: torch.randn(*shape, device=DEV).to(torch.bfloat16)
+    t = dict(q=mk(1, l, 1, 1, n), k=mk(1, l, 1, 1, n), value=mk(1, l, h, p), gate=mk(1, l, h, p),
+             dt=torch.rand(1, l, h, device=DEV) * 0.1, trap=mk(1, l, h), phase=rows[:, :, :h])
+    t["a"] = -t["dt"]
+    D = torch.ones(h, device=DEV)
+
+    def scan(tensors, reverse):
+        out = torch.empty(1, l, h, p, device=DEV, dtype=torch.bfloat16)
+        state = torch.empty(1, h, p, n, device=DEV)
+        args = _hip.ScanArgs(batch=1, length=l, heads=h, groups=1, rank=1, d_state=n, head_dim=p,
+                             num_angles=s, chunk=64, act_dtype=_hip.BF16,
+                             phase_mode=_hip.PHASE_GIVEN, norm_eps=1e-5, segments=1)
+        for name, x in dict(tensors, D=D, out=out, final_state=state).items():
+            setattr(args, name, _hip.tensor(x))
+        if reverse:
+            for name in (*tensors, "out"):
+                ops._backwards(getattr(args, name), l)
+        ws = _hip.scan_workspace(args, DEV)
+        _hip.call("m3_scan_fwd", args, DEV)
+        del ws
+        return out, state
+
+    got, state = scan(t, True)
+    flipped = {name: x.flip(1) for name, x in t.items() if name != "phase"}
+    flipped["phase"] = torch.empty_like(rows)[:, :, :h]
+    flipped["phase"].copy_(t["phase"].flip(1))
+    want, want_state = scan(flipped, False)
+    assert torch.equal(got, want.flip(1))
+    assert torch.equal(state, want_state)
