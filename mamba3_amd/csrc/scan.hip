@@ -2124,7 +2124,7 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   g.seg_len = static_cast<int>((len + 63) / 64 * 64);
   g.last_only = 0;
   g.perm = a.phase_mode != M3_PHASE_NONE && a.mimo_rotation != 0;
-  g.wlo = !pow2(a.d_state);
+  g.lo = !pow2(a.d_state);
   const bool norm = a.q_norm_w.ptr != nullptr && form16 < 0;
   const bool angles = a.phase_mode == M3_PHASE_ANGLES;
   const int64_t batch = a.batch > 0 ? a.batch : 0;

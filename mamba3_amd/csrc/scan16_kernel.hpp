@@ -44,6 +44,14 @@ namespace m3 {
 //   kProj   the other shapes in projection form: the normalized rows in FP32, rounded once after
 //           the rotation;
 //   kHook   the hook form: the given (normed) rows, phases given or none.
+//
+// LO: d_state no power of 2. Those calls are the recurrent scan's on rows that are not aligned, and
+// came from it: it holds the decay weights and the scaled values in FP32, rounding neither. Here
+// each becomes two 16-bit operands, the rounded value and the rounding error (for FP16 times 2^11,
+// in accumulators of its own, so that it stays a normal number), and two products. Output error
+// against 64 bits (bf16, 2 x 500 tokens; recurrent scan, one operand each, two weights alone, two
+// each): hook form d_state 96 rank 1 2.00e-3, 2.43e-3, 2.04e-3, 1.85e-3; projection form d_state
+// 112 rank 2 3.18e-3, 3.28e-3, 3.26e-3, 3.10e-3.
 
 constexpr int k16Threads = 1024;
 
@@ -58,17 +66,19 @@ constexpr int k16Threads = 1024;
 //   ZR      rank 1 the same; above it [64 rows][64] FP32: 256-byte rows, 16-byte chunks
 //           XOR-swizzled by row (z_off)
 //   WS      [64 t][80]: 160-byte rows
+//   WL, VL  (LO) the second operands of WS and VS, laid out as they are; ZR is 16-bit at every rank
 struct Lay16Rows {
   static constexpr int ROWS = 64, LQ = kNPad + 16, LS = kNPad, LV = kPPad, LW = kPPad + 16, ES = 2;
 };
-template <int R>
+template <int R, bool LO>
 struct Lay16 : Lay16Rows {
   static constexpr bool TWO = R > 1;              // the two-interval schedule
+  static constexpr bool ZF32 = TWO && !LO;        // ZR holds the FP32 gate
   static constexpr int QS = 0, QB = ROWS * LQ;    // one or two Qs tiles, QB elements apart
   static constexpr int KS = QS + (TWO ? 2 : 1) * QB * ES;
   static constexpr int VR = KS + ROWS * LQ * ES;
   static constexpr int ZR = VR + ROWS * LV * ES;
-  static constexpr int VS = ZR + ROWS * LV * (TWO ? 4 : ES);  // (ZR: FP32 above rank 1)
+  static constexpr int VS = ZR + ROWS * LV * (ZF32 ? 4 : ES);
   static constexpr int SB = VS + ROWS * LV * ES;
   static constexpr int WS = SB + kPPad * LS * ES;  // decay weights [t][s'] (s' permuted, below)
   static constexpr int FB = WS + ROWS * LW * ES;
@@ -82,11 +92,12 @@ struct Lay16 : Lay16Rows {
   // ranks above 1: the rounded mimo_x, mimo_z and mimo_out [R][P]
   static constexpr int MP = TWO ? R * kPPad : 0;
   static constexpr int MX = POFF + kSMax, MZ = MX + MP, MO = MZ + MP;
-  // form kProj: the decay weights' second halves, W - rnd(W) (g.wlo)
   static constexpr int WL = FB + 4 * (MO + MP);
-  static constexpr int bytes(bool wlo) { return wlo ? WL + ROWS * LW * ES : WL; }
-  static_assert(WL + ROWS * LW * ES <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
-  static_assert(FB % 16 == 0 && WS % 16 == 0 && SB % 16 == 0 && WL % 16 == 0 && (ANG * 4) % 16 == 0 &&
+  static constexpr int VL = WL + (LO ? ROWS * LW * ES : 0);
+  static constexpr int BYTES = VL + (LO ? ROWS * LV * ES : 0);
+  static_assert(BYTES <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
+  static_assert(FB % 16 == 0 && WS % 16 == 0 && SB % 16 == 0 && WL % 16 == 0 && VL % 16 == 0 &&
+                    (ANG * 4) % 16 == 0 &&
                     (CS0 * 4) % 16 == 0 && (MX * 4) % 16 == 0,
                 "alignment");
 };
@@ -120,14 +131,15 @@ __device__ __forceinline__ void score_tile16(int w, int& it, int& sj) {
   sj = w < 4 ? w : (k < 1 ? 0 : (k < 3 ? k - 1 : k - 3));
 }
 
-template <typename T, int R, Form16 F, bool SO>
+template <typename T, int R, Form16 F, bool SO, bool LO>
 __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a,
                                                             const ScanGeom g,
                                                             const float* __restrict__ prep) {
   static_assert(R == 1 || R == 2 || R == 4 || R == 8, "scan16_kernel: ranks 1, 2, 4 and 8");
   static_assert(F != kModel || R == 1 || R == 4, "scan16_kernel: the model's shape");
   using M = Mma<T>;
-  using Ly = Lay16<R>;
+  static_assert(F != kModel || !LO, "scan16_kernel: the model's d_state is a power of 2");
+  using Ly = Lay16<R, LO>;
   constexpr int TOK = 64 / R;  // tokens per 64-row sub-chunk (rows (token, rank), rank minor)
   using SB_ = ScBlk<TOK>;
   constexpr int LQ = Ly::LQ, LW = Ly::LW, CST = Ly::CST, ES = 2;
@@ -167,11 +179,21 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   T* Ks = lds_t<T>(smem, Ly::KS);
   T* VR = lds_t<T>(smem, Ly::VR);
   T* ZR = lds_t<T>(smem, Ly::ZR);
-  float* ZF = lds_t<float>(smem, Ly::ZR);  // above rank 1
+  float* ZF = lds_t<float>(smem, Ly::ZR);  // Ly::ZF32
   T* VS = lds_t<T>(smem, Ly::VS);
   T* Sb = lds_t<T>(smem, Ly::SB);
   T* WS = lds_t<T>(smem, Ly::WS);
   T* WL = lds_t<T>(smem, Ly::WL);
+  T* VL = lds_t<T>(smem, Ly::VL);
+  // LO: the factor of the second operands; other than 1 they have accumulators of their own
+  constexpr float kLo = sizeof(T) == 2 && std::is_same<T, _Float16>::value ? 2048.f : 1.f;
+  constexpr bool LOA = LO && kLo != 1.f;
+  auto low = [](f4 x) {
+    f4 y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = (x[i] - rnd<T>(x[i])) * kLo;
+    return y;
+  };
   float* F_ = lds_t<float>(smem, Ly::FB);
 
   // ---- lane roles
@@ -566,9 +588,11 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
 #pragma unroll
     for (int i = 0; i < 4; ++i) vq[i] *= ev;
     st_quad<T>(VS + v_off(vt, p0), vq);
+    if constexpr (LO) st_quad<T>(VL + v_off(vt, p0), low(vq));
   };
   // the gate of row vt -> ZR (rank 1 as loaded; above it silu of the rounded z * mimo_z in FP32, so
-  // that the interval with the staging has less of the transcendental work), its values -> VR,
+  // that the interval with the staging has less of the transcendental work, LO the product itself),
+  // its values -> VR,
   // the state at the sub-chunk's start, rounded -> Sb
   auto stage_out = [&] {
     if constexpr (!SO) {
@@ -578,8 +602,15 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         const f4 mz = *reinterpret_cast<const f4*>(F_ + Ly::MZ + (vt & (R - 1)) * kPPad + p0);
         f4 zq;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) zq[i] = silu_fast(mul_r<T>(raw_get<T>(rz, i), mz[i]));
-        *reinterpret_cast<f4*>(ZF + z_off(vt, p0)) = zq;
+        for (int i = 0; i < 4; ++i) {
+          const float zm = mul_r<T>(raw_get<T>(rz, i), mz[i]);
+          zq[i] = Ly::ZF32 ? silu_fast(zm) : zm;
+        }
+        if constexpr (Ly::ZF32) {
+          *reinterpret_cast<f4*>(ZF + z_off(vt, p0)) = zq;
+        } else {
+          st_quad<T>(ZR + v_off(vt, p0), zq);
+        }
       }
       *reinterpret_cast<u32x2*>(VR + v_off(vt, p0)) = (u32x2){rv[0], rv[1]};
 #pragma unroll
@@ -671,11 +702,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       // the intra product's K axis (below)
       const int wo = tq * LW + 32 * (sj >> 1) + 8 * lg + 4 * (sj & 1);
       st_quad<T>(WS + wo, wv);
-      if (ROWF && g.wlo) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) wv[i] -= rnd<T>(wv[i]);
-        st_quad<T>(WL + wo, wv);
-      }
+      if constexpr (LO) st_quad<T>(WL + wo, low(wv));
     }
   };
   auto carry = [&] {
@@ -686,6 +713,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       // The K axis of k-step kk, lane group lg: tokens kk + 4 lg + j (slots j) and
       // kk + 16 + 4 lg + j (slots 4 + j), so the 32 lanes of each read take 8 consecutive tokens
       const int xr = l16 >> 2, xc = 4 * (l16 & 3);
+      f4 sl[2] = {zero4(), zero4()};
 #pragma unroll
       for (int kk = 0; kk < 64; kk += 32) {  // the 64 rows
         const int r0 = kk + 4 * lg + xr;
@@ -699,16 +727,26 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
           const int vc = 16 * (spj0 + k) + xc;
-          const i16x4 vlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(VS + v_off(r0, vc)));
-          const i16x4 vhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) i16x4*)(VS + v_off(r0 + 16, vc)));
-          const typename M::v8 bv = __builtin_bit_cast(
-              typename M::v8,
-              (i16x8){vlo[0], vlo[1], vlo[2], vlo[3], vhi[0], vhi[1], vhi[2], vhi[3]});
-          st[k] = M::mma(av, bv, st[k]);
+          auto rows8 = [&](const T* v) {
+            const i16x4 vlo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) i16x4*)(v + v_off(r0, vc)));
+            const i16x4 vhi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) i16x4*)(v + v_off(r0 + 16, vc)));
+            return __builtin_bit_cast(
+                typename M::v8,
+                (i16x8){vlo[0], vlo[1], vlo[2], vlo[3], vhi[0], vhi[1], vhi[2], vhi[3]});
+          };
+          st[k] = M::mma(av, rows8(VS), st[k]);
+          if constexpr (LO) (LOA ? sl[k] : st[k]) = M::mma(av, rows8(VL), LOA ? sl[k] : st[k]);
         }
         __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (LOA) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) st[k][i] = fmaf(sl[k][i], 1.f / kLo, st[k][i]);
+        }
       }
     }
   };
@@ -717,7 +755,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     if constexpr (!SO) {
       const int it = w >> 2, pj = w & 3;
       const int tq = 16 * it + l16;
-      f4 yi = zero4(), ye = zero4();
+      f4 yi = zero4(), ye = zero4(), yl = zero4();
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
         if (2 * m > it) continue;
@@ -749,12 +787,16 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
         };
         bv = causal(bv);
         yi = M::mma(av, bv, yi);
-        if (ROWF && g.wlo) {
+        if constexpr (LO) {
           const typename M::v8 bl =
               *reinterpret_cast<const typename M::v8*>(WL + tq * LW + 32 * m + 8 * lg);
-          yi = M::mma(av, causal(bl), yi);
+          (LOA ? yl : yi) = M::mma(av, causal(bl), LOA ? yl : yi);
         }
         __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (LOA) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) yi[i] = fmaf(yl[i], 1.f / kLo, yi[i]);
       }
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
@@ -772,7 +814,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       const typename M::v4 v4 = *reinterpret_cast<const typename M::v4*>(VR + v_off(tq, pb));
       typename M::v4 z4;
       f4 sz;
-      if constexpr (R == 1) {
+      if constexpr (!Ly::ZF32) {
         z4 = *reinterpret_cast<const typename M::v4*>(ZR + v_off(tq, pb));
       } else {
         sz = *reinterpret_cast<const f4*>(ZF + z_off(tq, pb));
@@ -780,7 +822,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       f4 y;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float gate = R == 1 ? silu_fast(to_f(z4[i])) : sz[i];
+        const float gate = Ly::ZF32 ? sz[i] : silu_fast(to_f(z4[i]));
         y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * to_f(v4[i])) * gate;
       }
       if constexpr (R > 1) {
@@ -919,20 +961,21 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   }
 }
 
-template <typename T, int R, Form16 F, bool SO>
+template <typename T, int R, Form16 F, bool SO, bool LO>
 static int launch_one16(const m3_scan_args& a, const ScanGeom& g, const float* prep,
                         unsigned grid, hipStream_t stream) {
-  constexpr int kBytes = Lay16<R>::bytes(F == kProj && !SO);
+  constexpr int kBytes = Lay16<R, LO>::BYTES;
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan16_kernel<T, R, F, SO>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kBytes);
+    hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&scan16_kernel<T, R, F, SO, LO>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kBytes);
     if (e != hipSuccess) {
       return fail(M3_ELAUNCH, "m3_scan_fwd: hipFuncSetAttribute: %s", hipGetErrorString(e));
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((scan16_kernel<T, R, F, SO>), dim3(grid), dim3(k16Threads), kBytes,
+  hipLaunchKernelGGL((scan16_kernel<T, R, F, SO, LO>), dim3(grid), dim3(k16Threads), kBytes,
                      stream, a, g, prep);
   return check_launch("m3_scan_fwd");
 }
@@ -940,8 +983,14 @@ static int launch_one16(const m3_scan_args& a, const ScanGeom& g, const float* p
 template <typename T, int R, Form16 F>
 static int launch_form16(const m3_scan_args& a, const ScanGeom& g, const float* prep, bool so,
                          unsigned grid, hipStream_t stream) {
-  return so ? launch_one16<T, R, F, true>(a, g, prep, grid, stream)
-            : launch_one16<T, R, F, false>(a, g, prep, grid, stream);
+  if constexpr (F != kModel) {
+    if (g.lo) {
+      return so ? launch_one16<T, R, F, true, true>(a, g, prep, grid, stream)
+                : launch_one16<T, R, F, false, true>(a, g, prep, grid, stream);
+    }
+  }
+  return so ? launch_one16<T, R, F, true, false>(a, g, prep, grid, stream)
+            : launch_one16<T, R, F, false, false>(a, g, prep, grid, stream);
 }
 
 template <typename T, int R>

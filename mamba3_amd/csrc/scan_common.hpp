@@ -120,9 +120,8 @@ struct ScanGeom {
   // [B][L][G][R][2][128] in slot order, in the activation dtype or FP32 (form kProj), after the
   // regions above (byte offset)
   int form16, perm;
-  // form kProj: the decay weights as two 16-bit halves (d_state no power of 2: those calls came
-  // from the recurrent scan, which keeps them in FP32)
-  int wlo;
+  // d_state no power of 2: the kernels that hold no value in fewer bits than the recurrent scan
+  int lo;
   int64_t ws_qk;
   // projection form (the full-shape kernel): q, k, value, gate, dt, a, trap are slices of one
   // projection row; byte offsets of each slice from `proj`, the batch / token strides and the
