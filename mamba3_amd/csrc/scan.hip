@@ -338,12 +338,36 @@ struct Feed {
 
 // ------------------------------------------------------------------ prep
 
+// The scalar functions of a call, LO (d_state no power of 2: the calls that came from the recurrent
+// scan) that scan's library functions, else the hardware's.
+template <bool LO>
+__device__ __forceinline__ float exp_x(float x) {
+  return LO ? expf(x) : __expf(x);
+}
+template <bool LO>
+__device__ __forceinline__ float sigmoid_x(float x) {
+  return LO ? sigmoidf(x) : sigmoid_fast(x);
+}
+template <bool LO>
+__device__ __forceinline__ float silu_x(float x) {
+  return LO ? siluf(x) : silu_fast(x);
+}
+template <bool LO>
+__device__ __forceinline__ void dt_adt_x(bool raw, float dt_in, float a_in, float dt_bias, float& dt,
+                                         float& adt) {
+  if constexpr (LO) {
+    dt_adt(raw, dt_in, a_in, dt_bias, dt, adt);
+  } else {
+    dt_adt_fast(raw, dt_in, a_in, dt_bias, dt, adt);
+  }
+}
+
 // The scalar block of sub-chunk c of (batch, head) bh (one wave, lane = token): dt, adt, trap
 // from the raw projection or given (model.py:195-198), gamma = dt sigmoid(trap), scale = gamma +
 // dt' (1 - sigmoid(trap')) of the next token, 0 at the last token (ops.py:659-671) and, `cut`, at
 // the last of a segment (the next segment starts with it as its endpoint term), the within-chunk
 // cumsum of adt by a wave scan, and the decay products the scan uses.
-template <int TOK, int TPT>
+template <int TOK, int TPT, bool LO>
 __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __restrict__ o,
                                              int c, int lane, float dt_bias, float dt_in,
                                              float a_in, float tr_in, float dtn_in,
@@ -357,8 +381,8 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
   const bool raw_dt = a.raw_dt != 0;
   float dt = 0.f, adt = 0.f, tr = 0.f;
   if (tv) {
-    dt_adt_fast(raw_dt, dt_in, a_in, dt_bias, dt, adt);
-    tr = sigmoid_fast(tr_in);
+    dt_adt_x<LO>(raw_dt, dt_in, a_in, dt_bias, dt, adt);
+    tr = sigmoid_x<LO>(tr_in);
   }
   // right = dt' (1 - sigmoid(trap')) of the next token: lane + 1's; the last lane's from the
   // token after the sub-chunk (dtn_in, trn_in)
@@ -366,8 +390,8 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
   float right = __shfl_down(own, 1);
   if (lane == TOK - 1) {
     float dn, an;
-    dt_adt_fast(raw_dt, dtn_in, 0.f, dt_bias, dn, an);
-    right = dn * (1.f - sigmoid_fast(trn_in));
+    dt_adt_x<LO>(raw_dt, dtn_in, 0.f, dt_bias, dn, an);
+    right = dn * (1.f - sigmoid_x<LO>(trn_in));
   }
   if (!nv) right = 0.f;
   const float gamma = dt * tr;
@@ -390,11 +414,11 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
     o[B::CUM + lane] = cv;
     o[B::SCL + lane] = tv ? scale : 0.f;
     o[B::GAM + lane] = gamma;
-    o[B::BSC + lane] = tv ? scale * __expf(cend - cv) : 0.f;
+    o[B::BSC + lane] = tv ? scale * exp_x<LO>(cend - cv) : 0.f;
     if ((lane & (TPT - 1)) == 0) o[B::CEND + lane / TPT] = cend;
   }
   if (lane == 0) {
-    o[B::ECL] = __expf(cum_last);
+    o[B::ECL] = exp_x<LO>(cum_last);
     o[B::CL] = cum_last;
   }
 }
@@ -403,7 +427,7 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
 // token lane % TOK), `o` the lane's head's block, `live` false for lanes past the last head
 // (they compute on a valid head's inputs and store nothing). The arithmetic and its order are
 // scalar_block's (a segment's scan is the wave scan's first row), so the blocks are identical.
-template <int TOK, int TPT>
+template <int TOK, int TPT, bool LO>
 __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* __restrict__ o,
                                                  int c, int lane, bool live, float dt_bias,
                                                  float dt_in, float a_in, float tr_in,
@@ -419,15 +443,15 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
   const bool raw_dt = a.raw_dt != 0;
   float dt = 0.f, adt = 0.f, tr = 0.f;
   if (tv) {
-    dt_adt_fast(raw_dt, dt_in, a_in, dt_bias, dt, adt);
-    tr = sigmoid_fast(tr_in);
+    dt_adt_x<LO>(raw_dt, dt_in, a_in, dt_bias, dt, adt);
+    tr = sigmoid_x<LO>(tr_in);
   }
   const float own = dt * (1.f - tr);
   float right = __shfl_down(own, 1);
   if (j == TOK - 1) {
     float dn, an;
-    dt_adt_fast(raw_dt, dtn_in, 0.f, dt_bias, dn, an);
-    right = dn * (1.f - sigmoid_fast(trn_in));
+    dt_adt_x<LO>(raw_dt, dtn_in, 0.f, dt_bias, dn, an);
+    right = dn * (1.f - sigmoid_x<LO>(trn_in));
   }
   if (!nv) right = 0.f;
   const float gamma = dt * tr;
@@ -441,10 +465,10 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
     o[B::CUM + j] = cv;
     o[B::SCL + j] = tv ? scale : 0.f;
     o[B::GAM + j] = gamma;
-    o[B::BSC + j] = tv ? scale * __expf(cend - cv) : 0.f;
+    o[B::BSC + j] = tv ? scale * exp_x<LO>(cend - cv) : 0.f;
     if ((j & (TPT - 1)) == 0) o[B::CEND + j / TPT] = cend;
     if (j == 0) {
-      o[B::ECL] = __expf(cum_last);
+      o[B::ECL] = exp_x<LO>(cum_last);
       o[B::CL] = cum_last;
     }
   }
@@ -473,7 +497,7 @@ constexpr int norm_rows() {
 }
 constexpr int kAngQuads = 4;  // (4-token group, angle) pairs per lane of prep_kernel
 
-template <typename T, int R>
+template <typename T, int R, bool LO>
 __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const ScanGeom g,
                                                    float* __restrict__ ws, int nb_norm,
                                                    int nb_ang, int head_groups) {
@@ -773,7 +797,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
           const int j = lane & (TOK - 1);
           for (int hb = w * HPW; hb < hn; hb += 4 * HPW) {
             const int hh = hb + lane / TOK, hc = min(hh, hn - 1);
-            scalar_block_seg<TOK, TPT>(
+            scalar_block_seg<TOK, TPT, LO>(
                 a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
                 c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
                 s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
@@ -781,7 +805,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
         } else {
           for (int hh = w; hh < hn; hh += 4) {
             const int h = h0 + hh, j = min(lane, TOK - 1);
-            scalar_block<TOK, TPT>(
+            scalar_block<TOK, TPT, LO>(
                 a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
                 lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
                 s_in[2][TOK][hh], cut);
@@ -807,7 +831,14 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
 // last k and phase block sums but no outputs: the stores of Qs, VR, ZR, Sb and the output are left
 // out, and with them (dead code) the q math, the scores, the decay weights, the intra and inter
 // products and the epilogue.
-template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false>
+// LO (FP32): d_state no power of 2. Those calls came from the recurrent scan and are no further from
+// 64 bits than there: its functions (exp_x, sincos_of), and sums taken apart from what they are
+// added to (a matrix instruction rounds at the size of its accumulator four times). Errors of 2 x
+// 500 tokens, hook form, output and state: d_state 96 rank 1 recurrent 1.5e-7 and 2.4e-7, without
+// these 1.9e-7 and 1.5e-7, with them 1.2e-7 and 1.2e-7; rank 8 1.4e-7 and 2.4e-7, 1.3e-7 and 3.2e-7,
+// 0.9e-7 and 1.4e-7; given phases of 10^5 at rank 1 1.8e-7 and 2.5e-7, 3e-4 and 1.5e-3, 1.2e-7 and
+// 1.3e-7.
+template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false, bool LO = false>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, const ScanGeom g,
                                                         const float* __restrict__ prep) {
   using M = Mma<T>;
@@ -817,7 +848,8 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   constexpr int WPR = kWaves / RT;     // waves sharing one query row tile
   constexpr int TOK = ROWS / R;        // tokens per sub-chunk
   constexpr bool F32 = sizeof(T) == 4;
-  static_assert(F32 || !(FULL || SHAPE || SO), "16-bit calls of those forms take scan16_kernel");
+  static_assert(F32 || !(FULL || SHAPE || SO || LO), "16-bit calls of those forms take scan16_kernel");
+  static_assert(!LO || !(FULL || SHAPE), "the model's d_state is a power of 2");
   constexpr int ES = sizeof(T);
   constexpr int LQ = Lay::LQ, LR = Lay::LR, LP = Lay::LP, NP = kNPad, CST = Lay::CST;
   using SB_ = ScBlk<TOK>;
@@ -1116,7 +1148,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
   if (ph_on && nsub > 0) {
     float pa[TPL];
     angles_of(pa);
-    phase_stage<PG, TPL, CST, false, F32>(csb(0), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
+    phase_stage<PG, TPL, CST, false, F32, LO ? kFull : kFast>(csb(0), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
                                      scb(0) + SB_::DTV, 0, L, pg, lane, angles, pa, fph, fblk,
                                      blk_stride);
   }
@@ -1207,8 +1239,8 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       if constexpr (!KTR) {
         const int r0 = (2 * rp) / R, r1 = (2 * rp + 1) / R;
         const float cl = SC[SB_::CL];
-        const float e0 = SC[SB_::SCL + r0] * __expf(cl - SC[SB_::CUM + r0]);
-        const float e1 = SC[SB_::SCL + r1] * __expf(cl - SC[SB_::CUM + r1]);
+        const float e0 = SC[SB_::SCL + r0] * exp_x<LO>(cl - SC[SB_::CUM + r0]);
+        const float e1 = SC[SB_::SCL + r1] * exp_x<LO>(cl - SC[SB_::CUM + r1]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int n = n0 + i;
@@ -1399,8 +1431,10 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
         for (int kk = 0; kk < NP / 16; ++kk) {
           const f4 kv = *reinterpret_cast<const f4*>(Ks + (16 * sj + l16) * LQ + 16 * kk + 4 * lg);
+          f4 sum = LO ? zero4() : acc[sj];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[sj] = M::mma(kv[i], qf[kk][i], acc[sj]);
+          for (int i = 0; i < 4; ++i) sum = M::mma(kv[i], qf[kk][i], sum);
+          acc[sj] = LO ? acc[sj] + sum : sum;
         }
       }
     }
@@ -1437,13 +1471,19 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           st[k] = M::mma(av, bv, st[k]);
         }
       } else {
+        f4 sum = LO ? zero4() : st[k];
 #pragma unroll
         for (int kk = 0; kk < ROWS; kk += 16) {
           const f4 kv = *reinterpret_cast<const f4*>(KT + nrow * LR + swz<ROWS>(kk + 4 * lg, nrow >> KSH));
           const f4 vv = *reinterpret_cast<const f4*>(VT + prow * LR + swz<ROWS>(kk + 4 * lg, prow >> VSH));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) st[k] = M::mma(kv[i], vv[i], st[k]);
+          for (int i = 0; i < 4; ++i) sum = M::mma(kv[i], vv[i], sum);
         }
+        if constexpr (LO) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum[i] += st[k][i];
+        }
+        st[k] = sum;
       }
     }
     if constexpr (FULL || SHAPE) loads_vz();
@@ -1451,7 +1491,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     if (ph_on && c + 1 < nsub) {
       float pa[TPL];
       angles_of(pa);
-      phase_stage<PG, TPL, CST, false, F32>(csb(c + 1), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
+      phase_stage<PG, TPL, CST, false, F32, LO ? kFull : kFast>(csb(c + 1), ps, F + Lay::PBASE + ps, F + Lay::POFF + ps,
                                        scb(c + 1) + SB_::DTV, t0 + TOK, L, pg, lane, angles, pa,
                                        fph, fblk, blk_stride);
     }
@@ -1474,7 +1514,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       if (sj > it) continue;
       if (sj < it) {
         // strictly earlier tile: d = exp(cum_t - cend) * (scale_s exp(cend - cum_s)), both <= 1
-        const float at = __expf(cum_t - SC[SB_::CEND + sj]);
+        const float at = exp_x<LO>(cum_t - SC[SB_::CEND + sj]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int ts = (16 * sj + 4 * lg + i) / R;
@@ -1502,7 +1542,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int ts = (16 * sj + 4 * lg + i) / R;
-          const float lower = sc[i] * __expf(cum_t - cs[i]);
+          const float lower = sc[i] * exp_x<LO>(cum_t - cs[i]);
           const float d = tq_m > ts ? lower : (tq_m == ts ? gam_t : 0.f);
           wsc[sj][i] = acc[sj][i] * d;
         }
@@ -1510,7 +1550,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     }
     // Outputs, computed transposed (Y^T tiles, rows p, columns the row tile's 16 (token, rank)
     // rows): a lane holds 4 consecutive p of one row, stored as one vector.
-    const float ecum_t = __expf(cum_t);
+    const float ecum_t = exp_x<LO>(cum_t);
     const int rr = trow - tq * R;  // the lane's rank
 #pragma unroll
     for (int pq = 0; pq < kPT / WPR; ++pq) {
@@ -1559,8 +1599,10 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
         for (int kk = 0; kk < NP / 16; ++kk) {
           const f4 sv = *reinterpret_cast<const f4*>(Sb + pcol * LQ + 16 * kk + 4 * lg);
+          f4 sum = LO ? zero4() : ye;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) ye = M::mma(sv[i], qf[kk][i], ye);
+          for (int i = 0; i < 4; ++i) sum = M::mma(sv[i], qf[kk][i], sum);
+          ye = LO ? ye + sum : sum;
         }
       }
       // epilogue: row trow (token tq, rank rr), columns pb .. pb+3
@@ -1586,7 +1628,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
       f4 y;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * vv[i]) * silu_fast(zz[i]);
+        y[i] = (fmaf(ye[i], ecum_t, yi[i]) + Dh * vv[i]) * silu_x<LO>(zz[i]);
         if (R > 1) y[i] *= F[Lay::MO + rr * kPPad + pb + i];
       }
       if constexpr (R > 1) {
@@ -1983,7 +2025,13 @@ __global__ __launch_bounds__(kCompBlock) void compose_kernel(const m3_scan_args 
           __builtin_amdgcn_s_sleep(2);
         }
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        if (part >= 0) __sincosf(s_phig[g * S + j], &sn, &cs);
+        if (part >= 0) {
+          if (sizeof(T) == 4 && (N & (N - 1)) != 0) {
+            sincos_of<kFull>(s_phig[g * S + j], &sn, &cs);
+          } else {
+            __sincosf(s_phig[g * S + j], &sn, &cs);
+          }
+        }
         if (lead && tb < S) sg.in_phase[sh * S + tb] = s_phig[g * S + tb];
       }
 
@@ -2296,12 +2344,12 @@ static bool model_shape(const m3_scan_args& a, ScanGeom& g, int es) {
   return true;
 }
 
-template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false>
+template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false, bool LO = false>
 static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* prep, dim3 grid,
                          dim3 block, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SHAPE, SO>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&scan_kernel<T, R, FULL, SHAPE, SO, LO>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize,
                                        Layout<T>::BYTES);
     if (e != hipSuccess) {
@@ -2309,7 +2357,7 @@ static int launch_kernel(const m3_scan_args& a, const ScanGeom& g, const float* 
     }
     attr_set = true;
   }
-  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SHAPE, SO>), grid, block, Layout<T>::BYTES, stream,
+  hipLaunchKernelGGL((scan_kernel<T, R, FULL, SHAPE, SO, LO>), grid, block, Layout<T>::BYTES, stream,
                      a, g, prep);
   return check_launch("m3_scan_fwd");
 }
@@ -2360,9 +2408,16 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
     const int64_t nb_ang = (ang / 4 + 256 * kAngQuads - 1) / (256 * kAngQuads), nb_sc = blocks;
     if (run_prep && nb_norm + nb_ang + nb_sc > 0) {
       const dim3 pgrid(static_cast<unsigned>(nb_norm + nb_ang + nb_sc)), pblock(256);
-      hipLaunchKernelGGL((prep_kernel<T, R>), pgrid, pblock, 0, stream, a, g,
-                         static_cast<float*>(a.workspace), static_cast<int>(nb_norm),
-                         static_cast<int>(nb_ang), head_groups);
+      auto launch_prep = [&](auto lo) {
+        hipLaunchKernelGGL((prep_kernel<T, R, decltype(lo)::value>), pgrid, pblock, 0, stream, a, g,
+                           static_cast<float*>(a.workspace), static_cast<int>(nb_norm),
+                           static_cast<int>(nb_ang), head_groups);
+      };
+      if (g.lo) {
+        launch_prep(std::true_type{});
+      } else {
+        launch_prep(std::false_type{});
+      }
       int rc = check_launch("m3_scan_fwd (prep)");
       if (rc != M3_OK) return rc;
     }
@@ -2379,6 +2434,10 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
     if (prep != nullptr && model_shape(a, g, static_cast<int>(sizeof(T)))) {
       if (state_only) return launch_kernel<T, R, false, true, true>(a, g, prep, grid, block, stream);
       return launch_kernel<T, R, false, true>(a, g, prep, grid, block, stream);
+    }
+    if (g.lo) {
+      if (state_only) return launch_kernel<T, R, false, false, true, true>(a, g, prep, grid, block, stream);
+      return launch_kernel<T, R, false, false, false, true>(a, g, prep, grid, block, stream);
     }
     if (state_only) return launch_kernel<T, R, false, false, true>(a, g, prep, grid, block, stream);
   }

@@ -349,7 +349,8 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       } else {
         pa[0] = ANG[4 * ang_slot(pg >> 2, ps) + (pg & 3)];  // token pg of its 4-token group
       }
-      phase_stage<PG, TPL, CST, true, false>(cst(c), ps, F_ + Ly::PBASE + ps, F_ + Ly::POFF + ps,
+      phase_stage<PG, TPL, CST, true, false, GIVEN && LO ? kWide : kFast>(
+          cst(c), ps, F_ + Ly::PBASE + ps, F_ + Ly::POFF + ps,
                                              F_ + slot + SB_::DTV, c * TOK, L, pg, lane, !GIVEN, pa,
                                              fph, fblk, blk_stride);
     }

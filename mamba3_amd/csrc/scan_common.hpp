@@ -376,10 +376,34 @@ __device__ __forceinline__ int cs_col(int col, int tt) {
   return SWZ ? col ^ (4 * ((tt >> 4) & 3)) ^ (2 * ((tt >> 1) & 1)) : col;
 }
 
+// How a phase becomes cos and sin. kFast: the hardware functions (the phase times 1 / 2 pi in FP32:
+// an error of |phase| 2^-24, for phases reduced below a few turns). The calls that came from the
+// recurrent scan, which takes any given phase to full precision (LO), keep that: kFull the library's
+// functions (FP32), kWide the hardware functions of the turns reduced in 64 bits (16-bit: hook form;
+// the phase times 1 / 2 pi as two doubles, its product error folded in: exact to the hardware
+// functions' own error below 10^20).
+enum Trig { kFast, kFull, kWide };
+
+template <Trig TR>
+__device__ __forceinline__ void sincos_of(float x, float* s, float* c) {
+  if constexpr (TR == kFast) {
+    __sincosf(x, s, c);
+  } else if constexpr (TR == kFull) {
+    sincosf(x, s, c);
+  } else {
+    constexpr double kHi = 0x1.45f306dc9c883p-3, kLo = -0x1.6b01ec5417056p-57;  // 1 / 2 pi
+    const double xd = x, t = xd * kHi;
+    double r = (t - __builtin_rint(t)) + (__builtin_fma(xd, kHi, -t) + xd * kLo);
+    r -= __builtin_rint(r);
+    *s = __builtin_amdgcn_sinf(static_cast<float>(r));
+    *c = __builtin_amdgcn_cosf(static_cast<float>(r));
+  }
+}
+
 // Bounded phase (model.py:215-256) of tokens TPL pg .. TPL pg + TPL-1 of the sub-chunk at t0 for
 // angle ps: fmod-reduced increments summed within 64-token blocks, an fmod-reduced carry between
 // blocks, the running block sum and carry in pbase / poff; cos / sin into the table of angle ps.
-template <int PG, int TPL, int CST, bool SWZ, bool EXACT>
+template <int PG, int TPL, int CST, bool SWZ, bool EXACT, Trig TR>
 __device__ __forceinline__ void phase_stage(float* tab, int ps, float* pbase, float* poff,
                                             const float* dtv, int t0, int L, int pg, int lane,
                                             bool angles, const float (&pa)[TPL], float* fph,
@@ -453,7 +477,7 @@ __device__ __forceinline__ void phase_stage(float* tab, int ps, float* pbase, fl
   for (int i = 0; i < TPL; ++i) {
     const int tt = TPL * pg + i;
     float2 v;
-    __sincosf(ph[i], &v.y, &v.x);
+    sincos_of<TR>(ph[i], &v.y, &v.x);
     *reinterpret_cast<float2*>(tab + tt * CST + 2 * cs_col<SWZ>(ps, tt)) = v;
   }
 }

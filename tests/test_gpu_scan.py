@@ -338,3 +338,39 @@ def test_recurrent_scan_matches_oracle(shape, dtype):
     # equally accurate against FP32 (the accuracy checks) agree on fewer elements (97.1%)
     _check(dtype, y.cpu(), s.cpu(), y_ref, s_ref, inp, chunk,
            min_inside=0.96 if d_state >= 1024 else 0.985)
+
+
+@pytest.mark.parametrize("rank,d_state,span", [(1, 96, 6.0), (1, 100, 1e4), (2, 48, 1e6), (4, 112, 6.0),
+                                               (8, 80, 1e7)])
+@pytest.mark.parametrize("segments", [1, 4])
+def test_fp32_widths_no_power_of_two_are_exact(rank, d_state, span, segments, monkeypatch):
+    """FP32 at a d_state that is no power of 2, unsplit and split, against the float64 recurrence:
+    a few roundings of 2^-24 in each of some hundred decaying terms, 16 x 2^-24 for the whole; the
+    given phases count to full precision at any number of turns."""
+    from oracle.recurrence import recurrent_scan
+    monkeypatch.setattr(ops, "SCAN_SEGMENTS", segments)
+    length, heads = 256, 3
+    inp = _inputs(rank, torch.float32, batch=1, length=length, heads=heads, head_dim=32,
+                  d_state=d_state, seed=d_state, initial=False)
+    inp["phase"] = inp["phase"] * (span / 6)
+    q, k = (inp[n].double().expand(-1, -1, heads, -1, -1) + inp[n + "_bias"].double()
+            for n in ("q", "k"))
+    s = d_state // 4
+    i = torch.arange(s)
+    a, b = (2 * i, 2 * i + 1) if rank == 1 else (i, 2 * s + i)
+    cos, sin = (f(inp["phase"].double()).unsqueeze(-2) for f in (torch.cos, torch.sin))
+    for t in (q, k):
+        x, y = t[..., a].clone(), t[..., b].clone()
+        t[..., a], t[..., b] = x * cos - y * sin, x * sin + y * cos
+    mimo = {n: inp[n] for n in ("mimo_x", "mimo_z", "mimo_out") if n in inp}
+    want, want_state = recurrent_scan(q, k, inp["value"], inp["gate"], inp["adt"], inp["dt"],
+                                      inp["trap_logits"], inp["D"], **mimo)
+    dev = {n: (t.to(DEV) if isinstance(t, torch.Tensor) else t) for n, t in inp.items()}
+    with torch.inference_mode():
+        got, state = ops.mamba3_scan(**dev)
+    for name, x, ref in (("output", got, want), ("state", state, want_state)):
+        ref = torch.from_numpy(ref)
+        err = ((x.double().cpu() - ref).norm() / ref.norm()).item()
+        print(f"FP32 d_state {d_state} R={rank} span {span:g} segments {segments}: {name} {err:.2e}",
+              flush=True)
+        assert err <= 16 * 2.0 ** -24

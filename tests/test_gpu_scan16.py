@@ -134,6 +134,22 @@ def test_widths_no_power_of_two_are_as_exact_as_the_recurrent_scan(rank, d_state
     assert es <= 1.01 * rs
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rank,d_state,span", [(1, 96, 30.0), (1, 96, 1e4), (2, 48, 1e6), (8, 80, 1e7)])
+def test_given_phases_need_no_reduction(rank, d_state, span, dtype):
+    """Given phases of many turns at a d_state that is no power of 2: cos and sin to full
+    precision whatever the phase, as the recurrent scan takes them (the hardware functions alone
+    are off by 2^-24 of the phase: 0.06 at 1e6, where every bar here would be missed)."""
+    inp = _inputs(rank, dtype, batch=1, length=200, heads=3, groups=1, head_dim=32, d_state=d_state,
+                  angles=d_state // 4, bias=True, initial=True, seed=5)
+    inp["phase"] = inp["phase"] * (span / 6)
+    want, want_state = _oracle32(inp)
+    got, state = ops.mamba3_scan(**{n: (t.to(DEV) if isinstance(t, torch.Tensor) else t)
+                                    for n, t in inp.items()})
+    _close(got, want, dtype)
+    _close(state, want_state, dtype)
+
+
 @pytest.mark.parametrize("layout", ["padded", "head_major", "unaligned"])
 def test_hook_form_layouts(layout):
     """Rows padded to a longer token stride, q / k and value / gate as slices of one buffer,
