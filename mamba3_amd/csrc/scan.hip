@@ -396,7 +396,7 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
   if (!nv) right = 0.f;
   const float gamma = dt * tr;
   const float scale = gamma + right;
-  const float cum = wave_incl_scan(adt, lane);
+  const float cum = wave_incl_scan(LO && adt < kDecayLow ? kDecayLow : adt, lane);
   const float cum_last = readlane_f(cum, wn - 1);
   const float cv = tv ? cum : cum_last;
   // cum at the end of this lane's 16-row tile (TPT tokens), clamped to the last valid token
@@ -416,6 +416,10 @@ __device__ __forceinline__ void scalar_block(const m3_scan_args& a, float* __res
     o[B::GAM + lane] = gamma;
     o[B::BSC + lane] = tv ? scale * exp_x<LO>(cend - cv) : 0.f;
     if ((lane & (TPT - 1)) == 0) o[B::CEND + lane / TPT] = cend;
+  }
+  if constexpr (LO) {
+    const float sum = readlane_f(wave_incl_scan(adt, lane), wn - 1);
+    if (lane == 0) o[B::DEC] = sum;
   }
   if (lane == 0) {
     o[B::ECL] = exp_x<LO>(cum_last);
@@ -456,10 +460,14 @@ __device__ __forceinline__ void scalar_block_seg(const m3_scan_args& a, float* _
   if (!nv) right = 0.f;
   const float gamma = dt * tr;
   const float scale = gamma + right;
-  const float cum = seg_incl_scan<TOK>(adt, lane);
+  const float cum = seg_incl_scan<TOK>(LO && adt < kDecayLow ? kDecayLow : adt, lane);
   const float cum_last = __shfl(cum, s0 + wn - 1);
   const float cv = tv ? cum : cum_last;
   const float cend = __shfl(cv, s0 + min(j | (TPT - 1), wn - 1));
+  if constexpr (LO) {
+    const float sum = __shfl(seg_incl_scan<TOK>(adt, lane), s0 + wn - 1);
+    if (live && j == 0) o[B::DEC] = sum;
+  }
   if (live) {
     o[B::DTV + j] = dt;
     o[B::CUM + j] = cv;
@@ -1350,7 +1358,7 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
     // onto it
     {
       const float ecl = SC[SB_::ECL];
-      log_decay += SC[SB_::CL];
+      log_decay += SC[LO ? SB_::DEC : SB_::CL];
 #pragma unroll
       for (int k = 0; k < kTiles; ++k) {
 #pragma unroll

@@ -626,7 +626,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   auto decay_state = [&](const float* SC) {
     {
       const float ecl = SC[SB_::ECL];
-      log_decay += SC[SB_::CL];
+      log_decay += SC[LO ? SB_::DEC : SB_::CL];
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
 #pragma unroll

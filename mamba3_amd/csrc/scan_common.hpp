@@ -90,13 +90,20 @@ template <typename T> struct Layout {
 // Per-token scalar block of one sub-chunk of TOK tokens (floats, token-indexed arrays): dt, the
 // within-chunk cumsum of adt, the exp-trapezoid scale, gamma, scale * decay to the end of the
 // token's 16-row tile; then the cumsum at each tile end, exp of the last cumsum and the last
-// cumsum itself. The prep pass writes them; the scan copies them to LDS (and takes exp(cum) and
+// cumsum itself. LO (d_state no power of 2): the cumsum counts a step below kDecayLow as that, and
+// DEC holds the sum of the steps as they are. The prep pass writes them; the scan copies them to LDS (and takes exp(cum) and
 // scale * exp(cum_last - cum) from them itself, an exp per lane).
 template <int TOK> struct ScBlk {
   static constexpr int DTV = 0, CUM = TOK, SCL = 2 * TOK, GAM = 3 * TOK, BSC = 4 * TOK;
   static constexpr int CEND = 5 * TOK, ECL = 5 * TOK + 4, CL = 5 * TOK + 5;
+  static constexpr int DEC = 5 * TOK + 6;
   static constexpr int SIZE = 5 * TOK + 8;
 };
+
+// exp of it is 0 in FP32. A step that resets the state (adt = -inf, or any value far below this)
+// makes differences of a plain cumsum NaN, or loses the steps after it to the sum's rounding; the
+// recurrent scan, where the LO calls came from, multiplies by exp(adt) and takes it as it is.
+constexpr float kDecayLow = -104.f;
 
 // Per-launch values shared by host and device.
 struct ScanGeom {

@@ -374,3 +374,33 @@ def test_fp32_widths_no_power_of_two_are_exact(rank, d_state, span, segments, mo
         print(f"FP32 d_state {d_state} R={rank} span {span:g} segments {segments}: {name} {err:.2e}",
               flush=True)
         assert err <= 16 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rank,d_state", [(1, 96), (4, 48), (8, 80)])
+@pytest.mark.parametrize("low", [-float("inf"), torch.finfo(torch.float32).min, -1e4])
+@pytest.mark.parametrize("segments", [1, 4])
+def test_a_reset_leaves_the_steps_after_it_exact(low, rank, d_state, dtype, segments, monkeypatch):
+    """adt of -inf, the lowest FP32 value or -1e4 resets the state (exp(adt) is 0). At a d_state
+    that is no power of 2, where the recurrent scan took it, the tokens after it decay by their own
+    adt. Against the float64 recurrence: FP32 within 2^-16 (cum keeps a multiple of 104 in the
+    sub-chunk: 2^-24 x 208 in an exponent), bf16 at the 16-wave test's 3 x 2^-9."""
+    from oracle.recurrence import recurrent_scan
+    monkeypatch.setattr(ops, "SCAN_SEGMENTS", segments)
+    heads = 3
+    inp = _inputs(rank, dtype, batch=1, length=256, heads=heads, head_dim=32, d_state=d_state,
+                  seed=9, initial=False, phase=False, bias=False)
+    inp["adt"][:, [5, 100, 130, 200]] = low
+    mimo = {n: inp[n].to(dtype).float() if n != "mimo_out" else inp[n]
+            for n in ("mimo_x", "mimo_z", "mimo_out") if n in inp}
+    q, k = (inp[n].double().expand(-1, -1, heads, -1, -1) for n in ("q", "k"))
+    want, want_state = recurrent_scan(q, k, inp["value"].double(), inp["gate"].double(),
+                                      inp["adt"], inp["dt"], inp["trap_logits"].double(), inp["D"],
+                                      **mimo)
+    dev = {n: (t.to(DEV) if isinstance(t, torch.Tensor) else t) for n, t in inp.items()}
+    with torch.inference_mode():
+        got, state = ops.mamba3_scan(**dev)
+    bar = 2.0 ** -16 if dtype == torch.float32 else 3 * 2.0 ** -9
+    for x, ref in ((got, want), (state, want_state)):
+        ref = torch.from_numpy(ref)
+        assert ((x.double().cpu() - ref).norm() / ref.norm()).item() <= bar
