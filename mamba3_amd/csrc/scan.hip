@@ -2475,6 +2475,11 @@ static int sub_chunk_tokens(const m3_scan_args& a) {
 //   1 x 8192, 32 heads:  348; 4 170, 8 110, 16 124            3 x 3072, 24 heads: 144; 2 138, 3 109, 6 122
 //   1 x 61440, 24 heads: 2528; 8 596, 10 500, 16 609, 32 506  4 x 2048, 32 heads: 104; 2 112
 //   1 x 512, 64 heads:   38; 2 52, 4 52                       FP32 2 x 1024, 8 heads: 240; 4 149, 8 100, 16 84
+//
+// A count that does not divide the sequence is taken back as an explicit request only where it is
+// the choice for one of 1 .. kOwnCalls concurrent calls; for more calls the choice is among the
+// counts that divide it, which every request may name.
+constexpr int kOwnCalls = 4;
 constexpr double kStateOnly = 0.53, kCompose = 4.5, kPerSeg = 0.11, kWalk = 0.02;
 
 struct Segments {
@@ -2484,6 +2489,11 @@ struct Segments {
 static Segments cut(int64_t len, int64_t unit, int64_t count) {
   const int64_t ls = (len + count * unit - 1) / (count * unit) * unit;
   return Segments{static_cast<int>((len + ls - 1) / ls), static_cast<int>(ls)};
+}
+
+// Whether `count` segments divide the sequence (into whole phase blocks with angle increments).
+static bool divides(const m3_scan_args& a, int64_t count) {
+  return a.length % (count * (a.phase_mode == M3_PHASE_ANGLES ? 64 : 1)) == 0;
 }
 
 static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurrent) {
@@ -2499,7 +2509,7 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
     const Segments s = cut(len, unit, n);
     const int shortest = f32 ? (n <= 16 ? 2 : 4) : (n <= 8 ? 4 : 8);
     if (s.len < shortest * tok) break;
-    if (s.count != n) continue;
+    if (s.count != n || (concurrent > kOwnCalls && !divides(a, n))) continue;
     const double cost = rounds(n) * (2 * prologue + (1.0 + kStateOnly) * static_cast<double>(s.len / tok)) +
                         kCompose + kPerSeg * n + walk;
     if (cost < best_cost * (1.0 - 1e-9)) {
@@ -2535,12 +2545,11 @@ static Segments segments_for(const m3_scan_args& a, int concurrent = 1) {
   if (a.segments < 0) return Segments{-1, 0};
   const int64_t unit = a.phase_mode == M3_PHASE_ANGLES ? 64 : sub_chunk_tokens(a);
   if (a.segments == 0) return auto_segments(a, unit, concurrent > 1 ? concurrent : 1);
-  // an explicit count divides the sequence (into whole phase blocks), or is the library's own
-  // choice for a few concurrent calls (m3_scan_segments), whose last segment may be shorter
-  const int64_t align = a.phase_mode == M3_PHASE_ANGLES ? 64 : 1;
+  // an explicit count divides the sequence, or is the library's own choice (m3_scan_segments),
+  // whose last segment may be shorter
   if (a.segments <= kMaxSegments && static_cast<int64_t>(a.batch) * a.heads * a.segments <= INT32_MAX) {
-    if (len % (a.segments * align) == 0) return cut(len, unit, a.segments);
-    for (int c = 1; c <= 4; ++c) {
+    if (divides(a, a.segments)) return cut(len, unit, a.segments);
+    for (int c = 1; c <= kOwnCalls; ++c) {
       const Segments s = auto_segments(a, unit, c);
       if (s.count == a.segments) return s;
     }
@@ -2659,8 +2668,8 @@ static int launch_scan_r(const m3_scan_args& a, bool rows, hipStream_t stream) {
   const Segments s = segments_for(a);
   if (s.count < 0) {
     return fail(M3_EUNSUPPORTED,
-                "m3_scan_fwd: %d segments need 1 < segments <= 256 dividing L into whole "
-                "64-token blocks (angle phases)",
+                "m3_scan_fwd: %d segments: a request is 1 < segments <= 256 dividing L (into whole "
+                "64-token blocks with angle phases), or a count m3_scan_segments gave",
                 a.segments);
   }
   if (s.count > 1) return launch_segmented<T, R>(a, s, rows, stream);

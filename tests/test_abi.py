@@ -260,6 +260,38 @@ def test_scan_segment_choice_on_the_host(lib):
     assert lib.m3_scan_segments(ctypes.byref(args), 0, ctypes.byref(g)) == 1
 
 
+def _with_angles(args: _hip.ScanArgs) -> _hip.ScanArgs:
+    """The hook-form arguments with angle increments (segments on 64-token blocks)."""
+    args.phase_mode, args.num_angles = _hip.PHASE_ANGLES, 16
+    args.phase.ptr, args.phase.dtype = 0x90000000, _hip.BF16
+    for i, stride in enumerate((args.length * 16, 16, 1)):
+        args.phase.stride[i] = stride
+    return args
+
+
+@pytest.mark.parametrize("angles", [False, True])
+def test_the_chosen_segment_count_can_be_passed_back(lib, angles):
+    """m3_scan_segments' answer for any number of concurrent calls is a request m3_scan_fwd takes:
+    with a workspace that is too small it stops there (4), not at the count (2)."""
+    g = ctypes.c_int(0)
+    split = 0
+    for batch, heads in ((1, 8), (1, 24), (2, 16), (4, 8), (1, 64)):
+        for length in (500, 1033, 1055, 1777, 2500, 4097, 6144, 10007, 65537):
+            for concurrent in range(1, 17):
+                args = _hook_scan_args(batch, length, heads, 0)
+                if angles:
+                    _with_angles(args)
+                assert lib.m3_scan_segments(ctypes.byref(args), concurrent, ctypes.byref(g)) == 0
+                args.segments = chosen = g.value
+                split += chosen > 1
+                what = (batch, heads, length, concurrent, chosen)
+                assert lib.m3_scan_segments(ctypes.byref(args), 1, ctypes.byref(g)) == 0, what
+                assert g.value == chosen, what
+                assert lib.m3_scan_fwd(ctypes.byref(args), None) == 4, what
+                assert b"workspace" in lib.m3_last_error()
+    assert split > 100
+
+
 def test_scan_backwards_token_strides_on_the_host(lib):
     """Per-token tensors may run backwards (the reverse scan), but all of them together."""
     args = _hook_scan_args(1, 128, 2, 1)
