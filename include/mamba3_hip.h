@@ -90,7 +90,9 @@ typedef struct {
   int32_t mimo_rotation;  /* 0: SISO adjacent pairs (2i, 2i+1); 1: MIMO quarters (i, 2S + i) */
   int32_t raw_dt;         /* 0: dt / a are FP32 dt / adt; 1: raw logits (see above) */
   int32_t phase_mode;     /* M3_PHASE_* */
-  int32_t segments;       /* 0: the library picks; 1: one pass per (b, h); G > 1: G segments */
+  int32_t segments;       /* 0: the library picks; 1: one pass per (b, h); G > 1: at most G segments,
+                             of ceil(L / G) tokens rounded up to whole sub-chunks (64 / R tokens in 16
+                             bits, 32 / R in FP32; 64 with angles) */
   float norm_eps;
   m3_tensor q, k;                   /* [B, L, G, R, N] */
   m3_tensor q_norm_w, k_norm_w;     /* [N] optional (C_norm.weight / B_norm.weight) */
@@ -120,9 +122,10 @@ typedef struct {
 /* Bytes of device workspace m3_scan_fwd needs for these arguments (0 is possible). */
 int m3_scan_workspace_size(const m3_scan_args* args, size_t* bytes);
 /*
- * The segment count m3_scan_fwd uses for these arguments when `concurrent_calls` calls of this
- * shape run on the GPU at once (1: alone); with args->segments == 0 the library picks it, else
- * the explicit request is checked. A caller running such calls together (the two directions of
+ * The segments request for these arguments when `concurrent_calls` calls of this shape run on the
+ * GPU at once (1: alone): with args->segments == 0 the library's choice, else the explicit request
+ * itself, after a check (it divides L, into whole 64-token blocks with angles, or is a choice given
+ * for 1 to 4 concurrent calls). m3_scan_fwd takes every answer as args->segments. A caller running such calls together (the two directions of
  * a bidirectional layer) passes the result as args->segments before sizing the workspace.
  * No counterpart in the reference, whose portable scan has no segments (ops.py:544-822).
  */

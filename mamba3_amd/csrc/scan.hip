@@ -2545,7 +2545,8 @@ static Segments segments_for(const m3_scan_args& a, int concurrent = 1) {
   if (a.segments < 0) return Segments{-1, 0};
   const int64_t unit = a.phase_mode == M3_PHASE_ANGLES ? 64 : sub_chunk_tokens(a);
   if (a.segments == 0) return auto_segments(a, unit, concurrent > 1 ? concurrent : 1);
-  // an explicit count divides the sequence, or is the library's own choice (m3_scan_segments),
+  // an explicit count divides the sequence (its segments are rounded up to whole sub-chunks: of a
+  // count above what that leaves, fewer run), or is the library's own choice (m3_scan_segments),
   // whose last segment may be shorter
   if (a.segments <= kMaxSegments && static_cast<int64_t>(a.batch) * a.heads * a.segments <= INT32_MAX) {
     if (divides(a, a.segments)) return cut(len, unit, a.segments);
@@ -2836,7 +2837,8 @@ extern "C" int m3_scan_segments(const m3_scan_args* args, int concurrent_calls,
     return m3::fail(M3_EUNSUPPORTED, "m3_scan_segments: the requested %d segments cannot be met",
                     args->segments);
   }
-  *segments = G;
+  // an explicit request is answered with itself (it can be passed back as it is)
+  *segments = args->segments > 0 ? args->segments : G;
   return M3_OK;
 }
 

@@ -292,6 +292,18 @@ def test_the_chosen_segment_count_can_be_passed_back(lib, angles):
     assert split > 100
 
 
+@pytest.mark.parametrize("length,request_", [(1000, 10), (100, 4), (60, 4), (1050, 10)])
+def test_a_request_of_short_segments_is_answered_with_itself(lib, length, request_):
+    """Requests whose segments are not whole sub-chunks (64 tokens here; fewer segments run then):
+    accepted, and the answer can be passed back."""
+    g = ctypes.c_int(0)
+    args = _hook_scan_args(1, length, 2, request_)
+    for concurrent in (1, 2, 7):
+        assert lib.m3_scan_segments(ctypes.byref(args), concurrent, ctypes.byref(g)) == 0
+        assert g.value == request_
+    assert lib.m3_scan_fwd(ctypes.byref(args), None) == 4  # stops at the workspace, not the count
+
+
 def test_scan_backwards_token_strides_on_the_host(lib):
     """Per-token tensors may run backwards (the reverse scan), but all of them together."""
     args = _hook_scan_args(1, 128, 2, 1)
