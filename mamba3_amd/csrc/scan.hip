@@ -526,15 +526,19 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     const int l16 = tid & 15, row0 = blk * 16 * kNormRows + (tid >> 4);
     const int N = a.d_state;
     const bool in = 8 * l16 < N;  // lanes past column N load column 0 and count zeros
-    // rows_out (the 16-wave scan): lane l16 holds the slots 8 l16 .. 8 l16 + 7 (slot_col) instead
-    // of the columns, as two 4-column chunks at ca and cb (a pair's two columns with the MIMO
-    // rotation, interleaved below); a chunk past column N counts zeros
-    const bool rows_out = sizeof(T) == 2 && g.form16 >= 0;
-    const bool pairs = rows_out && g.perm && 8 * l16 < 2 * a.num_angles;
+    // rows_out (the 16-wave scan's forms kModel, kRows and kCopy): the finished rows; lane l16 holds the slots 8 l16 ..
+    // 8 l16 + 7 (slot_col) instead of the columns, as two 4-column chunks at ca and cb (a pair's two
+    // columns with the MIMO rotation, interleaved below). Form kProj, whose factors alone are
+    // written, reads the same chunks where the rows start on 8 bytes only; a chunk past column N
+    // counts zeros.
+    const bool rows_out = sizeof(T) == 2 && g.ws_qk >= 0;
+    const int perm = rows_out ? g.perm : 0;
+    const bool pairs = perm && 8 * l16 < 2 * a.num_angles;
     const bool in_b = 8 * l16 + 4 < N;
-    const int ca = !in ? 0 : pairs ? 4 * l16 : slot_col(8 * l16, g.perm, a.num_angles);
+    const int ca = !in ? 0 : pairs ? 4 * l16 : slot_col(8 * l16, perm, a.num_angles);
     const int cb = !in_b ? 0 : pairs ? 4 * l16 + 2 * a.num_angles
-                                     : slot_col(8 * l16 + 4, g.perm, a.num_angles);
+                                     : slot_col(8 * l16 + 4, perm, a.num_angles);
+    const bool chunks = sizeof(T) == 2 && g.form16 >= 0 && (perm || !g.vec_qk);
     // Rows (token, group, rank, q | k): a lane's rows row0 + 16 k all have row0's parity, so one
     // tensor (q or k). When 2 gr_n divides 16 they also share its (group, rank), the token
     // advancing by 8 / gr_n per k: the addresses follow from row0's by additions (a division
@@ -542,8 +546,8 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     // instructions). Rows past the end re-read the last batch row's last token.
     const int which = row0 & 1;
     const m3_tensor& xt = which ? a.k : a.q;
-    // (rows_out: the chunks are added to the row's start below)
-    const T* xbase = static_cast<const T*>(xt.ptr) + (in && !rows_out ? 8 * l16 : 0);
+    // (the chunks are added to the row's start below)
+    const T* xbase = static_cast<const T*>(xt.ptr) + (in && !chunks ? 8 * l16 : 0);
     const int64_t xs0 = xt.stride[0], xs1 = xt.stride[1];
     const bool step_rows = 16 % (2 * gr_n) == 0;
     const int dtok = step_rows ? 8 / gr_n : 0;
@@ -572,7 +576,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
       const int b2 = tok / L, t2 = tok - b2 * L;
       const m3_tensor& x = wh ? a.k : a.q;
       return static_cast<const T*>(x.ptr) + b2 * x.stride[0] + t2 * x.stride[1] +
-             g2i * x.stride[2] + r2 * x.stride[3] + (in && !rows_out ? 8 * l16 : 0);
+             g2i * x.stride[2] + r2 * x.stride[3] + (in && !chunks ? 8 * l16 : 0);
     };
     float ss[kNormRows];
     uint32_t w8[kNormRows][Words<T>::W8];
@@ -586,7 +590,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
       nw_r[1][0] = ldraw4(a.k_norm_w, ca);
       nw_r[1][1] = ldraw4(a.k_norm_w, cb);
     }
-    if (rows_out && !(g.vec_qk && !g.perm)) {
+    if (chunks) {
       if constexpr (sizeof(T) == 2) {
 #pragma unroll
         for (int k = 0; k < kNormRows; ++k) {
@@ -612,7 +616,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
 #pragma unroll
       for (int k = 0; k < kNormRows; ++k) {
         // rows past the end re-read an earlier row; their sums are not stored
-        const T* p = row_ptr(k) + (rows_out && in ? 8 * l16 : 0);
+        const T* p = row_ptr(k);
 #pragma unroll
         for (int j = 0; j < Words<T>::W8; j += 4) {
           const uint4 q = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint32_t*>(p) + j);
@@ -655,15 +659,14 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     }
     if constexpr (sizeof(T) == 2) {
       if (rows_out) {
-        // the rows themselves, 128 slots (zeros past the call's columns): rnd(x * factor * rnd(w))
-        // for the model's shape (model.py:48-55: F.rms_norm with the weight in the activation
-        // dtype, the result in it), the same product in FP32 for form kProj, the given values
-        // without norm weights (the hook form). Rows (token, group, rank, q | k).
+        // the rows themselves: rnd(x * factor * rnd(w)) (model.py:48-55: F.rms_norm with the weight
+        // in the activation dtype, the result in it), in FP32 unrounded (kRows), or x, zeros past
+        // column N (kCopy). Rows (token, group, rank, q | k).
         // The lane's tensor's weights (every row of the lane is q, or every row k) are chosen by
         // bit masks on the raw words: a select between two weight arrays by `which` became a
         // dynamically indexed array in scratch memory
         const bool norm = a.q_norm_w.ptr != nullptr;
-        float wl[8];
+        float wl[8] = {};
         if (nw_vec) {
           const uint32_t msk = 0u - static_cast<uint32_t>(which);
           const int wdt = which ? a.k_norm_w.dtype : a.q_norm_w.dtype;
@@ -676,16 +679,13 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
 #pragma unroll
             for (int e = 0; e < 4; ++e) wl[4 * h2 + e] = rnd<T>(v4[e]);
           }
-        } else {
+        } else if (norm) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            const int n = min((i < 4 ? ca : cb) + (i & 3), N - 1);
-            wl[i] = 1.f;
-            if (norm) {
-              const float wq = ldx(a.q_norm_w.ptr, a.q_norm_w.dtype, n * a.q_norm_w.stride[0]);
-              const float wk = ldx(a.k_norm_w.ptr, a.k_norm_w.dtype, n * a.k_norm_w.stride[0]);
-              wl[i] = rnd<T>(which ? wk : wq);
-            }
+            const int n = (i < 4 ? ca : cb) + (i & 3);  // (a chunk past column N: column 0's)
+            const float wq = ldx(a.q_norm_w.ptr, a.q_norm_w.dtype, n * a.q_norm_w.stride[0]);
+            const float wk = ldx(a.k_norm_w.ptr, a.k_norm_w.dtype, n * a.k_norm_w.stride[0]);
+            wl[i] = rnd<T>(which ? wk : wq);
           }
         }
         char* qk = reinterpret_cast<char*>(ws) + g.ws_qk;
@@ -705,11 +705,12 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
             y[2 * i] = pairs ? x[i] : x[2 * i];
             y[2 * i + 1] = pairs ? x[4 + i] : x[2 * i + 1];
           }
-          const int64_t o = static_cast<int64_t>(row) * kNPad + 8 * l16;
-          if (g.form16 == kProj) {
-            st_row8<float>(reinterpret_cast<float*>(qk) + o, y);
+          if (g.form16 == kRows) {
+            float* o = reinterpret_cast<float*>(qk) + static_cast<int64_t>(row) * N + 8 * l16;
+            if (in) *reinterpret_cast<f4*>(o) = (f4){y[0], y[1], y[2], y[3]};
+            if (in_b) *reinterpret_cast<f4*>(o + 4) = (f4){y[4], y[5], y[6], y[7]};
           } else {
-            st_row8<T>(reinterpret_cast<T*>(qk) + o, y);
+            st_row8<T>(reinterpret_cast<T*>(qk) + static_cast<int64_t>(row) * kNPad + 8 * l16, y);
           }
         }
       }
@@ -2075,16 +2076,18 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // The form in which scan16_kernel takes a call (Form16), -1 when it does not: a 16-bit call of up
 // to 128 columns, 64 values and 32 angles at ranks 1, 2, 4 and 8, whose q / k / value / gate /
-// out rows can be read and written 4 elements at a time, each token's row (of one group, rank or
-// head) below the next token's, and whose offsets within a batch row fit 32 bits (the loads run
-// up to two sub-chunks, 128 tokens, and a token group ahead). Projection form: norm weights,
-// biases, raw dt, angle increments; hook form: none of the norms, phases given or none.
+// out rows can be read and written 4 elements at a time, each token's row (of one group or head)
+// below the next token's, and whose offsets within a batch row fit 32 bits (the loads run up to
+// two sub-chunks, 128 tokens, and a token group ahead). Projection form: norm weights, biases, raw
+// dt, angle increments; hook form: none of the norms, phases given or none. Rank 1 with the MIMO
+// rotation takes the other kernels. `rows` false: without the workspace for prep's rows (kModel's
+// shape and the ranks above 1 then take kProj and kHook, which read the caller's).
 // Every such call is faster on it than on the kernel it took before (per call, scan_kernel then
 // scan16_kernel, 8 x 1024 tokens, 32 heads): hook form rank 1 80 -> 72 us, rank 2 184 -> 118,
 // rank 4 332 -> 207, rank 8 628 -> 392; projection form rank 2 140 -> 121, rank 8 487 -> 391,
 // d_state 64 rank 1 114 -> 67; the recurrent scan at d_state 96, 4 x 1500 tokens, 16 heads:
 // 21.6 ms -> 86 us.
-static int form16_of(const m3_scan_args& a) {
+static int form16_of(const m3_scan_args& a, bool rows) {
   if (a.act_dtype != M3_BF16 && a.act_dtype != M3_F16) return -1;
   if (a.rank != 1 && a.rank != 2 && a.rank != 4 && a.rank != 8) return -1;
   const int N = a.d_state, P = a.head_dim, S = a.num_angles;
@@ -2095,7 +2098,7 @@ static int form16_of(const m3_scan_args& a) {
   const bool rotates = a.phase_mode != M3_PHASE_NONE;
   // the MIMO pairs' columns come in chunks of 4 (4 S == N there, 2 S <= N otherwise: validated)
   if (rotates && (a.mimo_rotation ? S % 4 != 0 || 4 * S != N : 2 * S > N)) return -1;
-  if (rotates && S <= 0) return -1;
+  if (rotates && (S <= 0 || (a.rank == 1 && a.mimo_rotation))) return -1;
   const bool norm = a.q_norm_w.ptr != nullptr && a.k_norm_w.ptr != nullptr;
   const bool proj = norm && a.q_bias.ptr != nullptr && a.k_bias.ptr != nullptr &&
                     a.raw_dt != 0 && a.dt_bias.ptr != nullptr && a.phase_mode == M3_PHASE_ANGLES;
@@ -2128,8 +2131,7 @@ static int form16_of(const m3_scan_args& a) {
     }
   }
   const int64_t tok = 64 / a.rank, nsub = (len + tok - 1) / tok;
-  if (ahead * a.groups * a.rank * 2 * kNPad * 4 >= INT32_MAX ||
-      (nsub + 3) * (5 * tok + 8) * 4 >= INT32_MAX) {
+  if ((proj && ahead * a.groups * a.rank * 8 >= INT32_MAX) || (nsub + 3) * (5 * tok + 8) * 4 >= INT32_MAX) {
     return -1;
   }
   if (a.phase_mode == M3_PHASE_ANGLES && ahead * S * 4 >= (int64_t{1} << 30)) return -1;
@@ -2157,16 +2159,27 @@ static int form16_of(const m3_scan_args& a) {
       (a.initial_k.stride[2] < 0 || (a.rank * a.initial_k.stride[2] + N) * 2 >= (int64_t{1} << 30))) {
     return -1;
   }
-  if (!proj) return kHook;
-  return N == kNPad && P == kPPad && S == kSMax && a.groups == 1 && (a.rank == 1 || a.rank == 4) &&
-                 (a.mimo_rotation != 0) == (a.rank > 1)
-             ? kModel
-             : kProj;
+  if (proj && rows && N == kNPad && P == kPPad && S == kSMax && a.groups == 1 &&
+      (a.rank == 1 || a.rank == 4) && (a.mimo_rotation != 0) == (a.rank > 1) &&
+      ahead * a.rank * 2 * kNPad * 2 < INT32_MAX) {
+    return kModel;
+  }
+  if (rows && a.rank > 1 && ahead * a.groups * a.rank * 2 * N * 4 < INT32_MAX) {
+    if (proj) return kRows;
+    if (a.heads >= 16 * a.groups && int64_t{2} * a.batch * len * a.groups * a.rank < INT32_MAX) return kCopy;
+  }
+  // the caller's rows: the ranks of a token's row below the next token's
+  for (const m3_tensor* t : {&a.q, &a.k}) {
+    const int64_t s1 = t->stride[1] < 0 ? -t->stride[1] : t->stride[1];
+    const int64_t span = (a.rank - 1) * t->stride[3] + N;
+    if (a.rank > 1 && t->stride[3] < 0) return -1;
+    if (len > 1 ? s1 < span : span * 2 >= INT32_MAX) return -1;
+  }
+  return proj ? kProj : kHook;
 }
 
 // Prep workspace regions (floats, each 16-byte aligned) and the sub-chunk geometry; returns the
-// workspace size in bytes. `form16`: form16_of(a), or -1 for a layout without the 16-wave scan's
-// rows.
+// workspace size in bytes. `form16`: form16_of(a).
 static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   const int rows = a.act_dtype == M3_F32 ? Mma<float>::ROWS : Mma<__bf16>::ROWS;
   const int rank = a.rank > 0 ? a.rank : 1;
@@ -2181,7 +2194,7 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   g.last_only = 0;
   g.perm = a.phase_mode != M3_PHASE_NONE && a.mimo_rotation != 0;
   g.lo = !pow2(a.d_state);
-  const bool norm = a.q_norm_w.ptr != nullptr && form16 < 0;
+  const bool norm = a.q_norm_w.ptr != nullptr && form16 != kModel && form16 != kRows;
   const bool angles = a.phase_mode == M3_PHASE_ANGLES;
   const int64_t batch = a.batch > 0 ? a.batch : 0;
   int64_t off = 0;
@@ -2197,10 +2210,10 @@ static size_t ws_layout(const m3_scan_args& a, ScanGeom& g, int form16) {
   // the projection form's 32-bit offsets run up to two sub-chunk strides past the end
   g.ws_bytes = bytes < (int64_t{1} << 30) ? static_cast<int>(bytes) : -1;
   g.ws_qk = -1;
-  if (form16 < 0) return static_cast<size_t>(bytes);
+  if (form16 != kModel && form16 != kRows && form16 != kCopy) return static_cast<size_t>(bytes);
   g.ws_qk = (bytes + 255) / 256 * 256;  // 256-byte aligned
-  return static_cast<size_t>(g.ws_qk + batch * len * a.groups * a.rank * 2 * kNPad *
-                                           (form16 == kProj ? 4 : 2));
+  return static_cast<size_t>(g.ws_qk + batch * len * a.groups * a.rank * 2 *
+                                           (form16 == kRows ? a.d_state * 4 : kNPad * 2));
 }
 
 template <typename T>
@@ -2399,7 +2412,7 @@ static int launch_pass(const m3_scan_args& a, hipStream_t stream, bool run_prep,
     }
     prep = static_cast<const float*>(a.workspace);
     const int64_t tokens = static_cast<int64_t>(a.batch) * a.length;
-    const int64_t nrow = g.ws_norm >= 0 || g.form16 >= 0 ? tokens * 2 * a.groups * a.rank : 0;
+    const int64_t nrow = g.ws_norm >= 0 || g.ws_qk >= 0 ? tokens * 2 * a.groups * a.rank : 0;
     const int64_t ang = g.ws_ang >= 0 ? static_cast<int64_t>(a.batch) * g.L4 * a.num_angles * 4 : 0;
     // scalar-block workgroups: one per sub-chunk and group of heads. A call of many sub-chunks
     // fills the GPU with all its heads in one group (8 heads each there, 4 times the workgroups,
@@ -2534,7 +2547,7 @@ static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
       (a.phase_mode == M3_PHASE_NONE || a.mimo_rotation == 0 || a.d_state % 16 == 0)) {
     return true;
   }
-  return rows && form16_of(a) >= 0;
+  return rows && form16_of(a, true) >= 0;
 }
 
 static Segments segments_for(const m3_scan_args& a, int concurrent = 1) {
@@ -2581,7 +2594,7 @@ static SegPlan plan_segments(const m3_scan_args& a, const Segments& s, bool rows
   SegPlan sp{};
   ScanGeom g{};
   auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-  sp.prep_bytes = up(ws_layout(a, g, rows ? form16_of(a) : -1));
+  sp.prep_bytes = up(ws_layout(a, g, form16_of(a, rows)));
   const size_t es = a.act_dtype == M3_F32 ? 4 : 2;
   const size_t pairs = static_cast<size_t>(a.batch) * a.heads, segs = pairs * s.count;
   size_t off = sp.prep_bytes;
@@ -2639,7 +2652,7 @@ static int launch_segmented(const m3_scan_args& a, const Segments& s, bool rows,
   a1.block_phase = angles ? contiguous(sg.seg_blk, M3_F32, {B, H, sg.nblk, S}) : m3_tensor{};
   a1.final_k = contiguous(sg.seg_k, a.act_dtype, {BG, H, R, N});
   const Split first{G, s.len, 0}, second{G, s.len, 1};
-  const int form16 = rows ? form16_of(a) : -1;
+  const int form16 = form16_of(a, rows);
   int rc = launch_pass<T, R>(a1, stream, true, form16, &first, /*state_only=*/true);
   if (rc != M3_OK) return rc;
 
@@ -2674,7 +2687,7 @@ static int launch_scan_r(const m3_scan_args& a, bool rows, hipStream_t stream) {
                 a.segments);
   }
   if (s.count > 1) return launch_segmented<T, R>(a, s, rows, stream);
-  return launch_pass<T, R>(a, stream, true, rows ? form16_of(a) : -1);
+  return launch_pass<T, R>(a, stream, true, form16_of(a, rows));
 }
 
 template <typename T>
@@ -2797,7 +2810,7 @@ size_t scan_need(const m3_scan_args& a, bool rows) {
   const Segments s = segments_for(a);
   if (s.count > 1) return plan_segments(a, s, rows).total_bytes;
   ScanGeom g{};
-  return ws_layout(a, g, rows ? form16_of(a) : -1);
+  return ws_layout(a, g, form16_of(a, rows));
 }
 
 int scan_run(const m3_scan_args& a, bool rows, hipStream_t stream) {

@@ -10,7 +10,7 @@ namespace m3 {
 // one another's LDS, MFMA and transcendental latency. A sub-chunk is 64 rows (token, rank), rank
 // minor: 64 / R tokens, whose decay weights, phases and scalars are per token and whose output
 // sums the token's R rows (times mimo_out). The work of a sub-chunk c, between workgroup barriers:
-//   staging   every wave: row qt's q / k (bias and rotation on prep's rows; waves 0-7 the slots
+//   staging   every wave: row qt's q / k (norm, bias and rotation; waves 0-7 the slots
 //             that can rotate, waves 8-15 the others) -> Qs, Ks; row vt's values scaled for the
 //             carry -> VS;
 //   start     row vt's gate and value -> ZR, VR; the wave's two state tiles, rounded -> Sb, decayed;
@@ -30,20 +30,30 @@ namespace m3 {
 // the priority of the later waves (s_setprio) measured 2-5% slower.
 // Same mathematics and rounding points as scan_kernel (whose header lists them).
 //
-// Slots. prep writes the q / k rows with their columns in slot order: the rotation's pairs first,
-// a pair's two columns side by side (slots 2j, 2j + 1 of angle j), then the other columns, zeros
-// up to 128. The products sum over the columns, so any common order of q, k and the state gives
-// the same result, and one staging code serves both rotations (adjacent pairs, and the MIMO
-// pairs (j, j + 2S)) and every d_state; slot_col() maps a slot back for the bias, the state and
-// the last k. Slots 0-63 go through the rotation with phase 0 past the call's angles (cos 1,
-// sin 0: the value itself).
+// Slots. The columns are taken in slot order: the rotation's pairs first, a pair's two columns side
+// by side (slots 2j, 2j + 1 of angle j), then the other columns, zeros up to 128. The products sum
+// over the columns, so any common order of q, k and the state gives the same result, and one
+// staging code serves both rotations (adjacent pairs, and above rank 1 the MIMO pairs (j, j + 2S))
+// and every d_state; slot_col() maps a slot back to its column. Slots 0-63 go through the rotation
+// with phase 0 past the call's angles (cos 1, sin 0: the value itself).
 //
-// Forms (F), by what prep's rows hold:
+// Forms (F), by where the q / k rows come from:
 //   kModel  the model's own shape (N = 128, P = 64, 32 angles, ranks 1 and 4) in projection form:
-//           rows rounded after the RMSNorm (the reference's rounding point, model.py:48-55);
-//   kProj   the other shapes in projection form: the normalized rows in FP32, rounded once after
-//           the rotation;
-//   kHook   the hook form: the given (normed) rows, phases given or none.
+//           prep's rows in slot order, rounded after the RMSNorm (the reference's rounding point,
+//           model.py:48-55);
+//   kRows   the other shapes in projection form above rank 1: prep's rows in slot order in FP32, of
+//           d_state slots, rounded once after the rotation;
+//   kProj   those at rank 1, and any that have no workspace for rows: the caller's rows, normalized
+//           in FP32 by prep's factors;
+//   kCopy   the hook form (normed rows, phases given or none) above rank 1 where 16 heads or more
+//           share a row: prep's copies in slot order;
+//   kHook   the hook form elsewhere, and with no workspace for rows: the caller's rows.
+// The caller's rows are read as they lie, above rank 1 by two loads of two columns where prep's take
+// one of four slots. Measured (32 heads, d_state 128): hook form, rank 2, one group (4 x 2048)
+// kCopy 172 us, kHook 192; 32 groups (2 x 1024) 102 and 85; rank 4, 32 groups (4 x 2048) 511 and
+// 362; 8 heads at rank 4 (1 x 32768) 355 and 304. Projection form (8 x 1024) kRows 121 us at rank 2
+// and 384 at rank 8, kProj, whose normalization at every head spills registers, 147 and 494; at rank
+// 1 and d_state 64 73 and 74, with 13.6 and 5.7 MiB of workspace.
 //
 // LO: d_state no power of 2. Those calls are the recurrent scan's on rows that are not aligned, and
 // came from it: it holds the decay weights and the scaled values in FP32, rounding neither. Here
@@ -92,13 +102,15 @@ struct Lay16 : Lay16Rows {
   // ranks above 1: the rounded mimo_x, mimo_z and mimo_out [R][P]
   static constexpr int MP = TWO ? R * kPPad : 0;
   static constexpr int MX = POFF + kSMax, MZ = MX + MP, MO = MZ + MP;
-  static constexpr int WL = FB + 4 * (MO + MP);
+  static constexpr int NW = MO + MP;  // form kProj: the rounded norm weights of q and k, by slot
+  static constexpr int WL = FB + 4 * (NW + 2 * kNPad);
   static constexpr int VL = WL + (LO ? ROWS * LW * ES : 0);
   static constexpr int BYTES = VL + (LO ? ROWS * LV * ES : 0);
   static_assert(BYTES <= 160 * 1024, "scan16 LDS layout exceeds 160 KiB");
   static_assert(FB % 16 == 0 && WS % 16 == 0 && SB % 16 == 0 && WL % 16 == 0 && VL % 16 == 0 &&
                     (ANG * 4) % 16 == 0 &&
-                    (CS0 * 4) % 16 == 0 && (MX * 4) % 16 == 0,
+                    (CS0 * 4) % 16 == 0 && (MX * 4) % 16 == 0 &&
+                    (NW * 4) % 16 == 0,
                 "alignment");
 };
 
@@ -143,10 +155,12 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   constexpr int TOK = 64 / R;  // tokens per 64-row sub-chunk (rows (token, rank), rank minor)
   using SB_ = ScBlk<TOK>;
   constexpr int LQ = Ly::LQ, LW = Ly::LW, CST = Ly::CST, ES = 2;
-  constexpr bool ROWF = F == kProj;   // prep's rows are FP32
-  constexpr bool GIVEN = F == kHook;  // phases given (or none), no increments
-  constexpr int RB = kNPad * (ROWF ? 4 : 2);  // bytes of one q or k row
+  constexpr bool PREP = F == kModel || F == kRows || F == kCopy;  // prep's rows; else the caller's
+  constexpr bool ROWF = F == kRows;   // in FP32
+  constexpr bool NORM = F == kProj;   // to be normalized here
+  constexpr bool GIVEN = F == kHook || F == kCopy;  // phases given (or none), no increments
   const int N = F == kModel ? kNPad : a.d_state;
+  const int RB = ROWF ? N * 4 : kNPad * 2;  // bytes of one of prep's rows
   const int P = F == kModel ? kPPad : a.head_dim;
   const int S = F == kModel ? kSMax : a.num_angles;
   // phase: PG lanes per angle, TPL tokens per lane, on the first PG / 2 waves (32 angles)
@@ -171,7 +185,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   const int nsub = (L + TOK - 1) / TOK;
   const int GRP = F == kModel ? 1 : a.groups;
   const int grp = F == kModel ? 0 : h / (H / GRP);
-  const int perm = F == kModel ? (R > 1 ? 1 : 0) : g.perm;
+  const int perm = R == 1 ? 0 : F == kModel ? 1 : g.perm;
   auto col = [&](int slot) { return slot_col(slot, perm, S); };
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -238,14 +252,39 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
   const int p0c = p0 < P ? p0 : 0;
   const int o_v = gv.o0 + (vt / R) * gv.step + p0c * ES;
   const int o_z = gz.o0 + (vt / R) * gz.step + p0c * ES;
-  // prep's q / k rows of batch row b: row (token, group, rank) at 2 RB bytes, k after q
+  // prep's q / k rows of batch row b: row (token, group, rank) at 2 RB bytes, k after q; 32 rows on: 32
+  // / R tokens
   const int tok_qk = GRP * R * 2 * RB;
-  const __amdgpu_buffer_rsrc_t rs_qk = make_rsrc(
-      reinterpret_cast<const char*>(prep) + g.ws_qk +
-          (static_cast<int64_t>(b) * a.length + tok0) * tok_qk,
-      L * tok_qk);
-  // row (token qt / R, rank qt % R) of this group, slot n0 of q; 32 rows on: 32 / R tokens
-  const int o_qk = (qt / R) * tok_qk + (grp * R + qr) * 2 * RB + n0 * (ROWF ? 4 : 2);
+  const __amdgpu_buffer_rsrc_t rs_qk =
+      PREP ? make_rsrc(reinterpret_cast<const char*>(prep) + g.ws_qk +
+                           (static_cast<int64_t>(b) * a.length + tok0) * tok_qk,
+                       L * tok_qk)
+           : make_rsrc(nullptr, 0);
+  // the caller's rows: the columns of slots n0 .. n0 + 3, which above rank 1 are two words `d2`
+  // bytes apart (a MIMO pair's columns; the words of two pairs are put side by side at the staging,
+  // v_perm selectors selA and selB); lanes past column N read past every extent (kOut: not moved
+  // with the token). prep's norm factors (q, k) of the same row.
+  constexpr int kOut = INT32_MIN;  // as an unsigned offset 2^31, the extents are below it
+  const bool in_n = (PREP && !ROWF) || n0 < N;
+  // (prep's rows run forwards, less than 2^31 bytes: a lane may start at kOut and move with the token)
+  const int o_qk =
+      in_n ? (qt / R) * tok_qk + (grp * R + qr) * 2 * RB + n0 * (ROWF ? 4 : ES) : kOut;
+  const bool pair = !PREP && perm && n0 < 2 * S;
+  const int c0q = col(n0), d2 = (pair ? 2 * S : 2) * ES;
+  const uint32_t selA = pair ? 0x05040100u : 0x03020100u, selB = pair ? 0x07060302u : 0x07060504u;
+  const int qr_s = PREP ? 0 : static_cast<int>(a.q.stride[3]);
+  const int kr_s = PREP ? 0 : static_cast<int>(a.k.stride[3]);
+  const Rows none{make_rsrc(nullptr, 0), 0, 0};
+  const Rows gq = PREP ? none : rows_of(a.q, grp * a.q.stride[2], (R - 1) * qr_s + N, ES);
+  const Rows gk = PREP ? none : rows_of(a.k, grp * a.k.stride[2], (R - 1) * kr_s + N, ES);
+  const int o_q = gq.o0 + (qt / R) * gq.step + (qr * qr_s + c0q) * ES;
+  const int o_k = gk.o0 + (qt / R) * gk.step + (qr * kr_s + c0q) * ES;
+  const int tok_n = GRP * R * 8;
+  const __amdgpu_buffer_rsrc_t rs_n =
+      NORM ? make_rsrc(prep + g.ws_norm + (static_cast<int64_t>(b) * a.length + tok0) * GRP * R * 2,
+                       L * tok_n)
+           : make_rsrc(nullptr, 0);
+  const int o_n = (qt / R) * tok_n + (grp * R + qr) * 8;
   const int scw = g.scw;
   // side words (waves 0-3, one float pair per lane): the scalar block
   const int q2 = 2 * tid;
@@ -286,18 +325,38 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
                     : nullptr;
   const int64_t blk_stride = a.block_phase.stride[2];
 
-  // q / k words: rows qt and qt + 32, q and k, 4 slots each
+  // q / k words: rows qt and qt + 32, q and k, 4 slots each; their norm factors
   using RowT = std::conditional_t<ROWF, float, T>;
   constexpr int QW = ROWF ? 4 : 2;
   uint32_t rq[2][QW], rk[2][QW], rv[2], rz[2];
+  u32x2 fac[2];
   float2 side = make_float2(0.f, 0.f);
   float4 ang = make_float4(0.f, 0.f, 0.f, 0.f);
   auto load_qk = [&](int t0) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int o = o_qk + (t0 + (32 / R) * j) * tok_qk;
-      bload_words<QW>(rq[j], rs_qk, o);
-      bload_words<QW>(rk[j], rs_qk, o + RB);
+      const int tj = t0 + (32 / R) * j;
+      if constexpr (PREP) {
+        const int o = o_qk + tj * tok_qk;
+        bload_words<QW>(rq[j], rs_qk, o);
+        bload_words<QW>(rk[j], rs_qk, o + RB);
+      } else {
+        auto row = [&](uint32_t (&w2)[2], const Rows& x, int o) {
+          const int oo = in_n ? o + tj * x.step : kOut;
+          if constexpr (R == 1) {
+            bload_words<2>(w2, x.rs, oo);
+          } else {
+            w2[0] = __builtin_amdgcn_raw_buffer_load_b32(x.rs, oo, 0, 0);
+            w2[1] = __builtin_amdgcn_raw_buffer_load_b32(x.rs, oo + d2, 0, 0);
+          }
+        };
+        row(rq[j], gq, o_q);
+        row(rk[j], gk, o_k);
+        if constexpr (NORM) {
+          fac[j] = __builtin_bit_cast(
+              u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs_n, o_n + tj * tok_n, 0, 0));
+        }
+      }
     }
   };
   auto load_vz = [&](int t0) {
@@ -394,7 +453,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
     return make_rsrc(static_cast<const char*>(t.ptr) + h * t.stride[0] * es, n * es);
   };
   // biases of the lane's 4 slots, rank qr (slots past the call's columns read past the extent)
-  const bool bias = F != kHook || a.q_bias.ptr != nullptr;
+  const bool bias = !GIVEN || a.q_bias.ptr != nullptr;
   uint32_t bq_r[4] = {0u, 0u, 0u, 0u}, bk_r[4] = {0u, 0u, 0u, 0u};
   if (bias) {
     const int qs = static_cast<int>(a.q_bias.stride[1]), ks = static_cast<int>(a.k_bias.stride[1]);
@@ -455,7 +514,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
                             b * a.dt.stride[0] + tok0 * a.dt.stride[1] + h * a.dt.stride[2]);
     const RawX tr_r = ldraw(a.trap.ptr, a.trap.dtype,
                             b * a.trap.stride[0] + tok0 * a.trap.stride[1] + h * a.trap.stride[2]);
-    const RawX db_r = F == kHook ? RawX{0u, 0u}
+    const RawX db_r = GIVEN ? RawX{0u, 0u}
                                  : ldraw(a.dt_bias.ptr, a.dt_bias.dtype, h * a.dt_bias.stride[0]);
     const int kr_s = static_cast<int>(a.initial_k.stride[2]);
     const __amdgpu_buffer_rsrc_t rs_v =
@@ -490,7 +549,7 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       }
     }
     float dt0, adt0;
-    dt_adt(F != kHook, decode(dt_r, a.dt.dtype), 0.f, decode(db_r, F == kHook ? 0 : a.dt_bias.dtype),
+    dt_adt(!GIVEN, decode(dt_r, a.dt.dtype), 0.f, decode(db_r, GIVEN ? 0 : a.dt_bias.dtype),
            dt0, adt0);
     const float c0 = dt0 * (1.f - sigmoidf(decode(tr_r, a.trap.dtype)));
 #pragma unroll
@@ -506,9 +565,17 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       }
     }
   }
+  // norm weights, slot tid % 128 of q (threads 0-127) or k
+  float nw = 0.f;
+  if constexpr (NORM) {
+    const m3_tensor& t = tid < kNPad ? a.q_norm_w : a.k_norm_w;
+    const int sl = tid & (kNPad - 1);
+    if (tid < 2 * kNPad && sl < N) nw = rnd<T>(ldx(t.ptr, t.dtype, col(sl) * t.stride[0]));
+  }
   __builtin_amdgcn_sched_barrier(0);
   put_side(sc0);
   load_side(1);
+  if (NORM && tid < 2 * kNPad) F_[Ly::NW + tid] = nw;
   if (tid < kSMax) {
     F_[Ly::PBASE + tid] = 0.f;
     F_[Ly::POFF + tid] = po;
@@ -545,10 +612,28 @@ __global__ __launch_bounds__(k16Threads) void scan16_kernel(const m3_scan_args a
       // (n0 + 2, n0 + 3), angles n0 / 2 and n0 / 2 + 1, adjacent in the cos / sin table row
       const int rw = qt + 32 * j, tt = rw / R;
       f4 q, k;
+      if constexpr (!PREP && R > 1) {
+        const uint32_t q0 = rq[j][0], q1 = rq[j][1], k0 = rk[j][0], k1 = rk[j][1];
+        rq[j][0] = __builtin_amdgcn_perm(q1, q0, selA);
+        rq[j][1] = __builtin_amdgcn_perm(q1, q0, selB);
+        rk[j][0] = __builtin_amdgcn_perm(k1, k0, selA);
+        rk[j][1] = __builtin_amdgcn_perm(k1, k0, selB);
+      }
+      if constexpr (NORM) {
+        const float fq = __uint_as_float(fac[j][0]), fk = __uint_as_float(fac[j][1]);
+        const f4 wq = *reinterpret_cast<const f4*>(F_ + Ly::NW + n0);
+        const f4 wk = *reinterpret_cast<const f4*>(F_ + Ly::NW + kNPad + n0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        q[i] = raw_get<RowT>(rq[j], i) + bq[i];
-        k[i] = raw_get<RowT>(rk[j], i) + bk[i];
+        for (int i = 0; i < 4; ++i) {
+          q[i] = fmaf(raw_get<T>(rq[j], i) * fq, wq[i], bq[i]);
+          k[i] = fmaf(raw_get<T>(rk[j], i) * fk, wk[i], bk[i]);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          q[i] = raw_get<RowT>(rq[j], i) + bq[i];
+          k[i] = raw_get<RowT>(rk[j], i) + bk[i];
+        }
       }
       if (rot) {
         const f4 cv = *reinterpret_cast<const f4*>(CSt + tt * CST + 2 * cs_col<true>(n0 >> 1, tt));
@@ -999,6 +1084,10 @@ static int launch_rank16(const m3_scan_args& a, const ScanGeom& g, const float* 
                          unsigned grid, hipStream_t stream) {
   if constexpr (R == 1 || R == 4) {
     if (g.form16 == kModel) return launch_form16<T, R, kModel>(a, g, prep, so, grid, stream);
+  }
+  if constexpr (R > 1) {
+    if (g.form16 == kRows) return launch_form16<T, R, kRows>(a, g, prep, so, grid, stream);
+    if (g.form16 == kCopy) return launch_form16<T, R, kCopy>(a, g, prep, so, grid, stream);
   }
   if (g.form16 == kProj) return launch_form16<T, R, kProj>(a, g, prep, so, grid, stream);
   return launch_form16<T, R, kHook>(a, g, prep, so, grid, stream);

@@ -123,9 +123,9 @@ struct ScanGeom {
   int segs, seg_len, last_only;
   int ws_bytes;  // workspace bytes when below 2^31 (the projection form addresses it in 32 bits)
   // the 16-wave kernel (scan16_kernel): its form (Form16, -1: the call takes another kernel),
-  // whether the columns are permuted into slots (the MIMO rotation), and the q / k rows
-  // [B][L][G][R][2][128] in slot order, in the activation dtype or FP32 (form kProj), after the
-  // regions above (byte offset)
+  // whether the columns are permuted into slots (the MIMO rotation), and the q / k rows [B][L][G][R][2]
+  // in slot order, 128 slots in the activation dtype (forms kModel, kCopy) or d_state in FP32 (kRows),
+  // after the regions above (byte offset)
   int form16, perm;
   // d_state no power of 2: the kernels that hold no value in fewer bits than the recurrent scan
   int lo;
@@ -489,8 +489,8 @@ __device__ __forceinline__ void phase_stage(float* tab, int ps, float* pbase, fl
   }
 }
 
-// What prep's q / k rows hold and where a 16-wave call's inputs come from (scan16_kernel.hpp).
-enum Form16 { kModel, kProj, kHook };
+// Where a 16-wave call's q / k rows come from (scan16_kernel.hpp).
+enum Form16 { kModel, kRows, kProj, kCopy, kHook };
 
 // The column of slot `slot`: the identity, or with the MIMO pairs (perm: S angles, columns j and
 // 2S + j) their two columns side by side first, then the columns S .. 2S - 1 and 3S ..

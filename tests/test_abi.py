@@ -304,6 +304,24 @@ def test_a_request_of_short_segments_is_answered_with_itself(lib, length, reques
     assert lib.m3_scan_fwd(ctypes.byref(args), None) == 4  # stops at the workspace, not the count
 
 
+def test_hook_form_workspace_holds_no_rows(lib):
+    """The hook form reads the caller's q and k rows as they lie: its workspace (scalar blocks, and
+    what a split adds) does not grow with the number of q / k groups."""
+    size = ctypes.c_size_t(0)
+
+    def ws(groups):
+        args = _hook_scan_args(4, 4096, 32, 1)
+        args.groups = groups
+        for t in (args.q, args.k):
+            for i, stride in enumerate((4096 * groups * 64, groups * 64, 64, 64, 1)):
+                t.stride[i] = stride
+        assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+        return size.value
+
+    assert ws(32) == ws(1)
+    assert ws(1) == 4 * 32 * 64 * (5 * 64 + 8) * 4  # 64 sub-chunks of 64 tokens per head
+
+
 def test_scan_backwards_token_strides_on_the_host(lib):
     """Per-token tensors may run backwards (the reverse scan), but all of them together."""
     args = _hook_scan_args(1, 128, 2, 1)

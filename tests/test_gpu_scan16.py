@@ -176,6 +176,38 @@ def test_hook_form_layouts(layout):
     _close(state, want_state.cpu(), torch.bfloat16)
 
 
+@pytest.mark.parametrize("rank,groups,d_state,angles,length,layout", [
+    (1, 4, 64, 16, 70, "groups_first"), (2, 4, 128, 32, 70, "groups_first"),
+    (2, 2, 128, 32, 45, "ranks_first"), (4, 1, 48, 12, 33, "ranks_first"),
+    (8, 4, 16, 4, 19, "q_k_apart"), (4, 2, 112, 0, 40, "q_k_apart"),
+    (1, 2, 100, 25, 130, "q_k_apart"), (1, 1, 128, 32, 70, "pairs_j_2s"),
+])
+def test_hook_form_row_layouts(rank, groups, d_state, angles, length, layout):
+    """q and k rows as they lie in the caller's buffers: groups ahead of tokens, ranks ahead of
+    tokens (whose rows pass the next token's: another kernel), q and k with strides of their own,
+    and rank 1 with the MIMO pairs (another kernel). Against the oracle."""
+    inp = _inputs(rank, torch.bfloat16, batch=2, length=length, heads=4, groups=groups, head_dim=32,
+                  d_state=d_state, angles=angles, bias=True, initial=True, seed=length)
+    if layout == "pairs_j_2s":
+        inp["mimo_rotation"] = True
+    want, want_state = _oracle32(inp)
+    dev = {n: (t.to(DEV) if isinstance(t, torch.Tensor) else t) for n, t in inp.items()}
+    if layout == "q_k_apart":
+        for name, extra in (("q", 4), ("k", 20)):
+            t = dev[name]
+            wide = torch.full((*t.shape[:2], groups + 1, rank, d_state + extra), float("nan"),
+                              dtype=t.dtype, device=DEV)
+            wide[:, :, :groups, :, :d_state] = t
+            dev[name] = wide[:, :, :groups, :, :d_state]
+    elif layout != "pairs_j_2s":
+        axis = 2 if layout == "groups_first" else 3
+        for name in ("q", "k"):
+            dev[name] = dev[name].transpose(1, axis).contiguous().transpose(1, axis)
+    got, state = ops.mamba3_scan(**dev)
+    _close(got, want, torch.bfloat16)
+    _close(state, want_state, torch.bfloat16)
+
+
 @pytest.mark.parametrize("rank,d_model,d_state,length,reverse", [
     (1, 96, 96, 70, False), (1, 40, 96, 129, True), (2, 64, 128, 40, False),
     (4, 64, 96, 33, True), (8, 96, 128, 20, False), (4, 128, 128, 1, False),
