@@ -2168,12 +2168,12 @@ static int form16_of(const m3_scan_args& a, bool rows) {
     if (proj) return kRows;
     if (a.heads >= 16 * a.groups && int64_t{2} * a.batch * len * a.groups * a.rank < INT32_MAX) return kCopy;
   }
-  // the caller's rows: the ranks of a token's row below the next token's
+  // the caller's rows: the ranks of a token's row below the next token's (also of one token: the
+  // rows after it are read, as zeros, past the extent)
   for (const m3_tensor* t : {&a.q, &a.k}) {
     const int64_t s1 = t->stride[1] < 0 ? -t->stride[1] : t->stride[1];
     const int64_t span = (a.rank - 1) * t->stride[3] + N;
-    if (a.rank > 1 && t->stride[3] < 0) return -1;
-    if (len > 1 ? s1 < span : span * 2 >= INT32_MAX) return -1;
+    if ((a.rank > 1 && t->stride[3] < 0) || s1 < span) return -1;
   }
   return proj ? kProj : kHook;
 }

@@ -181,11 +181,13 @@ def test_hook_form_layouts(layout):
     (2, 2, 128, 32, 45, "ranks_first"), (4, 1, 48, 12, 33, "ranks_first"),
     (8, 4, 16, 4, 19, "q_k_apart"), (4, 2, 112, 0, 40, "q_k_apart"),
     (1, 2, 100, 25, 130, "q_k_apart"), (1, 1, 128, 32, 70, "pairs_j_2s"),
+    (1, 1, 128, 32, 1, "one_token"), (4, 4, 64, 16, 1, "one_token"), (1, 1, 96, 24, 1, "one_token"),
 ])
 def test_hook_form_row_layouts(rank, groups, d_state, angles, length, layout):
     """q and k rows as they lie in the caller's buffers: groups ahead of tokens, ranks ahead of
     tokens (whose rows pass the next token's: another kernel), q and k with strides of their own,
-    and rank 1 with the MIMO pairs (another kernel). Against the oracle."""
+    rank 1 with the MIMO pairs (another kernel), and one token whose stride is 0. Against the
+    oracle."""
     inp = _inputs(rank, torch.bfloat16, batch=2, length=length, heads=4, groups=groups, head_dim=32,
                   d_state=d_state, angles=angles, bias=True, initial=True, seed=length)
     if layout == "pairs_j_2s":
@@ -199,6 +201,10 @@ def test_hook_form_row_layouts(rank, groups, d_state, angles, length, layout):
                               dtype=t.dtype, device=DEV)
             wide[:, :, :groups, :, :d_state] = t
             dev[name] = wide[:, :, :groups, :, :d_state]
+    elif layout == "one_token":
+        for name in ("q", "k"):
+            t = dev[name]
+            dev[name] = t.as_strided(t.shape, (t.stride(0), 0, *t.stride()[2:]))
     elif layout != "pairs_j_2s":
         axis = 2 if layout == "groups_first" else 3
         for name in ("q", "k"):
