@@ -119,7 +119,14 @@ typedef struct {
   size_t workspace_bytes;
 } m3_scan_args;
 
-/* Bytes of device workspace m3_scan_fwd needs for these arguments (0 is possible). */
+/*
+ * Bytes of device workspace m3_scan_fwd needs for these arguments (0 is possible): by the dimensions,
+ * modes, which optional tensors are set, and the addresses and strides of q, k, value, gate, out and
+ * a given phase. Those may be unset (NULL); at a d_state that is a power of 2 the answer then holds
+ * for any buffers. At any other d_state it is then 0, with which the call takes a slow route (the
+ * recurrent scan, about 10 us a token): set them before the query. A workspace below the answer is
+ * used by slower routes that need less, where there are any.
+ */
 int m3_scan_workspace_size(const m3_scan_args* args, size_t* bytes);
 /*
  * The segments request for these arguments when `concurrent_calls` calls of this shape run on the

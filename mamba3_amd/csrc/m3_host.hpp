@@ -25,8 +25,8 @@ int check_tensor(const m3_tensor& t, const char* name, int dims, int64_t inner_e
 // After a launch: translate hipGetLastError into a status.
 int check_launch(const char* what);
 
-// Workspace bytes of a scan call and the call itself (scan.hip). `rows` false: without the 16-wave
-// kernel, whose q / k rows take most of a 16-bit call's workspace.
+// Workspace bytes of a scan call and the call itself (scan.hip). `rows` false: by the routes that need
+// least, without copies of the q / k rows, and at a d_state that is no power of 2 the recurrent scan.
 size_t scan_need(const m3_scan_args& a, bool rows);
 int scan_run(const m3_scan_args& a, bool rows, hipStream_t stream);
 

@@ -2081,7 +2081,9 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // two sub-chunks, 128 tokens, and a token group ahead). Projection form: norm weights, biases, raw
 // dt, angle increments; hook form: none of the norms, phases given or none. Rank 1 with the MIMO
 // rotation takes the other kernels. `rows` false: without the workspace for prep's rows (kModel's
-// shape and the ranks above 1 then take kProj and kHook, which read the caller's).
+// shape and the ranks above 1 then take kProj and kHook, which read the caller's). A required tensor
+// that is not set yet (a workspace query ahead of the buffers) counts as one that fits; at a d_state
+// no power of 2, whose other route needs no workspace, as one that does not.
 // Every such call is faster on it than on the kernel it took before (per call, scan_kernel then
 // scan16_kernel, 8 x 1024 tokens, 32 heads): hook form rank 1 80 -> 72 us, rank 2 184 -> 118,
 // rank 4 332 -> 207, rank 8 628 -> 392; projection form rank 2 140 -> 121, rank 8 487 -> 391,
@@ -2101,14 +2103,15 @@ static int form16_of(const m3_scan_args& a, bool rows) {
   if (rotates && (S <= 0 || (a.rank == 1 && a.mimo_rotation))) return -1;
   const bool norm = a.q_norm_w.ptr != nullptr && a.k_norm_w.ptr != nullptr;
   const bool proj = norm && a.q_bias.ptr != nullptr && a.k_bias.ptr != nullptr &&
-                    a.raw_dt != 0 && a.dt_bias.ptr != nullptr && a.phase_mode == M3_PHASE_ANGLES;
+                    a.raw_dt != 0 && a.phase_mode == M3_PHASE_ANGLES;
   const bool hook = a.q_norm_w.ptr == nullptr && a.k_norm_w.ptr == nullptr && a.raw_dt == 0 &&
                     a.phase_mode != M3_PHASE_ANGLES;
   if (!proj && !hook) return -1;
   const int64_t len = a.length, ahead = len + 256;
   // rows of `dims` outer axes (extents in `ext`) read `span` elements at a time
   auto rows_ok = [&](const m3_tensor& t, std::initializer_list<int64_t> ext, int64_t span) {
-    if (t.ptr == nullptr || reinterpret_cast<uintptr_t>(t.ptr) % 8 != 0) return false;
+    if (t.ptr == nullptr) return pow2(N);
+    if (reinterpret_cast<uintptr_t>(t.ptr) % 8 != 0) return false;
     int i = 0;
     for (int64_t e : ext) {
       if (e > 1 && t.stride[i] % 4 != 0) return false;
@@ -2127,7 +2130,7 @@ static int form16_of(const m3_scan_args& a, bool rows) {
   // range or make a second token alias the first
   if (len == 1) {
     for (const m3_tensor* t : {&a.value, &a.gate, &a.out}) {
-      if ((t->stride[1] < 0 ? -t->stride[1] : t->stride[1]) < P) return -1;
+      if (t->ptr != nullptr && (t->stride[1] < 0 ? -t->stride[1] : t->stride[1]) < P) return -1;
     }
   }
   const int64_t tok = 64 / a.rank, nsub = (len + tok - 1) / tok;
@@ -2135,7 +2138,7 @@ static int form16_of(const m3_scan_args& a, bool rows) {
     return -1;
   }
   if (a.phase_mode == M3_PHASE_ANGLES && ahead * S * 4 >= (int64_t{1} << 30)) return -1;
-  if (a.phase_mode == M3_PHASE_GIVEN) {
+  if (a.phase_mode == M3_PHASE_GIVEN && (a.phase.ptr != nullptr || !pow2(N))) {
     const int64_t s1 = a.phase.stride[1] < 0 ? -a.phase.stride[1] : a.phase.stride[1];
     const int64_t span = (S - 1) * a.phase.stride[3] + 1;
     if (a.phase.ptr == nullptr || a.phase.stride[3] < 0 || s1 < span ||
@@ -2171,6 +2174,7 @@ static int form16_of(const m3_scan_args& a, bool rows) {
   // the caller's rows: the ranks of a token's row below the next token's (also of one token: the
   // rows after it are read, as zeros, past the extent)
   for (const m3_tensor* t : {&a.q, &a.k}) {
+    if (t->ptr == nullptr) continue;
     const int64_t s1 = t->stride[1] < 0 ? -t->stride[1] : t->stride[1];
     const int64_t span = (a.rank - 1) * t->stride[3] + N;
     if ((a.rank > 1 && t->stride[3] < 0) || s1 < span) return -1;
@@ -2536,14 +2540,15 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
 // The shapes the chunked MFMA kernels tile: up to 128 columns, 64 values and 32 angles at ranks 1,
 // 2, 4 and 8, with d_state a power of 2; in FP32 also any other, with the MIMO rotation where its
 // pairs lie whole 8-column lanes apart (d_state 96, 4 x 1500 tokens, 16 heads: 21.7 ms on the
-// recurrent scan, 185 us here); and the 16-wave kernel's calls at every d_state it takes
-// (`rows`: its workspace rows are allowed). Others take the recurrent scan (rscan.hip).
+// recurrent scan, 185 us here); and the 16-wave kernel's calls at every d_state it takes. Others
+// take the recurrent scan (rscan.hip), and so does every d_state that is no power of 2 with `rows`
+// false (the least workspace).
 static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
   const bool fits = a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
                     a.num_angles <= kSMax &&
                     (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8);
   if (fits && pow2(a.d_state)) return true;
-  if (fits && a.act_dtype == M3_F32 && a.q.ptr != nullptr &&
+  if (fits && rows && a.act_dtype == M3_F32 && a.q.ptr != nullptr &&
       (a.phase_mode == M3_PHASE_NONE || a.mimo_rotation == 0 || a.d_state % 16 == 0)) {
     return true;
   }
@@ -2817,7 +2822,10 @@ int scan_run(const m3_scan_args& a, bool rows, hipStream_t stream) {
   int rc = validate_scan(a);
   if (rc != M3_OK) return rc;
   if (a.batch == 0) return M3_OK;
-  if (!tiled_shape(a, rows)) return launch_recurrent_scan(a, stream);
+  if (!tiled_shape(a, rows)) {
+    if (!rscan_fits(a)) return fail(M3_EUNSUPPORTED, "m3_scan_fwd: no kernel without a workspace");
+    return launch_recurrent_scan(a, stream);
+  }
   switch (a.act_dtype) {
     case M3_F32: return launch_scan<float>(a, rows, stream);
     case M3_BF16: return launch_scan<__bf16>(a, rows, stream);
@@ -2858,5 +2866,13 @@ extern "C" int m3_scan_segments(const m3_scan_args* args, int concurrent_calls,
 extern "C" int m3_scan_fwd(const m3_scan_args* args, hipStream_t stream) {
   m3::clear_error();
   if (args == nullptr) return m3::fail(M3_EINVAL, "m3_scan_fwd: args is NULL");
-  return m3::scan_run(*args, true, stream);
+  const int rc = m3::scan_run(*args, true, stream);
+  if (rc != M3_EWORKSPACE) return rc;
+  // (nothing was launched) less workspace than the query's answer: the routes that need least, where
+  // it covers them
+  const size_t least = m3::scan_need(*args, false);
+  const bool given = args->workspace != nullptr && m3::aligned16(args->workspace);
+  if (least > 0 && (!given || args->workspace_bytes < least)) return rc;
+  m3::clear_error();
+  return m3::scan_run(*args, false, stream);
 }

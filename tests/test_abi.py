@@ -322,6 +322,69 @@ def test_hook_form_workspace_holds_no_rows(lib):
     assert ws(1) == 4 * 32 * 64 * (5 * 64 + 8) * 4  # 64 sub-chunks of 64 tokens per head
 
 
+def _model_scan_args(batch, length, heads, rank, bound, d_state=128, dtype=_hip.BF16):
+    """The model's projection form; `bound`: with its buffers at fake addresses."""
+    n, p, s = d_state, 64, d_state // 4
+    width = 2 * heads * p + 2 * n * rank + 3 * heads + s
+    width += -width % 8
+    args = _hip.ScanArgs(batch=batch, length=length, heads=heads, groups=1, rank=rank, d_state=n,
+                         head_dim=p, num_angles=s, chunk=256, act_dtype=dtype,
+                         mimo_rotation=int(rank > 1), raw_dt=1, phase_mode=_hip.PHASE_ANGLES,
+                         norm_eps=1e-5, segments=0)
+    for name in ("q_norm_w", "k_norm_w", "q_bias", "k_bias"):
+        t = getattr(args, name)
+        t.ptr, t.dtype = 0x1000, _hip.F32
+        for i, stride in enumerate((rank * n, n, 1) if "bias" in name else (1,)):
+            t.stride[i] = stride
+    if bound:
+        token = (length * width, width)
+        for i, (name, strides) in enumerate({
+                "q": (n * rank, n, 1), "k": (n * rank, n, 1), "value": (p, 1), "gate": (p, 1),
+                "dt": (1,), "a": (1,), "trap": (1,), "phase": (1,), "out": (p, 1)}.items()):
+            t = getattr(args, name)
+            t.ptr, t.dtype = 0x10000000 * (i + 1), dtype
+            lead = token if name != "out" else (length * heads * p, heads * p)
+            for j, stride in enumerate((*lead, *strides)):
+                t.stride[j] = stride
+        args.dt_bias.ptr, args.dt_bias.dtype, args.dt_bias.stride[0] = 0x2000, _hip.F32, 1
+    return args
+
+
+@pytest.mark.parametrize("rank", [1, 2, 4])
+@pytest.mark.parametrize("batch,length,heads", [(8, 1024, 32), (1, 4096, 16)])
+def test_workspace_query_ahead_of_the_buffers(lib, batch, length, heads, rank):
+    """The answer for arguments whose buffers are not set yet covers the call with any buffers: the
+    bound call's own need (its route must not depend on what the query could not know), and that of
+    rows on odd elements."""
+    size = ctypes.c_size_t(0)
+
+    def need(args):
+        assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+        return size.value
+
+    ahead = need(_model_scan_args(batch, length, heads, rank, False))
+    bound = _model_scan_args(batch, length, heads, rank, True)
+    assert ahead == need(bound) > 0
+    for t in (bound.q, bound.k):
+        t.ptr += 2
+    assert need(bound) <= ahead
+
+
+def test_widths_no_power_of_two_need_a_workspace_once_bound(lib):
+    """d_state 96 runs on the tiled kernels, with a workspace and split where that pays; a query
+    ahead of the buffers answers 0, with which the call takes the recurrent scan."""
+    size, g = ctypes.c_size_t(0), ctypes.c_int(0)
+    for dtype in (_hip.BF16, _hip.F32):
+        args = _model_scan_args(1, 4096, 4, 1, False, 96, dtype)
+        assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+        assert size.value == 0
+        args = _model_scan_args(1, 4096, 4, 1, True, 96, dtype)
+        assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+        assert size.value > 0
+        assert lib.m3_scan_segments(ctypes.byref(args), 1, ctypes.byref(g)) == 0
+        assert g.value > 1
+
+
 def test_scan_backwards_token_strides_on_the_host(lib):
     """Per-token tensors may run backwards (the reverse scan), but all of them together."""
     args = _hook_scan_args(1, 128, 2, 1)

@@ -303,3 +303,42 @@ def test_reversed_call_with_far_given_phases():
     want, want_state = scan(flipped, False)
     assert torch.equal(got, want.flip(1))
     assert torch.equal(state, want_state)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rank,d_state", [(1, 96), (4, 48), (2, 128), (4, 128), (1, 128)])
+def test_a_workspace_below_the_answer(rank, d_state, dtype):
+    """A call with less workspace than the query asks for takes the routes that need less: at a
+    d_state that is no power of 2 none at all; in 16 bits above rank 1, and for the model's shape,
+    without the q / k rows. Below that it is refused."""
+    torch.manual_seed(rank + d_state)
+    mixer = Mamba3(256, d_state=d_state, depth=1, mimo_rank=rank).eval().to(DEV).layers[0].mixer
+    proj = torch.randn(2, 300, mixer.in_proj.weight.shape[0], device=DEV).to(dtype)
+    with torch.inference_mode():
+        call = ops.ScanCall(proj, mixer, want_cache=True)
+        call.launch()
+        want = [t.clone() for t in (call.out, call.final_state, call.final_k)]
+        full = call.args.workspace_bytes
+        power = d_state & (d_state - 1) == 0
+        rows = 2 * 300 * rank * 2 * (2 if rank in (1, 4) else 4) * d_state
+        least = 0 if not power else full - rows if dtype == torch.bfloat16 else full
+        if power and dtype == torch.bfloat16:
+            least += 2 * 300 * rank * 2 * 4  # the norm factors in the rows' place
+        for t in (call.out, call.final_state, call.final_k):
+            t.fill_(float("nan"))
+        # (each region is rounded up to 256 bytes at most)
+        call.args.workspace_bytes = min(full, least + 512) if power else 0
+        if not power:
+            call.args.workspace = None
+        call.launch()
+        for got, ref in zip((call.out, call.final_state, call.final_k), want):
+            if dtype == torch.bfloat16:
+                # the model's shape is rounded after its norm, the others are not
+                bar = 3 * 2.0 ** -9
+            else:
+                bar = 1e-6
+            assert _error(got, ref.cpu()) <= bar
+        if power:
+            call.args.workspace_bytes = least // 2
+            with pytest.raises(_hip.HipError, match="workspace"):
+                call.launch()
