@@ -145,8 +145,9 @@ int m3_scan_fwd(const m3_scan_args* args, hipStream_t stream);
  * harnesses that forbid hipMalloc). The call uses the library's own device scratch, one static
  * array of M3_SCRATCH_BYTES per GPU, held until the process ends; args->workspace and
  * args->workspace_bytes are ignored. It allocates, frees and synchronises nothing. A call that
- * needs more than M3_SCRATCH_BYTES (m3_scan_workspace_size) runs unsplit, then without prepared
- * rows, where that fits, and fails with M3_EWORKSPACE only if nothing does. Every call
+ * needs more than M3_SCRATCH_BYTES (m3_scan_workspace_size) runs by the first of these that fits: split
+ * without copies of the q / k rows, unsplit, unsplit without copies, the recurrent scan (a d_state
+ * that is no power of 2). It fails with M3_EWORKSPACE only if none does. Every call
  * on one GPU uses that GPU's one scratch, which keeps the last call's contents: calls that overlap
  * in time on one GPU (on different streams) race, so the caller must order them.
  */

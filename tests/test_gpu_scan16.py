@@ -243,10 +243,10 @@ def test_projection_form_shapes(rank, d_model, d_state, length, reverse):
 
 
 def test_scan_without_room_for_rows():
-    """m3_scan_fwd_noalloc's calls too large for the q / k rows run on the kernels that keep
-    none: the same result as the workspace call."""
+    """A hook call whose q and k alone would fill m3_scan_fwd_noalloc's scratch: its rows are read as
+    they lie, and the result is the workspace call's."""
     torch.manual_seed(3)
-    b, l, h, n, p, r = 20, 1024, 2, 64, 16, 8  # 20 x 1024 x 8 x 2 x 128 x 2 B = 84 MB of rows
+    b, l, h, n, p, r = 20, 1024, 2, 64, 16, 8  # q, k at 128 slots: 84 MB
     mk = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)
     q, k, v, z, tr = mk(b, l, 1, r, n), mk(b, l, 1, r, n), mk(b, l, h, p), mk(b, l, h, p), mk(b, l, h)
     dt = torch.rand(b, l, h, device=DEV) * 0.1
@@ -342,3 +342,49 @@ def test_a_workspace_below_the_answer(rank, d_state, dtype):
             call.args.workspace_bytes = least // 2
             with pytest.raises(_hip.HipError, match="workspace"):
                 call.launch()
+
+
+def test_noalloc_keeps_the_split():
+    """A call whose q / k rows outgrow the scratch (1 x 32768 tokens, rank 2, FP32 rows: 67 MB) stays
+    split, reading the caller's rows: bit for bit m3_scan_fwd's result with a workspace that has no
+    room for the rows, which keeps the split; an unsplit scan sums in another order."""
+    torch.manual_seed(4)
+    mixer = Mamba3(128, d_state=128, depth=1, mimo_rank=2).eval().to(DEV).layers[0].mixer
+    proj = torch.randn(1, 32768, mixer.in_proj.weight.shape[0], device=DEV).to(torch.bfloat16)
+    with torch.inference_mode():
+        call = ops.ScanCall(proj, mixer, want_cache=True)
+        assert call.args.workspace_bytes > _hip.SCRATCH_BYTES
+        call.launch()
+        out = call.out.clone()
+        call.args.workspace_bytes = _hip.SCRATCH_BYTES
+        call.launch()
+        want = [t.clone() for t in (call.out, call.final_state, call.final_phase, call.final_k)]
+        for t in (call.out, call.final_state, call.final_phase, call.final_k):
+            t.fill_(float("nan"))
+        args = type(call.args).from_buffer_copy(call.args)
+        args.workspace, args.workspace_bytes = None, 0
+        _hip.call("m3_scan_fwd_noalloc", args, DEV)
+    for got, ref in zip((call.out, call.final_state, call.final_phase, call.final_k), want):
+        assert torch.equal(got, ref)
+    _close(call.out, out.cpu(), torch.bfloat16)
+
+
+def test_noalloc_ends_at_the_recurrent_scan():
+    """FP32 at a d_state that is no power of 2, more scalar blocks than the scratch holds (800 x 64
+    heads x 64 tokens, 68 MB): the recurrent scan, which needs no scratch, as the workspace call."""
+    torch.manual_seed(6)
+    b, l, h, n, p = 800, 64, 64, 96, 4
+    mk = lambda *s: torch.randn(*s, device=DEV)
+    t = dict(q=mk(b, l, 1, 1, n), k=mk(b, l, 1, 1, n), value=mk(b, l, h, p), gate=mk(b, l, h, p),
+             dt=torch.rand(b, l, h, device=DEV) * 0.1, trap=mk(b, l, h), D=torch.ones(h, device=DEV))
+    t["a"] = -t["dt"]
+    want, want_state = ops.mamba3_scan(t["q"], t["k"], t["value"], t["gate"], t["a"], t["dt"],
+                                       t["trap"], t["D"])
+    out, state = torch.empty_like(want), torch.empty_like(want_state)
+    args = _hip.ScanArgs(batch=b, length=l, heads=h, groups=1, rank=1, d_state=n, head_dim=p,
+                         chunk=64, act_dtype=_hip.F32, phase_mode=_hip.PHASE_NONE, norm_eps=1e-5)
+    for name, x in dict(t, out=out, final_state=state).items():
+        setattr(args, name, _hip.tensor(x))
+    _hip.call("m3_scan_fwd_noalloc", args, DEV)
+    assert _error(out, want.cpu()) <= 1e-6
+    assert _error(state, want_state.cpu()) <= 1e-6
