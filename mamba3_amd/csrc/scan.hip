@@ -532,7 +532,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     // written, reads the same chunks where the rows start on 8 bytes only; a chunk past column N
     // counts zeros.
     const bool rows_out = sizeof(T) == 2 && g.ws_qk >= 0;
-    const int perm = rows_out ? g.perm : 0;
+    const int perm = R > 1 && rows_out ? g.perm : 0;
     const bool pairs = perm && 8 * l16 < 2 * a.num_angles;
     const bool in_b = 8 * l16 + 4 < N;
     const int ca = !in ? 0 : pairs ? 4 * l16 : slot_col(8 * l16, perm, a.num_angles);
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
         // The lane's tensor's weights (every row of the lane is q, or every row k) are chosen by
         // bit masks on the raw words: a select between two weight arrays by `which` became a
         // dynamically indexed array in scratch memory
-        const bool norm = a.q_norm_w.ptr != nullptr;
+        const bool norm = R == 1 || a.q_norm_w.ptr != nullptr;
         float wl[8] = {};
         if (nw_vec) {
           const uint32_t msk = 0u - static_cast<uint32_t>(which);
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
             y[2 * i] = pairs ? x[i] : x[2 * i];
             y[2 * i + 1] = pairs ? x[4 + i] : x[2 * i + 1];
           }
-          if (g.form16 == kRows) {
+          if (R > 1 && g.form16 == kRows) {
             float* o = reinterpret_cast<float*>(qk) + static_cast<int64_t>(row) * N + 8 * l16;
             if (in) *reinterpret_cast<f4*>(o) = (f4){y[0], y[1], y[2], y[3]};
             if (in_b) *reinterpret_cast<f4*>(o + 4) = (f4){y[4], y[5], y[6], y[7]};
@@ -767,66 +767,71 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
     const int s1_dt = static_cast<int>(a.dt.stride[1]), s2_dt = static_cast<int>(a.dt.stride[2]);
     const int s1_a = static_cast<int>(a.a.stride[1]), s2_a = static_cast<int>(a.a.stride[2]);
     const int s1_tr = static_cast<int>(a.trap.stride[1]), s2_tr = static_cast<int>(a.trap.stride[2]);
-    auto heads_of = [&](auto hg) {
+    // the inputs of heads h0 .. h0 + hn - 1, hg at a time, into LDS (the scalar blocks below are one
+    // copy of code for both sizes; with one each, and the copies of MIMO rows in rank 1's code, prep
+    // took 34.8 us instead of 34.1 at 8 x 8192 tokens of 32 heads, and 40.9 instead of 40.0 at rank 4,
+    // 8 x 4096)
+    auto stage = [&](auto hg, int h0, int hn) {
       constexpr int HG = decltype(hg)::value, NE = (TOK + 1) * HG, NIT = (NE + 255) / 256;
-      for (int h0 = hgi * hpg; h0 < h_end; h0 += HG) {
-        const int hn = min(HG, h_end - h0);
-        // raw loads of every element first (clamped to valid tokens / heads), then decode and store
-        RawX rd[NIT], ra[NIT], rt[NIT];
-        // dt_bias with the batch (inside the per-head loop below, after its stores, each head's
-        // load would be a round trip of its own)
-        const RawX rdb = a.raw_dt != 0
-                             ? ldraw(a.dt_bias.ptr, a.dt_bias.dtype,
-                                     (h0 + min(tid & (HG - 1), hn - 1)) * a.dt_bias.stride[0])
-                             : RawX{0u, 0u};
+      // raw loads of every element first (clamped to valid tokens / heads), then decode and store
+      RawX rd[NIT], ra[NIT], rt[NIT];
+      // dt_bias with the batch (inside the per-head loop below, after its stores, each head's
+      // load would be a round trip of its own)
+      const RawX rdb = a.raw_dt != 0
+                           ? ldraw(a.dt_bias.ptr, a.dt_bias.dtype,
+                                   (h0 + min(tid & (HG - 1), hn - 1)) * a.dt_bias.stride[0])
+                           : RawX{0u, 0u};
 #pragma unroll
-        for (int k = 0; k < NIT; ++k) {
-          const int e = min(tid + 256 * k, NE - 1);
-          const int j = e / HG, hh = e - j * HG;
-          const int t = min(c * TOK + j, L - 1), h = h0 + min(hh, hn - 1);
-          rd[k] = ldraw(base_dt, a.dt.dtype, t * s1_dt + h * s2_dt);
-          ra[k] = ldraw(base_a, a.a.dtype, t * s1_a + h * s2_a);
-          rt[k] = ldraw(base_tr, a.trap.dtype, t * s1_tr + h * s2_tr);
-        }
-#pragma unroll
-        for (int k = 0; k < NIT; ++k) {
-          const int e = tid + 256 * k;
-          if (e < NE) {
-            const int j = e / HG, hh = e - j * HG;
-            s_in[0][j][hh] = decode(rd[k], a.dt.dtype);
-            s_in[1][j][hh] = decode(ra[k], a.a.dtype);
-            s_in[2][j][hh] = decode(rt[k], a.trap.dtype);
-          }
-        }
-        if (tid < HG) s_db[tid] = a.raw_dt != 0 ? decode(rdb, a.dt_bias.dtype) : 0.f;
-        __syncthreads();
-        if constexpr (TOK <= 16) {
-          // 64 / TOK heads per wave (one wave per head would leave most lanes idle)
-          constexpr int HPW = 64 / TOK;
-          const int j = lane & (TOK - 1);
-          for (int hb = w * HPW; hb < hn; hb += 4 * HPW) {
-            const int hh = hb + lane / TOK, hc = min(hh, hn - 1);
-            scalar_block_seg<TOK, TPT, LO>(
-                a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
-                c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
-                s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
-          }
-        } else {
-          for (int hh = w; hh < hn; hh += 4) {
-            const int h = h0 + hh, j = min(lane, TOK - 1);
-            scalar_block<TOK, TPT, LO>(
-                a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
-                lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
-                s_in[2][TOK][hh], cut);
-          }
-        }
-        __syncthreads();
+      for (int k = 0; k < NIT; ++k) {
+        const int e = min(tid + 256 * k, NE - 1);
+        const int j = e / HG, hh = e - j * HG;
+        const int t = min(c * TOK + j, L - 1), h = h0 + min(hh, hn - 1);
+        rd[k] = ldraw(base_dt, a.dt.dtype, t * s1_dt + h * s2_dt);
+        ra[k] = ldraw(base_a, a.a.dtype, t * s1_a + h * s2_a);
+        rt[k] = ldraw(base_tr, a.trap.dtype, t * s1_tr + h * s2_tr);
       }
+#pragma unroll
+      for (int k = 0; k < NIT; ++k) {
+        const int e = tid + 256 * k;
+        if (e < NE) {
+          const int j = e / HG, hh = e - j * HG;
+          s_in[0][j][hh] = decode(rd[k], a.dt.dtype);
+          s_in[1][j][hh] = decode(ra[k], a.a.dtype);
+          s_in[2][j][hh] = decode(rt[k], a.trap.dtype);
+        }
+      }
+      if (tid < HG) s_db[tid] = a.raw_dt != 0 ? decode(rdb, a.dt_bias.dtype) : 0.f;
     };
-    if (hpg <= 8) {
-      heads_of(std::integral_constant<int, 8>{});
-    } else {
-      heads_of(std::integral_constant<int, HG_MAX>{});
+    const int hg = hpg <= 8 ? 8 : HG_MAX;
+    for (int h0 = hgi * hpg; h0 < h_end; h0 += hg) {
+      const int hn = min(hg, h_end - h0);
+      if (hg == 8) {
+        stage(std::integral_constant<int, 8>{}, h0, hn);
+      } else {
+        stage(std::integral_constant<int, HG_MAX>{}, h0, hn);
+      }
+      __syncthreads();
+      if constexpr (TOK <= 16) {
+        // 64 / TOK heads per wave (one wave per head would leave most lanes idle)
+        constexpr int HPW = 64 / TOK;
+        const int j = lane & (TOK - 1);
+        for (int hb = w * HPW; hb < hn; hb += 4 * HPW) {
+          const int hh = hb + lane / TOK, hc = min(hh, hn - 1);
+          scalar_block_seg<TOK, TPT, LO>(
+              a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h0 + hc) * g.nsub + c) * g.scw,
+              c, lane, hh < hn, s_db[hc], s_in[0][j][hc], s_in[1][j][hc], s_in[2][j][hc],
+              s_in[0][TOK][hc], s_in[2][TOK][hc], cut);
+        }
+      } else {
+        for (int hh = w; hh < hn; hh += 4) {
+          const int h = h0 + hh, j = min(lane, TOK - 1);
+          scalar_block<TOK, TPT, LO>(
+              a, ws + g.ws_sc + (static_cast<int64_t>(b * a.heads + h) * g.nsub + c) * g.scw, c,
+              lane, s_db[hh], s_in[0][j][hh], s_in[1][j][hh], s_in[2][j][hh], s_in[0][TOK][hh],
+              s_in[2][TOK][hh], cut);
+        }
+      }
+      __syncthreads();
     }
   }
 }
