@@ -2547,12 +2547,14 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
 // pairs lie whole 8-column lanes apart (d_state 96, 4 x 1500 tokens, 16 heads: 21.7 ms on the
 // recurrent scan, 185 us here); and the 16-wave kernel's calls at every d_state it takes. Others
 // take the recurrent scan (rscan.hip), and so does every d_state that is no power of 2 with `rows`
-// false (the least workspace).
+// false (the least workspace), and one token, its whole call one kernel there (31 us with the
+// Python host, 36 as prep and scan; 4 tokens 63 and 36).
 static bool tiled_shape(const m3_scan_args& a, bool rows = true) {
   const bool fits = a.d_state >= 4 && a.d_state <= kNPad && a.head_dim <= kPPad &&
                     a.num_angles <= kSMax &&
                     (a.rank == 1 || a.rank == 2 || a.rank == 4 || a.rank == 8);
   if (fits && pow2(a.d_state)) return true;
+  if (a.length == 1) return false;
   if (fits && rows && a.act_dtype == M3_F32 && a.q.ptr != nullptr &&
       (a.phase_mode == M3_PHASE_NONE || a.mimo_rotation == 0 || a.d_state % 16 == 0)) {
     return true;

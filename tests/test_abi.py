@@ -383,6 +383,10 @@ def test_widths_no_power_of_two_need_a_workspace_once_bound(lib):
         assert size.value > 0
         assert lib.m3_scan_segments(ctypes.byref(args), 1, ctypes.byref(g)) == 0
         assert g.value > 1
+        # one token: the recurrent scan
+        args = _model_scan_args(1, 1, 4, 1, True, 96, dtype)
+        assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+        assert size.value == 0
 
 
 def test_scan_backwards_token_strides_on_the_host(lib):
