@@ -450,8 +450,9 @@ def test_noalloc_scan_rejects_calls_beyond_its_scratch(lib):
 
 
 def test_recurrent_shapes_need_no_workspace(lib):
-    """Shapes the MFMA scan does not tile take the recurrent scan, which needs no workspace and
-    cannot be split into segments; d_state below 4 is refused."""
+    """Shapes the MFMA scans do not tile take the recurrent scan, which needs no workspace and
+    cannot be split into segments (d_state 256, and 96 as long as its buffers are not set);
+    d_state below 4 is refused."""
     def args(**kw):
         base = dict(batch=2, length=100, heads=2, groups=1, rank=1, d_state=96, head_dim=32,
                     num_angles=24, chunk=64, act_dtype=_hip.BF16, mimo_rotation=0, raw_dt=0,
@@ -461,6 +462,10 @@ def test_recurrent_shapes_need_no_workspace(lib):
     need = ctypes.c_size_t(123)
     assert lib.m3_scan_workspace_size(ctypes.byref(args()), ctypes.byref(need)) == 0
     assert need.value == 0
+    assert lib.m3_scan_workspace_size(ctypes.byref(args(d_state=256)), ctypes.byref(need)) == 0
+    assert need.value == 0
+    assert lib.m3_scan_fwd(ctypes.byref(args(d_state=256, segments=4)), None) == 2
+    assert b"segments" in lib.m3_last_error()
     assert lib.m3_scan_workspace_size(ctypes.byref(args(d_state=128, num_angles=32, head_dim=64)),
                                       ctypes.byref(need)) == 0
     assert need.value > 0

@@ -319,7 +319,8 @@ def test_config1_parity():
     torch.testing.assert_close(steps, want[:, 960:], **F32)
 
 
-# Models whose shapes the MFMA scan does not tile (the recurrent scan), and whose decode step
+# Models whose shapes the MFMA scans do not tile (the recurrent scan; d_state 96, which they do, but
+# whose one-token calls are not theirs), and whose decode step
 # runs on the step kernels (d_state 256) or as a one-token recurrent scan (d_state not a power
 # of 2, rank 3; d_state 1024, whose 256 KiB state is updated in final_state instead of LDS;
 # rank 16, read out in two groups of 8): forward, prefill and steps against the oracle.

@@ -1,5 +1,6 @@
 """Sequences the library splits into segments of which the last is shorter: split against
-unsplit, over ranks, dtypes, given and walked phases, starts and widths."""
+unsplit, over ranks, dtypes, walked phases (projection form), given or no phases (hook form),
+starts and widths."""
 
 from __future__ import annotations
 
@@ -31,7 +32,7 @@ def _segments(call) -> int:
     (128, 128, 4, 2, 1001),
     (96, 64, 2, 1, 2049),    # one token in the last sub-chunk
     (64, 128, 8, 1, 700),
-    (128, 96, 1, 3, 1500),   # d_state no power of two (FP32: the recurrent scan, never split)
+    (128, 96, 1, 3, 1500),   # d_state no power of two
     (256, 48, 4, 1, 900),
 ])
 def test_split_matches_unsplit(d_model, d_state, rank, batch, length, dtype, monkeypatch):
@@ -50,11 +51,9 @@ def test_split_matches_unsplit(d_model, d_state, rank, batch, length, dtype, mon
             blocks = torch.full((batch, mixer.nheads, (length + 63) // 64, mixer.num_angles),
                                 float("nan"), device=DEV)
             decay = torch.full((batch, mixer.nheads), float("nan"), device=DEV)
-            tiled = d_state & (d_state - 1) == 0 or dtype != torch.float32
-            if tiled:
-                call.args.block_phase = _hip.tensor(blocks)
-                call.args.final_decay = _hip.tensor(decay)
-                assert (_segments(call) > 1) == (segs == 0)
+            call.args.block_phase = _hip.tensor(blocks)
+            call.args.final_decay = _hip.tensor(decay)
+            assert (_segments(call) > 1) == (segs == 0)
             call.launch()
             res[segs] = (call.out, call.final_state, call.final_phase, call.final_k, blocks, decay)
             back = ops.ScanCall(proj, mixer, reverse=True)
@@ -64,9 +63,8 @@ def test_split_matches_unsplit(d_model, d_state, rank, batch, length, dtype, mon
     for i in (0, 1, 3, 6, 7):
         _close(split[i], one[i], dtype)
     assert torch.equal(split[2], one[2]), "the phase carry differs from the unsplit scan's"
-    if tiled:
-        assert torch.equal(split[4], one[4])
-        _close(split[5], one[5], torch.float32)
+    assert torch.equal(split[4], one[4])
+    _close(split[5], one[5], torch.float32)
 
 
 def test_two_concurrent_calls_take_the_librarys_ragged_count():
@@ -102,3 +100,56 @@ def test_ragged_rows_read_only_their_own(d_model, d_state, rank, length, dtype, 
         call.launch()
     for got, ref in zip((call.out, call.final_state, call.final_phase, call.final_k), want):
         assert torch.equal(got[:1], ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rank,d_state,groups,length,given,initial,segments", [
+    (1, 128, 1, 1777, True, True, 0),    # 64-token sub-chunks in 16 bits, 32 in FP32
+    (2, 128, 1, 1000, True, False, 0),   # 32 and 16: cuts off the 64-token phase blocks
+    (2, 64, 2, 1000, False, True, 10),   # a request of 100 tokens a segment, rounded up
+    (4, 128, 1, 601, True, True, 0),     # 16 and 8
+    (4, 64, 4, 555, False, False, 5),
+    (8, 128, 1, 333, True, True, 0),     # 8 and 4
+    (8, 16, 2, 260, False, True, 13),
+    (1, 96, 2, 1500, True, True, 0),     # d_state no power of two
+    (4, 48, 1, 700, True, True, 7),
+])
+def test_hook_split_matches_unsplit(rank, d_state, groups, length, given, initial, segments, dtype,
+                                    monkeypatch):
+    """The hook form, split (the state-only first pass, segments on sub-chunks of 64 / rank tokens)
+    against unsplit: given phases or none, with and without a start, over the q / k row sources
+    (2 heads to a group or 16), and by the routes without copies of the rows."""
+    g = torch.Generator(DEV).manual_seed(length)
+    heads, p, s = 16 if groups == 1 else 2 * groups, 32, d_state // 4
+    mk = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    q, k = (mk(1, length, groups, rank, d_state).to(dtype) for _ in range(2))
+    v, z, tr = mk(1, length, heads, p).to(dtype), mk(1, length, heads, p).to(dtype), mk(1, length, heads)
+    dt = torch.rand(1, length, heads, generator=g, device=DEV) * 0.1
+    kw = dict(phase=mk(1, length, heads, s), mimo_rotation=rank > 1) if given else {}
+    if rank > 1:
+        kw.update({m: mk(heads, rank, p).to(dtype).float() for m in ("mimo_x", "mimo_z", "mimo_out")})
+    if initial:
+        kw.update(initial_state=mk(1, heads, p, d_state), initial_k=mk(1, heads, rank, d_state).to(dtype),
+                  initial_value=mk(1, heads, p).to(dtype))
+    sizes = {}
+    query = _hip.scan_workspace
+
+    def scan(segs, short=0):
+        monkeypatch.setattr(ops, "SCAN_SEGMENTS", segs)
+
+        def workspace(args, device):
+            ws = query(args, device)
+            sizes[segs] = args.workspace_bytes
+            args.workspace_bytes -= short
+            return ws
+        monkeypatch.setattr(_hip, "scan_workspace", workspace)
+        return ops.mamba3_scan(q, k, v, z, -dt, dt, tr, torch.ones(heads, device=DEV), **kw)
+
+    one, split = scan(1), scan(segments)
+    assert sizes[segments] > sizes[1], "not split"
+    for got, want in zip(split, one):
+        _close(got, want, dtype)
+    if dtype == torch.bfloat16 and rank > 1 and groups == 1 and d_state & (d_state - 1) == 0:
+        # 256 bytes short of the copies of the rows: they are read as they lie
+        for got, want in zip(scan(segments, 256), split):
+            assert torch.equal(got, want)

@@ -302,9 +302,10 @@ def test_chunk_state_in_place(shape):
     assert torch.equal(st, out)  # in place and out of place agree bit for bit
 
 
-# Shapes outside the MFMA kernel's tiles (d_state not a power of 2 or above 128, head_dim above
-# 64, ranks 3, 5, 6, 7): the recurrent scan. FP32 within 1e-4 of the oracle's chunked scan (the
-# same recurrence, summed in another order); 16-bit at the 16-bit parity bar.
+# Shapes outside the MFMA kernels' tiles (d_state above 128, head_dim above 64, ranks 3, 5, 6, 7 and
+# above 8; in 16 bits a d_state no multiple of 4): the recurrent scan; and d_state 96 and 20, which
+# the MFMA kernels take, beside it. FP32 within 1e-4 of the oracle's chunked scan (the same
+# recurrence, summed in another order); 16-bit at the 16-bit parity bar.
 RECURRENT = [
     # (rank, d_state, head_dim, heads, length)
     (1, 256, 64, 2, 150),
@@ -317,6 +318,7 @@ RECURRENT = [
     (1, 1024, 64, 2, 70),   # 256 KiB state: updated in final_state
     (16, 128, 64, 2, 50),   # rank 16: two readout groups
     (12, 64, 32, 1, 40),    # rank 12: a partial second group
+    (1, 22, 24, 2, 60),     # 16 bits: rows on 4 bytes; FP32: the MFMA kernel
 ]
 
 
@@ -341,14 +343,15 @@ def test_recurrent_scan_matches_oracle(shape, dtype):
 
 
 @pytest.mark.parametrize("rank,d_state,span", [(1, 96, 6.0), (1, 100, 1e4), (2, 48, 1e6), (4, 112, 6.0),
-                                               (8, 80, 1e7)])
+                                               (8, 80, 1e7), (2, 12, 1e5), (4, 24, 6.0)])
 @pytest.mark.parametrize("segments", [1, 4])
 def test_fp32_widths_no_power_of_two_are_exact(rank, d_state, span, segments, monkeypatch):
     """FP32 at a d_state that is no power of 2, unsplit and split, against the float64 recurrence:
     a few roundings of 2^-24 in each of some hundred decaying terms, 16 x 2^-24 for the whole; the
-    given phases count to full precision at any number of turns."""
+    given phases count to full precision at any number of turns. The MIMO pairs at d_state 12 and 24,
+    no multiple of 16, are the recurrent scan's, which is not split."""
     from oracle.recurrence import recurrent_scan
-    monkeypatch.setattr(ops, "SCAN_SEGMENTS", segments)
+    monkeypatch.setattr(ops, "SCAN_SEGMENTS", segments if d_state not in (12, 24) else 1)
     length, heads = 256, 3
     inp = _inputs(rank, torch.float32, batch=1, length=length, heads=heads, head_dim=32,
                   d_state=d_state, seed=d_state, initial=False)
