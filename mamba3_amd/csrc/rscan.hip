@@ -1,5 +1,7 @@
-// Mamba-3 scan for the shapes the chunked MFMA kernel (scan.hip) does not tile: d_state not a
-// power of 2 or above 128, head_dim above 64, more than 32 angles, ranks 3, 5, 6 and 7.
+// Mamba-3 scan for the shapes the chunked MFMA kernels (scan.hip, scan16_kernel.hpp) do not tile:
+// d_state above 128, head_dim above 64, more than 32 angles, ranks 3, 5, 6, 7 and above 8; and, of a
+// d_state up to 128 that is no power of 2, the 16-bit rows that cannot be read 4 elements at a time,
+// the MIMO pairs at no multiple of 16, one token, and calls without the workspace those need.
 // The reference takes any d_state >= 4 and any rank on its portable path (model.py:545-548,
 // ops.py:544-822); this kernel gives those shapes a GPU path.
 //

@@ -846,12 +846,13 @@ __global__ __launch_bounds__(256) void prep_kernel(const m3_scan_args a, const S
 // out, and with them (dead code) the q math, the scores, the decay weights, the intra and inter
 // products and the epilogue.
 // LO (FP32): d_state no power of 2. Those calls came from the recurrent scan and are no further from
-// 64 bits than there: its functions (exp_x, sincos_of), and sums taken apart from what they are
-// added to (a matrix instruction rounds at the size of its accumulator four times). Errors of 2 x
-// 500 tokens, hook form, output and state: d_state 96 rank 1 recurrent 1.5e-7 and 2.4e-7, without
-// these 1.9e-7 and 1.5e-7, with them 1.2e-7 and 1.2e-7; rank 8 1.4e-7 and 2.4e-7, 1.3e-7 and 3.2e-7,
-// 0.9e-7 and 1.4e-7; given phases of 10^5 at rank 1 1.8e-7 and 2.5e-7, 3e-4 and 1.5e-3, 1.2e-7 and
-// 1.3e-7.
+// 64 bits than there: its functions (exp_x, sincos_of), the carry's sum taken apart from the state it
+// is added to (a matrix instruction rounds at the size of its accumulator four times), and the
+// scores' and the inter product's in two halves. Errors of 2 x 500 tokens, hook form, output and
+// state: d_state 96 rank 1 recurrent 1.5e-7 and 2.4e-7, without these 1.9e-7 and 1.5e-7, with them
+// 1.4e-7 and 1.2e-7; rank 8 1.4e-7 and 2.4e-7, 1.3e-7 and 3.2e-7, 0.9e-7 and 1.4e-7; given phases of
+// 10^5 at rank 1 1.8e-7 and 2.5e-7, 3e-4 and 1.5e-3, 1.4e-7 and 1.3e-7. Time, 16 x 2048 tokens, 32
+// heads: 985 us without, 1,220 with; 1,367 with eight sums each, whose registers spill (output 1.2e-7).
 template <typename T, int R, bool FULL, bool SHAPE = false, bool SO = false, bool LO = false>
 __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, const ScanGeom g,
                                                         const float* __restrict__ prep) {
@@ -1442,14 +1443,15 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
           acc[sj] = M::mma(av, qv[kk], acc[sj]);
         }
       } else {
+        f4 half = zero4();
 #pragma unroll
         for (int kk = 0; kk < NP / 16; ++kk) {
           const f4 kv = *reinterpret_cast<const f4*>(Ks + (16 * sj + l16) * LQ + 16 * kk + 4 * lg);
-          f4 sum = LO ? zero4() : acc[sj];
+          f4& sum = LO && kk < NP / 32 ? half : acc[sj];
 #pragma unroll
           for (int i = 0; i < 4; ++i) sum = M::mma(kv[i], qf[kk][i], sum);
-          acc[sj] = LO ? acc[sj] + sum : sum;
         }
+        if constexpr (LO) acc[sj] += half;
       }
     }
     // K~^T V products of the state carry, issued early (they depend only on staged tiles),
@@ -1610,14 +1612,15 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(const m3_scan_args a, co
 #pragma unroll
           for (int i = 0; i < 4; ++i) yi = M::mma(vv[i], wsc[sj][i], yi);
         }
+        f4 half = zero4();
 #pragma unroll
         for (int kk = 0; kk < NP / 16; ++kk) {
           const f4 sv = *reinterpret_cast<const f4*>(Sb + pcol * LQ + 16 * kk + 4 * lg);
-          f4 sum = LO ? zero4() : ye;
+          f4& sum = LO && kk < NP / 32 ? half : ye;
 #pragma unroll
           for (int i = 0; i < 4; ++i) sum = M::mma(sv[i], qf[kk][i], sum);
-          ye = LO ? ye + sum : sum;
         }
+        if constexpr (LO) ye += half;
       }
       // epilogue: row trow (token tq, rank rr), columns pb .. pb+3
       const int pb = 16 * pj + 4 * lg;
