@@ -2093,10 +2093,11 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // that is not set yet (a workspace query ahead of the buffers) counts as one that fits; at a d_state
 // no power of 2, whose other route needs no workspace, as one that does not.
 // Every such call is faster on it than on the kernel it took before (per call, scan_kernel then
-// scan16_kernel, 8 x 1024 tokens, 32 heads): hook form rank 1 80 -> 72 us, rank 2 184 -> 118,
-// rank 4 332 -> 207, rank 8 628 -> 392; projection form rank 2 140 -> 121, rank 8 487 -> 391,
-// d_state 64 rank 1 114 -> 67; the recurrent scan at d_state 96, 4 x 1500 tokens, 16 heads:
-// 21.6 ms -> 86 us.
+// scan16_kernel, 8 x 1024 tokens, 32 heads): hook form rank 1 80 -> 71 us, rank 2 184 -> 120,
+// rank 4 332 -> 200, rank 8 628 -> 359; projection form rank 2 140 -> 120, rank 8 487 -> 381,
+// d_state 64 rank 1 114 -> 73; hook form of 32 groups, 4 x 4096 tokens, 518 -> 235, of 64 groups at
+// rank 8, 64 heads, 1,678 -> 858; the recurrent scan at d_state 96, 4 x 1500 tokens, 16 heads: 21.6
+// ms -> 77 us.
 static int form16_of(const m3_scan_args& a, bool rows) {
   if (a.act_dtype != M3_BF16 && a.act_dtype != M3_F16) return -1;
   if (a.rank != 1 && a.rank != 2 && a.rank != 4 && a.rank != 8) return -1;
@@ -2548,7 +2549,7 @@ static Segments auto_segments(const m3_scan_args& a, int64_t unit, int concurren
 // The shapes the chunked MFMA kernels tile: up to 128 columns, 64 values and 32 angles at ranks 1,
 // 2, 4 and 8, with d_state a power of 2; in FP32 also any other, with the MIMO rotation where its
 // pairs lie whole 8-column lanes apart (d_state 96, 4 x 1500 tokens, 16 heads: 21.7 ms on the
-// recurrent scan, 185 us here); and the 16-wave kernel's calls at every d_state it takes. Others
+// recurrent scan, 216 us here); and the 16-wave kernel's calls at every d_state it takes. Others
 // take the recurrent scan (rscan.hip), and so does every d_state that is no power of 2 with `rows`
 // false (the least workspace), and one token, its whole call one kernel there (31 us with the
 // Python host, 36 as prep and scan; 4 tokens 63 and 36).

@@ -58,7 +58,8 @@ namespace m3 {
 // LO: d_state no power of 2. Those calls are the recurrent scan's on rows that are not aligned, and
 // came from it: it holds the decay weights and the scaled values in FP32, rounding neither. Here
 // each becomes two 16-bit operands, the rounded value and the rounding error (for FP16 times 2^11,
-// in accumulators of its own, so that it stays a normal number), and two products. Output error
+// in accumulators of its own, so that it stays a normal number; above 65504 it overflows, as at a
+// power of 2), and two products. Output error
 // against 64 bits (bf16, 2 x 500 tokens; recurrent scan, one operand each, two weights alone, two
 // each): hook form d_state 96 rank 1 2.00e-3, 2.43e-3, 2.04e-3, 1.85e-3; projection form d_state
 // 112 rank 2 3.18e-3, 3.28e-3, 3.26e-3, 3.10e-3.
