@@ -153,3 +153,57 @@ def test_hook_split_matches_unsplit(rank, d_state, groups, length, given, initia
         # 256 bytes short of the copies of the rows: they are read as they lie
         for got, want in zip(scan(segments, 256), split):
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("segments", [1, 3])
+@pytest.mark.parametrize("rank,d_state,groups,length", [
+    (1, 128, 1, 195), (1, 64, 4, 99), (2, 128, 4, 75), (2, 128, 1, 75), (4, 48, 2, 45), (8, 128, 1, 27),
+    (1, 96, 16, 195)])
+def test_hook_rows_read_only_their_own(rank, d_state, groups, length, segments, monkeypatch):
+    """The hook form's rows end with their batch row and group: the next batch row all NaN, the
+    other groups' q and k NaN beside the first's, the workspace all bits set before the call."""
+    monkeypatch.setattr(ops, "SCAN_SEGMENTS", segments)
+    g = torch.Generator(DEV).manual_seed(length)
+    heads, p, s = 16, 32, d_state // 4
+    mk = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    dtype = torch.bfloat16
+    t = dict(q=mk(2, length, groups, rank, d_state).to(dtype), k=mk(2, length, groups, rank, d_state).to(dtype),
+             value=mk(2, length, heads, p).to(dtype), gate=mk(2, length, heads, p).to(dtype),
+             dt=torch.rand(2, length, heads, generator=g, device=DEV) * 0.1,
+             trap_logits=mk(2, length, heads), phase=mk(2, length, heads, s))
+    t["adt"] = -t["dt"]
+    kw = dict(D=torch.ones(heads, device=DEV), mimo_rotation=rank > 1)
+    if rank > 1:
+        kw.update({m: mk(heads, rank, p) for m in ("mimo_x", "mimo_z", "mimo_out")})
+    query = _hip.scan_workspace
+
+    def dirty(args, device):
+        ws = query(args, device)
+        ws.fill_(255)
+        return ws
+    monkeypatch.setattr(_hip, "scan_workspace", dirty)
+    want, want_state = ops.mamba3_scan(**{n: x[:1].contiguous() for n, x in t.items()}, **kw)
+    for name, x in t.items():
+        x[1] = float("nan")
+        if name in ("q", "k") and groups > 1:
+            x[0, :, 1:] = float("nan")
+    got, state = ops.mamba3_scan(**t, **kw)
+    own = heads // groups  # the heads of the first group
+    assert torch.equal(got[:1, :, :own], want[:, :, :own])
+    assert torch.equal(state[:1, :own], want_state[:, :own])
+    assert torch.isfinite(want.float()).all()
+
+
+@pytest.mark.parametrize("concurrent", [5, 7, 12])
+@pytest.mark.parametrize("length", [1055, 2048])
+def test_many_concurrent_calls(concurrent, length):
+    """More concurrent calls than the library takes ragged counts back for: its answer is one that
+    divides the sequence, or no split, and the call runs."""
+    torch.manual_seed(length)
+    mixer = Mamba3(256, d_state=128, depth=1).eval().to(DEV).layers[0].mixer
+    proj = torch.randn(1, length, mixer.in_proj.weight.shape[0], device=DEV).to(torch.bfloat16)
+    with torch.inference_mode():
+        got = ops.scan_projection(proj, mixer, concurrent=concurrent)
+        want = ops.scan_projection(proj, mixer)
+    _close(got[0], want[0], torch.bfloat16)
+    _close(got[1], want[1], torch.bfloat16)
