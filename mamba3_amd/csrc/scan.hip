@@ -2176,7 +2176,9 @@ static int form16_of(const m3_scan_args& a, bool rows) {
       ahead * a.rank * 2 * kNPad * 2 < INT32_MAX) {
     return kModel;
   }
-  if (rows && a.rank > 1 && ahead * a.groups * a.rank * 2 * N * 4 < INT32_MAX) {
+  // prep's rows of one batch row, in 32 bits
+  const int64_t row_bytes = proj ? N * 4 : kNPad * 2;
+  if (rows && a.rank > 1 && ahead * a.groups * a.rank * 2 * row_bytes < INT32_MAX) {
     if (proj) return kRows;
     if (a.heads >= 16 * a.groups && int64_t{2} * a.batch * len * a.groups * a.rank < INT32_MAX) return kCopy;
   }

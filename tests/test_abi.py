@@ -389,6 +389,22 @@ def test_widths_no_power_of_two_need_a_workspace_once_bound(lib):
         assert size.value == 0
 
 
+@pytest.mark.parametrize("length,copies", [(500_000, True), (530_000, False)])
+def test_row_copies_stay_within_32_bits(lib, length, copies):
+    """The hook form above rank 1 copies its rows (512 bytes per token and rank, q and k) while those
+    of one batch row are below 2^31 bytes, whatever d_state is; beyond that it reads the caller's."""
+    size = ctypes.c_size_t(0)
+    args = _hook_scan_args(1, length, 16, 1)
+    args.rank, args.d_state = 8, 16
+    for t in (args.q, args.k):
+        for i, stride in enumerate((length * 128, 128, 128, 16, 1)):
+            t.stride[i] = stride
+    assert lib.m3_scan_workspace_size(ctypes.byref(args), ctypes.byref(size)) == 0
+    scalars = 16 * -(-length // 8) * (5 * 8 + 8) * 4  # 16 heads, sub-chunks of 8 tokens
+    assert size.value >= scalars
+    assert (size.value >= scalars + length * 8 * 512) == copies
+
+
 def test_scan_backwards_token_strides_on_the_host(lib):
     """Per-token tensors may run backwards (the reverse scan), but all of them together."""
     args = _hook_scan_args(1, 128, 2, 1)
